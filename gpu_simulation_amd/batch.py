@@ -3,10 +3,10 @@
 The reference evaluates one circuit per ``RingIsingCudaBackend.energy_and_grad``
 call (``cpp/ising_cuda_backend.cu:429-442``).  :class:`RingIsingBatch` wraps the
 extension's batch object (C ABI ``rie_batch_*``): circuits of different qubit
-counts (2..14), layer counts and fields share one persistent launch of the
-whole-circuit kernel (structured_adjoint) and grouped FP64-MFMA product-tree
-launches (dense_scan, ``num_qubits <= dense_max_qubits``), optionally replayed
-from a HIP graph, with gradient-descent or Adam steps on the device.
+counts (2..14), layer counts and fields run together: one launch of the
+whole-circuit kernel per qubit count (structured_adjoint) and grouped FP64-MFMA
+product-tree launches (dense_scan, ``num_qubits <= dense_max_qubits``), optionally
+replayed from a HIP graph, with gradient-descent or Adam steps on the device.
 
 Parameters of circuit ``i`` have the reference's per-circuit layout, shape
 ``(L_i, n_i, 2)`` with ``[..., 0] = theta_RY`` and ``[..., 1] = phi_RZ``; the

@@ -39,8 +39,8 @@ HIP_FLAGS = [
     f"-I{INCLUDE}",
     f"-I{CSRC}",
 ]
-HIP_SOURCES = ["rie_kernels.hip", "rie_dense.hip", "rie_batch.hip", "rie_mlp.hip",
-               "rie_noalloc.hip", "rie_engine.cpp", "rie_batch.cpp", "rie_mlp.cpp"]
+HIP_SOURCES = ["rie_kernels.hip", "rie_dense.hip", "rie_batch.hip", "rie_regcircuit.hip",
+               "rie_mlp.hip", "rie_noalloc.hip", "rie_engine.cpp", "rie_batch.cpp", "rie_mlp.cpp"]
 
 
 def _run_parallel(commands: list[list[str]], verbose: bool) -> None:

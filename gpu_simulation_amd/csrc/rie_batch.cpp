@@ -3,13 +3,16 @@
 //
 // Circuits with n <= dense_max_qubits take the dense_scan product tree
 // (rie_dense.hip, one grouped FP64-MFMA GEMM launch per tree level and tile
-// class for all of them); the others run in one persistent launch of the
-// whole-circuit kernel (rie_batch.hip) whose workgroups take circuits from a
-// longest-first (LPT) schedule built on the host from per-layer costs.  The
-// two parts run concurrently on two streams (two branches of one graph when
-// captured).  Parameters, energies and gradients of all circuits are packed
-// in device arrays owned by the batch: circuit i's 2 n_i L_i parameters start
-// at offset[i], in the reference's per-circuit layout (l n + w) 2 + {0, 1}
+// class for all of them).  The others take the whole-circuit kernels: up to
+// 13 qubits one launch per qubit count with every state in registers
+// (rie_regcircuit.hip), one workgroup per circuit, deepest first; 14 qubits one
+// persistent launch (rie_batch.hip) whose workgroups take circuits from a
+// longest-first (LPT) schedule built on the host.  The launches are spread over
+// four streams (branches of one graph when captured), so the tail of one
+// qubit count's deep circuits overlaps the others' work.  Parameters, energies
+// and gradients of all circuits are packed in device arrays owned by the
+// batch: circuit i's 2 n_i L_i parameters start at offset[i], in the
+// reference's per-circuit layout (l n + w) 2 + {0, 1}
 // (cpp/ising_cuda_structured_adjoint_modes.inc:73-77).
 //
 // The reference evaluates one circuit per call (RingIsingCudaBackend::
@@ -67,9 +70,10 @@ struct Batch {
     int device = 0;
     int num_cus = 0;
     hipStream_t s_own = nullptr;
-    hipStream_t s_aux = nullptr;
+    static constexpr int kAux = 3;  // streams beside the caller's
+    hipStream_t s_aux[kAux] = {};
     hipEvent_t ev_fork = nullptr;
-    hipEvent_t ev_join = nullptr;
+    hipEvent_t ev_join[kAux] = {};
     hipEvent_t ev_t0 = nullptr;
     hipEvent_t ev_t1 = nullptr;
     double *d_params = nullptr;
@@ -82,9 +86,27 @@ struct Batch {
     double *d_history = nullptr;
     size_t history_cap = 0;
 
-    // structured part: persistent launch
+    // structured part
     std::vector<int> sids;
-    std::vector<BatchJob> jobs_g;  // with gradients, indexed like sids
+    // up to kRegMaxQubits: one launch per qubit count, states in registers
+    struct RegGroup {
+        int n;
+        int first;  // in d_reg_g / d_reg_e
+        int count;
+    };
+    std::vector<RegGroup> reg_groups;   // largest n first
+    std::vector<RegJob> reg_jobs;       // with gradients, grouped, deepest first
+    std::vector<RecordJob> rec_jobs;    // indexed like reg_jobs
+    std::vector<int> reg_of;            // circuit -> reg_jobs index, or -1
+    int reg_layers = 0;                 // records of one evaluation
+    RegJob *d_reg_g = nullptr;
+    RegJob *d_reg_e = nullptr;
+    RecordJob *d_rec_jobs = nullptr;
+    int *d_layer_job = nullptr;
+    double *d_rec = nullptr;
+    // above: persistent launch
+    std::vector<int> gids;
+    std::vector<BatchJob> jobs_g;  // with gradients, indexed like gids
     BatchJob *d_jobs_g = nullptr;
     BatchJob *d_jobs_e = nullptr;  // energy only
     int *d_order = nullptr;
@@ -94,7 +116,6 @@ struct Batch {
     int scratch_slots = 0;
     int grid = 0;
     int threads = 512;
-    int max_lds_n = 0;
     int grid_limit = 0;  // 0: every CU
     int wg_per_cu = 1;
     int chunk_by_n[kMaxN + 1];
@@ -117,6 +138,7 @@ struct Batch {
     std::string report = "{}";
 
     void build_structured();
+    void build_register_jobs();
     void build_dense();
     void repartition(int split);
     void release_structured();
@@ -133,6 +155,8 @@ struct Batch {
     void ensure_history(size_t entries);
     void ensure_adam();
     std::string config_json() const;
+    // whether anything runs beside the persistent launch
+    bool parts_beside() const { return !dids.empty() || !reg_groups.empty(); }
 };
 
 Batch::Batch(size_t count_, const int *nq, const int *nl, const double *fields, int dense_max_qubits)
@@ -169,19 +193,18 @@ Batch::Batch(size_t count_, const int *nq, const int *nl, const double *fields, 
     }
     for (int q = 0; q <= kMaxN; ++q) {
         chunk_by_n[q] = 3;
-        // modelled per-layer cost: amplitude updates, with a floor for the
-        // barrier-bound small states and a factor for the global-scratch ones
-        const double amps = std::ldexp(1.0, q);
-        cost_per_layer[q] = q * std::max(amps, 1024.0) * (q > kBatchMaxLdsQubits ? 3.0 : 1.0);
+        cost_per_layer[q] = q * std::ldexp(1.0, q);  // modelled: amplitude updates
     }
     check(hipGetDevice(&device), "hipGetDevice");
     hipDeviceProp_t prop;
     check(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
     num_cus = prop.multiProcessorCount;
     check(hipStreamCreateWithFlags(&s_own, hipStreamNonBlocking), "hipStreamCreate");
-    check(hipStreamCreateWithFlags(&s_aux, hipStreamNonBlocking), "hipStreamCreate");
     check(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming), "hipEventCreate");
-    check(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming), "hipEventCreate");
+    for (int a = 0; a < kAux; ++a) {
+        check(hipStreamCreateWithFlags(&s_aux[a], hipStreamNonBlocking), "hipStreamCreate");
+        check(hipEventCreateWithFlags(&ev_join[a], hipEventDisableTiming), "hipEventCreate");
+    }
     check(hipEventCreate(&ev_t0), "hipEventCreate");
     check(hipEventCreate(&ev_t1), "hipEventCreate");
     d_params = (double *)device_alloc(sizeof(double) * total, "alloc batch params");
@@ -219,8 +242,10 @@ Batch::~Batch() {
     if (s_own != nullptr) {
         (void)hipStreamSynchronize(s_own);
     }
-    if (s_aux != nullptr) {
-        (void)hipStreamSynchronize(s_aux);
+    for (hipStream_t s : s_aux) {
+        if (s != nullptr) {
+            (void)hipStreamSynchronize(s);
+        }
     }
     invalidate_graph();
     release_structured();
@@ -232,7 +257,7 @@ Batch::~Batch() {
     device_free(d_v);
     device_free(d_step);
     device_free(d_history);
-    for (hipEvent_t ev : {ev_fork, ev_join, ev_t0, ev_t1}) {
+    for (hipEvent_t ev : {ev_fork, ev_join[0], ev_join[1], ev_join[2], ev_t0, ev_t1}) {
         if (ev != nullptr) {
             (void)hipEventDestroy(ev);
         }
@@ -240,8 +265,10 @@ Batch::~Batch() {
     if (s_own != nullptr) {
         (void)hipStreamDestroy(s_own);
     }
-    if (s_aux != nullptr) {
-        (void)hipStreamDestroy(s_aux);
+    for (hipStream_t s : s_aux) {
+        if (s != nullptr) {
+            (void)hipStreamDestroy(s);
+        }
     }
 }
 
@@ -259,6 +286,19 @@ void Batch::release_structured() {
     device_free(d_order);
     device_free(d_wg_begin);
     device_free(d_scratch);
+    device_free(d_reg_g);
+    device_free(d_reg_e);
+    device_free(d_rec_jobs);
+    device_free(d_layer_job);
+    device_free(d_rec);
+    d_reg_g = d_reg_e = nullptr;
+    d_rec_jobs = nullptr;
+    d_layer_job = nullptr;
+    d_rec = nullptr;
+    reg_groups.clear();
+    reg_jobs.clear();
+    rec_jobs.clear();
+    reg_layers = 0;
     d_jobs_g = d_jobs_e = nullptr;
     d_order = d_wg_begin = nullptr;
     d_scratch = nullptr;
@@ -266,19 +306,85 @@ void Batch::release_structured() {
     grid = 0;
 }
 
-// Longest-first schedule of the structured circuits over `grid` workgroups.
+// Jobs and records of the circuits whose states fit in registers.
+void Batch::build_register_jobs() {
+    std::vector<int> ids;
+    for (int i : sids) {
+        if (n[(size_t)i] <= kRegMaxQubits) {
+            ids.push_back(i);
+        }
+    }
+    reg_of.assign(count, -1);
+    if (ids.empty()) {
+        return;
+    }
+    std::stable_sort(ids.begin(), ids.end(), [&](int a, int b) {
+        return n[(size_t)a] != n[(size_t)b] ? n[(size_t)a] > n[(size_t)b]
+                                            : L[(size_t)a] > L[(size_t)b];
+    });
+    size_t bytes = 0;
+    for (int i : ids) {
+        bytes += circuit_record_bytes(n[(size_t)i], L[(size_t)i]);
+    }
+    d_rec = (double *)device_alloc(bytes, "alloc batch records");
+    std::vector<int> layer_job;
+    double *rec = d_rec;
+    for (int i : ids) {
+        const int q = n[(size_t)i];
+        const int layers = L[(size_t)i];
+        if (reg_groups.empty() || reg_groups.back().n != q) {
+            reg_groups.push_back({q, (int)reg_jobs.size(), 0});
+        }
+        reg_groups.back().count += 1;
+        reg_of[(size_t)i] = (int)reg_jobs.size();
+        layer_job.insert(layer_job.end(), (size_t)layers, (int)reg_jobs.size());
+        rec_jobs.push_back({d_params + poff[(size_t)i], rec, q, reg_layers});
+        reg_jobs.push_back({rec, d_energy + i, d_grad + poff[(size_t)i], nullptr, nullptr,
+                            h[(size_t)i], layers, 0});
+        reg_layers += layers;
+        rec += circuit_record_bytes(q, layers) / sizeof(double);
+    }
+    std::vector<RegJob> energy_only = reg_jobs;
+    for (auto &j : energy_only) {
+        j.grad = nullptr;
+    }
+    const size_t job_bytes = sizeof(RegJob) * reg_jobs.size();
+    d_reg_g = (RegJob *)device_alloc(job_bytes, "alloc batch jobs");
+    d_reg_e = (RegJob *)device_alloc(job_bytes, "alloc batch jobs");
+    d_rec_jobs = (RecordJob *)device_alloc(sizeof(RecordJob) * rec_jobs.size(), "alloc batch jobs");
+    d_layer_job = (int *)device_alloc(sizeof(int) * layer_job.size(), "alloc batch layers");
+    check(hipMemcpy(d_reg_g, reg_jobs.data(), job_bytes, hipMemcpyHostToDevice),
+          "upload batch jobs");
+    check(hipMemcpy(d_reg_e, energy_only.data(), job_bytes, hipMemcpyHostToDevice),
+          "upload batch jobs");
+    check(hipMemcpy(d_rec_jobs, rec_jobs.data(), sizeof(RecordJob) * rec_jobs.size(),
+                    hipMemcpyHostToDevice),
+          "upload batch jobs");
+    check(hipMemcpy(d_layer_job, layer_job.data(), sizeof(int) * layer_job.size(),
+                    hipMemcpyHostToDevice),
+          "upload batch layers");
+}
+
+// Register jobs, and a longest-first schedule of the larger circuits over
+// `grid` workgroups.
 void Batch::build_structured() {
     invalidate_graph();
     release_structured();
+    build_register_jobs();
     jobs_g.clear();
-    if (sids.empty()) {
+    gids.clear();
+    for (int i : sids) {
+        if (n[(size_t)i] > kRegMaxQubits) {
+            gids.push_back(i);
+        }
+    }
+    if (gids.empty()) {
         return;
     }
     const int cap = grid_limit > 0 ? grid_limit : num_cus * wg_per_cu;
-    grid = (int)std::min<size_t>(sids.size(), (size_t)std::max(1, cap));
-    max_lds_n = 0;
+    grid = (int)std::min<size_t>(gids.size(), (size_t)std::max(1, cap));
     int max_global_n = 0;
-    for (int i : sids) {
+    for (int i : gids) {
         BatchJob j{};
         j.n = n[(size_t)i];
         j.layers = L[(size_t)i];
@@ -290,14 +396,10 @@ void Batch::build_structured() {
         j.drift = nullptr;
         j.scale = nullptr;
         jobs_g.push_back(j);
-        if (j.n <= kBatchMaxLdsQubits) {
-            max_lds_n = std::max(max_lds_n, j.n);
-        } else {
-            max_global_n = std::max(max_global_n, j.n);
-        }
+        max_global_n = std::max(max_global_n, j.n);
     }
     // LPT: heaviest first onto the least-loaded workgroup
-    std::vector<int> idx(sids.size());
+    std::vector<int> idx(gids.size());
     for (size_t k = 0; k < idx.size(); ++k) {
         idx[k] = (int)k;
     }
@@ -347,7 +449,7 @@ void Batch::build_structured() {
         scratch_stride = (uint64_t)2 << max_global_n;
         // one slot per workgroup of the persistent grid, and at least as many
         // as the autotuner's one-circuit-per-workgroup probes use
-        scratch_slots = std::max(grid, std::min((int)sids.size(), num_cus));
+        scratch_slots = std::max(grid, std::min((int)gids.size(), num_cus));
         d_scratch = (double2 *)device_alloc(sizeof(double2) * scratch_stride * scratch_slots,
                                             "alloc batch scratch");
     }
@@ -365,24 +467,45 @@ void Batch::build_dense() {
 }
 
 void Batch::issue_eval(hipStream_t s, bool want_grad) {
-    launch_coef(d_params, d_coef, (int)(total / 2), s);
-    check_launch("batch coef");
-    const bool both = grid > 0 && !dids.empty();
-    if (both) {
-        check(hipEventRecord(ev_fork, s), "record fork");
-        check(hipStreamWaitEvent(s_aux, ev_fork, 0), "wait fork");
+    if (!gids.empty() || !dids.empty()) {
+        launch_coef(d_params, d_coef, (int)(total / 2), s);
+        check_launch("batch coef");
     }
-    if (grid > 0) {
+    if (reg_layers > 0) {
+        launch_circuit_records(d_rec_jobs, RecordJob{}, d_layer_job, reg_layers, s);
+        check_launch("batch records");
+    }
+    // part i of the evaluation runs on stream i mod 4 (0: s itself): the
+    // largest circuits first, each stream's parts one after the other
+    const int parts = (gids.empty() ? 0 : 1) + (dids.empty() ? 0 : 1) + (int)reg_groups.size();
+    const int used = std::min(parts - 1, kAux);
+    if (used > 0) {
+        check(hipEventRecord(ev_fork, s), "record fork");
+        for (int a = 0; a < used; ++a) {
+            check(hipStreamWaitEvent(s_aux[a], ev_fork, 0), "wait fork");
+        }
+    }
+    int part = 0;
+    auto next_stream = [&]() {
+        const int k = part++ % (kAux + 1);
+        return k == 0 ? s : s_aux[k - 1];
+    };
+    if (!gids.empty()) {
         launch_batch_structured(want_grad ? d_jobs_g : d_jobs_e, BatchJob{}, d_order, d_wg_begin,
-                                grid, threads, max_lds_n, d_scratch, scratch_stride, s);
+                                grid, threads, d_scratch, scratch_stride, next_stream());
         check_launch("batch structured");
     }
     if (!dids.empty()) {
-        dense.run(both ? s_aux : s, want_grad);
-        if (both) {
-            check(hipEventRecord(ev_join, s_aux), "record join");
-            check(hipStreamWaitEvent(s, ev_join, 0), "wait join");
-        }
+        dense.run(next_stream(), want_grad);
+    }
+    for (const RegGroup &g : reg_groups) {
+        launch_regcircuit(g.n, (want_grad ? d_reg_g : d_reg_e) + g.first, RegJob{}, g.count,
+                          next_stream());
+        check_launch("batch circuits");
+    }
+    for (int a = 0; a < used; ++a) {
+        check(hipEventRecord(ev_join[a], s_aux[a]), "record join");
+        check(hipStreamWaitEvent(s, ev_join[a], 0), "wait join");
     }
 }
 
@@ -470,18 +593,28 @@ void Batch::run_per_circuit(hipStream_t s, bool want_grad) {
         }
     }
     size_t di = 0;
-    size_t si = 0;
+    size_t gi = 0;
     for (size_t i = 0; i < count; ++i) {
+        if (reg_of[i] >= 0) {
+            RegJob j = reg_jobs[(size_t)reg_of[i]];
+            RecordJob r = rec_jobs[(size_t)reg_of[i]];
+            r.first_layer = 0;
+            if (!want_grad) {
+                j.grad = nullptr;
+            }
+            launch_circuit_records(nullptr, r, nullptr, j.layers, s);
+            launch_regcircuit(n[i], nullptr, j, 1, s);
+            continue;
+        }
         launch_coef(d_params + poff[i], d_coef + poff[i] / 2, n[i] * L[i], s);
         if (dense_flag[i]) {
             dense_single[di++]->run(s, want_grad);
         } else {
-            BatchJob j = jobs_g[si++];
+            BatchJob j = jobs_g[gi++];
             if (!want_grad) {
                 j.grad = nullptr;
             }
-            launch_batch_structured(nullptr, j, nullptr, nullptr, 1, threads,
-                                    j.n <= kBatchMaxLdsQubits ? j.n : 0, d_scratch,
+            launch_batch_structured(nullptr, j, nullptr, nullptr, 1, threads, d_scratch,
                                     scratch_stride, s);
         }
     }
@@ -574,7 +707,8 @@ void Batch::autotune(size_t repeats) {
     std::vector<std::vector<std::vector<double>>> c(
         kMaxN + 1, std::vector<std::vector<double>>(3, std::vector<double>(5, 0.0)));
     std::vector<double> layers_of_n(kMaxN + 1, 0.0);
-    for (size_t k = 0; k < sids.size(); ++k) {
+    // circuits above kRegMaxQubits: the register kernels have no shape to tune
+    for (size_t k = 0; k < gids.size(); ++k) {
         layers_of_n[(size_t)jobs_g[k].n] += jobs_g[k].layers;
     }
     bool first_n = true;
@@ -586,13 +720,13 @@ void Batch::autotune(size_t repeats) {
             }
             std::vector<BatchJob> probe;
             int max_l = 0;
-            for (size_t k = 0; k < sids.size() && (int)probe.size() < num_cus; ++k) {
+            for (size_t k = 0; k < gids.size() && (int)probe.size() < num_cus; ++k) {
                 if (jobs_g[k].n == q) {
                     probe.push_back(jobs_g[k]);
                     max_l = std::max(max_l, jobs_g[k].layers);
                 }
             }
-            if ((int)probe.size() > scratch_slots && q > kBatchMaxLdsQubits) {
+            if ((int)probe.size() > scratch_slots) {
                 probe.resize((size_t)scratch_slots);
             }
             device_free(d_probe);
@@ -609,10 +743,9 @@ void Batch::autotune(size_t repeats) {
                     check(hipMemcpy(d_probe, probe.data(), sizeof(BatchJob) * probe.size(),
                                     hipMemcpyHostToDevice),
                           "upload probe");
-                    const int lds_n = q <= kBatchMaxLdsQubits ? q : 0;
                     const double ms = time_ms(repeats, [&](hipStream_t s) {
                         launch_batch_structured(d_probe, BatchJob{}, nullptr, nullptr,
-                                                (int)probe.size(), T, lds_n, d_scratch,
+                                                (int)probe.size(), T, d_scratch,
                                                 scratch_stride, s);
                         check_launch("autotune probe");
                     });
@@ -629,7 +762,8 @@ void Batch::autotune(size_t repeats) {
     }
     device_free(d_probe);
     rep << "}";
-    if (!sids.empty()) {
+    measured = measured || !sids.empty();
+    if (!gids.empty()) {
         // one thread count for the launch: least total modelled work
         double best = -1.0;
         int best_ti = 1;
@@ -666,7 +800,6 @@ void Batch::autotune(size_t repeats) {
             chunk_by_n[q] = bk;
             cost_per_layer[q] = c[(size_t)q][(size_t)best_ti][(size_t)bk];
         }
-        measured = true;
     }
     // per split: the dense tile for D >= 64 and the structured launch's grid
     // (with a dense part running beside it, leave it CUs); the fastest whole
@@ -700,16 +833,13 @@ void Batch::autotune(size_t repeats) {
             build_dense();
         }
         std::vector<int> grid_opts;
-        if (!sids.empty()) {
-            if (!dids.empty()) {
+        if (!gids.empty()) {
+            if (parts_beside()) {
                 for (int f : {1, 2, 3, 4}) {
                     grid_opts.push_back(num_cus * f / 4);
                 }
             } else {
                 grid_opts.push_back(num_cus);
-                if (max_lds_n <= 11) {
-                    grid_opts.push_back(2 * num_cus);  // two workgroups per CU fit in LDS
-                }
             }
         } else {
             grid_opts.push_back(0);

@@ -1,14 +1,13 @@
-// Whole-circuit structured adjoint kernels for small circuits (n <= 14), one
-// workgroup per circuit at a time, and the optimizer-step kernels of a batch.
+// Whole-circuit structured adjoint kernel for 14 qubits, whose states do not fit
+// one workgroup's registers (rie_regcircuit.hip serves fewer qubits), and the
+// optimizer-step kernels of a batch.
 //
-// One launch runs a list of circuits of different qubit and layer counts:
-// workgroup b evaluates circuits order[wg_begin[b] .. wg_begin[b+1]) one after
-// the other (a persistent grid with a host-side longest-first schedule), each
-// circuit entirely on chip: psi and lambda in LDS for n <= 12, in a per-
-// workgroup global scratch of 2 * 2^n amplitudes (L2 / MALL resident) for
-// n = 13, 14.  The same kernel with one circuit serves an engine's n <= 12
-// path.  The ring-CNOT layers cost no data movement: they only change the
-// linear frame in which the amplitudes are stored (FrameTables below).
+// One launch runs a list of circuits of different layer counts: workgroup b
+// evaluates circuits order[wg_begin[b] .. wg_begin[b+1]) one after the other (a
+// persistent grid with a host-side longest-first schedule), psi and lambda in
+// a per-workgroup global scratch of 2 * 2^n amplitudes (L2 / MALL resident).
+// The ring-CNOT layers cost no data movement: they only change the linear frame
+// in which the amplitudes are stored (FrameTables below).
 //
 // Per layer, the rotations are applied in chunks of K consecutive wires:
 // each thread holds the 2^K amplitudes of one group in registers, applies the
@@ -16,8 +15,7 @@
 // sweeps of the state instead of n (the rotation-chunk width of the
 // reference's structured kernels, cpp/ising_cuda_rotation_kernels.cu:95-308,
 // and its backward counterpart, cpp/ising_cuda_statevector_grad_kernels.cu:
-// 440-587).  LDS slots are padded by one amplitude per 16 to spread the
-// strided accesses of a group over the LDS banks.
+// 440-587).
 #include <hip/hip_runtime.h>
 
 #include "rie_kernels.hpp"
@@ -35,11 +33,6 @@ constexpr int max_chunk() {
 template <int kThreads>
 constexpr int clamp_chunk(int k) {
     return k < max_chunk<kThreads>() ? k : max_chunk<kThreads>();
-}
-
-template <bool kLds>
-__device__ __forceinline__ uint32_t slot(uint32_t i) {
-    return kLds ? i + (i >> 4) : i;
 }
 
 __device__ __forceinline__ uint32_t parity(uint32_t x) { return (uint32_t)__popc(x) & 1u; }
@@ -169,7 +162,7 @@ __device__ __forceinline__ void build_chunk_rz(double2 *rzt, int n, int K, const
 // ceil(n / K) * 2^K <= 64 for n <= 14, K <= 4
 constexpr int kBatchRzEntries = 64;
 
-template <int K, int kThreads, bool kLds>
+template <int K, int kThreads>
 __device__ __forceinline__ void chunk_fwd(double2 *st, int n, int w0, const WireCoef *lc,
                                           const FrameTables &ft, int fb, const double2 *rz) {
     constexpr int A = 1 << K;
@@ -185,7 +178,7 @@ __device__ __forceinline__ void chunk_fwd(double2 *st, int n, int w0, const Wire
         double2 a[A];
 #pragma unroll
         for (int o = 0; o < A; ++o) {
-            a[o] = st[slot<kLds>(base ^ member_offset<K>(cg, o))];
+            a[o] = st[base ^ member_offset<K>(cg, o)];
         }
 #pragma unroll
         for (int j = 0; j < K; ++j) {
@@ -198,14 +191,14 @@ __device__ __forceinline__ void chunk_fwd(double2 *st, int n, int w0, const Wire
         }
 #pragma unroll
         for (int o = 0; o < A; ++o) {
-            st[slot<kLds>(base ^ member_offset<K>(cg, o))] = cmul(a[o], rz[o]);
+            st[base ^ member_offset<K>(cg, o)] = cmul(a[o], rz[o]);
         }
     }
 }
 
 // Un-rotates wires [w0, w0 + K) on (cur, lam) and leaves each wire's
 // per-wave gradient sums in red[wave][2w], red[wave][2w + 1].
-template <int K, int kThreads, bool kLds>
+template <int K, int kThreads>
 __device__ __forceinline__ void chunk_bwd(double2 *cur, double2 *lam, int n, int w0,
                                           const WireCoef *lc, const FrameTables &ft, int fb,
                                           double (*red)[kRedCols], const double2 *rz) {
@@ -227,7 +220,7 @@ __device__ __forceinline__ void chunk_bwd(double2 *cur, double2 *lam, int n, int
         double2 l[A];
 #pragma unroll
         for (int o = 0; o < A; ++o) {
-            const uint32_t i = slot<kLds>(base ^ member_offset<K>(cg, o));
+            const uint32_t i = base ^ member_offset<K>(cg, o);
             const double2 z = rz[o];
             const double2 zc = make_double2(z.x, -z.y);
             c[o] = cmul(cur[i], zc);
@@ -253,7 +246,7 @@ __device__ __forceinline__ void chunk_bwd(double2 *cur, double2 *lam, int n, int
         }
 #pragma unroll
         for (int o = 0; o < A; ++o) {
-            const uint32_t i = slot<kLds>(base ^ member_offset<K>(cg, o));
+            const uint32_t i = base ^ member_offset<K>(cg, o);
             cur[i] = c[o];
             lam[i] = l[o];
         }
@@ -271,47 +264,47 @@ __device__ __forceinline__ void chunk_bwd(double2 *cur, double2 *lam, int n, int
     }
 }
 
-template <int kThreads, bool kLds>
+template <int kThreads>
 __device__ __forceinline__ void chunk_fwd_any(int K, double2 *st, int n, int w0,
                                               const WireCoef *lc, const FrameTables &ft,
                                               int fb, const double2 *rz) {
     switch (K) {
         case 1:
-            chunk_fwd<1, kThreads, kLds>(st, n, w0, lc, ft, fb, rz);
+            chunk_fwd<1, kThreads>(st, n, w0, lc, ft, fb, rz);
             break;
         case 2:
-            chunk_fwd<clamp_chunk<kThreads>(2), kThreads, kLds>(st, n, w0, lc, ft, fb, rz);
+            chunk_fwd<clamp_chunk<kThreads>(2), kThreads>(st, n, w0, lc, ft, fb, rz);
             break;
         case 3:
-            chunk_fwd<clamp_chunk<kThreads>(3), kThreads, kLds>(st, n, w0, lc, ft, fb, rz);
+            chunk_fwd<clamp_chunk<kThreads>(3), kThreads>(st, n, w0, lc, ft, fb, rz);
             break;
         default:
-            chunk_fwd<max_chunk<kThreads>(), kThreads, kLds>(st, n, w0, lc, ft, fb, rz);
+            chunk_fwd<max_chunk<kThreads>(), kThreads>(st, n, w0, lc, ft, fb, rz);
             break;
     }
 }
 
-template <int kThreads, bool kLds>
+template <int kThreads>
 __device__ __forceinline__ void chunk_bwd_any(int K, double2 *cur, double2 *lam, int n, int w0,
                                               const WireCoef *lc, const FrameTables &ft, int fb,
                                               double (*red)[kRedCols], const double2 *rz) {
     switch (K) {
         case 1:
-            chunk_bwd<1, kThreads, kLds>(cur, lam, n, w0, lc, ft, fb, red, rz);
+            chunk_bwd<1, kThreads>(cur, lam, n, w0, lc, ft, fb, red, rz);
             break;
         case 2:
-            chunk_bwd<clamp_chunk<kThreads>(2), kThreads, kLds>(cur, lam, n, w0, lc, ft, fb, red, rz);
+            chunk_bwd<clamp_chunk<kThreads>(2), kThreads>(cur, lam, n, w0, lc, ft, fb, red, rz);
             break;
         case 3:
-            chunk_bwd<clamp_chunk<kThreads>(3), kThreads, kLds>(cur, lam, n, w0, lc, ft, fb, red, rz);
+            chunk_bwd<clamp_chunk<kThreads>(3), kThreads>(cur, lam, n, w0, lc, ft, fb, red, rz);
             break;
         default:
-            chunk_bwd<max_chunk<kThreads>(), kThreads, kLds>(cur, lam, n, w0, lc, ft, fb, red, rz);
+            chunk_bwd<max_chunk<kThreads>(), kThreads>(cur, lam, n, w0, lc, ft, fb, red, rz);
             break;
     }
 }
 
-template <int kThreads, bool kLds>
+template <int kThreads>
 __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, double2 *lam,
                                         FrameTables &ft, double (*red)[kRedCols], double2 *rzt) {
     const int n = job.n;
@@ -349,7 +342,7 @@ __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, doubl
             const WireCoef k = coef[w];
             v = cmul(v, ((j >> w) & 1) ? u1_of(k) : u0_of(k));
         }
-        cur[slot<kLds>(j)] = v;
+        cur[j] = v;
     }
     __syncthreads();
 
@@ -358,7 +351,7 @@ __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, doubl
         build_chunk_rz(rzt, n, K, lc);
         __syncthreads();
         for (int w0 = 0; w0 < n; w0 += K) {
-            chunk_fwd_any<kThreads, kLds>(K < n - w0 ? K : n - w0, cur, n, w0, lc, ft, fb,
+            chunk_fwd_any<kThreads>(K < n - w0 ? K : n - w0, cur, n, w0, lc, ft, fb,
                                           rzt + (w0 / K) * (1 << K));
             __syncthreads();
         }
@@ -372,17 +365,17 @@ __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, doubl
         for (int w = 0; w < n; ++w) {
             i |= parity(j & ft.r[fb][w]) << w;
         }
-        const double2 v = cur[slot<kLds>(j)];
+        const double2 v = cur[j];
         const double d = ham_diag(i, n);
         double fx = 0.0;
         double fy = 0.0;
         for (int w = 0; w < n; ++w) {
-            const double2 p = cur[slot<kLds>(j ^ ft.m[fb][w])];
+            const double2 p = cur[j ^ ft.m[fb][w]];
             fx += p.x;
             fy += p.y;
         }
         const double2 hv = make_double2(d * v.x - job.field * fx, d * v.y - job.field * fy);
-        lam[slot<kLds>(j)] = hv;
+        lam[j] = hv;
         e += v.x * hv.x + v.y * hv.y;
     }
     e = wave_sum(e);
@@ -409,7 +402,7 @@ __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, doubl
         build_chunk_rz(rzt, n, K, lc);
         __syncthreads();
         for (int w0 = 0; w0 < n; w0 += K) {
-            chunk_bwd_any<kThreads, kLds>(K < n - w0 ? K : n - w0, cur, lam, n, w0, lc, ft, fb,
+            chunk_bwd_any<kThreads>(K < n - w0 ? K : n - w0, cur, lam, n, w0, lc, ft, fb,
                                           red, rzt + (w0 / K) * (1 << K));
             __syncthreads();
         }
@@ -427,7 +420,7 @@ __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, doubl
         // the frame is the identity again
         double acc = 0.0;
         for (uint32_t i = t; i < N; i += kThreads) {
-            const double2 v = cur[slot<kLds>(i)];
+            const double2 v = cur[i];
             const double re = v.x - (i == 0 ? 1.0 : 0.0);
             acc += re * re + v.y * v.y;
         }
@@ -452,9 +445,7 @@ __device__ __forceinline__ void run_job(const BatchJob &job, double2 *cur, doubl
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void batch_structured_kernel(
     const BatchJob *__restrict__ jobs, BatchJob single, const int *__restrict__ order,
-    const int *__restrict__ wg_begin, double2 *scratch, uint64_t scratch_stride,
-    uint32_t lds_state) {
-    extern __shared__ double2 smem[];
+    const int *__restrict__ wg_begin, double2 *scratch, uint64_t scratch_stride) {
     __shared__ double red[kThreads / kWave][kRedCols];
     __shared__ FrameTables ft;
     __shared__ double2 rzt[kBatchRzEntries];
@@ -464,45 +455,29 @@ __global__ __launch_bounds__(kThreads) void batch_structured_kernel(
     for (int q = q0; q < q1; ++q) {
         const int idx = order != nullptr ? order[q] : q;
         const BatchJob job = jobs != nullptr ? jobs[idx] : single;
-        if (job.n <= kBatchMaxLdsQubits) {
-            run_job<kThreads, true>(job, smem, smem + lds_state, ft, red, rzt);
-        } else {
-            const uint64_t N = uint64_t{1} << job.n;
-            double2 *gs = scratch + (uint64_t)b * scratch_stride;
-            run_job<kThreads, false>(job, gs, gs + N, ft, red, rzt);
-        }
+        const uint64_t N = uint64_t{1} << job.n;
+        double2 *gs = scratch + (uint64_t)b * scratch_stride;
+        run_job<kThreads>(job, gs, gs + N, ft, red, rzt);
         __syncthreads();
     }
 }
 
-uint32_t batch_lds_state_amps(int max_lds_n) {
-    if (max_lds_n <= 0) {
-        return 0;
-    }
-    const uint32_t N = 1u << max_lds_n;
-    return N + (N >> 4);
-}
-
 void launch_batch_structured(const BatchJob *d_jobs, const BatchJob &single, const int *d_order,
-                             const int *d_wg_begin, int grid, int threads, int max_lds_n,
-                             double2 *scratch, uint64_t scratch_stride, hipStream_t s) {
-    const uint32_t lds_state = batch_lds_state_amps(max_lds_n);
-    const size_t bytes = sizeof(double2) * 2 * (size_t)lds_state;
+                             const int *d_wg_begin, int grid, int threads, double2 *scratch,
+                             uint64_t scratch_stride, hipStream_t s) {
     switch (threads) {
         case 256:
-            batch_structured_kernel<256><<<grid, 256, bytes, s>>>(d_jobs, single, d_order,
-                                                                  d_wg_begin, scratch,
-                                                                  scratch_stride, lds_state);
+            batch_structured_kernel<256><<<grid, 256, 0, s>>>(d_jobs, single, d_order, d_wg_begin,
+                                                              scratch, scratch_stride);
             break;
         case 512:
-            batch_structured_kernel<512><<<grid, 512, bytes, s>>>(d_jobs, single, d_order,
-                                                                  d_wg_begin, scratch,
-                                                                  scratch_stride, lds_state);
+            batch_structured_kernel<512><<<grid, 512, 0, s>>>(d_jobs, single, d_order, d_wg_begin,
+                                                              scratch, scratch_stride);
             break;
         default:
-            batch_structured_kernel<1024><<<grid, 1024, bytes, s>>>(d_jobs, single, d_order,
-                                                                    d_wg_begin, scratch,
-                                                                    scratch_stride, lds_state);
+            batch_structured_kernel<1024><<<grid, 1024, 0, s>>>(d_jobs, single, d_order,
+                                                                d_wg_begin, scratch,
+                                                                scratch_stride);
             break;
     }
 }

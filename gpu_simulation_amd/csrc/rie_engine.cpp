@@ -83,7 +83,7 @@ static int pass_grid(uint64_t tiles, int max_grid) {
 
 void Engine::build_plan() {
     passes.clear();
-    if (n <= kBatchMaxLdsQubits) {
+    if (n <= kEngineWholeQubits) {
         small = true;
         return;
     }
@@ -208,10 +208,14 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     d_params = (double *)device_alloc(sizeof(double) * num_params, "alloc params");
     d_grad = (double *)device_alloc(sizeof(double) * num_params, "alloc gradient");
     d_energy = (double *)device_alloc(sizeof(double) * 4, "alloc energy");
-    d_coef = (WireCoef *)device_alloc(sizeof(WireCoef) * (size_t)n * L, "alloc coefficients");
-
     if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
-        // the whole circuit lives in one workgroup's LDS
+        // the whole circuit lives in one workgroup's registers
+        d_rec = (double *)device_alloc(circuit_record_bytes(n, L), "alloc records");
+    } else {
+        d_coef = (WireCoef *)device_alloc(sizeof(WireCoef) * (size_t)n * L, "alloc coefficients");
+    }
+    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+        // no state buffers
     } else if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT) {
         // The stored schedule keeps every forward pass output; use it when it
         // fits comfortably in free device memory, else walk back by inverse gates.
@@ -289,6 +293,7 @@ Engine::~Engine() {
     device_free(d_grad);
     device_free(d_energy);
     device_free(d_coef);
+    device_free(d_rec);
     device_free(d_partials);
     device_free(d_epartials);
     device_free(d_drift);
@@ -1164,20 +1169,23 @@ void Engine::structured_backward_stored(hipStream_t s, const double *scale) {
 // Structured adjoint: whole-circuit path (n <= 12)
 // ---------------------------------------------------------------------------
 
+void Engine::small_records(const double *params, hipStream_t s) {
+    launch_circuit_records(nullptr, RecordJob{params, d_rec, n, 0}, nullptr, L, s);
+    check_launch("circuit records");
+}
+
 void Engine::small_run(hipStream_t s, bool want_grad, const double *scale, double *energy_out,
                        double *grad_out, double *drift_out) {
-    BatchJob job{};
-    job.n = n;
-    job.layers = L;
-    job.chunk = (int)std::min<size_t>(chunk_width, 4);
-    job.field = h;
-    job.coef = d_coef;
+    RegJob job{};
+    job.rec = d_rec;
     job.energy = energy_out;
     job.grad = want_grad ? grad_out : nullptr;
     job.drift = drift_out;
     job.scale = scale;
+    job.field = h;
+    job.layers = L;
     kt_begin(s);
-    launch_batch_structured(nullptr, job, nullptr, nullptr, 1, 256, n, nullptr, 0, s);
+    launch_regcircuit(n, nullptr, job, 1, s);
     check_launch("small_circuit");
     kt_end(s, "small_circuit", 0.0);
 }
@@ -1237,6 +1245,12 @@ void Engine::gate_backward(hipStream_t s, const double *scale) {
 // ---------------------------------------------------------------------------
 
 void Engine::forward_device(const double *params, double *energy, hipStream_t s, bool keep_lam) {
+    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+        small_records(params, s);
+        small_run(s, false, nullptr, energy, nullptr, nullptr);
+        resident = false;
+        return;
+    }
     launch_coef(params, d_coef, n * L, s);
     check_launch("coef");
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
@@ -1249,11 +1263,6 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
         launch_reduce_sum(d_epartials, (int)energy_partials, energy, s);
         check_launch("energy reduce");
         resident = true;
-        return;
-    }
-    if (small) {
-        small_run(s, false, nullptr, energy, nullptr, nullptr);
-        resident = false;
         return;
     }
     structured_forward(s, ckpt_every > 0);
@@ -1282,7 +1291,7 @@ void Engine::backward_device(const double *params, const double *scale, double *
         return;
     }
     if (small) {
-        launch_coef(params, d_coef, n * L, s);
+        small_records(params, s);
         small_run(s, true, scale, d_energy + 1, grad, nullptr);
         return;
     }
@@ -1302,6 +1311,11 @@ void Engine::eval_device(const double *params, double *energy, double *grad, hip
         check_launch("coef");
         structured_eval_fused(s, nullptr, energy, false);
         copy_grad_if_needed(grad, s);
+        return;
+    }
+    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+        small_records(params, s);
+        small_run(s, true, nullptr, energy, grad, nullptr);
         return;
     }
     forward_device(params, energy, s, true);
@@ -1348,7 +1362,7 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         stage_end(s, "dense_scan_ms");
     } else if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
         stage_begin(s);
-        launch_coef(d_params, d_coef, n * L, s);
+        small_records(d_params, s);
         stage_end(s, "zero_state_ms");
         stage_begin(s);
         small_run(s, want_grad, nullptr, d_energy, want_grad ? d_grad : nullptr, nullptr);
@@ -1421,16 +1435,17 @@ double Engine::inverse_walk_drift(const double *params, size_t count) {
     order_begin(s);
     check(hipMemcpyAsync(d_params, params, sizeof(double) * num_params, hipMemcpyHostToDevice, s),
           "upload params");
-    launch_coef(d_params, d_coef, n * L, s);
     if (d_drift == nullptr) {
         d_drift = (double *)device_alloc(sizeof(double) * 8200, "alloc drift");
     }
     double drift2 = 0.0;
     if (small) {
+        small_records(d_params, s);
         small_run(s, true, nullptr, d_energy, d_grad, d_drift);
         check(hipMemcpyAsync(&drift2, d_drift, sizeof(double), hipMemcpyDeviceToHost, s),
               "copy drift");
     } else {
+        launch_coef(d_params, d_coef, n * L, s);
         const int saved = schedule;
         schedule = RIE_SCHEDULE_INVERSE_WALK;
         structured_forward(s, ckpt_every > 0);
@@ -1643,10 +1658,11 @@ void Engine::benchmark_forward_graph(const double *params, size_t count, size_t 
     check(hipMemcpyAsync(d_params, params, sizeof(double) * num_params, hipMemcpyHostToDevice, s),
           "upload params");
     auto forward = [&]() {
-        launch_coef(d_params, d_coef, n * L, s);
         if (small) {
+            small_records(d_params, s);
             small_run_captured(s);
         } else {
+            launch_coef(d_params, d_coef, n * L, s);
             structured_forward(s, false);
         }
     };

@@ -132,6 +132,7 @@ struct Engine {
     double *d_grad = nullptr;
     double *d_energy = nullptr;
     WireCoef *d_coef = nullptr;
+    double *d_rec = nullptr;  // whole-circuit path: the layers' records
     double *d_partials = nullptr;
     double *d_epartials = nullptr;
     double *d_drift = nullptr;
@@ -223,6 +224,7 @@ struct Engine {
     double2 *lbuf(int i) const;         // stored schedule: lambda buffers 0 and 1
     void ensure_pool(size_t count);
     void set_schedule(int sched);
+    void small_records(const double *params, hipStream_t s);
     void small_run(hipStream_t s, bool want_grad, const double *scale, double *energy_out,
                    double *grad_out, double *drift_out);
     void small_run_captured(hipStream_t s);

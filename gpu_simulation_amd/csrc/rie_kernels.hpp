@@ -154,7 +154,8 @@ inline bool lay_fits(const LamLayout &L, int n, int first, int count) {
     return true;
 }
 
-// One independent circuit evaluated by a single workgroup (n <= 14).
+// One independent circuit evaluated by a single workgroup on global scratch
+// (n <= 14).
 struct BatchJob {
     int n;
     int layers;
@@ -168,8 +169,39 @@ struct BatchJob {
     const double *scale;   // optional chain-rule factor for grad (nullptr = 1)
 };
 
-constexpr int kBatchMaxLdsQubits = 12;  // psi and lambda in LDS
-constexpr int kBatchMaxQubits = 14;     // global-scratch variant above that
+constexpr int kRegMaxQubits = 13;  // states in the registers of one workgroup
+
+// One circuit (2 <= n <= kRegMaxQubits) evaluated in registers.
+struct RegJob {
+    const double *rec;     // layers records (circuit_record_bytes)
+    double *energy;        // 1 value
+    double *grad;          // 2 * n * layers values, or nullptr for energy only
+    double *drift;         // || walked state - |0> ||^2, or nullptr
+    const double *scale;   // optional chain-rule factor for grad (nullptr = 1)
+    double field;
+    int layers;
+    int reserved;
+};
+
+// Records of one circuit's layers from its parameters; first_layer: its first
+// layer's number within the launch.
+struct RecordJob {
+    const double *params;
+    double *rec;
+    int n;
+    int first_layer;
+};
+
+size_t circuit_record_bytes(int n, int layers);
+// total_layers records: of `single`, or of d_jobs[d_layer_job[i]] for layer i.
+void launch_circuit_records(const RecordJob *d_jobs, const RecordJob &single,
+                            const int *d_layer_job, int total_layers, hipStream_t s);
+// count circuits of n qubits: `single`, or d_jobs[0 .. count).
+void launch_regcircuit(int n, const RegJob *d_jobs, const RegJob &single, int count,
+                       hipStream_t s);
+
+constexpr int kEngineWholeQubits = 12;  // an engine's whole-circuit path (tile passes above)
+constexpr int kBatchMaxQubits = 14;     // whole-circuit kernels; above kRegMaxQubits on scratch
 
 // Widest rotation chunk per workgroup size: a backward group keeps 2 * 2^K
 // amplitudes in registers, and the register budget per thread halves each
@@ -183,14 +215,11 @@ void launch_coef(const double *d_params, WireCoef *d_coef, int count, hipStream_
 
 // Persistent whole-circuit kernel: workgroup b runs the circuits
 // d_order[d_wg_begin[b] .. d_wg_begin[b+1]) in turn (without d_wg_begin:
-// circuit b of d_jobs, or `single` when d_jobs is null).  threads is 256,
-// 512 or 1024; max_lds_n sizes the LDS (largest n <= 12 in the launch, 0 if
-// none); circuits with n > 12 use scratch + b * scratch_stride (2 * 2^n
-// amplitudes).
+// circuit b of d_jobs, or `single` when d_jobs is null) on scratch +
+// b * scratch_stride (2 * 2^n amplitudes).  threads is 256, 512 or 1024.
 void launch_batch_structured(const BatchJob *d_jobs, const BatchJob &single, const int *d_order,
-                             const int *d_wg_begin, int grid, int threads, int max_lds_n,
-                             double2 *scratch, uint64_t scratch_stride, hipStream_t s);
-uint32_t batch_lds_state_amps(int max_lds_n);
+                             const int *d_wg_begin, int grid, int threads, double2 *scratch,
+                             uint64_t scratch_stride, hipStream_t s);
 
 // Optimizer steps and helpers over packed arrays.
 void launch_gd_update(double *p, const double *g, uint64_t count, double lr, hipStream_t s);

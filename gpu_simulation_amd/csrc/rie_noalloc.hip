@@ -2,11 +2,11 @@
 // 2 <= n <= 14), for callers that cannot allocate device memory: code under
 // HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
 //
-// The whole circuit runs in one workgroup (batch_structured_kernel with a
-// single job): psi and lambda in LDS for n <= 12, in a 2 * 2^n-amplitude
-// global scratch for n = 13, 14.  Everything beyond the caller's inputs and
-// outputs -- the per-(layer, wire) coefficient table and that state scratch --
-// lives in the file-scope array `scratch` below, one copy per device, held
+// The whole circuit runs in one workgroup: psi and lambda in registers for
+// n <= 13 (regcircuit_kernel), in a 2 * 2^n-amplitude global scratch for n = 14
+// (batch_structured_kernel with a single job).  Everything beyond the caller's
+// inputs and outputs -- the layers' records, or the per-(layer, wire)
+// coefficient table and that state scratch -- lives in the file-scope array `scratch` below, one copy per device, held
 // until the process ends.  Its address on each device comes from
 // hipGetSymbolAddress once per device (with that device current) and is the
 // only form in which host code hands it to kernels.
@@ -35,6 +35,8 @@ static_assert(kNoAllocMaxQubits <= (size_t)kBatchMaxQubits, "the whole-circuit k
 constexpr size_t kCoefBytes = sizeof(WireCoef) * kNoAllocMaxQubits * kNoAllocMaxLayers;
 constexpr size_t kStateBytes = sizeof(double2) * 2 * (size_t{1} << kNoAllocMaxQubits);
 constexpr size_t kScratchBytes = kCoefBytes + kStateBytes;
+static_assert(sizeof(double) * 112 * kNoAllocMaxLayers <= kScratchBytes,
+              "the records of 13 qubits (the longest) fit");
 static_assert(kCoefBytes % 256 == 0, "the state region starts 256-byte aligned");
 static_assert(kScratchBytes == RIE_NOALLOC_SCRATCH_BYTES, "the size the header states");
 
@@ -96,13 +98,32 @@ rie_status rie_energy_and_grad_noalloc(size_t num_qubits, size_t num_layers, dou
         }
         const hipStream_t stream = static_cast<hipStream_t>(stream_handle);
         unsigned char *base = device_scratch();
+        const int layers = (int)num_layers;
+        if (num_qubits <= (size_t)kRegMaxQubits) {
+            double *rec = reinterpret_cast<double *>(base);
+            launch_circuit_records(nullptr, RecordJob{params_device, rec, (int)num_qubits, 0},
+                                   nullptr, layers, stream);
+            RegJob job{};
+            job.rec = rec;
+            job.energy = energy_device;
+            job.grad = gradient_device;  // nullptr: energy only
+            job.field = field;
+            job.layers = layers;
+            launch_regcircuit((int)num_qubits, nullptr, job, 1, stream);
+            const hipError_t err = hipGetLastError();
+            if (err != hipSuccess) {
+                fail(RIE_DEVICE_ERROR,
+                     std::string("allocation-free launch: ") + hipGetErrorString(err));
+            }
+            return;
+        }
         WireCoef *coef = reinterpret_cast<WireCoef *>(base);
         double2 *state = reinterpret_cast<double2 *>(base + kCoefBytes);
         const int n = (int)num_qubits;
-        launch_coef(params_device, coef, n * (int)num_layers, stream);
+        launch_coef(params_device, coef, n * layers, stream);
         BatchJob job{};
         job.n = n;
-        job.layers = (int)num_layers;
+        job.layers = layers;
         job.chunk = (int)std::min<size_t>(structured_rotation_chunk_width, 4);
         job.field = field;
         job.coef = coef;
@@ -110,9 +131,7 @@ rie_status rie_energy_and_grad_noalloc(size_t num_qubits, size_t num_layers, dou
         job.grad = gradient_device;  // nullptr: energy only
         job.drift = nullptr;
         job.scale = nullptr;
-        const bool in_lds = n <= kBatchMaxLdsQubits;
-        launch_batch_structured(nullptr, job, nullptr, nullptr, 1, 256, in_lds ? n : 0,
-                                in_lds ? nullptr : state, 0, stream);
+        launch_batch_structured(nullptr, job, nullptr, nullptr, 1, 256, state, 0, stream);
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) {
             fail(RIE_DEVICE_ERROR, std::string("allocation-free launch: ") + hipGetErrorString(err));

@@ -116,8 +116,9 @@ rie_status rie_energy_and_grad(size_t num_qubits, size_t num_layers, double fiel
  * whole circuit in one workgroup).  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It calls no
- * hipMalloc, hipFree or allocating library routine: the coefficient table and
- * the state scratch (n = 13, 14) live in a file-scope device array of
+ * hipMalloc, hipFree or allocating library routine: the layers' records (n <=
+ * 13) or the coefficient table and state scratch (n = 14) live in a file-scope
+ * device array of
  * RIE_NOALLOC_SCRATCH_BYTES per device, held until the process ends.  Every
  * call on a device shares that array, so calls that overlap on one device
  * race; serialize them (one stream, or wait between streams).
@@ -343,9 +344,9 @@ rie_status rie_engine_copy_state(rie_engine *engine, double *host_out, size_t nu
  * 429-442).  A batch holds `count` circuits with their own qubit count
  * (2..14), layer count and field; circuits with num_qubits <=
  * dense_max_qubits (0..8) use dense_scan, the others structured_adjoint.
- * All circuits are evaluated together: the structured ones in one persistent
- * launch, the dense ones level by level in grouped FP64-MFMA GEMM launches,
- * concurrently.  Parameters, energies and gradients live in device arrays
+ * All circuits are evaluated together: the structured ones in one launch per
+ * qubit count (14 qubits: one persistent launch), the dense ones level by
+ * level in grouped FP64-MFMA GEMM launches, concurrently.  Parameters, energies and gradients live in device arrays
  * owned by the batch; circuit i's 2*n_i*L_i parameters (and gradients) start
  * at offsets[i] and follow the single-circuit layout. */
 typedef struct rie_batch rie_batch;
@@ -393,8 +394,9 @@ rie_status rie_batch_run_per_circuit(rie_batch *batch, int compute_gradient, voi
 rie_status rie_batch_optimize(rie_batch *batch, int optimizer, double learning_rate, size_t steps,
                               int use_graph, double *energy_history_out, void *stream);
 
-/* Autotuner: times the whole-circuit kernel per qubit count for every
- * workgroup size (256/512/1024) and rotation-chunk width (1..4), then, for
+/* Autotuner: times the 14-qubit whole-circuit kernel for every workgroup size
+ * (256/512/1024) and rotation-chunk width (1..4) (fewer qubits have one shape
+ * per qubit count), then, for
  * each split of the circuits between dense_scan (num_qubits <= s) and the
  * whole-circuit kernel, s from the dense_max_qubits given at creation down to
  * 0 (see rie_batch_set_tune_split), the dense GEMM tile (32/64) and the share
@@ -409,7 +411,9 @@ rie_status rie_batch_autotune(rie_batch *batch, size_t repeats);
 rie_status rie_batch_set_tune_split(rie_batch *batch, int enabled);
 /* Manual configuration: threads 256/512/1024; chunk_by_n (15 values,
  * indexed by num_qubits, each 1..4) or NULL to keep; dense_tile 32/64;
- * structured_grid = workgroups of the persistent launch (0: one per CU). */
+ * structured_grid = workgroups of the persistent launch (0: one per CU).
+ * Threads, chunks and grid shape the 14-qubit launch; circuits of fewer
+ * qubits run in registers and have no such choice. */
 rie_status rie_batch_set_config(rie_batch *batch, int threads, const int *chunk_by_n,
                                 size_t chunk_len, int dense_tile, int structured_grid);
 /* Current configuration and the last autotuning measurements as JSON. */

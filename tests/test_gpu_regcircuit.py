@@ -1,0 +1,80 @@
+"""Whole-circuit kernels with the state in registers (2..13 qubits).
+
+Each qubit count has its own layout (register, lane and wave wires) and its own
+unrolled layer, so every one is checked against the FP64 CPU oracle: one, two
+and several layers, generic angles and those where the tangent form changes
+(half angles at 0, pi/4, pi/2, pi and their negatives, on every wire in turn).
+FP64 rounding over a few hundred gates is below 1e-13; the bound is the
+project's 1e-10.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from gpu_simulation_amd.batch import CircuitSpec, RingIsingBatch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+# the last pair straddles the switch of the tangent form at a half angle of pi/4
+SPECIAL = np.array([0.0, np.pi, -np.pi, 2 * np.pi, np.pi / 2, -np.pi / 2, 3 * np.pi / 2,
+                    np.nextafter(np.pi / 2, 4.0)])
+
+
+def _params(kind, layers, n, rng):
+    p = rng.uniform(-2 * np.pi, 4 * np.pi, (layers, n, 2))
+    if kind == "special":
+        k = np.arange(layers * n).reshape(layers, n)
+        p[..., 0] = SPECIAL[(k * 5 + k // 8) % len(SPECIAL)]
+        p[..., 1] = np.where(k % 3 == 0, SPECIAL[(k * 3) % len(SPECIAL)], p[..., 1])
+    return p
+
+
+@pytest.mark.parametrize("n", range(2, 14))
+def test_every_layout_matches_oracle(oracle, n):
+    rng = np.random.default_rng([9, n])
+    specs, params = [], []
+    for kind in ("generic", "special"):
+        for layers in (1, 2, 3, 6):
+            specs.append(CircuitSpec(n, layers, 0.6 + 0.1 * layers))
+            params.append(_params(kind, layers, n, rng))
+    print(f"case n={n}", flush=True)
+    batch = RingIsingBatch(specs, dense_max_qubits=0)
+    energies, grads = batch.energy_and_grad(params)
+    energy_only, _ = batch.energy_and_grad(params, compute_gradient=False)
+    assert np.array_equal(energy_only, energies)
+    for s, p, e, g in zip(specs, params, energies, grads):
+        e_ref, g_ref = oracle.energy_and_grad(n, s.layers, s.field, p)
+        assert abs(e - e_ref) <= TOL, (n, s.layers)
+        assert np.max(np.abs(np.ravel(g) - np.ravel(g_ref))) <= TOL, (n, s.layers)
+
+
+@pytest.mark.parametrize("n", [2, 5, 6, 7, 8, 9, 11, 12])
+def test_engine_calls_agree(oracle, backend_module, n):
+    # host call, device calls (one and two step), walk back to |0...0>
+    import torch
+
+    layers = 40 if n <= 8 else 9
+    p = np.random.default_rng([10, n]).uniform(0, 2 * np.pi, (layers, n, 2))
+    eng = backend_module.RingIsingCudaBackend(n, layers, 0.8, "structured_adjoint", 8, False)
+    print(f"case engine n={n}", flush=True)
+    out = eng.energy_and_grad(p.reshape(-1))
+    e_ref, g_ref = oracle.energy_and_grad(n, layers, 0.8, p)
+    assert abs(out["energy"] - e_ref) <= TOL
+    assert np.max(np.abs(np.asarray(out["gradient"]) - np.ravel(g_ref))) <= TOL
+    assert eng.inverse_walk_drift(p.reshape(-1)) <= 1e-12
+    d = torch.from_numpy(p.reshape(-1)).cuda()
+    e = torch.zeros(1, dtype=torch.float64, device="cuda")
+    g = torch.zeros_like(d)
+    scale = torch.full((1,), -2.0, dtype=torch.float64, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    eng.energy_and_grad_device(d.data_ptr(), e.data_ptr(), g.data_ptr(), stream)
+    torch.cuda.synchronize()
+    assert e.item() == out["energy"] and np.array_equal(g.cpu().numpy(), out["gradient"])
+    eng.forward_device(d.data_ptr(), e.data_ptr(), stream)
+    eng.backward_device(d.data_ptr(), scale.data_ptr(), g.data_ptr(), stream)
+    torch.cuda.synchronize()
+    assert e.item() == out["energy"]
+    assert np.array_equal(g.cpu().numpy(), -2.0 * np.asarray(out["gradient"]))
