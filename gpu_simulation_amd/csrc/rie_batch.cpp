@@ -125,7 +125,7 @@ struct Batch {
     // dense part
     std::vector<int> dids;
     DensePlan dense;
-    int dense_tile = 64;
+    int dense_tile = 64;  // reported only: the product tree has one tile shape
     std::vector<std::unique_ptr<DensePlan>> dense_single;
 
     // graphs
@@ -460,14 +460,14 @@ void Batch::build_dense() {
     dense_single.clear();
     std::vector<DenseSpec> specs;
     for (int i : dids) {
-        specs.push_back({n[(size_t)i], L[(size_t)i], h[(size_t)i], d_coef + poff[(size_t)i] / 2,
+        specs.push_back({n[(size_t)i], L[(size_t)i], h[(size_t)i], d_params + poff[(size_t)i],
                          d_energy + i, d_grad + poff[(size_t)i], nullptr});
     }
-    dense.build(specs, dense_tile);
+    dense.build(specs, specs.size());
 }
 
 void Batch::issue_eval(hipStream_t s, bool want_grad) {
-    if (!gids.empty() || !dids.empty()) {
+    if (!gids.empty()) {
         launch_coef(d_params, d_coef, (int)(total / 2), s);
         check_launch("batch coef");
     }
@@ -586,9 +586,9 @@ void Batch::run_per_circuit(hipStream_t s, bool want_grad) {
     if (dense_single.empty() && !dids.empty()) {
         for (int i : dids) {
             auto plan = std::make_unique<DensePlan>();
-            plan->build({{n[(size_t)i], L[(size_t)i], h[(size_t)i], d_coef + poff[(size_t)i] / 2,
+            plan->build({{n[(size_t)i], L[(size_t)i], h[(size_t)i], d_params + poff[(size_t)i],
                           d_energy + i, d_grad + poff[(size_t)i], nullptr}},
-                        dense_tile);
+                        dids.size());
             dense_single.push_back(std::move(plan));
         }
     }
@@ -606,17 +606,17 @@ void Batch::run_per_circuit(hipStream_t s, bool want_grad) {
             launch_regcircuit(n[i], nullptr, j, 1, s);
             continue;
         }
-        launch_coef(d_params + poff[i], d_coef + poff[i] / 2, n[i] * L[i], s);
         if (dense_flag[i]) {
             dense_single[di++]->run(s, want_grad);
-        } else {
-            BatchJob j = jobs_g[gi++];
-            if (!want_grad) {
-                j.grad = nullptr;
-            }
-            launch_batch_structured(nullptr, j, nullptr, nullptr, 1, threads, d_scratch,
-                                    scratch_stride, s);
+            continue;
         }
+        BatchJob j = jobs_g[gi++];
+        if (!want_grad) {
+            j.grad = nullptr;
+        }
+        launch_coef(d_params + poff[i], d_coef + poff[i] / 2, n[i] * L[i], s);
+        launch_batch_structured(nullptr, j, nullptr, nullptr, 1, threads, d_scratch,
+                                scratch_stride, s);
     }
     check_launch("per-circuit launches");
 }
@@ -801,36 +801,16 @@ void Batch::autotune(size_t repeats) {
             cost_per_layer[q] = c[(size_t)q][(size_t)best_ti][(size_t)bk];
         }
     }
-    // per split: the dense tile for D >= 64 and the structured launch's grid
-    // (with a dense part running beside it, leave it CUs); the fastest whole
-    // evaluation wins
+    // per split: the persistent launch's grid (leaving CUs to what runs beside
+    // it); the fastest whole evaluation wins
     double best_ms = -1.0;
     int best_grid = 0;
     int best_split = splits.front();
-    int best_tile = dense_tile;
     rep << ", \"split_ms\": {";
     for (size_t si = 0; si < splits.size(); ++si) {
         const int split = splits[si];
         if (split != dense_split || si == 0) {
             repartition(split);
-        }
-        bool big_dense = false;
-        for (int i : dids) {
-            big_dense = big_dense || n[(size_t)i] >= 6;
-        }
-        if (big_dense) {
-            const int tiles[2] = {32, 64};
-            double dense_ms[2] = {0.0, 0.0};
-            for (int k = 0; k < 2; ++k) {
-                dense_tile = tiles[k];
-                build_dense();
-                dense_ms[k] = time_ms(repeats, [&](hipStream_t s) {
-                    launch_coef(d_params, d_coef, (int)(total / 2), s);
-                    dense.run(s, true);
-                });
-            }
-            dense_tile = dense_ms[0] < dense_ms[1] ? 32 : 64;
-            build_dense();
         }
         std::vector<int> grid_opts;
         if (!gids.empty()) {
@@ -854,14 +834,12 @@ void Batch::autotune(size_t repeats) {
                 best_ms = ms;
                 best_grid = grid_limit;
                 best_split = split;
-                best_tile = dense_tile;
             }
         }
         rep << "}";
     }
     rep << "}";
     grid_limit = best_grid;
-    dense_tile = best_tile;
     repartition(best_split);
     rep << ", \"dense_max_qubits\": " << best_split << ", \"batch_ms\": " << best_ms << "}";
     report = rep.str();
@@ -1114,12 +1092,8 @@ rie_status rie_batch_set_config(rie_batch *batch, int threads, const int *chunk_
         rie::check(hipDeviceSynchronize(), "sync");
         b->threads = threads;
         b->grid_limit = structured_grid;
-        const bool tile_changed = b->dense_tile != dense_tile;
         b->dense_tile = dense_tile;
         b->build_structured();
-        if (tile_changed) {
-            b->build_dense();
-        }
     });
 }
 

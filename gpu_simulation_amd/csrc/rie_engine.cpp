@@ -1251,12 +1251,12 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
         resident = false;
         return;
     }
-    launch_coef(params, d_coef, n * L, s);
-    check_launch("coef");
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
-        dense_run(s, false, nullptr, energy, nullptr);
+        dense_run(s, false, params, nullptr, energy, nullptr);
         return;
     }
+    launch_coef(params, d_coef, n * L, s);
+    check_launch("coef");
     if (strategy == RIE_STRATEGY_INVERSE_WALK_GATE) {
         gate_forward(s);
         gate_hamiltonian(s);
@@ -1277,8 +1277,7 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
 void Engine::backward_device(const double *params, const double *scale, double *grad,
                              hipStream_t s) {
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
-        launch_coef(params, d_coef, n * L, s);
-        dense_run(s, true, scale, d_energy + 1, grad);
+        dense_run(s, true, params, scale, d_energy + 1, grad);
         return;
     }
     if (strategy == RIE_STRATEGY_INVERSE_WALK_GATE) {
@@ -1311,6 +1310,10 @@ void Engine::eval_device(const double *params, double *energy, double *grad, hip
         check_launch("coef");
         structured_eval_fused(s, nullptr, energy, false);
         copy_grad_if_needed(grad, s);
+        return;
+    }
+    if (strategy == RIE_STRATEGY_DENSE_SCAN) {
+        dense_run(s, true, params, nullptr, energy, grad);
         return;
     }
     if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
@@ -1357,8 +1360,7 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
     }
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
         stage_begin(s);
-        launch_coef(d_params, d_coef, n * L, s);
-        dense_run(s, want_grad, nullptr, d_energy, want_grad ? d_grad : nullptr);
+        dense_run(s, want_grad, d_params, nullptr, d_energy, want_grad ? d_grad : nullptr);
         stage_end(s, "dense_scan_ms");
     } else if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
         stage_begin(s);

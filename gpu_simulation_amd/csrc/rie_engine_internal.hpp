@@ -233,8 +233,8 @@ struct Engine {
     void gate_backward(hipStream_t s, const double *scale);
     void dense_init();
     void dense_free();
-    void dense_run(hipStream_t s, bool want_grad, const double *scale, double *energy_out,
-                   double *grad_out);
+    void dense_run(hipStream_t s, bool want_grad, const double *params, const double *scale,
+                   double *energy_out, double *grad_out);
 
     void forward_device(const double *params, double *energy, hipStream_t s, bool keep_lam);
     void backward_device(const double *params, const double *scale, double *grad, hipStream_t s);

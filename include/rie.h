@@ -399,8 +399,8 @@ rie_status rie_batch_optimize(rie_batch *batch, int optimizer, double learning_r
  * per qubit count), then, for
  * each split of the circuits between dense_scan (num_qubits <= s) and the
  * whole-circuit kernel, s from the dense_max_qubits given at creation down to
- * 0 (see rie_batch_set_tune_split), the dense GEMM tile (32/64) and the share
- * of CUs given to the structured launch; keeps the fastest whole evaluation
+ * 0 (see rie_batch_set_tune_split), the share of CUs given to the 14-qubit
+ * launch; keeps the fastest whole evaluation
  * and rebuilds the schedule with the measured costs.  The reference fixes the
  * strategy per call and its kernel shapes by qubit-count thresholds
  * (cpp/ising_cuda_rotation_kernels.cu:562-575). */
@@ -413,7 +413,8 @@ rie_status rie_batch_set_tune_split(rie_batch *batch, int enabled);
  * indexed by num_qubits, each 1..4) or NULL to keep; dense_tile 32/64;
  * structured_grid = workgroups of the persistent launch (0: one per CU).
  * Threads, chunks and grid shape the 14-qubit launch; circuits of fewer
- * qubits run in registers and have no such choice. */
+ * qubits run in registers, and the product tree has one tile shape, so
+ * dense_tile is only reported. */
 rie_status rie_batch_set_config(rie_batch *batch, int threads, const int *chunk_by_n,
                                 size_t chunk_len, int dense_tile, int structured_grid);
 /* Current configuration and the last autotuning measurements as JSON. */
