@@ -5,9 +5,10 @@
 // (rie_dense.hip, one grouped FP64-MFMA GEMM launch per tree level and tile
 // class for all of them).  The others take the whole-circuit kernels: up to
 // 13 qubits one launch per qubit count with every state in registers
-// (rie_regcircuit.hip), one workgroup per circuit, deepest first; 14 qubits one
-// persistent launch (rie_batch.hip) whose workgroups take circuits from a
-// longest-first (LPT) schedule built on the host.  The launches are spread over
+// (rie_regcircuit.hip), one workgroup per circuit, deepest first; 14 qubits a
+// forward launch of the same kind and a persistent adjoint launch whose
+// workgroups take circuits from a longest-first (LPT) schedule built on the
+// host.  The launches are spread over
 // four streams (branches of one graph when captured), so the tail of one
 // qubit count's deep circuits overlaps the others' work.  Parameters, energies
 // and gradients of all circuits are packed in device arrays owned by the
@@ -44,8 +45,6 @@ namespace {
 
 constexpr int kMaxN = kBatchMaxQubits;
 
-int max_chunk_for(int threads) { return batch_max_chunk(threads); }
-
 }  // namespace
 
 struct Batch {
@@ -79,7 +78,6 @@ struct Batch {
     double *d_params = nullptr;
     double *d_grad = nullptr;
     double *d_energy = nullptr;
-    WireCoef *d_coef = nullptr;
     double *d_m = nullptr;
     double *d_v = nullptr;
     int *d_step = nullptr;
@@ -96,7 +94,8 @@ struct Batch {
     };
     std::vector<RegGroup> reg_groups;   // largest n first
     std::vector<RegJob> reg_jobs;       // with gradients, grouped, deepest first
-    std::vector<RecordJob> rec_jobs;    // indexed like reg_jobs
+    std::vector<RecordJob> reg_rec;     // indexed like reg_jobs
+    std::vector<RecordJob> rec_jobs;    // every structured circuit
     std::vector<int> reg_of;            // circuit -> reg_jobs index, or -1
     int reg_layers = 0;                 // records of one evaluation
     RegJob *d_reg_g = nullptr;
@@ -104,28 +103,27 @@ struct Batch {
     RecordJob *d_rec_jobs = nullptr;
     int *d_layer_job = nullptr;
     double *d_rec = nullptr;
-    // above: persistent launch
+    // 14 qubits
     std::vector<int> gids;
-    std::vector<BatchJob> jobs_g;  // with gradients, indexed like gids
-    BatchJob *d_jobs_g = nullptr;
-    BatchJob *d_jobs_e = nullptr;  // energy only
+    std::vector<Reg14Job> jobs_g;    // with gradients, indexed like gids
+    std::vector<RecordJob> jobs_rec; // indexed like gids
+    Reg14Job *d_jobs_g = nullptr;
+    Reg14Job *d_jobs_e = nullptr;  // energy only
+    double2 *d_psi = nullptr;      // forward results of the 14-qubit circuits
     int *d_order = nullptr;
     int *d_wg_begin = nullptr;
     double2 *d_scratch = nullptr;
-    uint64_t scratch_stride = 0;
-    int scratch_slots = 0;
     int grid = 0;
-    int threads = 512;
+    int threads = 512;  // reported only, like chunk_by_n and dense_tile below:
+                        // the kernels have one shape per qubit count
     int grid_limit = 0;  // 0: every CU
-    int wg_per_cu = 1;
     int chunk_by_n[kMaxN + 1];
-    double cost_per_layer[kMaxN + 1];  // measured (autotuner) or modelled
     bool measured = false;
 
     // dense part
     std::vector<int> dids;
     DensePlan dense;
-    int dense_tile = 64;  // reported only: the product tree has one tile shape
+    int dense_tile = 64;
     std::vector<std::unique_ptr<DensePlan>> dense_single;
 
     // graphs
@@ -193,7 +191,6 @@ Batch::Batch(size_t count_, const int *nq, const int *nl, const double *fields, 
     }
     for (int q = 0; q <= kMaxN; ++q) {
         chunk_by_n[q] = 3;
-        cost_per_layer[q] = q * std::ldexp(1.0, q);  // modelled: amplitude updates
     }
     check(hipGetDevice(&device), "hipGetDevice");
     hipDeviceProp_t prop;
@@ -210,7 +207,6 @@ Batch::Batch(size_t count_, const int *nq, const int *nl, const double *fields, 
     d_params = (double *)device_alloc(sizeof(double) * total, "alloc batch params");
     d_grad = (double *)device_alloc(sizeof(double) * total, "alloc batch gradient");
     d_energy = (double *)device_alloc(sizeof(double) * count, "alloc batch energies");
-    d_coef = (WireCoef *)device_alloc(sizeof(WireCoef) * (total / 2), "alloc batch coefficients");
     d_step = (int *)device_alloc(sizeof(int), "alloc step counter");
     check(hipMemset(d_params, 0, sizeof(double) * total), "clear params");
     check(hipMemset(d_grad, 0, sizeof(double) * total), "clear gradient");
@@ -252,7 +248,6 @@ Batch::~Batch() {
     device_free(d_params);
     device_free(d_grad);
     device_free(d_energy);
-    device_free(d_coef);
     device_free(d_m);
     device_free(d_v);
     device_free(d_step);
@@ -286,6 +281,8 @@ void Batch::release_structured() {
     device_free(d_order);
     device_free(d_wg_begin);
     device_free(d_scratch);
+    device_free(d_psi);
+    d_psi = nullptr;
     device_free(d_reg_g);
     device_free(d_reg_e);
     device_free(d_rec_jobs);
@@ -298,22 +295,18 @@ void Batch::release_structured() {
     reg_groups.clear();
     reg_jobs.clear();
     rec_jobs.clear();
+    reg_rec.clear();
     reg_layers = 0;
     d_jobs_g = d_jobs_e = nullptr;
     d_order = d_wg_begin = nullptr;
     d_scratch = nullptr;
-    scratch_slots = 0;
     grid = 0;
 }
 
-// Jobs and records of the circuits whose states fit in registers.
+// Records of every structured circuit, jobs of those whose states fit in
+// registers.
 void Batch::build_register_jobs() {
-    std::vector<int> ids;
-    for (int i : sids) {
-        if (n[(size_t)i] <= kRegMaxQubits) {
-            ids.push_back(i);
-        }
-    }
+    std::vector<int> ids = sids;
     reg_of.assign(count, -1);
     if (ids.empty()) {
         return;
@@ -332,31 +325,42 @@ void Batch::build_register_jobs() {
     for (int i : ids) {
         const int q = n[(size_t)i];
         const int layers = L[(size_t)i];
+        const RegJob job{rec, d_energy + i, d_grad + poff[(size_t)i], nullptr, nullptr,
+                         h[(size_t)i], layers, 0};
+        const RecordJob record{d_params + poff[(size_t)i], rec, q, reg_layers};
+        layer_job.insert(layer_job.end(), (size_t)layers, (int)rec_jobs.size());
+        rec_jobs.push_back(record);
+        reg_layers += layers;
+        rec += circuit_record_bytes(q, layers) / sizeof(double);
+        if (q > kRegMaxQubits) {
+            gids.push_back(i);
+            jobs_g.push_back({job, nullptr});
+            jobs_rec.push_back(record);
+            continue;
+        }
         if (reg_groups.empty() || reg_groups.back().n != q) {
             reg_groups.push_back({q, (int)reg_jobs.size(), 0});
         }
         reg_groups.back().count += 1;
         reg_of[(size_t)i] = (int)reg_jobs.size();
-        layer_job.insert(layer_job.end(), (size_t)layers, (int)reg_jobs.size());
-        rec_jobs.push_back({d_params + poff[(size_t)i], rec, q, reg_layers});
-        reg_jobs.push_back({rec, d_energy + i, d_grad + poff[(size_t)i], nullptr, nullptr,
-                            h[(size_t)i], layers, 0});
-        reg_layers += layers;
-        rec += circuit_record_bytes(q, layers) / sizeof(double);
+        reg_jobs.push_back(job);
+        reg_rec.push_back(record);
     }
     std::vector<RegJob> energy_only = reg_jobs;
     for (auto &j : energy_only) {
         j.grad = nullptr;
     }
     const size_t job_bytes = sizeof(RegJob) * reg_jobs.size();
-    d_reg_g = (RegJob *)device_alloc(job_bytes, "alloc batch jobs");
-    d_reg_e = (RegJob *)device_alloc(job_bytes, "alloc batch jobs");
+    if (!reg_jobs.empty()) {
+        d_reg_g = (RegJob *)device_alloc(job_bytes, "alloc batch jobs");
+        d_reg_e = (RegJob *)device_alloc(job_bytes, "alloc batch jobs");
+        check(hipMemcpy(d_reg_g, reg_jobs.data(), job_bytes, hipMemcpyHostToDevice),
+              "upload batch jobs");
+        check(hipMemcpy(d_reg_e, energy_only.data(), job_bytes, hipMemcpyHostToDevice),
+              "upload batch jobs");
+    }
     d_rec_jobs = (RecordJob *)device_alloc(sizeof(RecordJob) * rec_jobs.size(), "alloc batch jobs");
     d_layer_job = (int *)device_alloc(sizeof(int) * layer_job.size(), "alloc batch layers");
-    check(hipMemcpy(d_reg_g, reg_jobs.data(), job_bytes, hipMemcpyHostToDevice),
-          "upload batch jobs");
-    check(hipMemcpy(d_reg_e, energy_only.data(), job_bytes, hipMemcpyHostToDevice),
-          "upload batch jobs");
     check(hipMemcpy(d_rec_jobs, rec_jobs.data(), sizeof(RecordJob) * rec_jobs.size(),
                     hipMemcpyHostToDevice),
           "upload batch jobs");
@@ -365,48 +369,31 @@ void Batch::build_register_jobs() {
           "upload batch layers");
 }
 
-// Register jobs, and a longest-first schedule of the larger circuits over
-// `grid` workgroups.
+// Jobs and records, and a longest-first schedule of the 14-qubit circuits'
+// adjoint sweeps over `grid` workgroups.
 void Batch::build_structured() {
     invalidate_graph();
     release_structured();
-    build_register_jobs();
     jobs_g.clear();
+    jobs_rec.clear();
     gids.clear();
-    for (int i : sids) {
-        if (n[(size_t)i] > kRegMaxQubits) {
-            gids.push_back(i);
-        }
-    }
+    build_register_jobs();
     if (gids.empty()) {
         return;
     }
-    const int cap = grid_limit > 0 ? grid_limit : num_cus * wg_per_cu;
+    const int cap = grid_limit > 0 ? grid_limit : num_cus;
     grid = (int)std::min<size_t>(gids.size(), (size_t)std::max(1, cap));
-    int max_global_n = 0;
-    for (int i : gids) {
-        BatchJob j{};
-        j.n = n[(size_t)i];
-        j.layers = L[(size_t)i];
-        j.chunk = std::min(chunk_by_n[j.n], max_chunk_for(threads));
-        j.field = h[(size_t)i];
-        j.coef = d_coef + poff[(size_t)i] / 2;
-        j.energy = d_energy + i;
-        j.grad = d_grad + poff[(size_t)i];
-        j.drift = nullptr;
-        j.scale = nullptr;
-        jobs_g.push_back(j);
-        max_global_n = std::max(max_global_n, j.n);
+    constexpr size_t kAmps = (size_t)1 << kMaxN;
+    d_psi = (double2 *)device_alloc(sizeof(double2) * kAmps * gids.size(), "alloc batch states");
+    for (size_t k = 0; k < gids.size(); ++k) {
+        jobs_g[k].psi = d_psi + kAmps * k;
     }
     // LPT: heaviest first onto the least-loaded workgroup
     std::vector<int> idx(gids.size());
     for (size_t k = 0; k < idx.size(); ++k) {
         idx[k] = (int)k;
     }
-    auto cost = [&](int k) {
-        const BatchJob &j = jobs_g[(size_t)k];
-        return (double)j.layers * cost_per_layer[j.n];
-    };
+    auto cost = [&](int k) { return (double)jobs_g[(size_t)k].base.layers; };
     std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return cost(a) > cost(b); });
     using Slot = std::pair<double, int>;
     std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> heap;
@@ -427,32 +414,26 @@ void Batch::build_structured() {
         order.insert(order.end(), lst.begin(), lst.end());
         begin.push_back((int)order.size());
     }
-    std::vector<BatchJob> jobs_e = jobs_g;
+    std::vector<Reg14Job> jobs_e = jobs_g;
     for (auto &j : jobs_e) {
-        j.grad = nullptr;
+        j.base.grad = nullptr;
     }
-    d_jobs_g = (BatchJob *)device_alloc(sizeof(BatchJob) * jobs_g.size(), "alloc batch jobs");
-    d_jobs_e = (BatchJob *)device_alloc(sizeof(BatchJob) * jobs_g.size(), "alloc batch jobs");
+    d_jobs_g = (Reg14Job *)device_alloc(sizeof(Reg14Job) * jobs_g.size(), "alloc batch jobs");
+    d_jobs_e = (Reg14Job *)device_alloc(sizeof(Reg14Job) * jobs_g.size(), "alloc batch jobs");
     d_order = (int *)device_alloc(sizeof(int) * order.size(), "alloc batch order");
     d_wg_begin = (int *)device_alloc(sizeof(int) * begin.size(), "alloc batch schedule");
-    check(hipMemcpy(d_jobs_g, jobs_g.data(), sizeof(BatchJob) * jobs_g.size(),
+    check(hipMemcpy(d_jobs_g, jobs_g.data(), sizeof(Reg14Job) * jobs_g.size(),
                     hipMemcpyHostToDevice),
           "upload batch jobs");
-    check(hipMemcpy(d_jobs_e, jobs_e.data(), sizeof(BatchJob) * jobs_e.size(),
+    check(hipMemcpy(d_jobs_e, jobs_e.data(), sizeof(Reg14Job) * jobs_e.size(),
                     hipMemcpyHostToDevice),
           "upload batch jobs");
     check(hipMemcpy(d_order, order.data(), sizeof(int) * order.size(), hipMemcpyHostToDevice),
           "upload batch order");
     check(hipMemcpy(d_wg_begin, begin.data(), sizeof(int) * begin.size(), hipMemcpyHostToDevice),
           "upload batch schedule");
-    if (max_global_n > 0) {
-        scratch_stride = (uint64_t)2 << max_global_n;
-        // one slot per workgroup of the persistent grid, and at least as many
-        // as the autotuner's one-circuit-per-workgroup probes use
-        scratch_slots = std::max(grid, std::min((int)gids.size(), num_cus));
-        d_scratch = (double2 *)device_alloc(sizeof(double2) * scratch_stride * scratch_slots,
-                                            "alloc batch scratch");
-    }
+    d_scratch = (double2 *)device_alloc(sizeof(double2) * kReg14Scratch * (size_t)grid,
+                                        "alloc batch scratch");
 }
 
 void Batch::build_dense() {
@@ -467,10 +448,6 @@ void Batch::build_dense() {
 }
 
 void Batch::issue_eval(hipStream_t s, bool want_grad) {
-    if (!gids.empty()) {
-        launch_coef(d_params, d_coef, (int)(total / 2), s);
-        check_launch("batch coef");
-    }
     if (reg_layers > 0) {
         launch_circuit_records(d_rec_jobs, RecordJob{}, d_layer_job, reg_layers, s);
         check_launch("batch records");
@@ -491,9 +468,9 @@ void Batch::issue_eval(hipStream_t s, bool want_grad) {
         return k == 0 ? s : s_aux[k - 1];
     };
     if (!gids.empty()) {
-        launch_batch_structured(want_grad ? d_jobs_g : d_jobs_e, BatchJob{}, d_order, d_wg_begin,
-                                grid, threads, d_scratch, scratch_stride, next_stream());
-        check_launch("batch structured");
+        launch_reg14(want_grad ? d_jobs_g : d_jobs_e, Reg14Job{}, d_order, d_wg_begin,
+                     (int)gids.size(), grid, d_scratch, next_stream());
+        check_launch("batch 14 qubits");
     }
     if (!dids.empty()) {
         dense.run(next_stream(), want_grad);
@@ -593,11 +570,10 @@ void Batch::run_per_circuit(hipStream_t s, bool want_grad) {
         }
     }
     size_t di = 0;
-    size_t gi = 0;
     for (size_t i = 0; i < count; ++i) {
         if (reg_of[i] >= 0) {
             RegJob j = reg_jobs[(size_t)reg_of[i]];
-            RecordJob r = rec_jobs[(size_t)reg_of[i]];
+            RecordJob r = reg_rec[(size_t)reg_of[i]];
             r.first_layer = 0;
             if (!want_grad) {
                 j.grad = nullptr;
@@ -610,13 +586,15 @@ void Batch::run_per_circuit(hipStream_t s, bool want_grad) {
             dense_single[di++]->run(s, want_grad);
             continue;
         }
-        BatchJob j = jobs_g[gi++];
+        const size_t k = (size_t)(std::find(gids.begin(), gids.end(), (int)i) - gids.begin());
+        Reg14Job j = jobs_g[k];
+        RecordJob r = jobs_rec[k];
+        r.first_layer = 0;
         if (!want_grad) {
-            j.grad = nullptr;
+            j.base.grad = nullptr;
         }
-        launch_coef(d_params + poff[i], d_coef + poff[i] / 2, n[i] * L[i], s);
-        launch_batch_structured(nullptr, j, nullptr, nullptr, 1, threads, d_scratch,
-                                scratch_stride, s);
+        launch_circuit_records(nullptr, r, nullptr, j.base.layers, s);
+        launch_reg14(nullptr, j, nullptr, nullptr, 1, 1, d_scratch, s);
     }
     check_launch("per-circuit launches");
 }
@@ -692,8 +670,6 @@ void Batch::autotune(size_t repeats) {
         }
         if (!splits.empty()) {
             splits.push_back(0);
-            // every circuit on the whole-circuit kernel while its costs are probed
-            repartition(0);
         }
     }
     if (splits.empty()) {
@@ -701,112 +677,13 @@ void Batch::autotune(size_t repeats) {
     }
     std::ostringstream rep;
     rep.precision(6);
-    rep << "{\"per_layer_us\": {";
-    const int thread_opts[3] = {256, 512, 1024};
-    // c[n][ti][K]: microseconds per layer of the slowest probe circuit
-    std::vector<std::vector<std::vector<double>>> c(
-        kMaxN + 1, std::vector<std::vector<double>>(3, std::vector<double>(5, 0.0)));
-    std::vector<double> layers_of_n(kMaxN + 1, 0.0);
-    // circuits above kRegMaxQubits: the register kernels have no shape to tune
-    for (size_t k = 0; k < gids.size(); ++k) {
-        layers_of_n[(size_t)jobs_g[k].n] += jobs_g[k].layers;
-    }
-    bool first_n = true;
-    BatchJob *d_probe = nullptr;
-    try {
-        for (int q = 2; q <= kMaxN; ++q) {
-            if (layers_of_n[(size_t)q] == 0.0) {
-                continue;
-            }
-            std::vector<BatchJob> probe;
-            int max_l = 0;
-            for (size_t k = 0; k < gids.size() && (int)probe.size() < num_cus; ++k) {
-                if (jobs_g[k].n == q) {
-                    probe.push_back(jobs_g[k]);
-                    max_l = std::max(max_l, jobs_g[k].layers);
-                }
-            }
-            if ((int)probe.size() > scratch_slots) {
-                probe.resize((size_t)scratch_slots);
-            }
-            device_free(d_probe);
-            d_probe = (BatchJob *)device_alloc(sizeof(BatchJob) * probe.size(), "alloc probe");
-            rep << (first_n ? "" : ", ") << "\"" << q << "\": {";
-            first_n = false;
-            for (int ti = 0; ti < 3; ++ti) {
-                const int T = thread_opts[ti];
-                rep << (ti ? ", " : "") << "\"" << T << "\": [";
-                for (int K = 1; K <= max_chunk_for(T); ++K) {
-                    for (auto &j : probe) {
-                        j.chunk = K;
-                    }
-                    check(hipMemcpy(d_probe, probe.data(), sizeof(BatchJob) * probe.size(),
-                                    hipMemcpyHostToDevice),
-                          "upload probe");
-                    const double ms = time_ms(repeats, [&](hipStream_t s) {
-                        launch_batch_structured(d_probe, BatchJob{}, nullptr, nullptr,
-                                                (int)probe.size(), T, d_scratch,
-                                                scratch_stride, s);
-                        check_launch("autotune probe");
-                    });
-                    c[(size_t)q][(size_t)ti][(size_t)K] = ms * 1e3 / max_l;
-                    rep << (K > 1 ? ", " : "") << c[(size_t)q][(size_t)ti][(size_t)K];
-                }
-                rep << "]";
-            }
-            rep << "}";
-        }
-    } catch (...) {
-        device_free(d_probe);
-        throw;
-    }
-    device_free(d_probe);
-    rep << "}";
     measured = measured || !sids.empty();
-    if (!gids.empty()) {
-        // one thread count for the launch: least total modelled work
-        double best = -1.0;
-        int best_ti = 1;
-        for (int ti = 0; ti < 3; ++ti) {
-            double work = 0.0;
-            for (int q = 2; q <= kMaxN; ++q) {
-                if (layers_of_n[(size_t)q] == 0.0) {
-                    continue;
-                }
-                double m = -1.0;
-                for (int K = 1; K <= max_chunk_for(thread_opts[ti]); ++K) {
-                    const double v = c[(size_t)q][(size_t)ti][(size_t)K];
-                    m = (m < 0.0 || v < m) ? v : m;
-                }
-                work += layers_of_n[(size_t)q] * m;
-            }
-            if (best < 0.0 || work < best) {
-                best = work;
-                best_ti = ti;
-            }
-        }
-        threads = thread_opts[best_ti];
-        for (int q = 2; q <= kMaxN; ++q) {
-            if (layers_of_n[(size_t)q] == 0.0) {
-                continue;
-            }
-            int bk = 1;
-            for (int K = 2; K <= max_chunk_for(threads); ++K) {
-                if (c[(size_t)q][(size_t)best_ti][(size_t)K] <
-                    c[(size_t)q][(size_t)best_ti][(size_t)bk]) {
-                    bk = K;
-                }
-            }
-            chunk_by_n[q] = bk;
-            cost_per_layer[q] = c[(size_t)q][(size_t)best_ti][(size_t)bk];
-        }
-    }
     // per split: the persistent launch's grid (leaving CUs to what runs beside
     // it); the fastest whole evaluation wins
     double best_ms = -1.0;
     int best_grid = 0;
     int best_split = splits.front();
-    rep << ", \"split_ms\": {";
+    rep << "{\"split_ms\": {";
     for (size_t si = 0; si < splits.size(); ++si) {
         const int split = splits[si];
         if (split != dense_split || si == 0) {
@@ -854,7 +731,7 @@ std::string Batch::config_json() const {
       << ", \"chunk_by_n\": {";
     bool first = true;
     for (int q = 2; q <= kMaxN; ++q) {
-        o << (first ? "" : ", ") << "\"" << q << "\": " << std::min(chunk_by_n[q], max_chunk_for(threads));
+        o << (first ? "" : ", ") << "\"" << q << "\": " << chunk_by_n[q];
         first = false;
     }
     o << "}, \"autotune\": " << report << "}";

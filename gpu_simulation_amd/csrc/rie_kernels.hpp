@@ -154,21 +154,6 @@ inline bool lay_fits(const LamLayout &L, int n, int first, int count) {
     return true;
 }
 
-// One independent circuit evaluated by a single workgroup on global scratch
-// (n <= 14).
-struct BatchJob {
-    int n;
-    int layers;
-    int chunk;             // wires per register chunk (1..4)
-    int reserved;
-    double field;
-    const WireCoef *coef;  // layers * n entries
-    double *energy;        // 1 value
-    double *grad;          // 2 * n * layers values, or nullptr for energy only
-    double *drift;         // || walked state - |0> ||^2, or nullptr
-    const double *scale;   // optional chain-rule factor for grad (nullptr = 1)
-};
-
 constexpr int kRegMaxQubits = 13;  // states in the registers of one workgroup
 
 // One circuit (2 <= n <= kRegMaxQubits) evaluated in registers.
@@ -200,26 +185,24 @@ void launch_circuit_records(const RecordJob *d_jobs, const RecordJob &single,
 void launch_regcircuit(int n, const RegJob *d_jobs, const RegJob &single, int count,
                        hipStream_t s);
 
-constexpr int kEngineWholeQubits = 12;  // an engine's whole-circuit path (tile passes above)
-constexpr int kBatchMaxQubits = 14;     // whole-circuit kernels; above kRegMaxQubits on scratch
+// 14 qubits: the forward sweep in registers, the adjoint sweep in two halves
+// through scratch (kReg14Scratch amplitudes per workgroup).
+struct Reg14Job {
+    RegJob base;
+    double2 *psi;  // 2^14 amplitudes, written by the forward sweep
+};
+constexpr size_t kReg14Scratch = (size_t)4 << 14;
+// count circuits (`single`, or d_jobs[0 .. count)); the adjoint sweep runs
+// them on `grid` workgroups: workgroup b takes d_order[d_wg_begin[b] ..
+// d_wg_begin[b + 1]) in turn (null: `single`).
+void launch_reg14(const Reg14Job *d_jobs, const Reg14Job &single, const int *d_order,
+                  const int *d_wg_begin, int count, int grid, double2 *scratch, hipStream_t s);
 
-// Widest rotation chunk per workgroup size: a backward group keeps 2 * 2^K
-// amplitudes in registers, and the register budget per thread halves each
-// time the workgroup doubles.
-constexpr int batch_max_chunk(int threads) {
-    return threads >= 1024 ? 2 : (threads >= 512 ? 3 : 4);
-}
+constexpr int kEngineWholeQubits = 12;  // an engine's whole-circuit path (tile passes above)
+constexpr int kBatchMaxQubits = 14;     // whole-circuit kernels
 
 // Coefficient table from device parameters: coef[i] from params[2i], params[2i+1].
 void launch_coef(const double *d_params, WireCoef *d_coef, int count, hipStream_t s);
-
-// Persistent whole-circuit kernel: workgroup b runs the circuits
-// d_order[d_wg_begin[b] .. d_wg_begin[b+1]) in turn (without d_wg_begin:
-// circuit b of d_jobs, or `single` when d_jobs is null) on scratch +
-// b * scratch_stride (2 * 2^n amplitudes).  threads is 256, 512 or 1024.
-void launch_batch_structured(const BatchJob *d_jobs, const BatchJob &single, const int *d_order,
-                             const int *d_wg_begin, int grid, int threads, double2 *scratch,
-                             uint64_t scratch_stride, hipStream_t s);
 
 // Optimizer steps and helpers over packed arrays.
 void launch_gd_update(double *p, const double *g, uint64_t count, double lr, hipStream_t s);

@@ -3,18 +3,18 @@
 // HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.
 //
 // The whole circuit runs in one workgroup: psi and lambda in registers for
-// n <= 13 (regcircuit_kernel), in a 2 * 2^n-amplitude global scratch for n = 14
-// (batch_structured_kernel with a single job).  Everything beyond the caller's
-// inputs and outputs -- the layers' records, or the per-(layer, wire)
-// coefficient table and that state scratch -- lives in the file-scope array `scratch` below, one copy per device, held
-// until the process ends.  Its address on each device comes from
-// hipGetSymbolAddress once per device (with that device current) and is the
-// only form in which host code hands it to kernels.
+// n <= 13, for n = 14 the adjoint sweep in two halves through a global scratch
+// (rie_regcircuit.hip).  Everything beyond the caller's inputs and outputs -- the
+// layers' records, and at n = 14 the state and that scratch -- lives in the
+// file-scope array `scratch` below, one copy per device, held until the process
+// ends.  Its address on each device comes from hipGetSymbolAddress once per
+// device (with that device current) and is the only form in which host code
+// hands it to kernels.
 //
 // Every call on a device shares that device's array: calls that overlap on
 // one device (different streams, or different host threads) race.  Nothing
-// in it needs to start at zero: the coefficient kernel writes every entry the
-// circuit reads, and the circuit kernel writes its initial state.
+// in it needs to start at zero: the records kernel writes every entry the
+// circuit reads, and the circuit kernels write the states they read.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,12 +32,9 @@ namespace {
 constexpr size_t kNoAllocMaxQubits = RIE_NOALLOC_MAX_QUBITS;
 constexpr size_t kNoAllocMaxLayers = RIE_NOALLOC_MAX_LAYERS;
 static_assert(kNoAllocMaxQubits <= (size_t)kBatchMaxQubits, "the whole-circuit kernel's limit");
-constexpr size_t kCoefBytes = sizeof(WireCoef) * kNoAllocMaxQubits * kNoAllocMaxLayers;
-constexpr size_t kStateBytes = sizeof(double2) * 2 * (size_t{1} << kNoAllocMaxQubits);
-constexpr size_t kScratchBytes = kCoefBytes + kStateBytes;
-static_assert(sizeof(double) * 112 * kNoAllocMaxLayers <= kScratchBytes,
-              "the records of 13 qubits (the longest) fit");
-static_assert(kCoefBytes % 256 == 0, "the state region starts 256-byte aligned");
+constexpr size_t kRecordBytes = 1024 * kNoAllocMaxLayers;  // at most 1 KB a layer
+constexpr size_t kStateBytes = sizeof(double2) * (size_t{1} << kNoAllocMaxQubits);
+constexpr size_t kScratchBytes = kRecordBytes + kStateBytes + sizeof(double2) * kReg14Scratch;
 static_assert(kScratchBytes == RIE_NOALLOC_SCRATCH_BYTES, "the size the header states");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -98,40 +95,27 @@ rie_status rie_energy_and_grad_noalloc(size_t num_qubits, size_t num_layers, dou
         }
         const hipStream_t stream = static_cast<hipStream_t>(stream_handle);
         unsigned char *base = device_scratch();
-        const int layers = (int)num_layers;
-        if (num_qubits <= (size_t)kRegMaxQubits) {
-            double *rec = reinterpret_cast<double *>(base);
-            launch_circuit_records(nullptr, RecordJob{params_device, rec, (int)num_qubits, 0},
-                                   nullptr, layers, stream);
-            RegJob job{};
-            job.rec = rec;
-            job.energy = energy_device;
-            job.grad = gradient_device;  // nullptr: energy only
-            job.field = field;
-            job.layers = layers;
-            launch_regcircuit((int)num_qubits, nullptr, job, 1, stream);
-            const hipError_t err = hipGetLastError();
-            if (err != hipSuccess) {
-                fail(RIE_DEVICE_ERROR,
-                     std::string("allocation-free launch: ") + hipGetErrorString(err));
-            }
-            return;
-        }
-        WireCoef *coef = reinterpret_cast<WireCoef *>(base);
-        double2 *state = reinterpret_cast<double2 *>(base + kCoefBytes);
         const int n = (int)num_qubits;
-        launch_coef(params_device, coef, n * layers, stream);
-        BatchJob job{};
-        job.n = n;
-        job.layers = layers;
-        job.chunk = (int)std::min<size_t>(structured_rotation_chunk_width, 4);
-        job.field = field;
-        job.coef = coef;
+        const int layers = (int)num_layers;
+        if (circuit_record_bytes(n, layers) > kRecordBytes) {
+            fail(RIE_DEVICE_ERROR, "internal: records exceed the scratch");
+        }
+        double *rec = reinterpret_cast<double *>(base);
+        launch_circuit_records(nullptr, RecordJob{params_device, rec, n, 0}, nullptr, layers,
+                               stream);
+        RegJob job{};
+        job.rec = rec;
         job.energy = energy_device;
         job.grad = gradient_device;  // nullptr: energy only
-        job.drift = nullptr;
-        job.scale = nullptr;
-        launch_batch_structured(nullptr, job, nullptr, nullptr, 1, 256, state, 0, stream);
+        job.field = field;
+        job.layers = layers;
+        if (n <= kRegMaxQubits) {
+            launch_regcircuit(n, nullptr, job, 1, stream);
+        } else {
+            double2 *psi = reinterpret_cast<double2 *>(base + kRecordBytes);
+            launch_reg14(nullptr, Reg14Job{job, psi}, nullptr, nullptr, 1, 1,
+                         psi + (size_t{1} << kNoAllocMaxQubits), stream);
+        }
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) {
             fail(RIE_DEVICE_ERROR, std::string("allocation-free launch: ") + hipGetErrorString(err));

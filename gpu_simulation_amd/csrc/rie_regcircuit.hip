@@ -168,19 +168,13 @@ __global__ __launch_bounds__(RegState<n>::kThreads) __attribute__((
         k = S::flips(rec);
     }
     for (int l = 1; l < L; ++l) {
-        S::sync();
-        st.put(ex, c);
-        S::sync();
-        st.template get<0>(ex, c);
+        st.template exchange<0>(ex, c);
         f = ring_fwd_c(f ^ k, n);
         const double *rec = ring.advance();
         st.forward_layer({rec, f}, c, ex);
         k = S::flips(rec);
     }
-    S::sync();
-    st.put(ex, c);
-    S::sync();
-    st.template get<1>(ex, c);
+    st.template exchange<1>(ex, c);
     f = ring_fwd_c(f ^ k, n);
 
     double2 lam[A];
@@ -201,32 +195,13 @@ __global__ __launch_bounds__(RegState<n>::kThreads) __attribute__((
     }
     const double gscale = job.scale != nullptr ? *job.scale : 1.0;
 
-    // psi and lambda through the inverse ring CNOT
-    auto inverse_ring = [&](auto kind) {
-        constexpr int k = decltype(kind)::value;
-        S::sync();
-        st.put(ex, c);
-        if constexpr (kSplit) {
-            S::sync();
-            st.template get<k>(ex, c);
-            S::sync();
-            st.put(ex, lam);
-            S::sync();
-            st.template get<k>(ex, lam);
-        } else {
-            st.put(ex + S::kBuf, lam);
-            S::sync();
-            st.template get<k>(ex, c);
-            st.template get<k>(ex + S::kBuf, lam);
-        }
-    };
     auto write_gradient = [&](int l, const double *rec, const double *sums, bool all_scaled) {
         if (t < 2 * n) {
             job.grad[(size_t)l * 2 * n + t] =
                 S::gradient_entry(t, rec, sums, f, k, all_scaled) * gscale;
         }
     };
-    inverse_ring(std::integral_constant<int, 3>{});
+    st.template exchange2<3, kSplit>(ex, c, lam);
     int l = L - 1;
     if (l > 0) {
         do {
@@ -237,7 +212,7 @@ __global__ __launch_bounds__(RegState<n>::kThreads) __attribute__((
             st.template adjoint_layer<true, kSplit>({rec, f}, c, lam, ex, sums + 32 * st.wave);
             S::sync();
             write_gradient(l, rec, sums, false);
-            inverse_ring(std::integral_constant<int, 2>{});
+            st.template exchange2<2, kSplit>(ex, c, lam);
         } while (--l > 0);
     }
     const double *rec = ring.advance();
@@ -270,12 +245,226 @@ __global__ __launch_bounds__(RegState<n>::kThreads) __attribute__((
     }
 }
 
+// ---------------------------------------------------------------------------
+// 14 qubits.  psi alone fits the registers of 1024 threads (64 VGPRs of 128),
+// psi and lambda together fill the whole register file.  So the forward sweep
+// runs in registers and leaves psi in memory; the adjoint sweep takes the two
+// halves (top wire 0 and 1) of both arrays through 512 threads' registers, one
+// after the other, 13 wires each, and moves them through a scratch of two copies
+// (L2 / MALL) once a layer: the read applies the inverse ring CNOT and, as it
+// meets both halves, un-rotates the top wire of the layer before.
+//
+// Bound by latency and L2: a layer of one circuit takes 69 us forward and back
+// against 212 for sweeps of chunks of three wires over the scratch.
+// ---------------------------------------------------------------------------
+
+constexpr uint32_t kHalf14 = 1u << 13;
+
+__global__ __launch_bounds__(1024) void reg14_forward_kernel(const Reg14Job *__restrict__ jobs,
+                                                             Reg14Job single) {
+    using S = RegState<14>;
+    extern __shared__ double2 ex[];
+    __shared__ __align__(16) double slots[3][S::kRec];
+    const Reg14Job job = uniform(jobs != nullptr ? jobs[blockIdx.x] : single);
+    const int t = threadIdx.x;
+    S st;
+    st.setup((uint32_t)(t & 63), (uint32_t)__builtin_amdgcn_readfirstlane(t >> 6));
+    const int L = job.base.layers;
+    RecordRing<S::kRec> ring{slots, job.base.rec, L, L, st.wave == 0,
+                             2 * min(t & 63, S::kRec / 2 - 1)};
+    ring.start();
+    S::sync();
+    double2 c[S::A];
+    const double *rec = ring.advance();
+    st.product_state({rec, 0u}, c);
+    uint32_t f = 0;
+    uint32_t k = S::flips(rec);
+    for (int l = 1; l < L; ++l) {
+        st.exchange<0>(ex, c);
+        f = ring_fwd_c(f ^ k, 14);
+        rec = ring.advance();
+        st.forward_layer({rec, f}, c, ex);
+        k = S::flips(rec);
+    }
+    st.exchange<1>(ex, c);
+    f = ring_fwd_c(f ^ k, 14);
+    // storage order without label flips
+    const uint32_t at = st.own ^ S::frame(f);
+#pragma unroll
+    for (int r = 0; r < S::A; ++r) {
+        job.psi[at ^ (64u * r)] = c[r];
+    }
+}
+
+// Storage position (both halves: bit 13 the top wire) that position s reads
+// through the inverse ring CNOT, from layout 1 or 2 of the halves.
+template <bool kLayout2>
+__host__ __device__ constexpr uint32_t source14(uint32_t s) {
+    using S = RegState<13, 1>;
+    const uint32_t i = ring_fwd_c(S::frame(s & (kHalf14 - 1u)) | (s & kHalf14), 14);
+    const uint32_t low = i & (kHalf14 - 1u);
+    return (kLayout2 ? S::storage2(low) : S::frame(low)) | (i & kHalf14);
+}
+
+// Workgroup b takes circuits order[wg_begin[b] .. wg_begin[b + 1]) in turn
+// (without wg_begin: `single`) on scratch + b * kReg14Scratch.
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void reg14_adjoint_kernel(
+    const Reg14Job *__restrict__ jobs, Reg14Job single, const int *__restrict__ order,
+    const int *__restrict__ wg_begin, double2 *scratch) {
+    using S = RegState<13, 1>;
+    constexpr int A = S::A;
+    constexpr uint32_t kAll = 2 * kHalf14;
+    extern __shared__ double2 ex[];
+    __shared__ __align__(16) double slots[3][S::kRec];
+    __shared__ double red[3][32 * 16];  // sums of (half, wave), three layers in turn
+    const int t = threadIdx.x;
+    S st;
+    st.setup((uint32_t)(t & 63), (uint32_t)__builtin_amdgcn_readfirstlane(t >> 6));
+    const uint32_t from1 = source14<false>(st.own);
+    const uint32_t from2 = source14<true>(st.own);
+    double2 *slot = scratch + (size_t)blockIdx.x * kReg14Scratch;
+    const int q0 = wg_begin != nullptr ? wg_begin[blockIdx.x] : 0;
+    const int q1 = wg_begin != nullptr ? wg_begin[blockIdx.x + 1] : 1;
+    for (int at = q0; at < q1; ++at) {
+        const Reg14Job job = uniform(jobs != nullptr ? jobs[order[at]] : single);
+        const int L = job.base.layers;
+        double2 c[A];
+        double2 lam[A];
+        double2 *next = slot + 2 * kAll;  // written now; each buffer: psi, lambda
+        const double2 *src_c = job.psi;
+        const double2 *src_l = slot + kAll;
+        double e = 0.0;
+        for (uint32_t h = 0; h < 2; ++h) {
+            st.outer = h;
+            const double2 *half = job.psi + h * kHalf14;
+#pragma unroll
+            for (int r = 0; r < A; ++r) {
+                c[r] = half[st.own + 64u * r];
+            }
+            e += st.hamiltonian_of(job.base.field, 0u, c, lam, half,
+                                   job.psi + (h ^ 1u) * kHalf14);
+            st.put(slot + kAll + h * kHalf14, lam);
+        }
+        e = wave_sum(e);
+        if (st.lane == 0) {
+            red[0][st.wave] = e;
+        }
+        S::sync();
+        if (t == 0) {
+            double acc = 0.0;
+            for (int w = 0; w < S::kWaves; ++w) {
+                acc += red[0][w];
+            }
+            *job.base.energy = acc;
+        }
+        S::sync();
+        if (job.base.grad == nullptr) {
+            continue;
+        }
+        const double gscale = job.base.scale != nullptr ? *job.base.scale : 1.0;
+        RecordRing<S::kRec> ring{slots, job.base.rec, L, 2 * L, st.wave == 0,
+                                 2 * min(t & 63, S::kRec / 2 - 1), L};
+        ring.start();
+        S::sync();
+        // One half through the inverse ring CNOT: with kTop the top wire's RY of
+        // the layer before (tangent tt) comes off on the way; returns this
+        // lane's share of that wire's dtheta sum.
+        auto load = [&](auto first, auto rotate, uint32_t h, double tt) {
+            constexpr bool kFirst = decltype(first)::value;
+            constexpr bool kRotate = decltype(rotate)::value;
+            uint32_t base = (kFirst ? from1 : from2) ^
+                            (h != 0 ? source14<!kFirst>(kHalf14) : 0u);
+            asm volatile("" : "+v"(base));
+            double s = 0.0;
+#pragma unroll
+            for (int r = 0; r < A; ++r) {
+                const uint32_t o = base ^ source14<!kFirst>(64u * r);
+                c[r] = src_c[o];
+                lam[r] = src_l[o];
+                if constexpr (!kFirst) {
+                    const double sign = (o & kHalf14) ? -1.0 : 1.0;
+                    double2 pc = src_c[o ^ kHalf14];
+                    pc = make_double2(sign * pc.x, sign * pc.y);
+                    s += lam[r].x * pc.x + lam[r].y * pc.y;
+                    if constexpr (kRotate) {
+                        double2 pl = src_l[o ^ kHalf14];
+                        pl = make_double2(sign * pl.x, sign * pl.y);
+                        c[r] = S::rot_with(c[r], pc, tt);
+                        lam[r] = S::rot_with(lam[r], pl, tt);
+                    }
+                    if ((r & 7) == 7) {
+                        hold_schedule();
+                    }
+                }
+            }
+            return s;
+        };
+        auto put_top = [&](double s, double *sums) {
+            const double v = wave_sum(s);
+            if (st.lane == 0) {
+                sums[13] = v;
+            }
+        };
+        auto write_gradient = [&](int l, const double *rec, const double *sums, uint32_t f,
+                                  uint32_t k) {
+            if (t < 28) {
+                job.base.grad[(size_t)l * 28 + t] =
+                    RegState<14>::gradient_entry(t, rec, sums, f, k, false) * gscale;
+            }
+        };
+        const std::true_type yes;
+        const std::false_type no;
+        uint32_t f = 0;  // labels of the layer before (l + 1), and its flips and record
+        uint32_t k = 0;
+        const double *rec = nullptr;
+        int parity = 0;  // sums of the layer before
+        for (int l = L - 1; l >= 0; --l) {
+            const double *before = rec;
+            const uint32_t f_before = f;
+            const uint32_t k_before = k;
+            const int now = parity == 2 ? 0 : parity + 1;
+            rec = ring.advance();
+            k = S::flips(rec);
+            f = ring_inv_c(f, 14) ^ k;
+            for (uint32_t h = 0; h < 2; ++h) {
+                st.outer = h;
+                const uint32_t v = st.wave | (h << 3);
+                if (l == L - 1) {
+                    load(yes, no, h, 0.0);
+                } else {
+                    const typename S::Rec kb{before, f_before};
+                    const double s = load(no, yes, h, kb.t(13));
+                    put_top(s, red[parity] + 32 * v);
+                }
+                st.adjoint_layer<true, true>({rec, f}, c, lam, ex, red[now] + 32 * v);
+                st.put(next + h * kHalf14, c);
+                st.put(next + kAll + h * kHalf14, lam);
+            }
+            S::sync();
+            if (l < L - 1) {
+                write_gradient(l + 1, before, red[parity], f_before, k_before);
+            }
+            src_c = next;
+            src_l = next + kAll;
+            next = next == slot ? slot + 2 * kAll : slot;
+            parity = now;
+        }
+        for (uint32_t h = 0; h < 2; ++h) {
+            const uint32_t v = st.wave | (h << 3);
+            put_top(load(no, no, h, 0.0), red[parity] + 32 * v);
+        }
+        S::sync();
+        write_gradient(0, rec, red[parity], f, k);
+        S::sync();
+    }
+}
+
 namespace {
 
 template <int n>
 void launch_one(const RegJob *d_jobs, const RegJob &single, int count, hipStream_t s) {
     using S = RegState<n>;
-    const size_t bytes = sizeof(double2) * (size_t)S::kBuf * (n >= 12 ? 1 : 2);
+    const size_t bytes = S::kExchangeBytes * (n >= 12 ? 1 : 2);
     if constexpr (n <= kEngineWholeQubits) {
         if (single.drift != nullptr) {
             regcircuit_kernel<n, true><<<count, S::kThreads, bytes, s>>>(d_jobs, single);
@@ -303,6 +492,13 @@ void launch_regcircuit(int n, const RegJob *d_jobs, const RegJob &single, int co
         case 12: launch_one<12>(d_jobs, single, count, s); break;
         default: launch_one<13>(d_jobs, single, count, s); break;
     }
+}
+
+void launch_reg14(const Reg14Job *d_jobs, const Reg14Job &single, const int *d_order,
+                  const int *d_wg_begin, int count, int grid, double2 *scratch, hipStream_t s) {
+    reg14_forward_kernel<<<count, 1024, RegState<14>::kExchangeBytes, s>>>(d_jobs, single);
+    reg14_adjoint_kernel<<<grid, 512, RegState<13, 1>::kExchangeBytes, s>>>(
+        d_jobs, single, d_order, d_wg_begin, scratch);
 }
 
 }  // namespace rie

@@ -1,5 +1,6 @@
-// A whole n-qubit state (2 <= n <= 13) in the registers of one workgroup of
-// 2^W waves: the gates, permutations and inner products of one layer.
+// A whole n-qubit state in the registers of one workgroup of 2^W waves: the
+// gates, permutations and inner products of one layer (2 <= n <= 13; 14 for psi
+// alone, and for psi and lambda in two halves that differ in the top wire).
 //
 // Why registers: a layer rotates every wire, so a state kept in LDS is read
 // and written once per group of wires (three or four times a layer for psi
@@ -54,7 +55,7 @@ constexpr int kRecLb = 48;
 constexpr int kRecReg = 64;
 
 __host__ __device__ constexpr int reg_bits(int n) {
-    return n <= 6 ? 0 : n == 7 ? 1 : n <= 10 ? 2 : n == 11 ? 3 : 4;
+    return n <= 6 ? 0 : n == 7 ? 1 : n <= 10 ? 2 : n == 11 ? 3 : 4;  // 12..14: 4
 }
 __host__ __device__ constexpr int wave_bits(int n) { return n <= 8 ? 0 : n - 6 - reg_bits(n); }
 __host__ __device__ constexpr int record_doubles(int n) {
@@ -180,7 +181,8 @@ __host__ __device__ constexpr int adjoint_order(int w, int R) {
     return w >= 6 + R ? w : w >= 6 ? w - 6 : w < 4 ? R + w : w == 5 ? R + 4 : R + 5;
 }
 
-template <int n>
+// O = 1: one half (top wire n fixed, `outer`) of an (n + 1)-qubit state.
+template <int n, int O = 0>
 struct RegState {
     static constexpr int R = reg_bits(n);
     static constexpr int W = wave_bits(n);
@@ -188,11 +190,16 @@ struct RegState {
     static constexpr int kWaves = 1 << W;
     static constexpr int kThreads = 64 << W;
     static constexpr int kLaneWires = n < 6 ? n : 6;
-    static constexpr int kRec = record_doubles(n);
+    static constexpr int kRec = record_doubles(n + O);
     static constexpr uint32_t kAmps = 1u << n;
     // LDS amplitudes of one exchange buffer (lanes beyond 2^n use theirs too)
     static constexpr uint32_t kBuf = kAmps < 64u ? 64u : kAmps;
-    static_assert(n >= 2 && n <= kRegMaxQubits && W <= R, "register layouts");
+    // 256 KB at 14 qubits: the exchanges move re and im in turn
+    static constexpr bool kPlanes = n > kRegMaxQubits;
+    static constexpr size_t kExchangeBytes = (kPlanes ? 8 : 16) * (size_t)kBuf;
+    static_assert(n >= 2 && n <= 14 && W <= R, "register layouts");
+    static_assert(O == 0 || (n == 13 && reg_bits(14) == R && wave_bits(14) == W + 1),
+                  "halves of 14 qubits");
 
     // storage bit of wire w in layout 1 (w itself) and in layout 2
     static constexpr int pos2(int w) {
@@ -255,6 +262,7 @@ struct RegState {
     uint32_t own;    // storage position of r = 0
     uint32_t from[4];
     bool active;     // lane holds an amplitude (n < 6: lanes below 2^n)
+    uint32_t outer = 0;  // the half (O = 1)
 
     __device__ __forceinline__ void setup(uint32_t lane_, uint32_t wave_) {
         lane = lane_;
@@ -286,24 +294,73 @@ struct RegState {
         }
     }
 
-    template <int kind>
-    __device__ __forceinline__ void get(const double2 *buf, double2 (&a)[A]) const {
-        uint32_t base = from[kind];
-        // formed here each time: A addresses held across the layers would
-        // spill at 12 and 13 qubits
-        asm volatile("" : "+v"(base));
+    // kinds 0..3 (see image), 4: wave bits <-> the W low register bits
+    template <int kind, typename T, typename F>
+    __device__ __forceinline__ void read(const T *buf, F &&store) const {
+        if constexpr (kind < 4) {
+            uint32_t base = from[kind];
+            // formed here each time: A addresses held across the layers would
+            // spill at 12 and 13 qubits
+            asm volatile("" : "+v"(base));
 #pragma unroll
-        for (int r = 0; r < A; ++r) {
-            a[r] = buf[base ^ image(kind, 64u * r)];
+            for (int r = 0; r < A; ++r) {
+                store(r, buf[base ^ image(kind, 64u * r)]);
+            }
+        } else {
+            constexpr uint32_t m = (1u << W) - 1u;
+#pragma unroll
+            for (uint32_t r = 0; r < (uint32_t)A; ++r) {
+                store((int)r, buf[lane + 64u * ((r & ~m) | wave) + 64u * A * (r & m)]);
+            }
         }
     }
 
-    // wave bits <-> the W low register bits
-    __device__ __forceinline__ void get_waves(const double2 *buf, double2 (&a)[A]) const {
-        constexpr uint32_t m = (1u << W) - 1u;
+    template <int kind>
+    __device__ __forceinline__ void get(const double2 *buf, double2 (&a)[A]) const {
+        read<kind>(buf, [&](int r, double2 v) { a[r] = v; });
+    }
+
+    // One array through LDS, after a barrier for earlier reads of buf.
+    template <int kind>
+    __device__ __forceinline__ void exchange(double2 *buf, double2 (&a)[A]) const {
+        if constexpr (kPlanes) {
+            double *plane = reinterpret_cast<double *>(buf);
+            sync();
 #pragma unroll
-        for (uint32_t r = 0; r < (uint32_t)A; ++r) {
-            a[r] = buf[lane + 64u * ((r & ~m) | wave) + 64u * A * (r & m)];
+            for (int r = 0; r < A; ++r) {
+                plane[own + 64u * r] = a[r].x;
+            }
+            sync();
+            read<kind>(plane, [&](int r, double v) { a[r].x = v; });
+            sync();
+#pragma unroll
+            for (int r = 0; r < A; ++r) {
+                plane[own + 64u * r] = a[r].y;
+            }
+            sync();
+            read<kind>(plane, [&](int r, double v) { a[r].y = v; });
+        } else {
+            sync();
+            put(buf, a);
+            sync();
+            get<kind>(buf, a);
+        }
+    }
+
+    // Two arrays, through one buffer in turn (kSplit) or two at once.
+    template <int kind, bool kSplit>
+    __device__ __forceinline__ void exchange2(double2 *buf, double2 (&a)[A],
+                                              double2 (&b)[A]) const {
+        if constexpr (kSplit) {
+            exchange<kind>(buf, a);
+            exchange<kind>(buf, b);
+        } else {
+            sync();
+            put(buf, a);
+            put(buf + kBuf, b);
+            sync();
+            get<kind>(buf, a);
+            get<kind>(buf + kBuf, b);
         }
     }
 
@@ -396,9 +453,10 @@ struct RegState {
         if constexpr (n > 3) {
             z = cmul(z, k.c(kRecLb + 2 * (int)(((x ^ k.f) >> 3) & 7u)));
         }
-        if constexpr (W > 0) {
-            constexpr uint32_t m = (1u << W) - 1u;
-            z = cmul(z, k.c(kRecReg + 2 * A + 2 * (int)(wave ^ ((k.f >> (6 + R)) & m))));
+        if constexpr (W + O > 0) {
+            constexpr uint32_t m = (1u << (W + O)) - 1u;
+            const uint32_t v = wave | (outer << W);
+            z = cmul(z, k.c(kRecReg + 2 * A + 2 * (int)(v ^ ((k.f >> (6 + R)) & m))));
         }
         return z;
     }
@@ -438,10 +496,7 @@ struct RegState {
             for (int j = 0; j < W; ++j) {
                 rot_reg<false>(a, j, k.t(6 + R + j));
             }
-            sync();  // earlier reads of buf are done
-            put(buf, a);
-            sync();
-            get_waves(buf, a);
+            exchange<4>(buf, a);
         }
         if constexpr (R == 1) {
             rot_reg<false>(a, 0, k.t(4));
@@ -654,21 +709,7 @@ struct RegState {
             }
         }
         if constexpr (W > 0) {
-            sync();
-            put(buf, c);
-            if constexpr (kSplit) {
-                sync();
-                get_waves(buf, c);
-                sync();
-                put(buf, l);
-                sync();
-                get_waves(buf, l);
-            } else {
-                put(buf + kBuf, l);
-                sync();
-                get_waves(buf, c);
-                get_waves(buf + kBuf, l);
-            }
+            exchange2<4, kSplit>(buf, c, l);
 #pragma unroll
             for (int j = 0; j < W; ++j) {
                 reg_wire(j, 6 + R + j);
@@ -718,6 +759,15 @@ struct RegState {
         sync();
         put(buf, c);
         sync();
+        return hamiltonian_of(field, f_mask, c, l, buf, nullptr);
+    }
+
+    // The same from a copy of psi in storage order (and, O = 1, of the other
+    // half's).
+    __device__ __forceinline__ double hamiltonian_of(double field, uint32_t f_mask,
+                                                     const double2 (&c)[A], double2 (&l)[A],
+                                                     const double2 *buf,
+                                                     const double2 *other) const {
         double e = 0.0;
 #pragma unroll
         for (int r = 0; r < A; ++r) {
@@ -750,8 +800,12 @@ struct RegState {
             for (int j = 0; j < W; ++j) {
                 add(buf[(own ^ ((uint32_t)(64 * A) << j)) + 64u * r]);
             }
-            const uint32_t i = (x | ((uint32_t)r << 6) | (wave << (6 + R))) ^ f_mask;
-            const double d = ham_diag((uint64_t)i, n);
+            if constexpr (O > 0) {
+                add(other[own + 64u * r]);
+            }
+            const uint32_t i =
+                (x | ((uint32_t)r << 6) | (wave << (6 + R)) | (outer << n)) ^ f_mask;
+            const double d = ham_diag((uint64_t)i, n + O);
             l[r] = make_double2(d * c[r].x - field * f.x, d * c[r].y - field * f.y);
             if (!active) {
                 l[r] = make_double2(0.0, 0.0);

@@ -116,9 +116,8 @@ rie_status rie_energy_and_grad(size_t num_qubits, size_t num_layers, double fiel
  * whole circuit in one workgroup).  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  It calls no
- * hipMalloc, hipFree or allocating library routine: the layers' records (n <=
- * 13) or the coefficient table and state scratch (n = 14) live in a file-scope
- * device array of
+ * hipMalloc, hipFree or allocating library routine: the layers' records and
+ * the state scratch (n = 14) live in a file-scope device array of
  * RIE_NOALLOC_SCRATCH_BYTES per device, held until the process ends.  Every
  * call on a device shares that array, so calls that overlap on one device
  * race; serialize them (one stream, or wait between streams).
@@ -132,7 +131,7 @@ rie_status rie_energy_and_grad(size_t num_qubits, size_t num_layers, double fiel
 #define RIE_NOALLOC_MAX_QUBITS 14
 #define RIE_NOALLOC_MAX_LAYERS 1024
 #define RIE_NOALLOC_SCRATCH_BYTES \
-    (32u * RIE_NOALLOC_MAX_QUBITS * RIE_NOALLOC_MAX_LAYERS + 32u * (1u << RIE_NOALLOC_MAX_QUBITS))
+    (1024u * RIE_NOALLOC_MAX_LAYERS + 80u * (1u << RIE_NOALLOC_MAX_QUBITS))
 rie_status rie_energy_and_grad_noalloc(size_t num_qubits, size_t num_layers, double field,
                                        const double *d_params, size_t num_params,
                                        size_t structured_rotation_chunk_width,
@@ -394,14 +393,10 @@ rie_status rie_batch_run_per_circuit(rie_batch *batch, int compute_gradient, voi
 rie_status rie_batch_optimize(rie_batch *batch, int optimizer, double learning_rate, size_t steps,
                               int use_graph, double *energy_history_out, void *stream);
 
-/* Autotuner: times the 14-qubit whole-circuit kernel for every workgroup size
- * (256/512/1024) and rotation-chunk width (1..4) (fewer qubits have one shape
- * per qubit count), then, for
- * each split of the circuits between dense_scan (num_qubits <= s) and the
- * whole-circuit kernel, s from the dense_max_qubits given at creation down to
- * 0 (see rie_batch_set_tune_split), the share of CUs given to the 14-qubit
- * launch; keeps the fastest whole evaluation
- * and rebuilds the schedule with the measured costs.  The reference fixes the
+/* Autotuner: for each split of the circuits between dense_scan (num_qubits <=
+ * s) and the whole-circuit kernels, s from the dense_max_qubits given at creation
+ * down to 0 (see rie_batch_set_tune_split), and each share of the CUs for the
+ * 14-qubit adjoint launch, times the whole evaluation and keeps the fastest.  The reference fixes the
  * strategy per call and its kernel shapes by qubit-count thresholds
  * (cpp/ising_cuda_rotation_kernels.cu:562-575). */
 rie_status rie_batch_autotune(rie_batch *batch, size_t repeats);
@@ -412,9 +407,9 @@ rie_status rie_batch_set_tune_split(rie_batch *batch, int enabled);
 /* Manual configuration: threads 256/512/1024; chunk_by_n (15 values,
  * indexed by num_qubits, each 1..4) or NULL to keep; dense_tile 32/64;
  * structured_grid = workgroups of the persistent launch (0: one per CU).
- * Threads, chunks and grid shape the 14-qubit launch; circuits of fewer
- * qubits run in registers, and the product tree has one tile shape, so
- * dense_tile is only reported. */
+ * structured_grid bounds the 14-qubit adjoint launch.  The kernels have one
+ * shape per qubit count: threads, chunk_by_n and dense_tile are checked and
+ * reported, nothing more. */
 rie_status rie_batch_set_config(rie_batch *batch, int threads, const int *chunk_by_n,
                                 size_t chunk_len, int dense_tile, int structured_grid);
 /* Current configuration and the last autotuning measurements as JSON. */

@@ -1,4 +1,4 @@
-"""Whole-circuit kernels with the state in registers (2..13 qubits).
+"""Whole-circuit kernels with the state in registers (2..13 qubits; 14 in halves).
 
 Each qubit count has its own layout (register, lane and wave wires) and its own
 unrolled layer, so every one is checked against the FP64 CPU oracle: one, two
@@ -32,7 +32,7 @@ def _params(kind, layers, n, rng):
     return p
 
 
-@pytest.mark.parametrize("n", range(2, 14))
+@pytest.mark.parametrize("n", range(2, 15))
 def test_every_layout_matches_oracle(oracle, n):
     rng = np.random.default_rng([9, n])
     specs, params = [], []
@@ -49,6 +49,22 @@ def test_every_layout_matches_oracle(oracle, n):
         e_ref, g_ref = oracle.energy_and_grad(n, s.layers, s.field, p)
         assert abs(e - e_ref) <= TOL, (n, s.layers)
         assert np.max(np.abs(np.ravel(g) - np.ravel(g_ref))) <= TOL, (n, s.layers)
+
+
+def test_fourteen_qubit_circuits_share_workgroups(oracle):
+    # more circuits than workgroups of the adjoint launch: each workgroup takes
+    # several of different depths in turn, on one scratch
+    specs = [CircuitSpec(14, layers, 0.4 + 0.1 * layers) for layers in (5, 1, 2, 4, 1, 3, 2)]
+    rng = np.random.default_rng(11)
+    params = [_params("generic", s.layers, 14, rng) for s in specs]
+    batch = RingIsingBatch(specs)
+    batch.native.set_config(512, None, 64, 3)
+    print("case 14 qubits, 7 circuits on 3 workgroups", flush=True)
+    energies, grads = batch.energy_and_grad(params)
+    for s, p, e, g in zip(specs, params, energies, grads):
+        e_ref, g_ref = oracle.energy_and_grad(14, s.layers, s.field, p)
+        assert abs(e - e_ref) <= TOL, s
+        assert np.max(np.abs(np.ravel(g) - np.ravel(g_ref))) <= TOL, s
 
 
 @pytest.mark.parametrize("n", [2, 5, 6, 7, 8, 9, 11, 12])
