@@ -220,13 +220,22 @@ constexpr int kMlpEpiNone = 0;      // C = op(A) op(B)
 constexpr int kMlpEpiBias = 1;      // C = A B + bias
 constexpr int kMlpEpiBiasGelu = 2;  // C = Z = A B + bias, act = GELU(Z)
 constexpr int kMlpEpiDGelu = 3;     // C = (A B^T) * GELU'(zin)
-// ta: A is stored K x M (use A^T); tb: B is stored N x K (use B^T).
-// Supported: (ta, tb) = (0, 0) with None/Bias/BiasGelu, (0, 1) with None/DGelu, (1, 0) None.
-void launch_mlp_gemm(bool ta, bool tb, int epi, const float *A, const float *B, float *C, int M,
-                     int N, int K, const float *bias, float *act, const float *zin, hipStream_t s);
-void launch_mlp_colsum(const float *X, int rows, int cols, float *out, hipStream_t s);
-void launch_mlp_mse(const float *Y, const float *T, int count, float *dY, float *partials,
-                    int blocks, float *loss_out, hipStream_t s);
+constexpr int kMlpEpiMse = 4;       // C = scale (A B + bias - targets), squares summed
+// Z = X W + bias (rows x cols, X: rows x K), act = GELU(Z) unless null.
+void launch_mlp_forward(const float *X, const float *W, const float *bias, float *Z, float *act,
+                        int rows, int cols, int K, hipStream_t s);
+// dY = 2 (X W + bias - T) / (rows cols), loss = mean of the squares; partials
+// holds mlp_mse_partials(rows, cols) values.
+void launch_mlp_output_loss(const float *X, const float *W, const float *bias, const float *T,
+                            float *dY, int rows, int cols, int K, float *partials,
+                            float *loss_out, hipStream_t s);
+size_t mlp_mse_partials(int rows, int cols);
+// dZ = (dY W^T) * GELU'(Z) (rows x cols; dY: rows x K, W: cols x K).
+void launch_mlp_backward_data(const float *dY, const float *W, const float *Z, float *dZ, int rows,
+                              int cols, int K, hipStream_t s);
+// dW = X^T dY (in x cols) and, right behind it, db = the column sums of dY.
+void launch_mlp_backward_weights(const float *X, const float *dY, float *dWb, int in, int cols,
+                                 int rows, hipStream_t s);
 void launch_mlp_adam(float *p, const float *g, float *m, float *v, int count, float lr, float b1,
                      float b2, float eps, int t, hipStream_t s);
 

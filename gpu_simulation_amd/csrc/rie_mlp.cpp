@@ -43,12 +43,12 @@ struct Mlp {
     float *d_dy = nullptr, *d_d2 = nullptr, *d_d1 = nullptr;
     float *d_partials = nullptr;
     float *d_loss = nullptr;
-    int mse_blocks = 0;
 
     void ensure_rows(int rows);
     void upload_rows(const float *x, const float *t, int rows);
-    void forward(int rows);
-    void backward(int rows);  // after forward; loss into d_loss, gradient into d_g
+    void hidden_layers(int rows);
+    void forward(int rows);  // outputs into d_y
+    void loss_and_grad(int rows, float *loss_out);  // device pointer; gradient into d_g
     void free_rows();
 };
 
@@ -128,8 +128,8 @@ void Mlp::ensure_rows(int rows) {
     d_dy = (float *)device_alloc(sizeof(float) * r * out, "alloc MLP rows");
     d_d2 = (float *)device_alloc(sizeof(float) * r * hidden, "alloc MLP rows");
     d_d1 = (float *)device_alloc(sizeof(float) * r * hidden, "alloc MLP rows");
-    mse_blocks = (int)std::min<size_t>(1024, (r * out + 255) / 256);
-    d_partials = (float *)device_alloc(sizeof(float) * mse_blocks, "alloc MLP partials");
+    d_partials = (float *)device_alloc(sizeof(float) * mlp_mse_partials(rows, out),
+                                       "alloc MLP partials");
     cap = rows;
 }
 
@@ -143,36 +143,29 @@ void Mlp::upload_rows(const float *x, const float *t, int rows) {
     }
 }
 
+void Mlp::hidden_layers(int rows) {
+    launch_mlp_forward(d_x, d_p + o_w1, d_p + o_b1, d_z1, d_a1, rows, hidden, in, s);
+    launch_mlp_forward(d_a1, d_p + o_w2, d_p + o_b2, d_z2, d_a2, rows, hidden, hidden, s);
+}
+
 void Mlp::forward(int rows) {
-    launch_mlp_gemm(false, false, kMlpEpiBiasGelu, d_x, d_p + o_w1, d_z1, rows, hidden, in,
-                    d_p + o_b1, d_a1, nullptr, s);
-    launch_mlp_gemm(false, false, kMlpEpiBiasGelu, d_a1, d_p + o_w2, d_z2, rows, hidden, hidden,
-                    d_p + o_b2, d_a2, nullptr, s);
-    launch_mlp_gemm(false, false, kMlpEpiBias, d_a2, d_p + o_w3, d_y, rows, out, hidden,
-                    d_p + o_b3, nullptr, nullptr, s);
+    hidden_layers(rows);
+    launch_mlp_forward(d_a2, d_p + o_w3, d_p + o_b3, d_y, nullptr, rows, out, hidden, s);
     check_launch("MLP forward");
 }
 
-void Mlp::backward(int rows) {
+void Mlp::loss_and_grad(int rows, float *loss_out) {
+    hidden_layers(rows);
     // loss = mean over all rows * out elements of (y - t)^2
-    launch_mlp_mse(d_y, d_t, rows * out, d_dy, d_partials, mse_blocks, d_loss, s);
-    // layer 3: dW3 = A2^T dY, db3 = colsum dY, dZ2 = (dY W3^T) * GELU'(Z2)
-    launch_mlp_gemm(true, false, kMlpEpiNone, d_a2, d_dy, d_g + o_w3, hidden, out, rows, nullptr,
-                    nullptr, nullptr, s);
-    launch_mlp_colsum(d_dy, rows, out, d_g + o_b3, s);
-    launch_mlp_gemm(false, true, kMlpEpiDGelu, d_dy, d_p + o_w3, d_d2, rows, hidden, out, nullptr,
-                    nullptr, d_z2, s);
-    // layer 2
-    launch_mlp_gemm(true, false, kMlpEpiNone, d_a1, d_d2, d_g + o_w2, hidden, hidden, rows,
-                    nullptr, nullptr, nullptr, s);
-    launch_mlp_colsum(d_d2, rows, hidden, d_g + o_b2, s);
-    launch_mlp_gemm(false, true, kMlpEpiDGelu, d_d2, d_p + o_w2, d_d1, rows, hidden, hidden,
-                    nullptr, nullptr, d_z1, s);
-    // layer 1
-    launch_mlp_gemm(true, false, kMlpEpiNone, d_x, d_d1, d_g + o_w1, in, hidden, rows, nullptr,
-                    nullptr, nullptr, s);
-    launch_mlp_colsum(d_d1, rows, hidden, d_g + o_b1, s);
-    check_launch("MLP backward");
+    launch_mlp_output_loss(d_a2, d_p + o_w3, d_p + o_b3, d_t, d_dy, rows, out, hidden, d_partials,
+                           loss_out, s);
+    // the packed gradient holds each bias right behind its weights
+    launch_mlp_backward_weights(d_a2, d_dy, d_g + o_w3, hidden, out, rows, s);
+    launch_mlp_backward_data(d_dy, d_p + o_w3, d_z2, d_d2, rows, hidden, out, s);
+    launch_mlp_backward_weights(d_a1, d_d2, d_g + o_w2, hidden, hidden, rows, s);
+    launch_mlp_backward_data(d_d2, d_p + o_w2, d_z1, d_d1, rows, hidden, hidden, s);
+    launch_mlp_backward_weights(d_x, d_d1, d_g + o_w1, in, hidden, rows, s);
+    check_launch("MLP loss and gradient");
 }
 
 }  // namespace rie
@@ -265,8 +258,7 @@ rie_status rie_mlp_loss_and_grad(rie_mlp *mlp, const float *inputs, const float 
             rie::fail(RIE_INVALID_ARGUMENT, "null pointer argument.");
         }
         m->upload_rows(inputs, targets, rows);
-        m->forward(rows);
-        m->backward(rows);
+        m->loss_and_grad(rows, m->d_loss);
         rie::check(hipMemcpyAsync(loss_out, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->s),
                    "download loss");
         if (grad_out != nullptr) {
@@ -298,13 +290,7 @@ rie_status rie_mlp_train(rie_mlp *mlp, const float *inputs, const float *targets
         }
         try {
             for (int t = 1; t <= steps; ++t) {
-                m->forward(rows);
-                m->backward(rows);
-                if (d_hist != nullptr) {
-                    rie::check(hipMemcpyAsync(d_hist + (t - 1), m->d_loss, sizeof(float),
-                                              hipMemcpyDeviceToDevice, m->s),
-                               "record loss");
-                }
+                m->loss_and_grad(rows, d_hist != nullptr ? d_hist + (t - 1) : m->d_loss);
                 rie::launch_mlp_adam(m->d_p, m->d_g, m->d_m, m->d_v, (int)m->count,
                                      learning_rate, 0.9f, 0.999f, 1e-8f, t, m->s);
                 rie::check_launch("MLP adam");

@@ -2,15 +2,25 @@
 // (forward, backward, Adam) and inference of x -> GELU(x W1 + b1) ->
 // GELU(. W2 + b2) -> . W3 + b3, all row-major with one sample per row.
 //
-// No counterpart in the reference.  The GEMMs are small (a few thousand rows
-// by 256), so one LDS-tiled FP32 kernel with fused epilogues serves every
-// product of the forward and backward pass:
+// No counterpart in the reference.  One GEMM on the FP32 matrix cores with
+// fused epilogues serves every product of the forward and backward pass:
 //   forward  Z = X W + b, A = GELU(Z)           (epilogue kBiasGelu / kBias)
+//   loss     dY = 2 / count (X W + b - T) and its squares (epilogue kMse)
 //   backward dA = dZn W^T, dZ = dA * GELU'(Z)     (transposed B, epilogue kDGelu)
-//            dW = A^T dZ                          (transposed A)
+//            [dW; db] = [A 1]^T dZ                (transposed A with a row of ones)
 // GELU is the exact form 0.5 x (1 + erf(x / sqrt 2)) (torch.nn.GELU's
 // default), evaluated with the device library's erff / expf.
+//
+// The products are small (a few hundred to a few thousand rows by 256), so what
+// bounds them is the number of workgroups and the chain over k: a workgroup
+// forms a 16 x 16 (or, from 512 such blocks of 32 x 32 on, 32 x 32) tile, its four
+// waves split k, and operands come straight from L2.  512 rows, 3-256-256-80: 842
+// us a loss and gradient through the host-array call with 64 x 64 LDS tiles (8 to
+// 32 workgroups), a column sum per bias in one thread per column (3 x 95 us) and
+// a serial loss sum; 135 us now.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "rie_kernels.hpp"
 
@@ -18,8 +28,7 @@ namespace rie {
 
 namespace {
 
-constexpr int kTile = 64;
-constexpr int kTK = 16;
+typedef float float4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float gelu(float x) {
     return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
@@ -33,154 +42,170 @@ __device__ __forceinline__ float gelu_grad(float x) {
 
 }  // namespace
 
-// C[M x N] = op(A)[M x K] * op(B)[K x N]; op(A) = A (M x K, lda) or A^T (A is
-// K x M); op(B) = B (K x N) or B^T (B is N x K).  256 threads, 4 x 4 outputs
-// each over a 64 x 64 tile.
-template <bool kTA, bool kTB, int kEpi>
-__global__ __launch_bounds__(256) void mlp_gemm_kernel(const float *__restrict__ A,
-                                                       const float *__restrict__ B,
-                                                       float *__restrict__ C, int M, int N, int K,
-                                                       const float *__restrict__ bias,
-                                                       float *__restrict__ act,
-                                                       const float *__restrict__ zin) {
-    __shared__ float as[kTK][kTile + 1];  // as[k][m]
-    __shared__ float bs[kTK][kTile + 1];  // bs[k][n]
+// C[M x N] = op(A)[M x K] * op(B)[K x N]; op(A) = A (M x K) or A^T (A is K x
+// Ma; row Ma of A^T, if M > Ma, is ones); op(B) = B (K x N) or B^T (B is N x K).
+// v_mfma_f32_16x16x4f32 lane layout: A[i][k] in lane i + 16k, B[k][j] in lane
+// j + 16k, D[4(lane / 16) + e][lane % 16] in element e.  A lane (i, g) holds k =
+// 4g .. 4g + 3 of a block of 16, one k per MFMA step, so an operand stored along
+// k is one 16-byte load (where its rows are 16-byte aligned: wide_a, wide_b).
+struct MlpGemm {
+    const float *A;
+    const float *B;
+    float *C;
+    int M;
+    int N;
+    int K;
+    int Ma;             // rows of A^T that A holds
+    int wide_a;
+    int wide_b;
+    const float *bias;
+    float *act;         // kBiasGelu: GELU(C)
+    const float *zin;   // kDGelu: Z; kMse: the targets
+    float *partials;    // kMse: a sum of squares per workgroup
+    float scale;        // kMse: 2 / count
+};
+
+template <bool kTA, bool kTB, int kEpi, int kSub>
+__global__ __launch_bounds__(256) void mlp_gemm_kernel(MlpGemm g) {
+    __shared__ float part[4][kSub * kSub][4][64];
+    __shared__ float red[4];
     const int t = threadIdx.x;
-    const int tm = (t / 16) * 4;
-    const int tn = (t % 16) * 4;
-    const int m0 = blockIdx.y * kTile;
-    const int n0 = blockIdx.x * kTile;
-    float acc[4][4];
+    const int lane = t & 63;
+    const int wave = t >> 6;
+    const int i = lane & 15;
+    const int q = lane >> 4;
+    const int m0 = blockIdx.y * 16 * kSub;
+    const int n0 = blockIdx.x * 16 * kSub;
+    float4_t acc[kSub][kSub];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int a = 0; a < kSub; ++a) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            acc[i][j] = 0.0f;
+        for (int b = 0; b < kSub; ++b) {
+            acc[a][b] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
         }
     }
-    for (int k0 = 0; k0 < K; k0 += kTK) {
-        for (int e = t; e < kTK * kTile; e += 256) {
-            const int kk = e / kTile;
-            const int mm = e % kTile;
-            const int gm = m0 + mm;
-            const int gk = k0 + kk;
-            float va = 0.0f;
-            if (gm < M && gk < K) {
-                va = kTA ? A[(size_t)gk * M + gm] : A[(size_t)gm * K + gk];
+    // four consecutive k of row (of the stored operand) r
+    auto along_k = [](const float *p, int r, int rows, int K, int k, bool wide, float (&v)[4]) {
+        if (r >= rows) {
+            v[0] = v[1] = v[2] = v[3] = 0.0f;
+        } else if (wide && k + 3 < K) {
+            const float4 x = *reinterpret_cast<const float4 *>(p + (size_t)r * K + k);
+            v[0] = x.x;
+            v[1] = x.y;
+            v[2] = x.z;
+            v[3] = x.w;
+        } else {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                v[m] = k + m < K ? p[(size_t)r * K + k + m] : 0.0f;
             }
-            as[kk][mm] = va;
-            const int gn = n0 + mm;
-            float vb = 0.0f;
-            if (gn < N && gk < K) {
-                vb = kTB ? B[(size_t)gn * K + gk] : B[(size_t)gk * N + gn];
-            }
-            bs[kk][mm] = vb;
         }
-        __syncthreads();
+    };
+    // column c of four consecutive rows k
+    auto down_k = [](const float *p, int c, int cols, int K, int k, float (&v)[4]) {
 #pragma unroll
-        for (int kk = 0; kk < kTK; ++kk) {
-            float a[4];
-            float b[4];
+        for (int m = 0; m < 4; ++m) {
+            v[m] = (c < cols && k + m < K) ? p[(size_t)(k + m) * cols + c] : 0.0f;
+        }
+    };
+#pragma unroll 2
+    for (int k0 = 16 * wave; k0 < g.K; k0 += 64) {
+        const int k = k0 + 4 * q;
+        float fa[kSub][4];
+        float fb[kSub][4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = as[kk][tm + i];
-                b[i] = bs[kk][tn + i];
+        for (int s = 0; s < kSub; ++s) {
+            const int row = m0 + 16 * s + i;
+            const int col = n0 + 16 * s + i;
+            if constexpr (kTA) {
+                down_k(g.A, row, g.Ma, g.K, k, fa[s]);
+                if (row == g.Ma) {
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        fa[s][m] = k + m < g.K ? 1.0f : 0.0f;
+                    }
+                }
+            } else {
+                along_k(g.A, row, g.M, g.K, k, g.wide_a != 0, fa[s]);
             }
+            if constexpr (kTB) {
+                along_k(g.B, col, g.N, g.K, k, g.wide_b != 0, fb[s]);
+            } else {
+                down_k(g.B, col, g.N, g.K, k, fb[s]);
+            }
+        }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+        for (int m = 0; m < 4; ++m) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+            for (int a = 0; a < kSub; ++a) {
+#pragma unroll
+                for (int b = 0; b < kSub; ++b) {
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[a][m], fb[b][m],
+                                                                     acc[a][b], 0, 0, 0);
                 }
             }
         }
-        __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gm = m0 + tm + i;
-        if (gm >= M) {
+    for (int s = 0; s < kSub * kSub; ++s) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            part[wave][s][e][lane] = acc[s / kSub][s % kSub][e];
+        }
+    }
+    __syncthreads();
+    float squares = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kSub * kSub; ++s) {
+        // wave w finishes element w of every lane
+        const int e = wave;
+        float v = (part[0][s][e][lane] + part[1][s][e][lane]) +
+                  (part[2][s][e][lane] + part[3][s][e][lane]);
+        const int gm = m0 + 16 * (s / kSub) + 4 * q + e;
+        const int gn = n0 + 16 * (s % kSub) + i;
+        if (gm >= g.M || gn >= g.N) {
             continue;
         }
+        const size_t o = (size_t)gm * g.N + gn;
+        if (kEpi == kMlpEpiBias || kEpi == kMlpEpiBiasGelu || kEpi == kMlpEpiMse) {
+            v += g.bias[gn];
+        }
+        if (kEpi == kMlpEpiDGelu) {
+            v *= gelu_grad(g.zin[o]);
+        }
+        if (kEpi == kMlpEpiMse) {
+            const float d = v - g.zin[o];
+            squares += d * d;
+            v = g.scale * d;
+        }
+        g.C[o] = v;
+        if (kEpi == kMlpEpiBiasGelu) {
+            g.act[o] = gelu(v);
+        }
+    }
+    if constexpr (kEpi == kMlpEpiMse) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int gn = n0 + tn + j;
-            if (gn >= N) {
-                continue;
-            }
-            const size_t o = (size_t)gm * N + gn;
-            float v = acc[i][j];
-            if (kEpi == kMlpEpiBias || kEpi == kMlpEpiBiasGelu) {
-                v += bias[gn];
-            }
-            if (kEpi == kMlpEpiDGelu) {
-                v *= gelu_grad(zin[o]);
-            }
-            C[o] = v;
-            if (kEpi == kMlpEpiBiasGelu) {
-                act[o] = gelu(v);
-            }
+        for (int off = 32; off > 0; off >>= 1) {
+            squares += __shfl_xor(squares, off, 64);
+        }
+        if (lane == 0) {
+            red[wave] = squares;
+        }
+        __syncthreads();
+        if (t == 0) {
+            g.partials[blockIdx.y * gridDim.x + blockIdx.x] =
+                (red[0] + red[1]) + (red[2] + red[3]);
         }
     }
 }
 
-void launch_mlp_gemm(bool ta, bool tb, int epi, const float *A, const float *B, float *C, int M,
-                     int N, int K, const float *bias, float *act, const float *zin,
-                     hipStream_t s) {
-    dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
-#define RIE_MLP_GEMM(TA, TB, EPI)                                                           \
-    mlp_gemm_kernel<TA, TB, EPI><<<grid, 256, 0, s>>>(A, B, C, M, N, K, bias, act, zin)
-    if (!ta && !tb) {
-        if (epi == kMlpEpiBias) {
-            RIE_MLP_GEMM(false, false, kMlpEpiBias);
-        } else if (epi == kMlpEpiBiasGelu) {
-            RIE_MLP_GEMM(false, false, kMlpEpiBiasGelu);
-        } else {
-            RIE_MLP_GEMM(false, false, kMlpEpiNone);
-        }
-    } else if (!ta && tb) {
-        if (epi == kMlpEpiDGelu) {
-            RIE_MLP_GEMM(false, true, kMlpEpiDGelu);
-        } else {
-            RIE_MLP_GEMM(false, true, kMlpEpiNone);
-        }
-    } else {
-        RIE_MLP_GEMM(true, false, kMlpEpiNone);
-    }
-#undef RIE_MLP_GEMM
-}
-
-// out[j] = sum_i X[i][j] over rows (fixed order: one thread per column,
-// rows in order), for bias gradients.
-__global__ void mlp_colsum_kernel(const float *__restrict__ X, int rows, int cols,
-                                  float *__restrict__ out) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= cols) {
-        return;
-    }
-    float acc = 0.0f;
-    for (int i = 0; i < rows; ++i) {
-        acc += X[(size_t)i * cols + j];
-    }
-    out[j] = acc;
-}
-
-void launch_mlp_colsum(const float *X, int rows, int cols, float *out, hipStream_t s) {
-    mlp_colsum_kernel<<<(cols + 127) / 128, 128, 0, s>>>(X, rows, cols, out);
-}
-
-// dY = (2 / count) (Y - T) and per-block partial sums of (Y - T)^2.
-__global__ __launch_bounds__(256) void mlp_mse_kernel(const float *__restrict__ Y,
-                                                      const float *__restrict__ T, int count,
-                                                      float *__restrict__ dY,
-                                                      float *__restrict__ partials) {
+// loss = sum of the workgroups' squares / count, in a fixed order.
+__global__ __launch_bounds__(256) void mlp_loss_kernel(const float *__restrict__ partials, int n,
+                                                       int count, float *__restrict__ loss_out) {
     __shared__ float red[4];
     float acc = 0.0f;
-    const float scale = 2.0f / (float)count;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-        const float d = Y[i] - T[i];
-        dY[i] = scale * d;
-        acc += d * d;
+    for (int i = threadIdx.x; i < n; i += 256) {
+        acc += partials[i];
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -191,25 +216,78 @@ __global__ __launch_bounds__(256) void mlp_mse_kernel(const float *__restrict__ 
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        partials[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+        loss_out[0] = ((red[0] + red[1]) + (red[2] + red[3])) / (float)count;
     }
 }
 
-__global__ void mlp_loss_kernel(const float *__restrict__ partials, int n, int count,
-                                float *__restrict__ loss_out) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        float acc = 0.0f;
-        for (int i = 0; i < n; ++i) {
-            acc += partials[i];
-        }
-        loss_out[0] = acc / (float)count;
+namespace {
+
+// 32 x 32 tiles read each operand half as often; below 512 of them the chip has
+// idle CUs and the shorter tiles win.
+constexpr int kWideTiles = 512;
+
+int sub_for(int M, int N) {
+    return (long)((M + 31) / 32) * ((N + 31) / 32) >= kWideTiles ? 2 : 1;
+}
+
+template <bool kTA, bool kTB, int kEpi>
+void gemm(const MlpGemm &g, hipStream_t s) {
+    const int sub = sub_for(g.M, g.N);
+    const int tile = 16 * sub;
+    dim3 grid((g.N + tile - 1) / tile, (g.M + tile - 1) / tile);
+    if (sub == 2) {
+        mlp_gemm_kernel<kTA, kTB, kEpi, 2><<<grid, 256, 0, s>>>(g);
+    } else {
+        mlp_gemm_kernel<kTA, kTB, kEpi, 1><<<grid, 256, 0, s>>>(g);
     }
 }
 
-void launch_mlp_mse(const float *Y, const float *T, int count, float *dY, float *partials,
-                    int blocks, float *loss_out, hipStream_t s) {
-    mlp_mse_kernel<<<blocks, 256, 0, s>>>(Y, T, count, dY, partials);
-    mlp_loss_kernel<<<1, 64, 0, s>>>(partials, blocks, count, loss_out);
+bool wide_rows(const float *p, int ld) {
+    return ld % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+}
+
+}  // namespace
+
+size_t mlp_mse_partials(int rows, int cols) {
+    // the 16 x 16 grid of fewer rows may be the larger one
+    const size_t wide = (size_t)((rows + 31) / 32) * ((cols + 31) / 32);
+    return std::max<size_t>(wide, 4 * (size_t)kWideTiles + (size_t)(cols + 15) / 16 * 2 +
+                                      (size_t)(rows + 15) / 16 * 2);
+}
+
+void launch_mlp_forward(const float *X, const float *W, const float *bias, float *Z, float *act,
+                        int rows, int cols, int K, hipStream_t s) {
+    MlpGemm g{X, W, Z, rows, cols, K, 0, wide_rows(X, K), 0, bias, act, nullptr, nullptr, 0.0f};
+    if (act != nullptr) {
+        gemm<false, false, kMlpEpiBiasGelu>(g, s);
+    } else {
+        gemm<false, false, kMlpEpiBias>(g, s);
+    }
+}
+
+void launch_mlp_output_loss(const float *X, const float *W, const float *bias, const float *T,
+                            float *dY, int rows, int cols, int K, float *partials,
+                            float *loss_out, hipStream_t s) {
+    const int count = rows * cols;
+    MlpGemm g{X, W, dY, rows, cols, K, 0, wide_rows(X, K), 0, bias, nullptr, T, partials,
+              2.0f / (float)count};
+    gemm<false, false, kMlpEpiMse>(g, s);
+    const int tile = 16 * sub_for(rows, cols);
+    const int n = ((rows + tile - 1) / tile) * ((cols + tile - 1) / tile);
+    mlp_loss_kernel<<<1, 256, 0, s>>>(partials, n, count, loss_out);
+}
+
+void launch_mlp_backward_data(const float *dY, const float *W, const float *Z, float *dZ, int rows,
+                              int cols, int K, hipStream_t s) {
+    MlpGemm g{dY, W, dZ, rows, cols, K, 0, wide_rows(dY, K), wide_rows(W, K), nullptr, nullptr, Z,
+              nullptr, 0.0f};
+    gemm<false, true, kMlpEpiDGelu>(g, s);
+}
+
+void launch_mlp_backward_weights(const float *X, const float *dY, float *dWb, int in, int cols,
+                                 int rows, hipStream_t s) {
+    MlpGemm g{X, dY, dWb, in + 1, cols, rows, in, 0, 0, nullptr, nullptr, nullptr, nullptr, 0.0f};
+    gemm<true, false, kMlpEpiNone>(g, s);
 }
 
 // Adam on the packed FP32 parameters (torch.optim.Adam arithmetic), step t.
