@@ -7,8 +7,8 @@
 // dispatched in order, so a caller lists the deepest circuits first.
 //
 // Bound by the latency of one workgroup's dependent FP64 and lane moves: a
-// layer of one circuit, forward and back, takes 1.1 us at 4 qubits, 2.5 at 8,
-// 14 at 12 and 22 at 13 (128 layers).  Before, with psi and lambda in LDS (a
+// layer of one circuit, forward and back, takes 1.0 us at 4 qubits, 2.5 at 8,
+// 11 at 12 and 22 at 13 (128 layers).  Before, with psi and lambda in LDS (a
 // sweep per chunk of wires, one barrier each, pair indexes computed per group)
 // or at 13 qubits in L2: 8, 15, 23 and 102 us.
 #include <hip/hip_runtime.h>
