@@ -21,11 +21,35 @@ namespace rie {
 // Records: one wave per (circuit, layer).
 // ---------------------------------------------------------------------------
 
+// 1 / sqrt(product of 1 + t_w^2), the scale that the tangent forms of a layer
+// leave out (each wire's factor is +-1 / sqrt(1 + t^2)), and that product.  In
+// twice the precision and rounded once: a product of rounded factors would let
+// the norm drift by a few ulp a layer.
+__device__ __forceinline__ double layer_scale(const double *t, int n, double &product) {
+#pragma clang fp contract(off)
+    double ph = 1.0;
+    double pl = 0.0;
+    for (int w = 0; w < n; ++w) {
+        const double t2 = t[w] * t[w];
+        const double sh = 1.0 + t2;
+        const double sl = (t2 - (sh - 1.0)) + fma(t[w], t[w], -t2);
+        const double h = ph * sh;
+        const double l = fma(ph, sh, -h) + (ph * sl + pl * sh);
+        ph = h + l;
+        pl = (h - ph) + l;
+    }
+    const double r = 1.0 / sqrt(ph);
+    const double r2 = r * r;
+    const double q = r2 * ph;
+    const double left = ((1.0 - q) - fma(r2, ph, -q)) - (fma(r, r, -r2) * ph + r2 * pl);
+    product = ph;
+    return r + 0.5 * r * left;
+}
+
 __global__ __launch_bounds__(256) void circuit_records_kernel(const RecordJob *__restrict__ jobs,
                                                               RecordJob single,
                                                               const int *__restrict__ layer_job,
                                                               int total_layers) {
-    __shared__ double sh_f[4][16];
     __shared__ double sh_t[4][16];
     __shared__ double2 sh_e[4][16];
     const int lane = threadIdx.x & 63;
@@ -41,13 +65,15 @@ __global__ __launch_bounds__(256) void circuit_records_kernel(const RecordJob *_
     const int W = wave_bits(n);
     const double *p = job.params + (size_t)l * 2 * n;
     bool flip = false;
+    bool negative = false;  // the factor cos or sin taken out
     if (lane < n) {
         double c;
         double s;
         sincos(0.5 * p[2 * lane], &s, &c);
         flip = fabs(s) > fabs(c);
-        sh_f[wave][lane] = flip ? s : c;
-        sh_t[wave][lane] = flip ? -c / s : s / c;
+        const double tangent = flip ? -c / s : s / c;
+        sh_t[wave][lane] = tangent;
+        negative = (flip ? s : c) < 0.0;
         double2 e;
         sincos(p[2 * lane + 1], &e.y, &e.x);
         // phase of logical bit 1: e, or with the flip's Z (diag(e, -1), its
@@ -55,14 +81,14 @@ __global__ __launch_bounds__(256) void circuit_records_kernel(const RecordJob *_
         sh_e[wave][lane] = flip ? make_double2(-e.x, e.y) : e;
     }
     const uint64_t flips = __ballot(flip);
+    const bool odd = (__popcll(__ballot(negative)) & 1) != 0;
     wave_lds_fence();
-    const double *f = sh_f[wave];
+    const double *tw = sh_t[wave];
     const double2 *e = sh_e[wave];
     double *rec = job.rec + (size_t)l * record_doubles(n);
-    double sigma = 1.0;
-    for (int w = 0; w < n; ++w) {
-        sigma *= f[w];
-    }
+    double ph;
+    double sigma = layer_scale(tw, n, ph);
+    sigma = odd ? -sigma : sigma;
     // phase tables: [first, first + count) wires of one entry's index bits
     int first = -1;
     int count = 0;
@@ -104,16 +130,13 @@ __global__ __launch_bounds__(256) void circuit_records_kernel(const RecordJob *_
         // when the adjoint sweep sums wire w's dtheta, both arrays still carry
         // the factors of w and of the wires after it in its order
         double g = 1.0;
-        if (w < n) {
-            double left = 1.0;
-            for (int v = 0; v < n; ++v) {
-                left *= adjoint_order(v, R) >= adjoint_order(w, R) ? f[v] : 1.0;
-            }
-            g = 1.0 / (left * left);
+        for (int v = 0; v < n; ++v) {
+            g *= w < n && adjoint_order(v, R) >= adjoint_order(w, R) ? fma(tw[v], tw[v], 1.0)
+                                                                      : 1.0;
         }
         double t = w < n ? sh_t[wave][w] : 0.0;
         if (w == kRecDphi) {
-            t = 1.0 / (sigma * sigma);
+            t = ph;
         } else if (w == kRecFlips) {
             t = (double)flips;
         }
