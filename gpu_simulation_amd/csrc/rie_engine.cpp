@@ -204,27 +204,36 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     check(hipEventCreate(&ev_b), "hipEventCreate");
     check(hipEventCreateWithFlags(&ev_last, hipEventDisableTiming), "hipEventCreate");
     build_plan();
+    // The gate-level strategy's results are those of the structured sweeps, so
+    // it runs on the same kernels; above kGateTileQubits, where their four state
+    // buffers and tables would take memory that two buffers leave free, gate by
+    // gate.  15 qubits x 2 layers through the host call: 849 us gate by gate
+    // (about 250 launches), 136 us on the tile passes.
+    const bool gate = strategy == RIE_STRATEGY_INVERSE_WALK_GATE;
+    whole = small && (gate || strategy == RIE_STRATEGY_STRUCTURED_ADJOINT);
+    on_tiles = !small && (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT ||
+                       (gate && n <= kGateTileQubits));
 
     d_params = (double *)device_alloc(sizeof(double) * num_params, "alloc params");
     d_grad = (double *)device_alloc(sizeof(double) * num_params, "alloc gradient");
     d_energy = (double *)device_alloc(sizeof(double) * 4, "alloc energy");
-    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+    if (whole) {
         // the whole circuit lives in one workgroup's registers
         d_rec = (double *)device_alloc(circuit_record_bytes(n, L), "alloc records");
     } else {
         d_coef = (WireCoef *)device_alloc(sizeof(WireCoef) * (size_t)n * L, "alloc coefficients");
     }
-    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+    if (whole) {
         // no state buffers
-    } else if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT) {
+    } else if (on_tiles) {
         // The stored schedule keeps every forward pass output; use it when it
         // fits comfortably in free device memory, else walk back by inverse gates.
         size_t free_b = 0;
         size_t total_b = 0;
         check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
         const double need = (double)stored_buffer_count() * (double)sizeof(double2) * (double)N;
-        schedule = (L > 1 && need <= 0.85 * (double)free_b) ? RIE_SCHEDULE_STORED
-                                                            : RIE_SCHEDULE_INVERSE_WALK;
+        schedule = (!gate && L > 1 && need <= 0.85 * (double)free_b) ? RIE_SCHEDULE_STORED
+                                                                     : RIE_SCHEDULE_INVERSE_WALK;
         ensure_pool(schedule == RIE_SCHEDULE_STORED ? stored_buffer_count() : 4);
         size_t part = 0;
         for (const auto &p : passes) {
@@ -716,7 +725,7 @@ bool Engine::gen_layouts() const {
 }
 
 bool Engine::gen_ready() const {
-    return gen_enabled && strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && !small && L >= 2 &&
+    return gen_enabled && on_tiles && L >= 2 &&
            n <= kChainMaxQubits && (int)passes.size() <= kChainMaxSets && d_chain_u != nullptr;
 }
 
@@ -945,8 +954,7 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, doubl
 }
 
 bool Engine::fused_eval() const {
-    return fuse_enabled && fuse_ready && strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && !small &&
-           L >= 2;
+    return fuse_enabled && fuse_ready && on_tiles && L >= 2;
 }
 
 void Engine::structured_hamiltonian_fused(hipStream_t s) {
@@ -1245,7 +1253,7 @@ void Engine::gate_backward(hipStream_t s, const double *scale) {
 // ---------------------------------------------------------------------------
 
 void Engine::forward_device(const double *params, double *energy, hipStream_t s, bool keep_lam) {
-    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+    if (whole) {
         small_records(params, s);
         small_run(s, false, nullptr, energy, nullptr, nullptr);
         resident = false;
@@ -1257,7 +1265,7 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
     }
     launch_coef(params, d_coef, n * L, s);
     check_launch("coef");
-    if (strategy == RIE_STRATEGY_INVERSE_WALK_GATE) {
+    if (!on_tiles) {
         gate_forward(s);
         gate_hamiltonian(s);
         launch_reduce_sum(d_epartials, (int)energy_partials, energy, s);
@@ -1280,18 +1288,18 @@ void Engine::backward_device(const double *params, const double *scale, double *
         dense_run(s, true, params, scale, d_energy + 1, grad);
         return;
     }
-    if (strategy == RIE_STRATEGY_INVERSE_WALK_GATE) {
+    if (whole) {
+        small_records(params, s);
+        small_run(s, true, scale, d_energy + 1, grad, nullptr);
+        return;
+    }
+    if (!on_tiles) {
         if (!resident) {
             forward_device(params, d_energy + 1, s, true);
         }
         gate_backward(s, scale);
         copy_grad_if_needed(grad, s);
         resident = false;
-        return;
-    }
-    if (small) {
-        small_records(params, s);
-        small_run(s, true, scale, d_energy + 1, grad, nullptr);
         return;
     }
     if (!resident) {
@@ -1316,7 +1324,7 @@ void Engine::eval_device(const double *params, double *energy, double *grad, hip
         dense_run(s, true, params, nullptr, energy, grad);
         return;
     }
-    if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+    if (whole) {
         small_records(params, s);
         small_run(s, true, nullptr, energy, grad, nullptr);
         return;
@@ -1362,13 +1370,25 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         stage_begin(s);
         dense_run(s, want_grad, d_params, nullptr, d_energy, want_grad ? d_grad : nullptr);
         stage_end(s, "dense_scan_ms");
-    } else if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT && small) {
+    } else if (whole) {
         stage_begin(s);
         small_records(d_params, s);
         stage_end(s, "zero_state_ms");
         stage_begin(s);
         small_run(s, want_grad, nullptr, d_energy, want_grad ? d_grad : nullptr, nullptr);
-        stage_end(s, want_grad ? "fused_circuit_ms" : "forward_apply_ms");
+        if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT) {
+            stage_end(s, want_grad ? "fused_circuit_ms" : "forward_apply_ms");
+        } else {
+            // the gate-level strategy's stages, all in that one launch
+            stage_end(s, "forward_apply_ms");
+            for (const char *name : {"hamiltonian_ms", "energy_dot_ms", "gradient_zero_ms",
+                                     "backward_sweep_ms"}) {
+                if (want_grad || name[0] == 'h' || name[0] == 'e') {
+                    stage_begin(s);
+                    stage_end(s, name);
+                }
+            }
+        }
     } else if (want_grad && fused_eval()) {
         stage_begin(s);
         launch_coef(d_params, d_coef, n * L, s);
@@ -1376,7 +1396,7 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         stage_end(s, "zero_state_ms");
         structured_eval_fused(s, nullptr, d_energy, true);
     } else {
-        const bool gate = strategy == RIE_STRATEGY_INVERSE_WALK_GATE;
+        const bool gate = !on_tiles;
         stage_begin(s);
         launch_coef(d_params, d_coef, n * L, s);
         check_launch("coef");

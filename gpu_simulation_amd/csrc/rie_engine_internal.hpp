@@ -56,6 +56,9 @@ struct PassPlan {
 
 class DensePlan;  // dense_scan buffers and launches (rie_dense.hpp)
 
+// Largest size that the gate-level strategy runs on the tile passes.
+constexpr int kGateTileQubits = 26;
+
 struct Engine {
     Engine(size_t num_qubits, size_t num_layers, double field, const std::string &strategy,
            size_t chunk_width, bool double_buffer);
@@ -78,7 +81,9 @@ struct Engine {
     int num_cus = 0;
     int max_grid = 0;
     hipStream_t own_stream = nullptr;
-    bool small = false;
+    bool small = false;  // n <= kEngineWholeQubits
+    bool whole = false;  // evaluations run the whole-circuit kernel
+    bool on_tiles = false;  // evaluations run the tile passes
     // register shape of the tile passes per pass kind: 4 = 256 threads x 16
     // registers, 3 = 512 threads x 8 registers (both 4096-amplitude tiles)
     // (defaults measured on MI355X at 30 qubits: the 512-thread shape is

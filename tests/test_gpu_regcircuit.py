@@ -94,3 +94,26 @@ def test_engine_calls_agree(oracle, backend_module, n):
     torch.cuda.synchronize()
     assert e.item() == out["energy"]
     assert np.array_equal(g.cpu().numpy(), -2.0 * np.asarray(out["gradient"]))
+
+
+@pytest.mark.parametrize("n,layers", [(2, 1), (9, 3), (14, 1), (14, 3), (17, 2), (27, 1)])
+def test_gate_level_strategy_over_its_paths(oracle, backend_module, n, layers):
+    # whole circuit, tile passes, and above 26 qubits gate by gate; at that size
+    # against the structured engine, which the headline tests hold to the oracle
+    p = np.random.default_rng([12, n]).uniform(0, 2 * np.pi, 2 * n * layers)
+    print(f"case gate n={n} L={layers}", flush=True)
+    eng = backend_module.RingIsingCudaBackend(n, layers, 1.1, "inverse_walk_cuQuantum", 8, False)
+    out = eng.energy_and_grad(p, True, True)
+    assert {"forward_apply_ms", "hamiltonian_ms", "energy_dot_ms",
+            "backward_sweep_ms"} <= set(out["timings_ms"])
+    if n <= 17:
+        e_ref, g_ref = oracle.energy_and_grad(n, layers, 1.1, p.reshape(layers, n, 2))
+    else:
+        ref = backend_module.RingIsingCudaBackend(n, layers, 1.1, "structured_adjoint", 8, False)
+        r = ref.energy_and_grad(p)
+        e_ref, g_ref = r["energy"], r["gradient"]
+    assert abs(out["energy"] - e_ref) <= TOL
+    assert np.max(np.abs(np.asarray(out["gradient"]) - np.ravel(g_ref))) <= TOL
+    assert abs(eng.energy_and_grad(p, False)["energy"] - e_ref) <= TOL
+    with pytest.raises((RuntimeError, ValueError)):
+        eng.final_state()
