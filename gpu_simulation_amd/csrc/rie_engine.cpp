@@ -190,9 +190,8 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     N = uint64_t{1} << n;
     num_params = (size_t)2 * n * L;
     check(hipGetDevice(&device), "hipGetDevice");
-    hipDeviceProp_t prop;
-    check(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
-    num_cus = prop.multiProcessorCount;
+    check(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, device),
+          "hipDeviceGetAttribute");
     // sixteen workgroups per CU (eight rounds of the two resident ones): the
     // tile passes balance better across CUs than with fewer, larger
     // workgroups (measured at 30 qubits: 2, 4, 8, 16, 32 per CU gave 28.2,
@@ -216,6 +215,11 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
 
     d_params = (double *)device_alloc(sizeof(double) * num_params, "alloc params");
     d_grad = (double *)device_alloc(sizeof(double) * num_params, "alloc gradient");
+    grad_dst = d_grad;
+    check(hipHostMalloc((void **)&h_params, sizeof(double) * (2 * num_params + 1), 0),
+          "alloc host staging");
+    h_grad = h_params + num_params;
+    h_energy = h_grad + num_params;
     d_energy = (double *)device_alloc(sizeof(double) * 4, "alloc energy");
     if (whole) {
         // the whole circuit lives in one workgroup's registers
@@ -300,6 +304,9 @@ Engine::~Engine() {
     }
     device_free(d_params);
     device_free(d_grad);
+    if (h_params != nullptr) {
+        (void)hipHostFree(h_params);
+    }
     device_free(d_energy);
     device_free(d_coef);
     device_free(d_rec);
@@ -877,7 +884,7 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, doubl
         check_launch("bwd_pass low gen");
         kt_end(s, "bwd_pass_low_gen", S);
         kt_begin(s);
-        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, 1, d_grad, scale, s);
+        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, 1, grad_dst, scale, s);
         check_launch("reduce_grad");
         kt_end(s, "reduce_grad", 0.0);
         for (int step = 0; step < K; ++step) {
@@ -906,10 +913,10 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, doubl
                 check_launch("bwd_pass high gen layer0");
                 kt_end(s, "bwd_pass_high_gen_layer0", S);
                 kt_begin(s);
-                launch_reduce_grad(d_partials, pp.grid, T, pp.g, 1, d_grad, scale, s);
+                launch_reduce_grad(d_partials, pp.grid, T, pp.g, 1, grad_dst, scale, s);
                 check_launch("reduce_grad");
                 launch_layer0_top_finish(d_tile_sums, tiles, l0_part, pp.grid, d_coef, n,
-                                         d_partials2, high_env_chunks, d_grad, scale, s,
+                                         d_partials2, high_env_chunks, grad_dst, scale, s,
                                          l0_energy_out);
                 check_launch("layer0_top_finish");
                 kt_end(s, "layer0_reduce", 0.0);
@@ -930,7 +937,7 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, doubl
             kt_end(s, "bwd_pass_high_gen", 2 * S);
             std::swap(lam, lam_other);
             kt_begin(s);
-            launch_reduce_grad(d_partials, pp.grid, T, pp.g, 1, d_grad, scale, s);
+            launch_reduce_grad(d_partials, pp.grid, T, pp.g, 1, grad_dst, scale, s);
             check_launch("reduce_grad");
             kt_end(s, "reduce_grad", 0.0);
         }
@@ -1058,7 +1065,7 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
         check_launch("bwd_pass gather");
         kt_end(s, "bwd_pass_low_cnot", S * (3.0 + (low_cur ? 1.0 : 0.0)));
         kt_begin(s);
-        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, l, d_grad, scale, s);
+        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, l, grad_dst, scale, s);
         check_launch("reduce_grad");
         kt_end(s, "reduce_grad", 0.0);
         cur = ncur;
@@ -1075,7 +1082,7 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
                 check_launch("bwd_pass");
                 kt_end(s, "bwd_pass_high_gen", 2 * S);
                 kt_begin(s);
-                launch_reduce_grad(d_partials, pp.grid, T, pp.g, l, d_grad, scale, s);
+                launch_reduce_grad(d_partials, pp.grid, T, pp.g, l, grad_dst, scale, s);
                 check_launch("reduce_grad");
                 kt_end(s, "reduce_grad", 0.0);
             }
@@ -1089,7 +1096,7 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
             check_launch("bwd_pass");
             kt_end(s, "bwd_pass_high", S * (3.0 + (write_cur ? 1.0 : 0.0)));
             kt_begin(s);
-            launch_reduce_grad(d_partials, passes[p].grid, T, passes[p].g, l, d_grad, scale, s);
+            launch_reduce_grad(d_partials, passes[p].grid, T, passes[p].g, l, grad_dst, scale, s);
             check_launch("reduce_grad");
             kt_end(s, "reduce_grad", 0.0);
         }
@@ -1122,7 +1129,7 @@ void Engine::layer0_gradients(hipStream_t s, const double2 *lam, const double *s
     kt_begin(s);
     launch_layer0_high_env(d_tile_sums, g0.num_tiles, d_coef, n, d_partials2, high_env_chunks, s);
     check_launch("layer0_high_env");
-    launch_layer0_finish(d_partials, grid0, d_partials2, high_env_chunks, d_coef, n, d_grad, scale,
+    launch_layer0_finish(d_partials, grid0, d_partials2, high_env_chunks, d_coef, n, grad_dst, scale,
                          s, l0_energy_out);
     check_launch("layer0_finish");
     kt_end(s, "layer0_reduce", 0.0);
@@ -1152,7 +1159,7 @@ void Engine::structured_backward_stored(hipStream_t s, const double *scale) {
         check_launch("bwd_pass gather");
         kt_end(s, "bwd_pass_low_cnot", 3 * S);
         kt_begin(s);
-        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, l, d_grad, scale, s);
+        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, l, grad_dst, scale, s);
         check_launch("reduce_grad");
         kt_end(s, "reduce_grad", 0.0);
         for (int j = K - 1; j >= 0; --j) {
@@ -1164,7 +1171,7 @@ void Engine::structured_backward_stored(hipStream_t s, const double *scale) {
             check_launch("bwd_pass");
             kt_end(s, gen ? "bwd_pass_high_gen" : "bwd_pass_high", (gen ? 2 : 3) * S);
             kt_begin(s);
-            launch_reduce_grad(d_partials, pp.grid, T, pp.g, l, d_grad, scale, s);
+            launch_reduce_grad(d_partials, pp.grid, T, pp.g, l, grad_dst, scale, s);
             check_launch("reduce_grad");
             kt_end(s, "reduce_grad", 0.0);
         }
@@ -1240,9 +1247,9 @@ void Engine::gate_backward(hipStream_t s, const double *scale) {
             const size_t base = ((size_t)l * n + w) * 2;
             const WireCoef *k = d_coef + (size_t)l * n + w;
             launch_gate_rz_step(pool[0], pool[1], n, w, k, d_partials, grid, s);
-            launch_reduce_to(d_partials, grid, d_grad + base + 1, scale, s);
+            launch_reduce_to(d_partials, grid, grad_dst + base + 1, scale, s);
             launch_gate_ry_step(pool[0], pool[1], n, w, k, d_partials, grid, s);
-            launch_reduce_to(d_partials, grid, d_grad + base, scale, s);
+            launch_reduce_to(d_partials, grid, grad_dst + base, scale, s);
         }
     }
     check_launch("gate backward");
@@ -1297,16 +1304,16 @@ void Engine::backward_device(const double *params, const double *scale, double *
         if (!resident) {
             forward_device(params, d_energy + 1, s, true);
         }
+        const GradTarget target(*this, grad);
         gate_backward(s, scale);
-        copy_grad_if_needed(grad, s);
         resident = false;
         return;
     }
     if (!resident) {
         forward_device(params, d_energy + 1, s, true);
     }
+    const GradTarget target(*this, grad);
     structured_backward(s, scale, false);
-    copy_grad_if_needed(grad, s);
     resident = false;
 }
 
@@ -1316,8 +1323,8 @@ void Engine::eval_device(const double *params, double *energy, double *grad, hip
     if (fused_eval()) {
         launch_coef(params, d_coef, n * L, s);
         check_launch("coef");
+        const GradTarget target(*this, grad);
         structured_eval_fused(s, nullptr, energy, false);
-        copy_grad_if_needed(grad, s);
         return;
     }
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
@@ -1331,13 +1338,6 @@ void Engine::eval_device(const double *params, double *energy, double *grad, hip
     }
     forward_device(params, energy, s, true);
     backward_device(params, nullptr, grad, s);
-}
-
-void Engine::copy_grad_if_needed(double *grad, hipStream_t s) {
-    if (grad != d_grad) {
-        check(hipMemcpyAsync(grad, d_grad, sizeof(double) * num_params, hipMemcpyDeviceToDevice, s),
-              "copy gradient");
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1357,10 +1357,12 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
     timings.clear();
     profiling = profile;
     auto t0 = std::chrono::steady_clock::now();
-    check(hipMemcpyAsync(d_params, params, sizeof(double) * num_params, hipMemcpyHostToDevice, s),
-          "upload params");
+    // Parameters, energy and gradient pass through pinned memory that the
+    // kernels read and write themselves (each value once): three copies of
+    // pageable memory cost 20 to 65 us a call, most of a small circuit's time.
+    std::memcpy(h_params, params, sizeof(double) * num_params);
+    const GradTarget target(*this, h_grad);
     if (profile) {
-        check(hipStreamSynchronize(s), "sync");
         const double host_ms =
             std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0)
                 .count();
@@ -1368,14 +1370,14 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
     }
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
         stage_begin(s);
-        dense_run(s, want_grad, d_params, nullptr, d_energy, want_grad ? d_grad : nullptr);
+        dense_run(s, want_grad, h_params, nullptr, h_energy, want_grad ? h_grad : nullptr);
         stage_end(s, "dense_scan_ms");
     } else if (whole) {
         stage_begin(s);
-        small_records(d_params, s);
+        small_records(h_params, s);
         stage_end(s, "zero_state_ms");
         stage_begin(s);
-        small_run(s, want_grad, nullptr, d_energy, want_grad ? d_grad : nullptr, nullptr);
+        small_run(s, want_grad, nullptr, h_energy, want_grad ? h_grad : nullptr, nullptr);
         if (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT) {
             stage_end(s, want_grad ? "fused_circuit_ms" : "forward_apply_ms");
         } else {
@@ -1391,14 +1393,14 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         }
     } else if (want_grad && fused_eval()) {
         stage_begin(s);
-        launch_coef(d_params, d_coef, n * L, s);
+        launch_coef(h_params, d_coef, n * L, s);
         check_launch("coef");
         stage_end(s, "zero_state_ms");
-        structured_eval_fused(s, nullptr, d_energy, true);
+        structured_eval_fused(s, nullptr, h_energy, true);
     } else {
         const bool gate = !on_tiles;
         stage_begin(s);
-        launch_coef(d_params, d_coef, n * L, s);
+        launch_coef(h_params, d_coef, n * L, s);
         check_launch("coef");
         stage_end(s, "zero_state_ms");
         stage_begin(s);
@@ -1416,7 +1418,7 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         }
         stage_end(s, "hamiltonian_ms");
         stage_begin(s);
-        launch_reduce_sum(d_epartials, (int)energy_partials, d_energy, s);
+        launch_reduce_sum(d_epartials, (int)energy_partials, h_energy, s);
         check_launch("energy reduce");
         stage_end(s, "energy_dot_ms");
         if (want_grad) {
@@ -1432,15 +1434,12 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         }
     }
     stage_begin(s);
-    check(hipMemcpyAsync(energy_out, d_energy, sizeof(double), hipMemcpyDeviceToHost, s),
-          "copy energy");
-    if (want_grad) {
-        check(hipMemcpyAsync(grad_out, d_grad, sizeof(double) * num_params, hipMemcpyDeviceToHost,
-                             s),
-              "copy gradient");
-    }
     order_end(s);
     check(hipStreamSynchronize(s), "synchronize");
+    *energy_out = *h_energy;
+    if (want_grad) {
+        std::memcpy(grad_out, h_grad, sizeof(double) * num_params);
+    }
     stage_end(s, "gradient_copy_ms");
     profiling = false;
     resident = false;

@@ -135,6 +135,10 @@ struct Engine {
     int schedule = RIE_SCHEDULE_INVERSE_WALK;
     double *d_params = nullptr;
     double *d_grad = nullptr;
+    double *grad_dst = nullptr;  // where the current call's gradient goes
+    double *h_params = nullptr;  // pinned: parameters, gradient, energy of host calls
+    double *h_grad = nullptr;
+    double *h_energy = nullptr;
     double *d_energy = nullptr;
     WireCoef *d_coef = nullptr;
     double *d_rec = nullptr;  // whole-circuit path: the layers' records
@@ -243,7 +247,6 @@ struct Engine {
 
     void forward_device(const double *params, double *energy, hipStream_t s, bool keep_lam);
     void backward_device(const double *params, const double *scale, double *grad, hipStream_t s);
-    void copy_grad_if_needed(double *grad, hipStream_t s);
     void eval_device(const double *params, double *energy, double *grad, hipStream_t s);
     void energy_and_grad_host(const double *params, size_t count, bool want_grad, bool profile,
                               double *energy_out, double *grad_out);
@@ -253,6 +256,15 @@ struct Engine {
                                  double *normal_ms, double *graph_ms);
     void copy_state(double *host_out, size_t count);
     std::string autotune(const double *params, size_t count, size_t repeats);
+
+    // Sends the gradient of the launches issued in its scope to dst.
+    struct GradTarget {
+        GradTarget(Engine &e, double *dst) : engine(e) { engine.grad_dst = dst; }
+        ~GradTarget() { engine.grad_dst = engine.d_grad; }
+        GradTarget(const GradTarget &) = delete;
+        GradTarget &operator=(const GradTarget &) = delete;
+        Engine &engine;
+    };
 };
 
 }  // namespace rie
