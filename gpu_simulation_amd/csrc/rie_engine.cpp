@@ -207,7 +207,7 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     // it runs on the same kernels; above kGateTileQubits, where their four state
     // buffers and tables would take memory that two buffers leave free, gate by
     // gate.  15 qubits x 2 layers through the host call: 849 us gate by gate
-    // (about 250 launches), 136 us on the tile passes.
+    // (about 250 launches), 75 us on the tile passes.
     const bool gate = strategy == RIE_STRATEGY_INVERSE_WALK_GATE;
     whole = small && (gate || strategy == RIE_STRATEGY_STRUCTURED_ADJOINT);
     on_tiles = !small && (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT ||
@@ -239,19 +239,22 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
         schedule = (!gate && L > 1 && need <= 0.85 * (double)free_b) ? RIE_SCHEDULE_STORED
                                                                      : RIE_SCHEDULE_INVERSE_WALK;
         ensure_pool(schedule == RIE_SCHEDULE_STORED ? stored_buffer_count() : 4);
-        size_t part = 0;
-        for (const auto &p : passes) {
-            part = std::max<size_t>(part, (size_t)p.grid * 2 * T);
-        }
         size_t eparts = 0;
         for (const auto &p : passes) {
+            part_stride = std::max<size_t>(part_stride, (size_t)p.grid * 2 * T);
             eparts += (size_t)p.grid;
         }
-        // the layer-0 contraction writes 48 values per workgroup of the low pass;
-        // inside the top group's pass, 2T + kTopL0Cols per workgroup of that pass
-        partial_count = std::max({part, eparts, (size_t)passes[0].grid * 48,
-                                  (size_t)passes.back().grid * (2 * T + kTopL0Cols)});
+        // A place for each pass's gradient partials (at most kGradReduceJobs:
+        // then they are reduced and the places used again), so that one launch
+        // reduces them all.  Behind them the layer-0 contraction's values: 48
+        // per workgroup of the low pass, kTopL0Cols per workgroup of the top
+        // group's pass.
+        part_slots = (int)std::min<size_t>(kGradReduceJobs, (size_t)L * passes.size());
+        const size_t l0_count =
+            std::max((size_t)passes[0].grid * 48, (size_t)passes.back().grid * kTopL0Cols);
+        partial_count = part_stride * (size_t)part_slots + l0_count;
         d_partials = (double *)device_alloc(sizeof(double) * partial_count, "alloc partials");
+        d_l0_partials = d_partials + part_stride * (size_t)part_slots;
         d_epartials = (double *)device_alloc(sizeof(double) * eparts, "alloc energy partials");
         epartial_count = eparts;
         const uint64_t tiles = passes[0].g.num_tiles;
@@ -261,8 +264,10 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
         tile_sum_count = L == 2 ? tiles * (Tile4Waves + 2) : tiles;
         d_tile_sums = (double2 *)device_alloc(sizeof(double2) * tile_sum_count, "alloc tile sums");
         if (L == 2) {
-            // the generated start's per-tile lambda addresses (read and write)
-            d_lam_tab = (uint64_t *)device_alloc(sizeof(uint64_t) * 2 * tiles, "alloc tile table");
+            // the generated start's per-tile lambda addresses: one table for
+            // the low pass (write), two for each high pass but the last
+            d_lam_tab = (uint64_t *)device_alloc(sizeof(uint64_t) * tiles * (2 * passes.size() - 3),
+                                                 "alloc tile tables");
         }
         d_chain = (CMat2 *)device_alloc(sizeof(CMat2) * kChainMaxSets * kChainTabEntries,
                                         "alloc chain tables");
@@ -445,7 +450,7 @@ void Engine::kt_flush() {
 // Structured adjoint: tile-pass path (n > 12)
 // ---------------------------------------------------------------------------
 
-void Engine::structured_forward(hipStream_t s, bool save_ckpts) {
+void Engine::structured_forward(hipStream_t s, bool save_ckpts, const double *params) {
     const double S = (double)sizeof(double2) * (double)N;
     const int K = (int)passes.size() - 1;  // high passes per layer (>= 1 for n > 12)
     if (L == 1) {
@@ -459,7 +464,7 @@ void Engine::structured_forward(hipStream_t s, bool save_ckpts) {
     }
     gen_fwd = gen_ready();
     if (gen_fwd) {
-        build_chain_tables(s);
+        build_chain_tables(s, params);
     }
     if (schedule == RIE_SCHEDULE_STORED) {
         // Every pass writes its own buffer; layer 1's first pass generates the
@@ -594,6 +599,31 @@ void Engine::require_partials(size_t count) const {
     }
 }
 
+// The gradient partials of the next tile pass go to the first free place.
+double *Engine::pass_partials() const {
+    return d_partials + part_stride * (size_t)greduce.count;
+}
+
+// Queue the reduction of the partials that a pass of layer l has just written;
+// with every place taken, reduce them.
+void Engine::queue_grad(const PassPlan &pp, int l, const double *scale, hipStream_t s) {
+    const PassGeom &g = pp.g;
+    greduce.job[greduce.count] = {pass_partials(), grad_dst + (size_t)l * 2 * n, pp.grid,
+                                  2 * g.rot_lo, 2 * (g.rot_hi - g.rot_lo), g.a, g.h0};
+    if (++greduce.count == part_slots) {
+        finish_grads(Layer0Reduce{}, scale, s);
+    }
+}
+
+// Reduce what is queued, with the layer-0 results (l0.lc0 null: none).
+void Engine::finish_grads(const Layer0Reduce &l0, const double *scale, hipStream_t s) {
+    kt_begin(s);
+    launch_reduce(greduce, T, l0, scale, s);
+    greduce.count = 0;
+    check_launch("reduce");
+    kt_end(s, l0.lc0 != nullptr ? "layer0_reduce" : "reduce_grad", 0.0);
+}
+
 int Engine::free_buffer(std::initializer_list<int> used) const {
     for (int i = 0; i < 4; ++i) {
         bool taken = false;
@@ -663,7 +693,7 @@ void Engine::launch_bwd(int l, bool gather, bool write_cur, const double2 *cur_i
     // one; the walk's one-sweep passes do not
     const bool prefetch = double_buffer && !write_cur;
     launch_bwd_pass(pass_r[gather ? RIE_PASS_BWD_LOW : RIE_PASS_BWD_HIGH], gather, write_cur, true,
-                    cur_in, lam_in, cur_out, lam_out, lc, pg, d_partials, pp.grid, s, pairs,
+                    cur_in, lam_in, cur_out, lam_out, lc, pg, pass_partials(), pp.grid, s, pairs,
                     pairs ? h : 0.0, gen_tab, gen_utab, prefetch, phase_free);
 }
 
@@ -742,8 +772,12 @@ bool Engine::gen_ready() const {
 // groups 0 .. j when the high passes run from the top group down (the stored
 // schedule and the walk), groups j .. K-1 when they run from the lowest group
 // up (the generated start, bottom_up).
-void Engine::build_chain_tables(hipStream_t s, int r_set0, bool bottom_up) {
-    ChainSetup cs{};
+// The tables are computed with the coefficients of params (the coefficient
+// table written too) or, null, with the table.  prep: the generated start's
+// parts, filled by the caller.
+void Engine::build_chain_tables(hipStream_t s, const double *params, int r_set0, bool bottom_up,
+                                ChainPrep prep) {
+    ChainSetup &cs = prep.cs;
     cs.n = n;
     cs.tiles = passes[0].g.num_tiles;
     const uint64_t all = (n >= 64) ? ~uint64_t{0} : ((uint64_t{1} << n) - 1);
@@ -800,15 +834,48 @@ void Engine::build_chain_tables(hipStream_t s, int r_set0, bool bottom_up) {
             fail(RIE_DEVICE_ERROR, "internal: chain tables do not fit this plan");
         }
     }
+    prep.params = params;
+    prep.coef = d_coef;
+    prep.coefs = n * L;
+    prep.tabs = d_chain;
+    prep.utab = d_chain_u;
+    // U_A of set 0 at the out-of-tile flips
+    prep.xtab = r_set0 > 0 ? d_chain_x : nullptr;
     kt_begin(s);
-    launch_chain_tables(d_coef, d_coef + n, cs, d_chain, d_chain_u, s);
-    check_launch("chain_tables");
-    if (r_set0 > 0) {
-        // U_A of set 0 at the out-of-tile flips
-        launch_chain_flips(d_coef, d_coef + n, cs, d_chain_x, s);
-        check_launch("chain_flips");
-    }
+    launch_chain_prep(prep, s);
+    check_launch("chain_prep");
     kt_end(s, "chain_tables", 0.0);
+    chain_rh = bottom_up ? 0 : rh;
+}
+
+// The backward's tables are the forward's unless the register shape changed in
+// between.  A capture records them all the same: its replay may follow an
+// evaluation with another shape.
+void Engine::rebuild_chain_tables(hipStream_t s) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool known = hipStreamIsCapturing(s, &capture) == hipSuccess;
+    if (!known) {
+        (void)hipGetLastError();  // the null stream beside a capture: as if captured
+    }
+    if (!known || capture != hipStreamCaptureStatusNone ||
+        chain_rh != pass_r[RIE_PASS_BWD_HIGH]) {
+        build_chain_tables(s);
+    }
+}
+
+// Start an evaluation of params: returns what the chain tables are to be
+// computed from.  Up to kPrepParamTiles tiles their launch computes the
+// coefficients itself, in each of its workgroups, from the parameters (one
+// launch less, 3 us; a table of its own pays once hundreds of workgroups would
+// read parameters that may lie in host memory).
+const double *Engine::start_coefs(const double *params, hipStream_t s) {
+    constexpr uint64_t kPrepParamTiles = 2048;
+    if (gen_ready() && passes[0].g.num_tiles <= kPrepParamTiles) {
+        return params;
+    }
+    launch_coef(params, d_coef, n * L, s);
+    check_launch("coef");
+    return nullptr;
 }
 
 bool Engine::gen_start_ready() const {
@@ -834,15 +901,57 @@ bool Engine::l0_in_pass_ready() const {
 // the high passes run from the lowest group up (gen_bottom_up: the last one
 // holds the top group's tiles); otherwise 2 S for it and the 1 S layer-0
 // contraction.
-void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, double *energy_out,
-                                       bool staged) {
+void Engine::structured_eval_gen_start(hipStream_t s, const double *params, const double *scale,
+                                       double *energy_out, bool staged) {
     const double S = (double)sizeof(double2) * (double)N;
     const int r_low = pass_r[RIE_PASS_BWD_LOW];
+    const int K = (int)passes.size() - 1;
+    const uint64_t tiles = passes[0].g.num_tiles;
     if (staged) {
         stage_begin(s);
     }
+    if (d_lam_tab == nullptr) {
+        fail(RIE_DEVICE_ERROR, "internal: no lambda tile table");
+    }
     const bool bottom_up = gen_bottom_up();
-    build_chain_tables(s, r_low, bottom_up);
+    PassGeom g0 = passes[0].g;
+    g0.pair_lo = 0;  // every adjacent pair inside the low tile
+    g0.pair_hi = T;
+    // lambda layouts: high pass j reads its tiles as contiguous blocks.  A
+    // tile's write addresses then differ from its read addresses, so the
+    // high passes alternate between two buffers instead of working in place.
+    const bool layouts = gen_layouts();
+    if (layouts) {
+        g0.lay_out = lam_layout_in(bottom_up ? 0 : K - 1, bottom_up);
+    }
+    // the tiles' lambda addresses: the low pass's (write), those of each high
+    // pass but the last when they run without phases (read and write), and
+    // those of the pass that contracts layer 0 (read)
+    ChainPrep prep{};
+    prep.tables[prep.table_count++] = {g0.a, g0.h0, g0.lay_out, d_lam_tab};
+    g0.tile_out = d_lam_tab;
+    double2 *phi_c = d_tile_sums + tiles * Tile4Waves;
+    uint64_t *lam_tile = reinterpret_cast<uint64_t *>(phi_c + tiles);
+    if (bottom_up) {
+        if ((size_t)high_env_chunks * 4 * (size_t)std::max(1, n - T) > partial2_count ||
+            tile_sum_count < tiles * (Tile4Waves + 2)) {
+            fail(RIE_DEVICE_ERROR, "internal: layer-0 partial buffer too small");
+        }
+        for (int j = 0; j + 1 < K; ++j) {
+            const PassGeom &g = passes[1 + (size_t)j].g;
+            uint64_t *tab = d_lam_tab + tiles * (size_t)(1 + 2 * j);
+            prep.tables[prep.table_count++] = {
+                g.a, g.h0, layouts ? lam_layout_in(j, bottom_up) : g.lay_in, tab};
+            prep.tables[prep.table_count++] = {
+                g.a, g.h0, layouts ? lam_layout_out(j, bottom_up) : g.lay_out, tab + tiles};
+        }
+        const PassGeom &g = passes[(size_t)K].g;
+        prep.tables[prep.table_count++] = {
+            g.a, g.h0, layouts ? lam_layout_in(K - 1, bottom_up) : g.lay_in, lam_tile};
+        prep.phi_c = phi_c;
+        prep.phi_h0 = g.h0;
+    }
+    build_chain_tables(s, params, r_low, bottom_up, prep);
     gen_fwd = false;
     final_ptr = nullptr;  // no state is written
     if (staged) {
@@ -853,40 +962,21 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, doubl
         stage_end(s, "gradient_zero_ms");
         stage_begin(s);
     }
-    PassGeom g0 = passes[0].g;
-    g0.pair_lo = 0;  // every adjacent pair inside the low tile
-    g0.pair_hi = T;
     double2 *lam = pool[0];
-    const int K = (int)passes.size() - 1;
-    // lambda layouts: high pass j reads its tiles as contiguous blocks.  A
-    // tile's write addresses then differ from its read addresses, so the
-    // high passes alternate between two buffers instead of working in place.
-    const bool layouts = gen_layouts();
     double2 *lam_other = layouts ? pool[1] : lam;
-    if (layouts) {
-        g0.lay_out = lam_layout_in(bottom_up ? 0 : K - 1, bottom_up);
-    }
     const bool l0_in_pass = bottom_up;
     // every X term is in lambda once the low pass is done: the high passes
     // add no pair terms (fuse_layer stays -1)
     fuse_layer = -1;
     l0_energy_out = energy_out;
+    greduce.count = 0;
     try {
-        require_partials((size_t)passes[0].grid * 2 * T);
-        if (d_lam_tab == nullptr) {
-            fail(RIE_DEVICE_ERROR, "internal: no lambda tile table");
-        }
         kt_begin(s);
-        launch_lam_tile_table(g0, g0.lay_out, d_lam_tab, s);
-        g0.tile_out = d_lam_tab;
-        launch_bwd_low_gen(r_low, lam, d_coef + n, g0, d_partials, passes[0].grid, s, h, d_chain,
-                           d_chain_u, d_chain_x);
+        launch_bwd_low_gen(r_low, lam, d_coef + n, g0, pass_partials(), passes[0].grid, s, h,
+                           d_chain, d_chain_u, d_chain_x);
         check_launch("bwd_pass low gen");
         kt_end(s, "bwd_pass_low_gen", S);
-        kt_begin(s);
-        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, 1, grad_dst, scale, s);
-        check_launch("reduce_grad");
-        kt_end(s, "reduce_grad", 0.0);
+        queue_grad(passes[0], 1, scale, s);
         for (int step = 0; step < K; ++step) {
             const int j = bottom_up ? step : K - 1 - step;
             const PassPlan &pp = passes[1 + (size_t)j];
@@ -896,50 +986,31 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *scale, doubl
                 gj.lay_out = lam_layout_out(j, bottom_up);
             }
             if (j == K - 1 && l0_in_pass) {
-                const uint64_t tiles = pp.g.num_tiles;
-                require_partials((size_t)pp.grid * (2 * T + kTopL0Cols));
-                if ((size_t)high_env_chunks * 4 * (size_t)std::max(1, n - T) > partial2_count ||
-                    tile_sum_count < tiles * (Tile4Waves + 2)) {
-                    fail(RIE_DEVICE_ERROR, "internal: layer-0 partial buffer too small");
-                }
-                double *l0_part = d_partials + (size_t)pp.grid * 2 * T;
-                double2 *phi_c = d_tile_sums + tiles * Tile4Waves;
-                uint64_t *lam_tile = reinterpret_cast<uint64_t *>(phi_c + tiles);
                 kt_begin(s);
-                launch_bwd_top_l0(lam, d_coef + n, gj, d_partials, pp.grid, s,
+                launch_bwd_top_l0(lam, d_coef + n, gj, pass_partials(), pp.grid, s,
                                   d_chain + (size_t)(1 + j) * kChainTabEntries,
-                                  d_chain_u + (size_t)(1 + j) * 2 * passes[0].g.num_tiles, d_coef,
-                                  phi_c, lam_tile, d_tile_sums, l0_part);
+                                  d_chain_u + (size_t)(1 + j) * 2 * tiles, d_coef, phi_c, lam_tile,
+                                  d_tile_sums, d_l0_partials);
                 check_launch("bwd_pass high gen layer0");
                 kt_end(s, "bwd_pass_high_gen_layer0", S);
-                kt_begin(s);
-                launch_reduce_grad(d_partials, pp.grid, T, pp.g, 1, grad_dst, scale, s);
-                check_launch("reduce_grad");
-                launch_layer0_top_finish(d_tile_sums, tiles, l0_part, pp.grid, d_coef, n,
-                                         d_partials2, high_env_chunks, grad_dst, scale, s,
-                                         l0_energy_out);
-                check_launch("layer0_top_finish");
-                kt_end(s, "layer0_reduce", 0.0);
+                queue_grad(pp, 1, scale, s);
+                finish_grads({d_coef, n, true, d_l0_partials, pp.grid, d_tile_sums, tiles,
+                              d_partials2, high_env_chunks, grad_dst, l0_energy_out},
+                             scale, s);
                 break;
             }
-            require_partials((size_t)pp.grid * 2 * T);
             kt_begin(s);
             if (bottom_up) {
                 // the phase-free sweep reads its tiles' lambda addresses from tables
-                launch_lam_tile_table(gj, gj.lay_in, d_lam_tab, s);
-                launch_lam_tile_table(gj, gj.lay_out, d_lam_tab + pp.g.num_tiles, s);
-                gj.tile_in = d_lam_tab;
-                gj.tile_out = d_lam_tab + pp.g.num_tiles;
+                gj.tile_in = d_lam_tab + tiles * (size_t)(1 + 2 * j);
+                gj.tile_out = gj.tile_in + tiles;
             }
             launch_bwd(1, false, false, nullptr, lam, nullptr, lam_other, (size_t)(1 + j), s, 1 + j,
                        &gj, bottom_up);
             check_launch("bwd_pass");
             kt_end(s, "bwd_pass_high_gen", 2 * S);
             std::swap(lam, lam_other);
-            kt_begin(s);
-            launch_reduce_grad(d_partials, pp.grid, T, pp.g, 1, grad_dst, scale, s);
-            check_launch("reduce_grad");
-            kt_end(s, "reduce_grad", 0.0);
+            queue_grad(pp, 1, scale, s);
         }
         if (!l0_in_pass) {
             layer0_gradients(s, lam, scale);
@@ -986,16 +1057,16 @@ void Engine::structured_hamiltonian_fused(hipStream_t s) {
 // once the last layer's adjoint passes have added their pair terms, and the
 // adjoint sweep is unitary, so at layer 0 <chi|mu> = <psi|H|psi>: the layer-0
 // contraction writes the energy.
-void Engine::structured_eval_fused(hipStream_t s, const double *scale, double *energy_out,
-                                   bool staged) {
+void Engine::structured_eval_fused(hipStream_t s, const double *params, const double *scale,
+                                   double *energy_out, bool staged) {
     if (gen_start_ready()) {
-        structured_eval_gen_start(s, scale, energy_out, staged);
+        structured_eval_gen_start(s, params, scale, energy_out, staged);
         return;
     }
     if (staged) {
         stage_begin(s);
     }
-    structured_forward(s, ckpt_every > 0);
+    structured_forward(s, ckpt_every > 0, params);
     if (staged) {
         stage_end(s, "forward_apply_ms");
         stage_begin(s);
@@ -1038,6 +1109,7 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
         structured_backward_stored(s, scale);
         return;
     }
+    greduce.count = 0;
     int cur = final_cur;  // -2 while the state lives in a checkpoint buffer
     const double2 *cur_in = final_state();
     int lam = lam_idx;
@@ -1056,18 +1128,14 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
         // written (the low pass still reads the state after layer 1).
         const bool gen = l == 1 && gen_fwd && !full_walk;
         if (gen) {
-            build_chain_tables(s);  // the register shapes may have changed since the forward
+            rebuild_chain_tables(s);
         }
         const bool low_cur = !gen && (only_low ? need_cur_after : true);
-        require_partials((size_t)passes[0].grid * 2 * T);
         kt_begin(s);
         launch_bwd(l, true, low_cur, cur_in, pool[lam], pool[ncur], pool[nlam], 0, s);
         check_launch("bwd_pass gather");
         kt_end(s, "bwd_pass_low_cnot", S * (3.0 + (low_cur ? 1.0 : 0.0)));
-        kt_begin(s);
-        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, l, grad_dst, scale, s);
-        check_launch("reduce_grad");
-        kt_end(s, "reduce_grad", 0.0);
+        queue_grad(passes[0], l, scale, s);
         cur = ncur;
         lam = nlam;
         if (gen) {
@@ -1075,30 +1143,22 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
             // groups 0 .. j rotated) holds the state each pass needs
             for (int j = (int)passes.size() - 2; j >= 0; --j) {
                 const PassPlan &pp = passes[1 + (size_t)j];
-                require_partials((size_t)pp.grid * 2 * T);
                 kt_begin(s);
                 launch_bwd(l, false, false, nullptr, pool[lam], nullptr, pool[lam],
                            (size_t)(1 + j), s, 1 + j);
                 check_launch("bwd_pass");
                 kt_end(s, "bwd_pass_high_gen", 2 * S);
-                kt_begin(s);
-                launch_reduce_grad(d_partials, pp.grid, T, pp.g, l, grad_dst, scale, s);
-                check_launch("reduce_grad");
-                kt_end(s, "reduce_grad", 0.0);
+                queue_grad(pp, l, scale, s);
             }
             continue;  // l == 1 is the last walked layer
         }
         for (size_t p = 1; p < passes.size(); ++p) {
             const bool write_cur = (p + 1 < passes.size()) || need_cur_after;
-            require_partials((size_t)passes[p].grid * 2 * T);
             kt_begin(s);
             launch_bwd(l, false, write_cur, pool[cur], pool[lam], pool[cur], pool[lam], p, s);
             check_launch("bwd_pass");
             kt_end(s, "bwd_pass_high", S * (3.0 + (write_cur ? 1.0 : 0.0)));
-            kt_begin(s);
-            launch_reduce_grad(d_partials, passes[p].grid, T, passes[p].g, l, grad_dst, scale, s);
-            check_launch("reduce_grad");
-            kt_end(s, "reduce_grad", 0.0);
+            queue_grad(passes[p], l, scale, s);
         }
         if (ckpt_next) {
             cur_in = ckpts[(size_t)l / ckpt_every - 1];
@@ -1108,7 +1168,9 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
         }
     }
     walked_cur = full_walk ? cur : -1;
-    if (!full_walk) {
+    if (full_walk) {
+        finish_grads(Layer0Reduce{}, scale, s);
+    } else {
         layer0_gradients(s, pool[lam], scale);
     }
 }
@@ -1117,22 +1179,17 @@ void Engine::layer0_gradients(hipStream_t s, const double2 *lam, const double *s
     const double S = (double)sizeof(double2) * (double)N;
     const PassGeom &g0 = passes[0].g;
     const int grid0 = passes[0].grid;
-    require_partials((size_t)grid0 * 48);
     if ((size_t)high_env_chunks * 4 * (size_t)std::max(1, n - T) > partial2_count) {
         fail(RIE_DEVICE_ERROR, "internal: layer-0 partial buffer too small");
     }
     kt_begin(s);
-    launch_layer0_contract(pass_r[RIE_PASS_LAYER0], lam, d_coef, g0, d_tile_sums, d_partials,
+    launch_layer0_contract(pass_r[RIE_PASS_LAYER0], lam, d_coef, g0, d_tile_sums, d_l0_partials,
                            grid0, s);
     check_launch("layer0_contract");
     kt_end(s, "layer0_contract", S);
-    kt_begin(s);
-    launch_layer0_high_env(d_tile_sums, g0.num_tiles, d_coef, n, d_partials2, high_env_chunks, s);
-    check_launch("layer0_high_env");
-    launch_layer0_finish(d_partials, grid0, d_partials2, high_env_chunks, d_coef, n, grad_dst, scale,
-                         s, l0_energy_out);
-    check_launch("layer0_finish");
-    kt_end(s, "layer0_reduce", 0.0);
+    finish_grads({d_coef, n, false, d_l0_partials, grid0, d_tile_sums, g0.num_tiles, d_partials2,
+                  high_env_chunks, grad_dst, l0_energy_out},
+                 scale, s);
 }
 
 
@@ -1147,33 +1204,26 @@ void Engine::structured_backward_stored(hipStream_t s, const double *scale) {
     const double S = (double)sizeof(double2) * (double)N;
     const int K = (int)passes.size() - 1;
     if (gen_fwd) {
-        build_chain_tables(s);  // the register shapes may have changed since the forward
+        rebuild_chain_tables(s);
     }
+    greduce.count = 0;
     int a = 0;  // lambda lives in lbuf(a)
     for (int l = L - 1; l >= 1; --l) {
         const int b = 1 - a;
         const bool gen = (l == 1 && gen_fwd);
-        require_partials((size_t)passes[0].grid * 2 * T);
         kt_begin(s);
         launch_bwd(l, true, false, fbuf(l, K), lbuf(a), nullptr, lbuf(b), 0, s);
         check_launch("bwd_pass gather");
         kt_end(s, "bwd_pass_low_cnot", 3 * S);
-        kt_begin(s);
-        launch_reduce_grad(d_partials, passes[0].grid, T, passes[0].g, l, grad_dst, scale, s);
-        check_launch("reduce_grad");
-        kt_end(s, "reduce_grad", 0.0);
+        queue_grad(passes[0], l, scale, s);
         for (int j = K - 1; j >= 0; --j) {
             const PassPlan &pp = passes[1 + j];
-            require_partials((size_t)pp.grid * 2 * T);
             kt_begin(s);
             launch_bwd(l, false, false, gen ? nullptr : fbuf(l, j), lbuf(b), nullptr, lbuf(b),
                        (size_t)(1 + j), s, gen ? 1 + j : -1);
             check_launch("bwd_pass");
             kt_end(s, gen ? "bwd_pass_high_gen" : "bwd_pass_high", (gen ? 2 : 3) * S);
-            kt_begin(s);
-            launch_reduce_grad(d_partials, pp.grid, T, pp.g, l, grad_dst, scale, s);
-            check_launch("reduce_grad");
-            kt_end(s, "reduce_grad", 0.0);
+            queue_grad(pp, l, scale, s);
         }
         a = b;
     }
@@ -1270,8 +1320,7 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
         dense_run(s, false, params, nullptr, energy, nullptr);
         return;
     }
-    launch_coef(params, d_coef, n * L, s);
-    check_launch("coef");
+    const double *prep = start_coefs(params, s);
     if (!on_tiles) {
         gate_forward(s);
         gate_hamiltonian(s);
@@ -1280,7 +1329,7 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
         resident = true;
         return;
     }
-    structured_forward(s, ckpt_every > 0);
+    structured_forward(s, ckpt_every > 0, prep);
     structured_hamiltonian(s, keep_lam);
     kt_begin(s);
     launch_reduce_sum(d_epartials, (int)energy_partials, energy, s);
@@ -1321,10 +1370,9 @@ void Engine::backward_device(const double *params, const double *scale, double *
 // when it applies, else the forward and backward halves.
 void Engine::eval_device(const double *params, double *energy, double *grad, hipStream_t s) {
     if (fused_eval()) {
-        launch_coef(params, d_coef, n * L, s);
-        check_launch("coef");
+        const double *prep = start_coefs(params, s);
         const GradTarget target(*this, grad);
-        structured_eval_fused(s, nullptr, energy, false);
+        structured_eval_fused(s, prep, nullptr, energy, false);
         return;
     }
     if (strategy == RIE_STRATEGY_DENSE_SCAN) {
@@ -1393,21 +1441,19 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         }
     } else if (want_grad && fused_eval()) {
         stage_begin(s);
-        launch_coef(h_params, d_coef, n * L, s);
-        check_launch("coef");
+        const double *prep = start_coefs(h_params, s);
         stage_end(s, "zero_state_ms");
-        structured_eval_fused(s, nullptr, h_energy, true);
+        structured_eval_fused(s, prep, nullptr, h_energy, true);
     } else {
         const bool gate = !on_tiles;
         stage_begin(s);
-        launch_coef(h_params, d_coef, n * L, s);
-        check_launch("coef");
+        const double *prep = start_coefs(h_params, s);
         stage_end(s, "zero_state_ms");
         stage_begin(s);
         if (gate) {
             gate_forward(s);
         } else {
-            structured_forward(s, want_grad && ckpt_every > 0);
+            structured_forward(s, want_grad && ckpt_every > 0, prep);
         }
         stage_end(s, "forward_apply_ms");
         stage_begin(s);

@@ -147,10 +147,14 @@ struct Engine {
     double *d_drift = nullptr;
     double2 *d_tile_sums = nullptr;  // layer-0 contraction: per-tile sums (tile_sum_count)
     uint64_t tile_sum_count = 0;
-    uint64_t *d_lam_tab = nullptr;  // generated start: per-tile lambda addresses (2 x tiles)
+    uint64_t *d_lam_tab = nullptr;  // generated start: per-tile lambda addresses of its passes
     double *d_partials2 = nullptr;   // layer-0 contraction: high-wire partials
     int high_env_chunks = 1;
     size_t partial_count = 0;    // capacity of d_partials (doubles)
+    size_t part_stride = 0;      // gradient partials of one tile pass
+    int part_slots = 0;          // passes whose partials fit
+    double *d_l0_partials = nullptr;  // in d_partials: the layer-0 contraction's values
+    GradReduce greduce{};        // passes whose partials wait to be reduced
     size_t epartial_count = 0;   // capacity of d_epartials
     size_t partial2_count = 0;   // capacity of d_partials2
     size_t energy_partials = 0;
@@ -204,26 +208,33 @@ struct Engine {
     void build_plan();
     const double2 *final_state() const;
     void require_partials(size_t count) const;
+    double *pass_partials() const;
+    void queue_grad(const PassPlan &pp, int l, const double *scale, hipStream_t s);
+    void finish_grads(const Layer0Reduce &l0, const double *scale, hipStream_t s);
     int free_buffer(std::initializer_list<int> used) const;
 
     void stage_begin(hipStream_t s);
     void stage_end(hipStream_t s, const char *name);
 
-    void structured_forward(hipStream_t s, bool save_ckpts);
+    void structured_forward(hipStream_t s, bool save_ckpts, const double *params = nullptr);
     void structured_hamiltonian(hipStream_t s, bool write_lam);
     bool fused_eval() const;
     void structured_hamiltonian_fused(hipStream_t s);
-    void structured_eval_fused(hipStream_t s, const double *scale, double *energy_out,
-                               bool staged);
+    void structured_eval_fused(hipStream_t s, const double *params, const double *scale,
+                               double *energy_out, bool staged);
     void launch_bwd(int l, bool gather, bool write_cur, const double2 *cur_in,
                     const double2 *lam_in, double2 *cur_out, double2 *lam_out, size_t p,
                     hipStream_t s, int gen_set = -1, const PassGeom *geom = nullptr,
                     bool phase_free = false);
     bool gen_ready() const;
     bool gen_start_ready() const;
-    void build_chain_tables(hipStream_t s, int r_set0 = -1, bool bottom_up = false);
-    void structured_eval_gen_start(hipStream_t s, const double *scale, double *energy_out,
-                                   bool staged);
+    void build_chain_tables(hipStream_t s, const double *params = nullptr, int r_set0 = -1,
+                            bool bottom_up = false, ChainPrep prep = {});
+    void rebuild_chain_tables(hipStream_t s);
+    const double *start_coefs(const double *params, hipStream_t s);
+    int chain_rh = 0;  // adjoint register shape of the tables, high passes from the top down
+    void structured_eval_gen_start(hipStream_t s, const double *params, const double *scale,
+                                   double *energy_out, bool staged);
     void structured_backward(hipStream_t s, const double *scale, bool full_walk);
     void structured_backward_stored(hipStream_t s, const double *scale);
     void layer0_gradients(hipStream_t s, const double2 *lam, const double *scale);

@@ -569,51 +569,6 @@ void launch_fwd_pass(int R, bool scatter, bool gen_init, const double2 *in, doub
 // Layer-1 states generated from the parameters (chain_site): tables.
 // ---------------------------------------------------------------------------
 
-// One workgroup per table set: the 2n site matrices in LDS, then the
-// register-run products tab[0, 2^R) and the chunk products C0 at tab[16 + v]
-// and C1 at tab[32 + v].
-__global__ __launch_bounds__(256) void chain_tables_kernel(const WireCoef *__restrict__ lc0,
-                                                           const WireCoef *__restrict__ lc1,
-                                                           ChainSetup cs, CMat2 *__restrict__ tabs) {
-    __shared__ CMat2 site[2 * 64];
-    const ChainSet st = cs.set[blockIdx.x];
-    const int n = cs.n;
-    for (int i = (int)threadIdx.x; i < 2 * n; i += (int)blockDim.x) {
-        const int w = i >> 1;
-        site[i] = chain_site(w, i & 1, lc0[w], lc1[w], ((st.rot >> w) & 1u) != 0,
-                             ((st.ry_only >> w) & 1u) == 0);
-    }
-    __syncthreads();
-    CMat2 *tab = tabs + (size_t)blockIdx.x * kChainTabEntries;
-    for (int e = (int)threadIdx.x; e < kChainTabEntries; e += (int)blockDim.x) {
-        int first;
-        int len;
-        int v;
-        if (e < kChainC0) {
-            first = st.r0;
-            len = st.R;
-            v = e;
-        } else if (e < kChainC1) {
-            first = st.c0_first;
-            len = st.c0_len;
-            v = e - kChainC0;
-        } else {
-            first = st.c1_first;
-            len = st.c1_len;
-            v = e - kChainC1;
-        }
-        if (len == 0 || v >= (1 << len)) {
-            continue;
-        }
-        CMat2 p = site[2 * first + (v & 1)];
-        for (int b = 1; b < len; ++b) {
-            const int w = first + b;
-            p = cmat_mul(p, site[2 * w + ((v >> b) & 1)]);
-        }
-        tab[e] = p;
-    }
-}
-
 // Product of the site matrices of wires [first, first + len) at the bits of
 // index i (the identity when len is 0).
 __device__ __forceinline__ CMat2 chain_segment(const CMat2 *site, int first, int len,
@@ -627,22 +582,130 @@ __device__ __forceinline__ CMat2 chain_segment(const CMat2 *site, int first, int
     return p;
 }
 
-// The tile-uniform segments of every tile: utab[2g] = U_A (wires [r0 + R, n)),
-// utab[2g + 1] = U_B, at the bits of tile g's base index.  grid.y: table set.
-__global__ __launch_bounds__(256) void chain_uniform_kernel(const WireCoef *__restrict__ lc0,
-                                                            const WireCoef *__restrict__ lc1,
-                                                            ChainSetup cs,
-                                                            CMat2 *__restrict__ utab) {
+// Everything that an evaluation derives from its parameters before its first
+// pass, in one launch whose workgroups take different parts.  A launch is bound by
+// its own 3 to 5 us here, not by the work: with this one and reduce_kernel in
+// place of one per part and pass, 17 qubits x 2 layers take 4 launches instead of
+// 13 and 78 us instead of 108 through the host call, 20 qubits x 4 layers 248
+// instead of 281.
+//   the coefficient table (all layers);
+//   per table set, from the 2n site matrices in LDS, the register-run products
+//   tab[0, 2^R) and the chunk products C0 at tab[16 + v] and C1 at tab[32 + v];
+//   per set and tile the uniform segments utab[2g] = U_A (wires [r0 + R, n)) and
+//   utab[2g + 1] = U_B, at the bits of tile g's base index;
+//   per tile the flipped segments of set 0 (see ChainPrep).  The sum over the
+//   pairs above the tile is one left-to-right walk over the sites T .. n-1 with
+//   three running products: A the plain prefix, C the prefix whose last site is
+//   flipped (a pair waiting for its partner), B the sum of prefixes with one
+//   completed flipped pair;
+//   per tile the lambda addresses of each pass, and the top pass's fixed-wire
+//   factor phi_C(g) = prod_{4 <= v < h} u_v(g_{v-3} ^ g_{v-4}).
+// With params the coefficients come from there, else from the table.
+__device__ __forceinline__ WireCoef coef_of(const double *__restrict__ params,
+                                            const WireCoef *__restrict__ coef, int i) {
+    if (params == nullptr) {
+        return coef[i];
+    }
+    WireCoef k;
+    sincos(0.5 * params[2 * i], &k.s, &k.c);
+    sincos(0.5 * params[2 * i + 1], &k.sh, &k.ch);
+    return k;
+}
+
+__global__ __launch_bounds__(256) void chain_prep_kernel(ChainPrep P) {
     __shared__ CMat2 site[2 * 64];
-    const ChainSet st = cs.set[blockIdx.y];
+    __shared__ WireCoef lc[2][64];
+    const ChainSetup &cs = P.cs;
     const int n = cs.n;
-    for (int i = (int)threadIdx.x; i < 2 * n; i += (int)blockDim.x) {
+    const int t = (int)threadIdx.x;
+    const int per_tile = (int)((cs.tiles + 255) / 256);  // workgroups of a per-tile part
+    int b = (int)blockIdx.x;
+    // the part of this workgroup, and its place there
+    int part = 0;
+    const int sizes[6] = {cs.count,
+                          cs.count * per_tile,
+                          P.xtab != nullptr ? per_tile : 0,
+                          P.table_count * per_tile,
+                          P.phi_c != nullptr ? per_tile : 0,
+                          P.params != nullptr ? (P.coefs + 255) / 256 : 0};
+    while (part < 5 && b >= sizes[part]) {
+        b -= sizes[part];
+        ++part;
+    }
+    if (part == 3) {
+        const LamTable &tab = P.tables[b / per_tile];
+        const uint64_t g = (uint64_t)(b % per_tile) * 256 + t;
+        if (g < cs.tiles) {
+            PassGeom G{};
+            G.a = tab.a;
+            G.h0 = tab.h0;
+            tab.out[g] = lay_addr(tile_base(g, G, Tile<4>::T), tab.layout);
+        }
+        return;
+    }
+    if (part == 5) {
+        const int i = b * 256 + t;
+        if (i < P.coefs) {
+            P.coef[i] = coef_of(P.params, nullptr, i);
+        }
+        return;
+    }
+    for (int i = t; i < 2 * n; i += 256) {
+        lc[i >= n][i >= n ? i - n : i] = coef_of(P.params, P.coef, i);
+    }
+    __syncthreads();
+    if (part == 4) {
+        const uint64_t g = (uint64_t)b * 256 + t;
+        if (g < cs.tiles) {
+            double2 f = make_double2(1.0, 0.0);
+            for (int v = 4; v < P.phi_h0; ++v) {
+                f = cmul(f, (((g >> (v - 3)) ^ (g >> (v - 4))) & 1u) ? u1_of(lc[0][v])
+                                                                     : u0_of(lc[0][v]));
+            }
+            P.phi_c[g] = f;
+        }
+        return;
+    }
+    const int set = part == 0 ? b : part == 1 ? b / per_tile : 0;
+    const ChainSet st = cs.set[set];
+    for (int i = t; i < 2 * n; i += 256) {
         const int w = i >> 1;
-        site[i] = chain_site(w, i & 1, lc0[w], lc1[w], ((st.rot >> w) & 1u) != 0,
+        site[i] = chain_site(w, i & 1, lc[0][w], lc[1][w], ((st.rot >> w) & 1u) != 0,
                              ((st.ry_only >> w) & 1u) == 0);
     }
     __syncthreads();
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (part == 0) {
+        CMat2 *tab = P.tabs + (size_t)set * kChainTabEntries;
+        for (int e = t; e < kChainTabEntries; e += 256) {
+            int first;
+            int len;
+            int v;
+            if (e < kChainC0) {
+                first = st.r0;
+                len = st.R;
+                v = e;
+            } else if (e < kChainC1) {
+                first = st.c0_first;
+                len = st.c0_len;
+                v = e - kChainC0;
+            } else {
+                first = st.c1_first;
+                len = st.c1_len;
+                v = e - kChainC1;
+            }
+            if (len == 0 || v >= (1 << len)) {
+                continue;
+            }
+            CMat2 p = site[2 * first + (v & 1)];
+            for (int k = 1; k < len; ++k) {
+                const int w = first + k;
+                p = cmat_mul(p, site[2 * w + ((v >> k) & 1)]);
+            }
+            tab[e] = p;
+        }
+        return;
+    }
+    const uint64_t g = (uint64_t)(part == 1 ? b % per_tile : b) * 256 + t;
     if (g >= cs.tiles) {
         return;
     }
@@ -650,45 +713,14 @@ __global__ __launch_bounds__(256) void chain_uniform_kernel(const WireCoef *__re
     G.a = st.ta;
     G.h0 = st.th0;
     const uint64_t base = tile_base(g, G, Tile<4>::T);
-    CMat2 *u = utab + ((size_t)blockIdx.y * cs.tiles + g) * 2;
-    u[0] = chain_segment(site, st.r0 + st.R, n - st.r0 - st.R, base);
-    u[1] = chain_segment(site, st.ub_first, st.ub_len, base);
-}
-
-void launch_chain_tables(const WireCoef *lc0, const WireCoef *lc1, const ChainSetup &cs,
-                         CMat2 *tabs, CMat2 *utab, hipStream_t s) {
-    chain_tables_kernel<<<cs.count, 256, 0, s>>>(lc0, lc1, cs, tabs);
-    const dim3 grid((unsigned)((cs.tiles + 255) / 256), (unsigned)cs.count);
-    chain_uniform_kernel<<<grid, 256, 0, s>>>(lc0, lc1, cs, utab);
-}
-
-// The flipped segments of table set 0 per tile (see launch_chain_flips in the
-// header).  The sum over the pairs above the tile is one left-to-right walk
-// over the sites T .. n-1 with three running products: A the plain prefix,
-// C the prefix whose last site is flipped (a pair waiting for its partner),
-// B the sum of prefixes with one completed flipped pair.
-__global__ __launch_bounds__(256) void chain_flip_kernel(const WireCoef *__restrict__ lc0,
-                                                         const WireCoef *__restrict__ lc1,
-                                                         ChainSetup cs, CMat2 *__restrict__ xtab) {
-    __shared__ CMat2 site[2 * 64];
-    const ChainSet st = cs.set[0];
-    const int n = cs.n;
-    for (int i = (int)threadIdx.x; i < 2 * n; i += (int)blockDim.x) {
-        const int w = i >> 1;
-        site[i] = chain_site(w, i & 1, lc0[w], lc1[w], ((st.rot >> w) & 1u) != 0,
-                             ((st.ry_only >> w) & 1u) == 0);
-    }
-    __syncthreads();
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= cs.tiles) {
+    if (part == 1) {
+        CMat2 *u = P.utab + ((size_t)set * cs.tiles + g) * 2;
+        u[0] = chain_segment(site, st.r0 + st.R, n - st.r0 - st.R, base);
+        u[1] = chain_segment(site, st.ub_first, st.ub_len, base);
         return;
     }
-    PassGeom G{};
-    G.a = st.ta;
-    G.h0 = st.th0;
     const int lo = st.r0 + st.R;  // the low tile's top: U_A covers wires [lo, n)
-    const uint64_t base = tile_base(g, G, Tile<4>::T);
-    CMat2 *x = xtab + g * kFlipSegments;
+    CMat2 *x = P.xtab + g * kFlipSegments;
     x[0] = chain_segment(site, lo, n - lo, base ^ (uint64_t{1} << lo));
     x[1] = chain_segment(site, lo, n - lo, base ^ (uint64_t{1} << (n - 1)));
     const CMat2 zero = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
@@ -696,9 +728,9 @@ __global__ __launch_bounds__(256) void chain_flip_kernel(const WireCoef *__restr
     CMat2 C = site[2 * lo + (int)(((base >> lo) & 1u) ^ 1u)];
     CMat2 B = zero;
     for (int v = lo + 1; v < n; ++v) {
-        const int b = (int)((base >> v) & 1u);
-        const CMat2 &sv = site[2 * v + b];
-        const CMat2 &sf = site[2 * v + (b ^ 1)];
+        const int bit = (int)((base >> v) & 1u);
+        const CMat2 &sv = site[2 * v + bit];
+        const CMat2 &sf = site[2 * v + (bit ^ 1)];
         B = cmat_add(cmat_mul(B, sv), cmat_mul(C, sf));
         C = cmat_mul(A, sf);
         A = cmat_mul(A, sv);
@@ -706,9 +738,12 @@ __global__ __launch_bounds__(256) void chain_flip_kernel(const WireCoef *__restr
     x[2] = B;
 }
 
-void launch_chain_flips(const WireCoef *lc0, const WireCoef *lc1, const ChainSetup &cs,
-                        CMat2 *xtab, hipStream_t s) {
-    chain_flip_kernel<<<(unsigned)((cs.tiles + 255) / 256), 256, 0, s>>>(lc0, lc1, cs, xtab);
+void launch_chain_prep(const ChainPrep &p, hipStream_t s) {
+    const int per_tile = (int)((p.cs.tiles + 255) / 256);
+    const int blocks = p.cs.count + per_tile * (p.cs.count + (p.xtab != nullptr ? 1 : 0) +
+                                                p.table_count + (p.phi_c != nullptr ? 1 : 0)) +
+                       (p.params != nullptr ? (p.coefs + 255) / 256 : 0);
+    chain_prep_kernel<<<blocks, 256, 0, s>>>(p);
 }
 
 // Y of the forward's low tile at row i (run bits zero): U_A . C0 . C1 with C0
@@ -2228,31 +2263,6 @@ void launch_ham_pass(int R, bool diag, bool read_lam, bool write_lam, const doub
 // Fixed-order reductions.
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(64) void reduce_grad_kernel(const double *__restrict__ partials,
-                                                         int num_blocks, int T, PassGeom G,
-                                                         int layer, double *__restrict__ grad,
-                                                         const double *__restrict__ scale) {
-    const int col = 2 * G.rot_lo + blockIdx.x;  // 2 * tile bit + component
-    const int j = col >> 1;
-    const int comp = col & 1;
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < num_blocks; b += 64) {
-        acc += partials[(uint64_t)b * (2 * T) + col];
-    }
-    acc = wave_sum(acc);
-    if (threadIdx.x == 0) {
-        const int wire = tile_wire(j, G);
-        const double f = scale != nullptr ? *scale : 1.0;
-        grad[((uint64_t)layer * G.n + wire) * 2 + comp] = acc * f;
-    }
-}
-
-void launch_reduce_grad(const double *partials, int num_blocks, int T, const PassGeom &g,
-                        int layer, double *grad, const double *scale, hipStream_t s) {
-    const int cols = 2 * (g.rot_hi - g.rot_lo);
-    reduce_grad_kernel<<<cols, 64, 0, s>>>(partials, num_blocks, T, g, layer, grad, scale);
-}
-
 __global__ __launch_bounds__(256) void reduce_sum_kernel(const double *__restrict__ values,
                                                          int count, double *__restrict__ out,
                                                          const double *__restrict__ scale) {
@@ -2698,49 +2708,6 @@ __global__ __launch_bounds__(512, 4) void layer0_contract_r3_kernel(
     }
 }
 
-// Environments of the high wires v in [12, n) from the per-tile sums S(g):
-// E_v[b] = sum_{g : bit v of (g << 12) = b} S(g) prod_{u >= 12, u != v} u_u(bit).
-// Block (v - 12, chunk) writes 4 doubles (E_v[0], E_v[1]) into partials.
-__global__ __launch_bounds__(256) void layer0_high_env_kernel(
-    const double2 *__restrict__ tile_sums, uint64_t num_tiles, const WireCoef *__restrict__ lc0,
-    int n, double *__restrict__ partials) {
-    constexpr int T = 12;
-    __shared__ double red[4][4];
-    const int v = T + blockIdx.y;
-    const int t = threadIdx.x;
-    double2 e0 = make_double2(0.0, 0.0);
-    double2 e1 = make_double2(0.0, 0.0);
-    const uint64_t stride = (uint64_t)gridDim.x * 256;
-    for (uint64_t g = (uint64_t)blockIdx.x * 256 + t; g < num_tiles; g += stride) {
-        double2 f = tile_sums[g];
-        for (int u = T; u < n; ++u) {
-            if (u != v) {
-                f = cmul(f, u_of(lc0[u], (int)((g >> (u - T)) & 1U)));
-            }
-        }
-        if ((g >> (v - T)) & 1U) {
-            e1.x += f.x;
-            e1.y += f.y;
-        } else {
-            e0.x += f.x;
-            e0.y += f.y;
-        }
-    }
-    const double vals[4] = {e0.x, e0.y, e1.x, e1.y};
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const double r = wave_sum(vals[c]);
-        if ((t & 63) == 0) {
-            red[t >> 6][c] = r;
-        }
-    }
-    __syncthreads();
-    if (t < 4) {
-        partials[((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + t] =
-            red[0][t] + red[1][t] + red[2][t] + red[3][t];
-    }
-}
-
 // Gradients of layer-0 wire w from its environments e = (E_w[0], E_w[1]) as
 // {re, im, re, im}: d u / d theta = (-s/2 e-, c/2 e+),
 // d u / d phi = (-i/2 c e-, +i/2 s e+), e-+ = e^{-+i phi/2}.  Wire 0 also
@@ -2769,40 +2736,6 @@ __device__ __forceinline__ void layer0_wire_result(const WireCoef &k, const doub
     }
 }
 
-// Layer-0 gradients from the environments of the low-tile contraction
-// (wires 0..11, per workgroup) and of layer0_high_env (wires 12..n-1).
-__global__ __launch_bounds__(64) void layer0_finish_kernel(
-    const double *__restrict__ low_partials, int low_blocks, const double *__restrict__ high_partials,
-    int high_chunks, const WireCoef *__restrict__ lc0, int n, double *__restrict__ grad,
-    const double *__restrict__ scale, double *__restrict__ energy_out) {
-    const int w = blockIdx.x;  // wire
-    const int t = threadIdx.x;
-    double e[4] = {0.0, 0.0, 0.0, 0.0};
-    if (w < 12) {
-        const int col = (w < 8) ? 4 * w : 32 + 4 * (w - 8);
-        for (int b = t; b < low_blocks; b += 64) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                e[c] += low_partials[(uint64_t)b * 48 + col + c];
-            }
-        }
-    } else {
-        for (int b = t; b < high_chunks; b += 64) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                e[c] += high_partials[((uint64_t)(w - 12) * high_chunks + b) * 4 + c];
-            }
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        e[c] = wave_sum(e[c]);
-    }
-    if (t == 0) {
-        layer0_wire_result(lc0[w], e, w, grad, scale, energy_out);
-    }
-}
-
 void launch_layer0_contract(int R, const double2 *lam, const WireCoef *lc0, const PassGeom &g,
                             double2 *tile_sums, double *partials, int grid, hipStream_t s) {
     if (R == 3) {
@@ -2810,22 +2743,6 @@ void launch_layer0_contract(int R, const double2 *lam, const WireCoef *lc0, cons
     } else {
         layer0_contract_kernel<<<grid, 256, 0, s>>>(lam, lc0, g, tile_sums, partials);
     }
-}
-
-void launch_layer0_high_env(const double2 *tile_sums, uint64_t num_tiles, const WireCoef *lc0,
-                            int n, double *partials, int chunks, hipStream_t s) {
-    if (n <= 12) {
-        return;
-    }
-    dim3 grid(chunks, n - 12);
-    layer0_high_env_kernel<<<grid, 256, 0, s>>>(tile_sums, num_tiles, lc0, n, partials);
-}
-
-void launch_layer0_finish(const double *low_partials, int low_blocks, const double *high_partials,
-                          int high_chunks, const WireCoef *lc0, int n, double *grad,
-                          const double *scale, hipStream_t s, double *energy_out) {
-    layer0_finish_kernel<<<n, 64, 0, s>>>(low_partials, low_blocks, high_partials, high_chunks,
-                                          lc0, n, grad, scale, energy_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -2846,7 +2763,7 @@ void launch_layer0_finish(const double *low_partials, int low_blocks, const doub
 // the register wires n-4 .. n-1 per thread (contract_reg4), the thread wires
 // from per-thread sums split by x = j_3 ^ parity(q_0, q_1, q_2) (wire 3's
 // factor is u_3(x)), the fixed wires 4 .. h-1 from per-tile sums S(g)
-// (layer0_fixed_env_kernel) and the per-tile product phi_c(g) of their factors.
+// (layer0_fixed_env) and the per-tile product phi_c(g) of their factors.
 // ---------------------------------------------------------------------------
 
 // q of top-tile offset o (bits 0..2: j_0..j_2, bits 3..11: j_h..j_{n-1})
@@ -2860,37 +2777,6 @@ __device__ __forceinline__ uint32_t top_q_of_offset(uint32_t o) {
 // Wire of q bit b in the top tile.
 __device__ __forceinline__ int top_wire(int b, int h) {
     return b < 3 ? b : h + (b - 3);
-}
-
-// Per top tile g: phi_c[g] = prod_{v = 4}^{h-1} u_v(j_v ^ j_{v-1}) (j_{3+m} =
-// bit m of g) and lam_tile[g], the address of the tile's base index in the
-// layout the pass reads.
-__global__ __launch_bounds__(256) void lam_tile_table_kernel(PassGeom G, LamLayout L,
-                                                             uint64_t *__restrict__ out) {
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < G.num_tiles) {
-        out[g] = lay_addr(tile_base(g, G, Tile<4>::T), L);
-    }
-}
-
-void launch_lam_tile_table(const PassGeom &g, const LamLayout &L, uint64_t *out, hipStream_t s) {
-    lam_tile_table_kernel<<<(unsigned)((g.num_tiles + 255) / 256), 256, 0, s>>>(g, L, out);
-}
-
-__global__ __launch_bounds__(256) void layer0_top_factor_kernel(const WireCoef *__restrict__ lc0,
-                                                                PassGeom G,
-                                                                double2 *__restrict__ phi_c,
-                                                                uint64_t *__restrict__ lam_tile) {
-    const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= G.num_tiles) {
-        return;
-    }
-    double2 f = make_double2(1.0, 0.0);
-    for (int v = 4; v < G.h0; ++v) {
-        f = cmul(f, u_of(lc0[v], (int)(((g >> (v - 3)) ^ (g >> (v - 4))) & 1u)));
-    }
-    phi_c[g] = f;
-    lam_tile[g] = lay_addr(tile_base(g, G, Tile<4>::T), G.lay_in);
 }
 
 // Per-block partials of the fused pass: layer-1 gradients as bwd_lam_kernel
@@ -3096,20 +2982,71 @@ __global__ __launch_bounds__(256, 2) void bwd_top_l0_kernel(
     }
 }
 
+void launch_bwd_top_l0(const double2 *lam_in, const WireCoef *layer_coef, const PassGeom &g,
+                       double *partials, int grid, hipStream_t s, const CMat2 *gen_tab,
+                       const CMat2 *gen_utab, const WireCoef *lc0, const double2 *phi_c,
+                       const uint64_t *lam_tile, double2 *tile_sums, double *l0_partials) {
+    if (g.a != 3 || g.h0 + 9 != g.n || g.h0 < 4 || g.rot_lo < 3 || g.lay_out.count != 0 ||
+        !lay_fits(g.lay_in, g.n, g.h0 + 5, 4)) {
+        throw std::invalid_argument("layer-0 contraction in a high pass: top group tiles only");
+    }
+    bwd_top_l0_kernel<<<grid, Tile<4>::THREADS, 0, s>>>(lam_in, layer_coef, g, partials, gen_tab,
+                                                        gen_utab, lc0, phi_c, lam_tile, tile_sums,
+                                                        l0_partials);
+}
+
+// Environments of the high wires v in [12, n) from the per-tile sums S(g):
+// E_v[b] = sum_{g : bit v of (g << 12) = b} S(g) prod_{u >= 12, u != v} u_u(bit).
+// One workgroup: wire v, the tiles of chunk `chunk` of `chunks`; 4 doubles
+// (E_v[0], E_v[1]) of its 4 waves to red.
+__device__ __forceinline__ void layer0_high_env(const double2 *__restrict__ tile_sums,
+                                                uint64_t num_tiles,
+                                                const WireCoef *__restrict__ lc0, int n, int v,
+                                                int chunk, int chunks, double *red) {
+    constexpr int T = 12;
+    const int t = threadIdx.x;
+    double2 e0 = make_double2(0.0, 0.0);
+    double2 e1 = make_double2(0.0, 0.0);
+    const uint64_t stride = (uint64_t)chunks * 256;
+    for (uint64_t g = (uint64_t)chunk * 256 + t; g < num_tiles; g += stride) {
+        double2 f = tile_sums[g];
+        for (int u = T; u < n; ++u) {
+            if (u != v) {
+                f = cmul(f, u_of(lc0[u], (int)((g >> (u - T)) & 1U)));
+            }
+        }
+        if ((g >> (v - T)) & 1U) {
+            e1.x += f.x;
+            e1.y += f.y;
+        } else {
+            e0.x += f.x;
+            e0.y += f.y;
+        }
+    }
+    const double vals[4] = {e0.x, e0.y, e1.x, e1.y};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const double r = wave_sum(vals[c]);
+        if ((t & 63) == 0) {
+            red[(t >> 6) * 4 + c] = r;
+        }
+    }
+}
+
 // Environments of the fixed wires v in [4, h) of the top-group tiles from the
 // per-tile sums (waves partials per tile):
 // E_v[b] = sum_{g : i_v(g) = b} S(g) prod_{u in [4, h), u != v} u_u(i_u(g)),
 // i_u(g) = j_u ^ j_{u-1}, j_{3+m} = bit m of g.  One thread per tile forms all
 // of them from prefix and suffix products of the tile's factors (one read of
-// the tile sums, O(h) products); block `chunk` writes 4 doubles per wire at
-// ((v - 4) * chunks + chunk) * 4.
+// the tile sums, O(h) products); 4 doubles per wire of each of the workgroup's
+// 4 waves go to red.
 constexpr int kMaxFixedWires = 18;  // h - 4 = n - 13 for n <= 31
 
-__global__ __launch_bounds__(256) void layer0_fixed_env_kernel(
-    const double2 *__restrict__ tile_sums, int waves, uint64_t num_tiles,
-    const WireCoef *__restrict__ lc0, int h, double *__restrict__ partials) {
+__device__ __forceinline__ void layer0_fixed_env(const double2 *__restrict__ tile_sums, int waves,
+                                                 uint64_t num_tiles,
+                                                 const WireCoef *__restrict__ lc0, int h,
+                                                 int chunk, int chunks, double *red) {
     constexpr int M = kMaxFixedWires;
-    __shared__ double red[4][4 * M];
     const int m = h - 4;
     const int t = threadIdx.x;
     double2 e0[M];
@@ -3119,8 +3056,8 @@ __global__ __launch_bounds__(256) void layer0_fixed_env_kernel(
         e0[i] = make_double2(0.0, 0.0);
         e1[i] = make_double2(0.0, 0.0);
     }
-    const uint64_t stride = (uint64_t)gridDim.x * 256;
-    for (uint64_t g = (uint64_t)blockIdx.x * 256 + t; g < num_tiles; g += stride) {
+    const uint64_t stride = (uint64_t)chunks * 256;
+    for (uint64_t g = (uint64_t)chunk * 256 + t; g < num_tiles; g += stride) {
         double2 f = tile_sums[g * waves];
         for (int w = 1; w < waves; ++w) {
             const double2 p = tile_sums[g * waves + w];
@@ -3161,85 +3098,160 @@ __global__ __launch_bounds__(256) void layer0_fixed_env_kernel(
             for (int c = 0; c < 4; ++c) {
                 const double r = wave_sum(vals[c]);
                 if ((t & 63) == 0) {
-                    red[t >> 6][4 * i + c] = r;
+                    red[(t >> 6) * (4 * m) + 4 * i + c] = r;
                 }
             }
         }
     }
+}
+
+// The sums that end an evaluation, in one launch whose workgroups take
+// different parts: the gradient entries of the queued passes from their
+// per-workgroup partials (2T values per workgroup, tile bit j's dtheta and dphi
+// at 2j, 2j + 1; one workgroup per entry), the layer-0 wires of the contraction's
+// own tile (per-workgroup values; one workgroup per wire), and the environments
+// of the wires fixed by its tiles, per chunk of tiles.  Where one chunk takes
+// all tiles (n <= 20) its workgroup writes those wires' results too, else
+// layer0_finish_kernel does.  Fixed order throughout.  Bound by
+// the latency of its strided reads (28 us at 27 qubits x 3 layers, where one
+// launch of 64 threads per entry and pass took 7 x 30).
+__global__ __launch_bounds__(256) void reduce_kernel(GradReduce jobs, int T, Layer0Reduce l0,
+                                                     const double *__restrict__ scale) {
+    __shared__ double red[4 * 4 * kMaxFixedWires];
+    const int t = (int)threadIdx.x;
+    int c = (int)blockIdx.x;
+    int k = 0;
+    while (k < jobs.count && c >= jobs.job[k].cols) {
+        c -= jobs.job[k].cols;
+        ++k;
+    }
+    if (k < jobs.count) {
+        const GradReduceJob &J = jobs.job[k];
+        const int col = J.first_col + c;
+        double acc = 0.0;
+        for (int b = t; b < J.blocks; b += 256) {
+            acc += J.partials[(uint64_t)b * (2 * T) + col];
+        }
+        acc = wave_sum(acc);
+        if ((t & 63) == 0) {
+            red[t >> 6] = acc;
+        }
+        __syncthreads();
+        if (t == 0) {
+            const int j = col >> 1;
+            const int wire = j < J.a ? j : J.h0 + (j - J.a);
+            const double f = scale != nullptr ? *scale : 1.0;
+            J.grad[2 * wire + (col & 1)] = ((red[0] + red[1]) + (red[2] + red[3])) * f;
+        }
+        return;
+    }
+    const int n = l0.n;
+    const int h = n - 9;  // the top group's tiles: wires 0..2 and [h, n), and 3 by its split
+    const int own = l0.top ? 13 : 12;
+    if (c < own) {
+        const int w = !l0.top || c < 4 ? c : h + (c - 4);
+        const int cols = l0.top ? kTopL0Cols : 48;
+        int col = w < 8 ? 4 * w : 32 + 4 * (w - 8);
+        if (l0.top) {
+            col = w < 3       ? 4 * w
+                  : w == 3    ? 48
+                  : w < h + 5 ? 4 * (3 + w - h)
+                              : 32 + 4 * (w - h - 5);
+        }
+        double e[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int b = t; b < l0.blocks; b += 256) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                e[q] += l0.partials[(uint64_t)b * cols + col + q];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            e[q] = wave_sum(e[q]);
+            if ((t & 63) == 0) {
+                red[(t >> 6) * 4 + q] = e[q];
+            }
+        }
+        __syncthreads();
+        if (t == 0) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                e[q] = (red[q] + red[4 + q]) + (red[8 + q] + red[12 + q]);
+            }
+            layer0_wire_result(l0.lc0[w], e, w, l0.grad, scale, l0.energy);
+        }
+        return;
+    }
+    // fixed wires [first, first + count)
+    c -= own;
+    const int chunk = c % l0.chunks;
+    int first = 4;
+    int count = h - 4;
+    if (l0.top) {
+        layer0_fixed_env(l0.tile_sums, Tile<4>::WAVES, l0.tiles, l0.lc0, h, chunk, l0.chunks, red);
+    } else {
+        first = 12 + c / l0.chunks;
+        count = 1;
+        layer0_high_env(l0.tile_sums, l0.tiles, l0.lc0, n, first, chunk, l0.chunks, red);
+    }
     __syncthreads();
-    for (int k = t; k < 4 * m; k += 256) {
-        partials[((uint64_t)(k >> 2) * gridDim.x + blockIdx.x) * 4 + (k & 3)] =
-            red[0][k] + red[1][k] + red[2][k] + red[3][k];
+    if (t < 4 * count) {
+        red[t] = (red[t] + red[4 * count + t]) + (red[8 * count + t] + red[12 * count + t]);
+    }
+    __syncthreads();
+    if (l0.chunks == 1) {
+        if (t < count) {
+            const double e[4] = {red[4 * t], red[4 * t + 1], red[4 * t + 2], red[4 * t + 3]};
+            layer0_wire_result(l0.lc0[first + t], e, first + t, l0.grad, scale, l0.energy);
+        }
+    } else if (t < 4 * count) {
+        const int i = first - (l0.top ? 4 : 12) + (t >> 2);
+        l0.env[((uint64_t)i * l0.chunks + chunk) * 4 + (t & 3)] = red[t];
     }
 }
 
-// Layer-0 gradients (and the energy) from the fused pass's per-block partials
-// and the fixed wires' chunks.
-__global__ __launch_bounds__(64) void layer0_finish_top_kernel(
-    const double *__restrict__ blk_partials, int blocks, const double *__restrict__ fixed_partials,
-    int chunks, const WireCoef *__restrict__ lc0, int n, double *__restrict__ grad,
-    const double *__restrict__ scale, double *__restrict__ energy_out) {
-    const int w = blockIdx.x;
-    const int t = threadIdx.x;
-    const int h = n - 9;
+// The fixed wires' results from their chunks (wire first + blockIdx.x).
+__global__ __launch_bounds__(64) void layer0_finish_kernel(Layer0Reduce l0, int first,
+                                                           const double *__restrict__ scale) {
+    const int w = first + (int)blockIdx.x;
+    const int t = (int)threadIdx.x;
     double e[4] = {0.0, 0.0, 0.0, 0.0};
-    if (w >= 4 && w < h) {
-        for (int b = t; b < chunks; b += 64) {
+    for (int b = t; b < l0.chunks; b += 64) {
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                e[c] += fixed_partials[((uint64_t)(w - 4) * chunks + b) * 4 + c];
-            }
-        }
-    } else {
-        const int col = w < 3        ? 4 * w
-                        : w == 3     ? 48
-                        : w < h + 5  ? 4 * (3 + w - h)
-                                     : 32 + 4 * (w - h - 5);
-        for (int b = t; b < blocks; b += 64) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                e[c] += blk_partials[(uint64_t)b * kTopL0Cols + col + c];
-            }
+        for (int q = 0; q < 4; ++q) {
+            e[q] += l0.env[((uint64_t)blockIdx.x * l0.chunks + b) * 4 + q];
         }
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        e[c] = wave_sum(e[c]);
+    for (int q = 0; q < 4; ++q) {
+        e[q] = wave_sum(e[q]);
     }
     if (t == 0) {
-        layer0_wire_result(lc0[w], e, w, grad, scale, energy_out);
+        layer0_wire_result(l0.lc0[w], e, w, l0.grad, scale, l0.energy);
     }
 }
 
-void launch_bwd_top_l0(const double2 *lam_in, const WireCoef *layer_coef, const PassGeom &g,
-                       double *partials, int grid, hipStream_t s, const CMat2 *gen_tab,
-                       const CMat2 *gen_utab, const WireCoef *lc0, double2 *phi_c,
-                       uint64_t *lam_tile, double2 *tile_sums, double *l0_partials) {
-    if (g.a != 3 || g.h0 + 9 != g.n || g.h0 < 4 || g.rot_lo < 3 || g.lay_out.count != 0 ||
-        !lay_fits(g.lay_in, g.n, g.h0 + 5, 4)) {
-        throw std::invalid_argument("layer-0 contraction in a high pass: top group tiles only");
+void launch_reduce(const GradReduce &jobs, int T, const Layer0Reduce &l0, const double *scale,
+                   hipStream_t s) {
+    int blocks = 0;
+    for (int k = 0; k < jobs.count; ++k) {
+        blocks += jobs.job[k].cols;
     }
-    layer0_top_factor_kernel<<<(unsigned)((g.num_tiles + 255) / 256), 256, 0, s>>>(lc0, g, phi_c,
-                                                                                  lam_tile);
-    bwd_top_l0_kernel<<<grid, Tile<4>::THREADS, 0, s>>>(lam_in, layer_coef, g, partials, gen_tab,
-                                                        gen_utab, lc0, phi_c, lam_tile, tile_sums,
-                                                        l0_partials);
-}
-
-void launch_layer0_top_finish(const double2 *tile_sums, uint64_t num_tiles, const double *blk_partials,
-                              int blocks, const WireCoef *lc0, int n, double *fixed_partials,
-                              int chunks, double *grad, const double *scale, hipStream_t s,
-                              double *energy_out) {
-    const int h = n - 9;
-    if (h - 4 > kMaxFixedWires) {
-        throw std::invalid_argument("layer-0 contraction in the top pass: too many fixed wires");
+    int fixed = 0;
+    if (l0.lc0 != nullptr) {
+        fixed = l0.n - (l0.top ? 13 : 12);
+        if (l0.top && fixed > kMaxFixedWires) {
+            throw std::invalid_argument(
+                "layer-0 contraction in the top pass: too many fixed wires");
+        }
+        blocks += l0.top ? 13 + (fixed > 0 ? l0.chunks : 0) : 12 + fixed * l0.chunks;
     }
-    if (h > 4) {
-        layer0_fixed_env_kernel<<<chunks, 256, 0, s>>>(tile_sums, Tile<4>::WAVES, num_tiles, lc0, h,
-                                                       fixed_partials);
+    if (blocks > 0) {
+        reduce_kernel<<<blocks, 256, 0, s>>>(jobs, T, l0, scale);
     }
-    layer0_finish_top_kernel<<<n, 64, 0, s>>>(blk_partials, blocks, fixed_partials, chunks, lc0, n,
-                                              grad, scale, energy_out);
+    if (fixed > 0 && l0.chunks > 1) {
+        layer0_finish_kernel<<<fixed, 64, 0, s>>>(l0, l0.top ? 4 : 12, scale);
+    }
 }
 
 // ---------------------------------------------------------------------------

@@ -49,7 +49,7 @@ struct PassGeom {
     LamLayout lay_in;
     LamLayout lay_out;
     // Per-tile lambda addresses, tile_in[g] = lay_addr(tile_base(g), lay_in)
-    // and tile_out[g] likewise (launch_lam_tile_table): the generated start's
+    // and tile_out[g] likewise (launch_chain_prep): the generated start's
     // phase-free high passes read them (tile_in, tile_out) and its low pass
     // stores through tile_out, so their tile loops do not evaluate a layout.
     const uint64_t *tile_in = nullptr;
@@ -298,8 +298,6 @@ struct ChainSetup {
 //   xtab[3g + 2] sum over w = T .. n - 2 of U_A at base ^ e_w ^ e_{w+1}
 //                                              (both bits above the tile)
 constexpr int kFlipSegments = 3;
-void launch_chain_flips(const WireCoef *lc0, const WireCoef *lc1, const ChainSetup &cs,
-                        CMat2 *xtab, hipStream_t s);
 // Generating low pass (two-layer circuits, layer 1's backward start): per low
 // tile the pre-CNOT state phi of layer 1 from chain table set 0 (tab, utab),
 // lambda = P^-1 H psi (the ZZ diagonal, the in-tile pairs [g.pair_lo,
@@ -310,10 +308,33 @@ void launch_bwd_low_gen(int R, double2 *lam_out, const WireCoef *layer_coef, con
                         double *partials, int grid, hipStream_t s, double field,
                         const CMat2 *tab, const CMat2 *utab, const CMat2 *xtab);
 
-// tabs: count * kChainTabEntries matrices, set i at tabs + i * kChainTabEntries;
-// utab: count * tiles * 2 matrices, set i at utab + i * tiles * 2.
-void launch_chain_tables(const WireCoef *lc0, const WireCoef *lc1, const ChainSetup &cs,
-                         CMat2 *tabs, CMat2 *utab, hipStream_t s);
+// Per-tile lambda addresses of one pass: out[g] = lay_addr(tile_base(g), layout)
+// for tiles of geometry (a, h0).
+struct LamTable {
+    int a;
+    int h0;
+    LamLayout layout;
+    uint64_t *out;
+};
+
+// What an evaluation prepares from its parameters (launch_chain_prep).
+// tabs: cs.count * kChainTabEntries matrices, set i at tabs + i *
+// kChainTabEntries; utab: cs.count * tiles * 2 matrices, set i at utab + i *
+// tiles * 2; xtab, tables and phi_c: the generated start's (null, none).
+struct ChainPrep {
+    const double *params;  // coefficients from here, and the table written; or
+    WireCoef *coef;        // (null) from the table
+    int coefs;             // entries of the table (n times the layers)
+    ChainSetup cs;
+    CMat2 *tabs;
+    CMat2 *utab;
+    CMat2 *xtab;
+    int table_count;
+    LamTable tables[2 * kChainMaxSets];
+    double2 *phi_c;
+    int phi_h0;
+};
+void launch_chain_prep(const ChainPrep &p, hipStream_t s);
 // Layer 1 (every wire rotated) and its ring CNOT as one write pass over the
 // low tiles; tab, utab: a set with r0 = 12 - R.
 void launch_gen_layer1(int R, double2 *out, const CMat2 *tab, const CMat2 *utab,
@@ -354,15 +375,11 @@ void launch_ham_pass_scattered(int R, const double2 *psi, double2 *lam_out, cons
 
 // Layer-0 gradients by contracting the adjoint state with the layer-0 product
 // state: one read pass over lambda (gathered through the inverse ring CNOT
-// per low tile, R = 4), a reduction of the per-tile sums over the high wires,
-// and the final per-wire assembly into grad[0 .. 2n).
+// per low tile); launch_reduce reduces its per-tile sums over the high wires and
+// assembles the results.
 // R: register shape of the contraction (4: 256 threads x 16, 3: 512 x 8).
 void launch_layer0_contract(int R, const double2 *lam, const WireCoef *lc0, const PassGeom &g,
                             double2 *tile_sums, double *partials, int grid, hipStream_t s);
-void launch_layer0_high_env(const double2 *tile_sums, uint64_t num_tiles, const WireCoef *lc0,
-                            int n, double *partials, int chunks, hipStream_t s);
-// energy_out (optional): Re <chi|mu>, the energy when lambda = H psi was carried
-// back complete (fused Hamiltonian: the pair terms are all added by then).
 // Waves of a 256-thread workgroup (register shape 4): the fused top pass
 // writes one sum per wave and tile.
 constexpr uint64_t Tile4Waves = 4;
@@ -373,27 +390,47 @@ constexpr int kTopL0Cols = 52;
 // lambda-only sweep of its wires, then, instead of storing lambda, the layer-0
 // contraction of its tiles (per-block partials: 2T layer-1 gradients in
 // partials, kTopL0Cols = 52 layer-0 values in l0_partials; per tile 4 wave
-// sums in tile_sums; phi_c and lam_tile: one value per tile, written first).
-// out[g] = lay_addr(tile_base(g, g_, T), L) for every tile of pass geometry g_.
-void launch_lam_tile_table(const PassGeom &g, const LamLayout &L, uint64_t *out, hipStream_t s);
-
+// sums in tile_sums; phi_c and lam_tile: one value per tile, from launch_chain_prep).
 void launch_bwd_top_l0(const double2 *lam_in, const WireCoef *layer_coef, const PassGeom &g,
                        double *partials, int grid, hipStream_t s, const CMat2 *gen_tab,
-                       const CMat2 *gen_utab, const WireCoef *lc0, double2 *phi_c,
-                       uint64_t *lam_tile, double2 *tile_sums, double *l0_partials);
-// The fixed wires' environments from tile_sums and the layer-0 gradients (and
-// energy) from the fused pass's partials.
-void launch_layer0_top_finish(const double2 *tile_sums, uint64_t num_tiles, const double *blk_partials,
-                              int blocks, const WireCoef *lc0, int n, double *fixed_partials,
-                              int chunks, double *grad, const double *scale, hipStream_t s,
-                              double *energy_out);
-void launch_layer0_finish(const double *low_partials, int low_blocks, const double *high_partials,
-                          int high_chunks, const WireCoef *lc0, int n, double *grad,
-                          const double *scale, hipStream_t s, double *energy_out = nullptr);
+                       const CMat2 *gen_utab, const WireCoef *lc0, const double2 *phi_c,
+                       const uint64_t *lam_tile, double2 *tile_sums, double *l0_partials);
 
-// grad[(layer*n + wire)*2 + comp] = (sum over blocks) * scale for the pass's wires.
-void launch_reduce_grad(const double *partials, int num_blocks, int T, const PassGeom &g,
-                        int layer, double *grad, const double *scale, hipStream_t s);
+// Reductions of several passes' gradient partials in one launch.
+struct GradReduceJob {
+    const double *partials;  // blocks * 2T values
+    double *grad;            // the layer's 2n values
+    int blocks;
+    int first_col;           // 2 rot_lo
+    int cols;                // 2 (rot_hi - rot_lo)
+    int a;                   // tile bit j is wire j (j < a) or h0 + j - a
+    int h0;
+};
+constexpr int kGradReduceJobs = 16;
+struct GradReduce {
+    int count;
+    GradReduceJob job[kGradReduceJobs];
+};
+// The layer-0 gradients (2n values at grad) and the energy from a contraction's
+// per-workgroup values and per-tile sums (lc0 null: none).  energy (optional):
+// Re <chi|mu>, the energy when lambda = H psi was carried back complete (fused
+// Hamiltonian: the pair terms are all added by then).
+struct Layer0Reduce {
+    const WireCoef *lc0;
+    int n;
+    bool top;                 // from launch_bwd_top_l0, else launch_layer0_contract
+    const double *partials;   // blocks * (top ? kTopL0Cols : 48) values
+    int blocks;
+    const double2 *tile_sums;
+    uint64_t tiles;
+    double *env;              // 4 * chunks values per fixed wire
+    int chunks;
+    double *grad;
+    double *energy;
+};
+// Both in one launch (two when chunks > 1).
+void launch_reduce(const GradReduce &jobs, int T, const Layer0Reduce &l0, const double *scale,
+                   hipStream_t s);
 
 // *out = sum of count values (fixed order).
 void launch_reduce_sum(const double *values, int count, double *out, hipStream_t s);
