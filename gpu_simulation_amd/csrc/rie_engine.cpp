@@ -106,13 +106,24 @@ void Engine::build_plan() {
     const int width = T - a;
     const int rest = n - T;
     const int groups = (rest + width - 1) / width;
+    // From three layers on, where the groups can leave a tile bit for the wire
+    // below them (at most width - 1 wires each, the top one exactly that many, so
+    // that each has it at tile bit a), the last layer's adjoint passes form H psi
+    // by themselves.  Left out: 13 to 19 qubits (the top group is narrower; a
+    // Hamiltonian pass costs 4 us there), 21, 29 and 30 (groups of width wires).
+    fold_ready = L >= 3 && rest >= width - 1 && rest <= groups * (width - 1);
     int g0 = T;
     for (int gi = 0; gi < groups; ++gi) {
-        const int bg = rest / groups + (gi < rest % groups ? 1 : 0);
+        int bg = rest / groups + (gi < rest % groups ? 1 : 0);
+        if (fold_ready) {
+            const int lower = rest - (width - 1);  // wires of the groups below the top one
+            bg = gi == groups - 1 ? width - 1
+                                  : lower / (groups - 1) + (gi < lower % (groups - 1) ? 1 : 0);
+        }
         PassGeom hg{};
         hg.n = n;
         hg.a = a;
-        hg.h0 = std::min(g0, n - width);
+        hg.h0 = std::min(fold_ready ? g0 - 1 : g0, n - width);
         hg.rot_lo = a + (g0 - hg.h0);
         hg.rot_hi = hg.rot_lo + bg;
         hg.num_tiles = tiles;
@@ -609,7 +620,8 @@ double *Engine::pass_partials() const {
 void Engine::queue_grad(const PassPlan &pp, int l, const double *scale, hipStream_t s) {
     const PassGeom &g = pp.g;
     greduce.job[greduce.count] = {pass_partials(), grad_dst + (size_t)l * 2 * n, pp.grid,
-                                  2 * g.rot_lo, 2 * (g.rot_hi - g.rot_lo), g.a, g.h0};
+                                  2 * g.rot_lo, 2 * (g.rot_hi - g.rot_lo), g.a, g.h0,
+                                  nullptr, 0, nullptr, 0};
     if (++greduce.count == part_slots) {
         finish_grads(Layer0Reduce{}, scale, s);
     }
@@ -639,16 +651,7 @@ int Engine::free_buffer(std::initializer_list<int> used) const {
 
 void Engine::structured_hamiltonian(hipStream_t s, bool write_lam) {
     const double2 *psi = final_state();
-    double2 *lam = nullptr;
-    if (write_lam) {
-        if (schedule == RIE_SCHEDULE_STORED && L > 1) {
-            lam_idx = -1;
-            lam = lbuf(0);
-        } else {
-            lam_idx = free_buffer({final_cur});
-            lam = pool[lam_idx];
-        }
-    }
+    double2 *lam = write_lam ? take_lam() : nullptr;
     size_t off = 0;
     const double S = (double)sizeof(double2) * (double)N;
     size_t total = 0;
@@ -687,14 +690,37 @@ void Engine::launch_bwd(int l, bool gather, bool write_cur, const double2 *cur_i
         gen_tab = d_chain + (size_t)gen_set * kChainTabEntries;
         gen_utab = d_chain_u + (size_t)gen_set * 2 * passes[0].g.num_tiles;
     }
-    const bool pairs = l == fuse_layer;
+    int ham = l == fuse_layer ? kHamPairs : kHamNone;
+    PassGeom folded = pg;
+    if (ham != kHamNone && fold_start) {
+        if (gather) {
+            ham = kHamStart;
+        } else {
+            // wires 0..11 are un-rotated, and going up from the lowest group
+            // so are those of the group below: their gradients take this
+            // pass's part where the layer's passes, the first of the
+            // evaluation, are reduced
+            const bool unrotated = p == 1 || fold_upwards;
+            const bool top = p + 1 == passes.size();
+            ham = top ? kHamFoldTop : kHamFold;
+            folded.fold_unrotated = unrotated;
+            if (unrotated) {
+                greduce.job[p - 1].above = pass_partials();
+                greduce.job[p - 1].above_blocks = pp.grid;
+            }
+            if (top) {
+                greduce.job[0].top = pass_partials();
+                greduce.job[0].top_blocks = pp.grid;
+            }
+        }
+    }
     // double buffering: the lambda-only passes load each workgroup's next tile
     // (lam of a high pass, the state of the gather pass) behind the current
     // one; the walk's one-sweep passes do not
     const bool prefetch = double_buffer && !write_cur;
     launch_bwd_pass(pass_r[gather ? RIE_PASS_BWD_LOW : RIE_PASS_BWD_HIGH], gather, write_cur, true,
-                    cur_in, lam_in, cur_out, lam_out, lc, pg, pass_partials(), pp.grid, s, pairs,
-                    pairs ? h : 0.0, gen_tab, gen_utab, prefetch, phase_free);
+                    cur_in, lam_in, cur_out, lam_out, lc, folded, pass_partials(), pp.grid, s, ham,
+                    ham != kHamNone ? h : 0.0, gen_tab, gen_utab, prefetch, phase_free);
 }
 
 // The generated start's lambda layouts.  The high passes run either from the
@@ -1032,19 +1058,21 @@ void Engine::structured_eval_gen_start(hipStream_t s, const double *params, cons
 }
 
 bool Engine::fused_eval() const {
-    return fuse_enabled && fuse_ready && on_tiles && L >= 2;
+    return fuse_enabled && (fuse_ready || fold_ready) && on_tiles && L >= 2;
+}
+
+// lambda goes where the unfused Hamiltonian puts it.
+double2 *Engine::take_lam() {
+    if (schedule == RIE_SCHEDULE_STORED && L > 1) {
+        lam_idx = -1;
+        return lbuf(0);
+    }
+    lam_idx = free_buffer({final_cur});
+    return pool[lam_idx];
 }
 
 void Engine::structured_hamiltonian_fused(hipStream_t s) {
-    // lambda goes where the unfused Hamiltonian puts it
-    double2 *lam = nullptr;
-    if (schedule == RIE_SCHEDULE_STORED) {
-        lam_idx = -1;
-        lam = lbuf(0);
-    } else {
-        lam_idx = free_buffer({final_cur});
-        lam = pool[lam_idx];
-    }
+    double2 *lam = take_lam();
     const double S = (double)sizeof(double2) * (double)N;
     kt_begin(s);
     launch_ham_pass_scattered(pass_r[RIE_PASS_HAM], final_state(), lam, ham_fused_g, h,
@@ -1053,10 +1081,30 @@ void Engine::structured_hamiltonian_fused(hipStream_t s) {
     kt_end(s, "ham_pass_fused", 2.0 * S);
 }
 
-// Energy and gradient with the fused Hamiltonian.  lambda = H psi is complete
-// once the last layer's adjoint passes have added their pair terms, and the
-// adjoint sweep is unitary, so at layer 0 <chi|mu> = <psi|H|psi>: the layer-0
-// contraction writes the energy.
+// The adjoint half of a fused evaluation: lambda = H psi is complete once the
+// last layer's adjoint passes have added their terms (with fold_ready all of
+// them: then its low pass starts lambda, else the Hamiltonian pass did).
+void Engine::structured_backward_fused(hipStream_t s, const double *scale, double *energy_out) {
+    fuse_layer = L - 1;
+    fold_start = fold_ready;
+    l0_energy_out = energy_out;
+    const auto reset = [this]() {
+        fuse_layer = -1;
+        fold_start = false;
+        l0_energy_out = nullptr;
+    };
+    try {
+        structured_backward(s, scale, false);
+    } catch (...) {
+        reset();
+        throw;
+    }
+    reset();
+}
+
+// Energy and gradient with the fused Hamiltonian.  The adjoint sweep is
+// unitary, so at layer 0 <chi|mu> = <psi|H|psi>: the layer-0 contraction writes
+// the energy.
 void Engine::structured_eval_fused(hipStream_t s, const double *params, const double *scale,
                                    double *energy_out, bool staged) {
     if (gen_start_ready()) {
@@ -1071,24 +1119,18 @@ void Engine::structured_eval_fused(hipStream_t s, const double *params, const do
         stage_end(s, "forward_apply_ms");
         stage_begin(s);
     }
-    structured_hamiltonian_fused(s);
+    if (fold_ready) {
+        take_lam();
+    } else {
+        structured_hamiltonian_fused(s);
+    }
     if (staged) {
         stage_end(s, "hamiltonian_ms");
         stage_begin(s);
         stage_end(s, "gradient_zero_ms");  // gradients are written, not accumulated
         stage_begin(s);
     }
-    fuse_layer = L - 1;
-    l0_energy_out = energy_out;
-    try {
-        structured_backward(s, scale, false);
-    } catch (...) {
-        fuse_layer = -1;
-        l0_energy_out = nullptr;
-        throw;
-    }
-    fuse_layer = -1;
-    l0_energy_out = nullptr;
+    structured_backward_fused(s, scale, energy_out);
     if (staged) {
         stage_end(s, "backward_sweep_ms");
         stage_begin(s);
@@ -1110,6 +1152,7 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
         return;
     }
     greduce.count = 0;
+    fold_upwards = true;
     int cur = final_cur;  // -2 while the state lives in a checkpoint buffer
     const double2 *cur_in = final_state();
     int lam = lam_idx;
@@ -1207,6 +1250,7 @@ void Engine::structured_backward_stored(hipStream_t s, const double *scale) {
         rebuild_chain_tables(s);
     }
     greduce.count = 0;
+    fold_upwards = false;
     int a = 0;  // lambda lives in lbuf(a)
     for (int l = L - 1; l >= 1; --l) {
         const int b = 1 - a;
@@ -1330,7 +1374,12 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
         return;
     }
     structured_forward(s, ckpt_every > 0, prep);
-    structured_hamiltonian(s, keep_lam);
+    // the adjoint passes form lambda themselves where they can
+    lam_deferred = keep_lam && fuse_enabled && fold_ready;
+    structured_hamiltonian(s, keep_lam && !lam_deferred);
+    if (lam_deferred) {
+        take_lam();
+    }
     kt_begin(s);
     launch_reduce_sum(d_epartials, (int)energy_partials, energy, s);
     check_launch("energy reduce");
@@ -1362,7 +1411,11 @@ void Engine::backward_device(const double *params, const double *scale, double *
         forward_device(params, d_energy + 1, s, true);
     }
     const GradTarget target(*this, grad);
-    structured_backward(s, scale, false);
+    if (lam_deferred) {
+        structured_backward_fused(s, scale, nullptr);
+    } else {
+        structured_backward(s, scale, false);
+    }
     resident = false;
 }
 

@@ -101,6 +101,12 @@ struct Engine {
     bool fuse_ready = false;   // the plan supports it
     bool fuse_enabled = true;  // caller's switch
     int fuse_layer = -1;       // layer whose adjoint passes add pair terms now
+    // L >= 3: that layer's adjoint passes form all of H psi, its low pass from
+    // the state alone, so no Hamiltonian pass runs and lambda is not read there.
+    bool fold_ready = false;    // the plan supports it
+    bool fold_start = false;    // the running backward does so
+    bool fold_upwards = false;  // its high passes run from the lowest group up
+    bool lam_deferred = false;  // the last forward left lambda to the backward
     // Layer-1 generation (L >= 2, n <= kChainMaxQubits): every state inside
     // layer 1 before its ring CNOT is a trace of a ring of 2x2 matrices over
     // the layer-0 product state, so layer 1's forward is one write pass and,
@@ -219,7 +225,9 @@ struct Engine {
     void structured_forward(hipStream_t s, bool save_ckpts, const double *params = nullptr);
     void structured_hamiltonian(hipStream_t s, bool write_lam);
     bool fused_eval() const;
+    double2 *take_lam();
     void structured_hamiltonian_fused(hipStream_t s);
+    void structured_backward_fused(hipStream_t s, const double *scale, double *energy_out);
     void structured_eval_fused(hipStream_t s, const double *params, const double *scale,
                                double *energy_out, bool staged);
     void launch_bwd(int l, bool gather, bool write_cur, const double2 *cur_in,

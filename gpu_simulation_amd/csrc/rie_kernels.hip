@@ -837,9 +837,15 @@ constexpr bool gather_pairs_reach() {
     return phase_first_bit<R, M>() + R - 1 >= Tile<R>::T - 4;
 }
 
-// kFullTile: pair_lo = 0 and pair_hi = T (the generating low pass), so the
-// range tests are resolved at compile time instead of held as uniform masks.
-template <int R, int M, bool kFullTile = false>
+// kFullTile: pair_lo = 0 and pair_hi = T (the generating low pass, and the low
+// pass that starts lambda), so the range tests are resolved at compile time
+// instead of held as uniform masks.
+// kRange: by uniform tests; kScaled (fold passes, pair_lo = 4): the pairs from
+// tile bit 4 on, those past pair_hi with factor 0, so that the register arrays
+// need no copies where control flow joins.
+enum class Pairs { kRange, kFullTile, kScaled };
+
+template <int R, int M, Pairs kPairs = Pairs::kRange>
 __device__ __forceinline__ void add_pair_terms(const double2 (&c)[Tile<R>::REGS],
                                                double2 (&l)[Tile<R>::REGS], const double2 *lds,
                                                uint32_t t, const PassGeom &G, uint32_t done,
@@ -855,13 +861,16 @@ __device__ __forceinline__ void add_pair_terms(const double2 (&c)[Tile<R>::REGS]
             continue;
         }
         const uint32_t m = 3u << j;
-        const bool in_range = kFullTile || (j >= G.pair_lo && j + 1 < G.pair_hi);
+        const bool in_range = kPairs == Pairs::kFullTile ||
+                              (kPairs == Pairs::kScaled ? j >= 4
+                                                        : j >= G.pair_lo && j + 1 < G.pair_hi);
+        const double f = kPairs == Pairs::kScaled && j + 1 >= G.pair_hi ? 0.0 : field;
         if (in_range && (m & done) == 0) {
 #pragma unroll
             for (int k = 0; k < Tile<R>::REGS; ++k) {
                 const double2 p = lds[lds_slot<R>(omap<R, M>(t, k) ^ m)];
-                l[k].x -= field * p.x;
-                l[k].y -= field * p.y;
+                l[k].x -= f * p.x;
+                l[k].y -= f * p.y;
             }
         }
     }
@@ -869,16 +878,231 @@ __device__ __forceinline__ void add_pair_terms(const double2 (&c)[Tile<R>::REGS]
 #pragma unroll
     for (int rb = 0; rb + 1 < R; ++rb) {
         const int j = lo + rb;
-        const bool in_range = kFullTile || (j >= G.pair_lo && j + 1 < G.pair_hi);
+        const bool in_range = kPairs == Pairs::kFullTile ||
+                              (kPairs == Pairs::kScaled ? j >= 4
+                                                        : j >= G.pair_lo && j + 1 < G.pair_hi);
+        const double f = kPairs == Pairs::kScaled && j + 1 >= G.pair_hi ? 0.0 : field;
         if (in_range && ((3u << j) & done) == 0) {
 #pragma unroll
             for (int k = 0; k < Tile<R>::REGS; ++k) {
                 const double2 p = c[k ^ (3 << rb)];
-                l[k].x -= field * p.x;
-                l[k].y -= field * p.y;
+                l[k].x -= f * p.x;
+                l[k].y -= f * p.y;
             }
         }
     }
+}
+
+constexpr bool ham_folds(int ham) { return ham == kHamFold || ham == kHamFoldTop; }
+
+// A high pass's pair terms of mapping M's window.
+template <int R, int M, int kHam>
+__device__ __forceinline__ void high_pair_terms(const double2 (&c)[Tile<R>::REGS],
+                                                double2 (&l)[Tile<R>::REGS], const double2 *lds,
+                                                uint32_t t, const PassGeom &G, uint32_t done,
+                                                double field) {
+    if constexpr (ham_folds(kHam)) {
+        add_pair_terms<R, M, Pairs::kScaled>(c, l, lds, t, G, done, field);
+    } else if constexpr (kHam == kHamPairs) {
+        add_pair_terms<R, M>(c, l, lds, t, G, done, field);
+    }
+}
+
+// The low (gather) pass's pair terms of mapping M's window.
+template <int R, int M, int kHam>
+__device__ __forceinline__ void gather_pair_terms(const double2 (&c)[Tile<R>::REGS],
+                                                  double2 (&l)[Tile<R>::REGS], const double2 *lds,
+                                                  uint32_t t, const PassGeom &G, uint32_t done,
+                                                  double field) {
+    if constexpr (kHam == kHamStart) {
+        add_pair_terms<R, M, Pairs::kFullTile>(c, l, lds, t, G, done, field);
+    } else if constexpr (kHam == kHamPairs && gather_pairs_reach<R, M>()) {
+        add_pair_terms<R, M>(c, l, lds, t, G, done, field);
+    }
+}
+
+// X_w X_v terms whose lower wire v a pass before this one has un-rotated: in the
+// frame of the state as it is now, X_v is O = U^dagger X U with the wire's
+// rotations U = RZ(phi) RY(theta),
+//   O = [[z, w], [conj(w), -z]], z = sin theta cos phi,
+//   w = cos theta cos phi + i sin phi.
+// The pass before took v's gradients without these terms; their part is
+// <c| dO/dtheta X_w |c> and <c| dO/dphi X_w |c>, formed here.
+struct FoldOp {
+    double z;
+    double wr;
+    double wi;
+    double tz;  // dO/dtheta (its w is real)
+    double tw;
+    double pz;  // dO/dphi
+    double pwr;
+    double pwi;
+};
+
+__device__ __forceinline__ FoldOp fold_op(const WireCoef &k) {
+    const double cp = k.ch * k.ch - k.sh * k.sh;
+    const double sp = 2.0 * k.ch * k.sh;
+    const double ct = k.c * k.c - k.s * k.s;
+    const double st = 2.0 * k.c * k.s;
+    return {st * cp, ct * cp, sp, ct * cp, -st * cp, -st * sp, -ct * sp, cp};
+}
+
+// An operator as one bit value sees it: (O c) = z a + w b with its own amplitude
+// a and the other one b (z and Im w change sign where the bit is set).
+struct FoldSide {
+    double z;
+    double wr;
+    double wi;
+};
+
+__device__ __forceinline__ FoldSide fold_side(const FoldOp &o, bool bit) {
+    return {bit ? -o.z : o.z, o.wr, bit ? -o.wi : o.wi};
+}
+
+__device__ __forceinline__ double2 fold_apply(const FoldSide &o, double2 a, double2 b) {
+    return make_double2(o.z * a.x + o.wr * b.x - o.wi * b.y,
+                        o.z * a.y + o.wr * b.y + o.wi * b.x);
+}
+
+// The expectation parts of <y| O |.>: sums of z's, Re w's and Im w's factors,
+// signs as for the bit clear.
+struct FoldSums {
+    double z = 0.0;
+    double wr = 0.0;
+    double wi = 0.0;
+    __device__ __forceinline__ void add(double2 y, double2 a, double2 b) {
+        z += y.x * a.x + y.y * a.y;
+        wr += y.x * b.x + y.y * b.y;
+        wi += y.y * b.x - y.x * b.y;
+    }
+    // gradient parts (times f), summed over the row into slots at, at + 1
+    __device__ __forceinline__ void finish(const FoldOp &o, bool bit, double f,
+                                           double *__restrict__ row_acc, int at, int lane) const {
+        const double sz = bit ? -z : z;
+        const double si = bit ? -wi : wi;
+        const double r = row_sums2(f * (o.tz * sz + o.tw * wr),
+                                   f * (o.pz * sz + o.pwr * wr + o.pwi * si), lane);
+        if ((lane & 15) < 2) {
+            row_acc[at + (lane & 1)] += r;
+        }
+    }
+};
+
+// Operators of a high pass's fold terms: ops[0] the wire below the group,
+// ops[1], ops[2] wires 0 and 1.
+__device__ __forceinline__ void build_fold_ops(FoldOp *ops, const WireCoef *__restrict__ lc,
+                                               const PassGeom &G, uint32_t t) {
+    if (t < 3) {
+        const int wire = t > 0 ? (int)t - 1 : tile_wire(3, G);
+        // a lower wire that is still rotated: plain X, no gradient part
+        ops[t] = t == 0 && !G.fold_unrotated ? FoldOp{0.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}
+                                             : fold_op(lc[wire]);
+    }
+}
+
+__device__ __forceinline__ double2 lane_xor8(double2 v) {
+    return make_double2(dpp_move<0x128>(v.x), dpp_move<0x128>(v.y));
+}
+
+__device__ __forceinline__ double2 lane_xor1(double2 v) {
+    return make_double2(dpp_move<0xB1>(v.x), dpp_move<0xB1>(v.y));
+}
+
+__device__ __forceinline__ double2 lane_xor2(double2 v) {
+    return make_double2(dpp_move<0x4E>(v.x), dpp_move<0x4E>(v.y));
+}
+
+// The fold passes' further terms (tile bit 4 the group's lowest wire, bit 3 the wire below
+// it, bits 0 and 1 wires 0 and 1, bit 11 of the top group's tile wire n - 1), each
+// in a mapping that holds its bits in registers and lanes, before the pass
+// un-rotates any of its rotated ones.  The gradient parts go to the slots of tile
+// bits 0..2, which no high pass rotates: those of wires 0 and 1 at 0..3, those of
+// the wire below the group at 4, 5 (GradReduceJob adds them to the wires' own).
+// A Hamiltonian pass and the low pass's read of lambda go (27 qubits x 3 layers:
+// 12.8 -> 11.9 ms; low pass 1.53 -> 1.41 ms, the Hamiltonian's 0.86 ms gone, the
+// top group's pass 1.61 -> 1.98 ms, the other group's 1.61 -> 1.43 with its
+// loads' steps formed per tile).  One kernel per combination of terms: with
+// branches around them the register arrays were copied and spilled (2.8 ms).
+// Wire n - 1's term (kHamFoldTop): mapping 0.  kStart: l becomes the term before
+// its factor -field, which the caller adds lambda to, else the term is added.
+template <int R, bool kStart>
+__device__ __forceinline__ void add_fold_top(const double2 (&c)[Tile<R>::REGS],
+                                             double2 (&l)[Tile<R>::REGS], uint32_t t,
+                                             const FoldOp *ops, double field,
+                                             double *__restrict__ row_acc) {
+    using TL = Tile<R>;
+    const bool b0 = (t & 1u) != 0;
+    const bool b1 = (t & 2u) != 0;
+    const FoldSide o0 = fold_side(ops[1], b0);
+    const FoldSide o1 = fold_side(ops[2], b1);
+    FoldSums s0;
+    FoldSums s1;
+#pragma unroll
+    for (int k = 0; k < TL::REGS; ++k) {
+        const double2 p0 = lane_xor1(c[k]);
+        const double2 u = fold_apply(o0, c[k], p0);
+        const double2 p1 = lane_xor2(u);
+        const double2 r = fold_apply(o1, u, p1);
+        double2 &dst = l[k ^ (TL::REGS / 2)];
+        if constexpr (kStart) {
+            dst = r;
+        } else {
+            dst.x -= field * r.x;
+            dst.y -= field * r.y;
+        }
+        // the two registers of a pair give the same expectation
+        if (k < TL::REGS / 2) {
+            const double2 y = c[k ^ (TL::REGS / 2)];
+            s1.add(y, u, p1);
+            s0.add(fold_apply(o1, y, lane_xor2(y)), c[k], p0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int lane = (int)(t & (kWave - 1));
+    s0.finish(ops[1], b0, -2.0 * field, row_acc, 0, lane);
+    s1.finish(ops[2], b1, -2.0 * field, row_acc, 2, lane);
+}
+
+// The pair below the group: mapping 2, whose registers hold tile bit 4 and (R = 3) bit 3, a lane
+// bit for R = 4.
+template <int R>
+__device__ __forceinline__ void add_fold_lower(const double2 (&c)[Tile<R>::REGS],
+                                               double2 (&l)[Tile<R>::REGS], uint32_t t,
+                                               const FoldOp *ops, double field,
+                                               double *__restrict__ row_acc) {
+    using TL = Tile<R>;
+    constexpr int kBit4 = 1 << (4 - phase_first_bit<R, 2>());
+    auto flip3 = [&](int k) {
+        if constexpr (R == 4) {
+            return lane_xor8(c[k]);
+        } else {
+            return c[k ^ 1];
+        }
+    };
+    const bool lane_bit = R == 4 && (t & 8u) != 0;
+    const FoldSide o = fold_side(ops[0], lane_bit);
+    FoldSums sums;
+#pragma unroll
+    for (int k = 0; k < TL::REGS; ++k) {
+        const double2 a = c[k ^ kBit4];
+        const double2 b = flip3(k ^ kBit4);
+        const bool reg_bit = R == 3 && (k & 1) != 0;
+        const FoldSide ok = {reg_bit ? -o.z : o.z, o.wr, reg_bit ? -o.wi : o.wi};
+        const double2 r = fold_apply(ok, a, b);
+        l[k].x -= field * r.x;
+        l[k].y -= field * r.y;
+        // the two registers of a pair (k, k ^ kBit4) give the same expectation
+        if ((k & kBit4) == 0) {
+            if (reg_bit) {
+                sums.z -= c[k].x * a.x + c[k].y * a.y;
+                sums.wr += c[k].x * b.x + c[k].y * b.y;
+                sums.wi -= c[k].y * b.x - c[k].x * b.y;
+            } else {
+                sums.add(c[k], a, b);
+            }
+        }
+    }
+    sums.finish(ops[0], lane_bit, -2.0 * field, row_acc, 4, (int)(t & (kWave - 1)));
 }
 
 // Loads one tile of (cur, lam) into the first mapping of the adjoint pass:
@@ -891,13 +1115,14 @@ __device__ __forceinline__ void add_pair_terms(const double2 (&c)[Tile<R>::REGS]
 // kReady, high passes: lam of the tile is already in l (prefetched); low
 // (gather) pass: c already holds the tile's state as loaded from the two
 // image runs (load_cur_gather), before its placement through LDS.
-template <int R, bool kGather, bool kHam, bool kGen = false, bool kReady = false>
+template <int R, bool kGather, int kHam, bool kGen = false, bool kReady = false>
 __device__ __forceinline__ void bwd_load_tile(double2 (&c)[Tile<R>::REGS],
                                               double2 (&l)[Tile<R>::REGS],
                                               const double2 *cur_in, const double2 *lam_in,
                                               uint64_t base, const TileAddr &ta,
                                               const PassGeom &G, double2 *lds, uint32_t t,
-                                              double field,
+                                              double field, const FoldOp *fold_ops,
+                                              double *__restrict__ row_acc,
                                               const CMat2 *__restrict__ gen_tab = nullptr,
                                               const CMat2 *gen_chunks = nullptr,
                                               const CMat2 *__restrict__ gen_u = nullptr,
@@ -916,20 +1141,24 @@ __device__ __forceinline__ void bwd_load_tile(double2 (&c)[Tile<R>::REGS],
 #pragma unroll
         for (int k = 0; k < TL::REGS; ++k) {
             const uint64_t src = (k < TL::REGS / 2 ? run : run1) + ((uint64_t)k << (T - R));
-            l[k] = lam_in[src];
+            if constexpr (kHam != kHamStart) {
+                l[k] = lam_in[src];
+            }
             if constexpr (!kReady) {
                 c[k] = cur_in[src];
             }
         }
-        __syncthreads();
+        if constexpr (kHam != kHamStart) {
+            __syncthreads();
 #pragma unroll
-        for (int k = 0; k < TL::REGS; ++k) {
-            lds[lds_slot<R>(ring_inv32(omap<R, 0>(t, k), T))] = l[k];
-        }
-        __syncthreads();
+            for (int k = 0; k < TL::REGS; ++k) {
+                lds[lds_slot<R>(ring_inv32(omap<R, 0>(t, k), T))] = l[k];
+            }
+            __syncthreads();
 #pragma unroll
-        for (int k = 0; k < TL::REGS; ++k) {
-            l[k] = lds[lds_slot<R>(omap<R, 1>(t, k))];
+            for (int k = 0; k < TL::REGS; ++k) {
+                l[k] = lds[lds_slot<R>(omap<R, 1>(t, k))];
+            }
         }
         __syncthreads();
 #pragma unroll
@@ -941,33 +1170,68 @@ __device__ __forceinline__ void bwd_load_tile(double2 (&c)[Tile<R>::REGS],
         for (int k = 0; k < TL::REGS; ++k) {
             c[k] = lds[lds_slot<R>(omap<R, 1>(t, k))];
         }
-        if constexpr (kHam && gather_pairs_reach<R, 1>()) {
-            // the LDS still holds the gathered tile of cur in offset order
-            add_pair_terms<R, 1>(c, l, lds, t, G, 0u, field);
+        if constexpr (kHam == kHamStart) {
+            // H's diagonal at P(i) from the pre-CNOT index i (see
+            // bwd_low_gen_kernel): 2 walls - n, walls = p + (i_0 ^ (p & 1)) + i_0
+            // with p = popcount(i >> 2); the register bits are i's bits 0 .. R - 1
+            const int p0 = (int)__popcll((base | omap<R, 1>(t, 0)) >> 2);
+#pragma unroll
+            for (int k = 0; k < TL::REGS; ++k) {
+                const int p = p0 + __builtin_popcount((unsigned)k >> 2);
+                const int b0 = k & 1;
+                const double d = (double)(2 * (p + (b0 ^ (p & 1)) + b0) - G.n);
+                l[k] = make_double2(d * c[k].x, d * c[k].y);
+            }
         }
+        // the LDS still holds the gathered tile of cur in offset order
+        gather_pair_terms<R, 1, kHam>(c, l, lds, t, G, 0u, field);
     } else {
         // row: the index of register 0 (the state's address, the chain's
         // argument); lambda may sit in another layout (lam_ta, lam_base)
         const uint64_t row = base + ta.offA;
         const TileAddr &la = lam_ta != nullptr ? *lam_ta : ta;
         const uint64_t lrow = (lam_ta != nullptr ? lam_base : base) + la.offA;
+        // wire n - 1's term starts lambda before most of it is loaded: beside all
+        // the loaded values its operators would not fit the registers
+        constexpr bool kTermFirst = kHam == kHamFoldTop && !kReady;
 #pragma unroll
         for (int k = 0; k < TL::REGS; ++k) {
-            if constexpr (!kReady) {
+            if constexpr (!kReady && !kTermFirst) {
                 l[k] = load_stream(lam_in + lrow + k * la.strideA);
             }
             if constexpr (!kGen) {
                 c[k] = cur_in[row + k * ta.strideA];
             }
         }
+        if constexpr (kTermFirst) {
+            constexpr int kEarly = R == 4 ? 6 : 0;
+            double2 early[kEarly > 0 ? kEarly : 1];
+#pragma unroll
+            for (int k = 0; k < kEarly; ++k) {
+                early[k] = load_stream(lam_in + lrow + k * la.strideA);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            add_fold_top<R, true>(c, l, t, fold_ops, field, row_acc);
+#pragma unroll
+            for (int k = 0; k < TL::REGS; ++k) {
+                double2 x;
+                if (k < kEarly) {
+                    x = early[k < kEarly ? k : 0];
+                } else {
+                    x = load_stream(lam_in + lrow + k * la.strideA);
+                }
+                l[k].x = x.x - field * l[k].x;
+                l[k].y = x.y - field * l[k].y;
+            }
+        }
         if constexpr (kGen) {
             const CMat2 y = chain_y_high<R>(gen_chunks, gen_u, row, G);
             chain_fill<R>(c, gen_tab, y);
         }
-        if constexpr (kHam) {
+        if constexpr (kHam != kHamNone) {
             // only the pair straddling the load window's lower edge needs
             // a copy of the tile in LDS
-            if (G.pair_lo <= T - R - 1 && G.pair_hi >= T - R + 1) {
+            if (ham_folds(kHam) || (G.pair_lo <= T - R - 1 && G.pair_hi >= T - R + 1)) {
                 __syncthreads();
 #pragma unroll
                 for (int k = 0; k < TL::REGS; ++k) {
@@ -975,12 +1239,15 @@ __device__ __forceinline__ void bwd_load_tile(double2 (&c)[Tile<R>::REGS],
                 }
                 __syncthreads();
             }
-            add_pair_terms<R, 0>(c, l, lds, t, G, 0u, field);
+            if constexpr (kHam == kHamFoldTop && kReady) {
+                add_fold_top<R, false>(c, l, t, fold_ops, field, row_acc);
+            }
+            high_pair_terms<R, 0, kHam>(c, l, lds, t, G, 0u, field);
         }
     }
 }
 
-template <int R, bool kGather, bool kWriteCur, bool kWriteLam, bool kHam>
+template <int R, bool kGather, bool kWriteCur, bool kWriteLam, int kHam>
 __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pass_kernel(
     const double2 *cur_in, const double2 *lam_in, double2 *cur_out, double2 *lam_out,
     const WireCoef *__restrict__ lc, PassGeom G, double *__restrict__ partials, double field) {
@@ -993,6 +1260,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
     __shared__ double acc[ROWS][2 * T];
     __shared__ double2 rz_tab[TL::P * TL::REGS];
     __shared__ WireCoef tile_coef[T];
+    __shared__ FoldOp fold_ops[3];  // high passes with pair terms
     const uint32_t t = threadIdx.x;
     const int lane = t & (kWave - 1);
     double *row_acc = acc[t / 16];
@@ -1000,6 +1268,9 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
         acc[i / (2 * T)][i % (2 * T)] = 0.0;
     }
     build_rz_tables<R>(rz_tab, lc, G, t);
+    if constexpr (ham_folds(kHam)) {
+        build_fold_ops(fold_ops, lc, G, t);
+    }
     if (t < (uint32_t)T) {
         const bool rot = (int)t >= G.rot_lo && (int)t < G.rot_hi;
         tile_coef[t] = rot ? lc[tile_wire((int)t, G)] : WireCoef{1.0, 0.0, 1.0, 0.0};
@@ -1014,7 +1285,8 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
         const uint64_t base = tile_base(g, G, T);
         double2 c[TL::REGS];
         double2 l[TL::REGS];
-        bwd_load_tile<R, kGather, kHam>(c, l, cur_in, lam_in, base, ta, G, lds, tl, field);
+        bwd_load_tile<R, kGather, kHam>(c, l, cur_in, lam_in, base, ta, G, lds, tl, field,
+                                        fold_ops, row_acc);
 
         // lam is exchanged before cur, so the LDS holds cur for the pair terms
         if constexpr (kGather) {
@@ -1023,28 +1295,20 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
             phase_bwd<R, 1, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
             exchange<R, 1, 2>(l, lds, tl);
             exchange<R, 1, 2>(c, lds, tl);
-            if constexpr (kHam && gather_pairs_reach<R, 2>()) {
-                add_pair_terms<R, 2>(c, l, lds, tl, G, w1, field);
-            }
+            gather_pair_terms<R, 2, kHam>(c, l, lds, tl, G, w1, field);
             phase_bwd<R, 2, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
             if constexpr (TL::P == 4) {
                 exchange<R, 2, 3>(l, lds, tl);
                 exchange<R, 2, 3>(c, lds, tl);
-                if constexpr (kHam && gather_pairs_reach<R, 3>()) {
-                    add_pair_terms<R, 3>(c, l, lds, tl, G, w1 | w2, field);
-                }
+                gather_pair_terms<R, 3, kHam>(c, l, lds, tl, G, w1 | w2, field);
                 phase_bwd<R, 3, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
                 exchange<R, 3, 0>(l, lds, tl);
                 exchange<R, 3, 0>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 0>(c, l, lds, tl, G, w1 | w2 | window_mask<R, 3>(), field);
-                }
+                gather_pair_terms<R, 0, kHam>(c, l, lds, tl, G, w1 | w2 | window_mask<R, 3>(), field);
             } else {
                 exchange<R, 2, 0>(l, lds, tl);
                 exchange<R, 2, 0>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 0>(c, l, lds, tl, G, w1 | w2, field);
-                }
+                gather_pair_terms<R, 0, kHam>(c, l, lds, tl, G, w1 | w2, field);
             }
             phase_bwd<R, 0, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
             const uint64_t row = base + ta.offA;
@@ -1064,14 +1328,13 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
             if constexpr (TL::P == 3) {
                 exchange<R, 0, 1>(l, lds, tl);
                 exchange<R, 0, 1>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 1>(c, l, lds, tl, G, w0, field);
-                }
+                high_pair_terms<R, 1, kHam>(c, l, lds, tl, G, w0, field);
                 phase_bwd<R, 1, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
                 exchange<R, 1, 2>(l, lds, tl);
                 exchange<R, 1, 2>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 2>(c, l, lds, tl, G, w0 | window_mask<R, 1>(), field);
+                high_pair_terms<R, 2, kHam>(c, l, lds, tl, G, w0 | window_mask<R, 1>(), field);
+                if constexpr (ham_folds(kHam)) {
+                    add_fold_lower<R>(c, l, tl, fold_ops, field, row_acc);
                 }
                 phase_bwd<R, 2, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
             } else {
@@ -1079,9 +1342,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
                 if (G.rot_lo < R) {
                     exchange<R, 0, 1>(l, lds, tl);
                     exchange<R, 0, 1>(c, lds, tl);
-                    if constexpr (kHam) {
-                        add_pair_terms<R, 1>(c, l, lds, tl, G, done, field);
-                    }
+                    high_pair_terms<R, 1, kHam>(c, l, lds, tl, G, done, field);
                     phase_bwd<R, 1, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
                     done |= window_mask<R, 1>();
                     exchange<R, 1, 2>(l, lds, tl);
@@ -1090,16 +1351,15 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
                     exchange<R, 0, 2>(l, lds, tl);
                     exchange<R, 0, 2>(c, lds, tl);
                 }
-                if constexpr (kHam) {
-                    add_pair_terms<R, 2>(c, l, lds, tl, G, done, field);
+                high_pair_terms<R, 2, kHam>(c, l, lds, tl, G, done, field);
+                if constexpr (ham_folds(kHam)) {
+                    add_fold_lower<R>(c, l, tl, fold_ops, field, row_acc);
                 }
                 phase_bwd<R, 2, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
                 done |= window_mask<R, 2>();
                 exchange<R, 2, 3>(l, lds, tl);
                 exchange<R, 2, 3>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 3>(c, l, lds, tl, G, done, field);
-                }
+                high_pair_terms<R, 3, kHam>(c, l, lds, tl, G, done, field);
                 phase_bwd<R, 3, kGather, !kGather>(c, l, tile_coef, row_acc, lane, rz_tab);
             }
             const uint64_t row = base + ta.offC;
@@ -1353,10 +1613,6 @@ __device__ __forceinline__ void scale_regs(double2 (&l)[Tile<R>::REGS], double s
 // bits that ride along).  In mappings 0 and 2 tile bit 3 is lane bit 3, so
 // its pair partner is the lane 8 apart in the same row of 16: DPP row_ror:8
 // brings it over without an LDS exchange.
-__device__ __forceinline__ double2 lane_xor8(double2 v) {
-    return make_double2(dpp_move<0x128>(v.x), dpp_move<0x128>(v.y));
-}
-
 // Tile bit 3: RZ^dagger on both states (window 1's phase table at register
 // index 8 or 0; none with kPhased = false), its gradients as in grad_window,
 // then RY^dagger of bit 3 on lam (before window 2's: they commute).  One lane
@@ -1482,7 +1738,7 @@ __device__ __forceinline__ void apply_tile_phase(double2 (&l)[Tile<R>::REGS], co
 // kPhaseFree (generated high passes, R = 4): the table set generates the
 // state without the RZ of the pass's own wires, so lambda takes the tile's
 // combined phase once (apply_tile_phase) and the windows none.
-template <int R, bool kGather, bool kHam, bool kGen, bool kPrefetch = false, bool kPhaseFree = false>
+template <int R, bool kGather, int kHam, bool kGen, bool kPrefetch = false, bool kPhaseFree = false>
 __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_lam_kernel(
     const double2 *cur_in, const double2 *lam_in, double2 *lam_out,
     const WireCoef *__restrict__ lc, PassGeom G, double *__restrict__ partials, double field,
@@ -1496,6 +1752,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
     __shared__ double acc[ROWS][2 * T];
     __shared__ double2 rz_tab[TL::P * TL::REGS];
     __shared__ WireCoef tile_coef[T];
+    __shared__ FoldOp fold_ops[3];  // high passes with pair terms
     // phase-free sweep: RY^dagger of lambda's window bits (4..11) in tangent
     // form, its scale applied once before the store
     __shared__ double tan_t[kPhaseFree ? T : 1];
@@ -1510,6 +1767,9 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
         acc[i / (2 * T)][i % (2 * T)] = 0.0;
     }
     build_rz_tables<R>(rz_tab, lc, G, t);
+    if constexpr (ham_folds(kHam)) {
+        build_fold_ops(fold_ops, lc, G, t);
+    }
     if (t < (uint32_t)T) {
         const bool rot = (int)t >= G.rot_lo && (int)t < G.rot_hi;
         tile_coef[t] = rot ? lc[tile_wire((int)t, G)] : WireCoef{1.0, 0.0, 1.0, 0.0};
@@ -1532,7 +1792,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
     const TileAddr ta_in = lay_tile_addr(ta, kGather ? LamLayout{} : G.lay_in);
     const TileAddr ta_out = lay_tile_addr(ta, kGather ? LamLayout{} : G.lay_out);
     static_assert(!(kPrefetch && kGather && kGen), "the gather pass reads the state");
-    static_assert(!kPhaseFree || (kGen && !kGather && !kHam && TL::P == 3),
+    static_assert(!kPhaseFree || (kGen && !kGather && kHam == kHamNone && TL::P == 3),
                   "phase-free sweep: generated high passes of register shape 4 without pairs");
     constexpr bool kPhased = !kPhaseFree;
 
@@ -1564,9 +1824,13 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
         // would be spilled)
         TileAddr tla = ta;
         TileAddr tla_in = ta_in;
-        if constexpr (kPrefetch) {
+        if constexpr (kPrefetch || ham_folds(kHam)) {
             asm volatile("" : "+v"(tla.offA));
             asm volatile("" : "+v"(tla_in.offA));
+        }
+        if constexpr (ham_folds(kHam)) {
+            asm volatile("" : "+s"(tla.strideA));
+            asm volatile("" : "+s"(tla_in.strideA));
         }
         const uint64_t base = tile_base(g, G, T);
         double2 c[TL::REGS];
@@ -1582,7 +1846,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
             }
         }
         bwd_load_tile<R, kGather, kHam, kGen, kPrefetch>(c, l, cur_in, lam_in, base, tla, G, lds,
-                                                         tl, field, gen_tab, gen_chunks,
+                                                         tl, field, fold_ops, row_acc, gen_tab, gen_chunks,
                                                          gen_utab + 2 * g,
                                                          kPhaseFree ? G.tile_in[g]
                                                                     : lay_addr(base, G.lay_in),
@@ -1609,21 +1873,15 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
             if constexpr (TL::P == 4) {
                 exchange<R, 1, 2>(l, lds, tl);
                 exchange<R, 1, 2>(c, lds, tl);
-                if constexpr (kHam && gather_pairs_reach<R, 2>()) {
-                    add_pair_terms<R, 2>(c, l, lds, tl, G, w1, field);
-                }
+                gather_pair_terms<R, 2, kHam>(c, l, lds, tl, G, w1, field);
                 grad_window<R, 2>(c, l, lc, G, row_acc, lane, rz_tab);
                 exchange<R, 2, 3>(l, lds, tl);
                 exchange<R, 2, 3>(c, lds, tl);
-                if constexpr (kHam && gather_pairs_reach<R, 3>()) {
-                    add_pair_terms<R, 3>(c, l, lds, tl, G, w1 | w2, field);
-                }
+                gather_pair_terms<R, 3, kHam>(c, l, lds, tl, G, w1 | w2, field);
                 grad_window<R, 3>(c, l, lc, G, row_acc, lane, rz_tab);
                 exchange<R, 3, 0>(l, lds, tl);
                 exchange<R, 3, 0>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 0>(c, l, lds, tl, G, w1 | w2 | window_mask<R, 3>(), field);
-                }
+                gather_pair_terms<R, 0, kHam>(c, l, lds, tl, G, w1 | w2 | window_mask<R, 3>(), field);
                 grad_window<R, 0>(c, l, lc, G, row_acc, lane, rz_tab);
                 prefetch_next();
                 ry_inv_window<R, 0>(l, tile_coef);
@@ -1639,15 +1897,11 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
                 // mapping 0 for the store
                 exchange<R, 1, 0>(l, lds, tl);
                 exchange<R, 1, 0>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 0>(c, l, lds, tl, G, w1, field);
-                }
+                gather_pair_terms<R, 0, kHam>(c, l, lds, tl, G, w1, field);
                 grad_window<R, 0>(c, l, lc, G, row_acc, lane, rz_tab);
                 exchange<R, 0, 2>(l, lds, tl);
                 exchange<R, 0, 2>(c, lds, tl);
-                if constexpr (kHam && gather_pairs_reach<R, 2>()) {
-                    add_pair_terms<R, 2>(c, l, lds, tl, G, w1 | window_mask<R, 0>(), field);
-                }
+                gather_pair_terms<R, 2, kHam>(c, l, lds, tl, G, w1 | window_mask<R, 0>(), field);
                 grad_window<R, 2>(c, l, lc, G, row_acc, lane, rz_tab);
                 prefetch_next();
                 ry_inv_window<R, 2>(l, tile_coef);
@@ -1670,13 +1924,17 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
                 // exchanges
                 exchange<R, 0, 2>(l, lds, tl);
                 exchange<R, 0, 2>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 2>(c, l, lds, tl, G, w0, field);
+                high_pair_terms<R, 2, kHam>(c, l, lds, tl, G, w0, field);
+                if constexpr (ham_folds(kHam)) {
+                    add_fold_lower<R>(c, l, tl, fold_ops, field, row_acc);
                 }
                 grad_window<R, 2, kPhased, kPhaseFree>(c, l, lc, G, row_acc, lane, rz_tab);
                 // unconditional: an unrotated bit 3 has phase 1 and the
                 // identity in tile_coef, and its gradient slot is not read
-                grad_ry_lane_bit3<R, kPhased>(c, l, row_acc, lane, rz_tab, tile_coef[3]);
+                // (with fold terms it is the wire below the group)
+                if constexpr (!ham_folds(kHam)) {
+                    grad_ry_lane_bit3<R, kPhased>(c, l, row_acc, lane, rz_tab, tile_coef[3]);
+                }
                 prefetch_next();
                 if constexpr (kPhaseFree) {
                     ry_inv_window_tan<R, 2>(l, tan_t, form_b);
@@ -1699,9 +1957,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
                 if (w1_rot) {
                     exchange<R, 0, 1>(l, lds, tl);
                     exchange<R, 0, 1>(c, lds, tl);
-                    if constexpr (kHam) {
-                        add_pair_terms<R, 1>(c, l, lds, tl, G, done, field);
-                    }
+                    high_pair_terms<R, 1, kHam>(c, l, lds, tl, G, done, field);
                     grad_window<R, 1>(c, l, lc, G, row_acc, lane, rz_tab);
                     done |= window_mask<R, 1>();
                     exchange<R, 1, 2>(l, lds, tl);
@@ -1710,16 +1966,15 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_la
                     exchange<R, 0, 2>(l, lds, tl);
                     exchange<R, 0, 2>(c, lds, tl);
                 }
-                if constexpr (kHam) {
-                    add_pair_terms<R, 2>(c, l, lds, tl, G, done, field);
+                high_pair_terms<R, 2, kHam>(c, l, lds, tl, G, done, field);
+                if constexpr (ham_folds(kHam)) {
+                    add_fold_lower<R>(c, l, tl, fold_ops, field, row_acc);
                 }
                 grad_window<R, 2>(c, l, lc, G, row_acc, lane, rz_tab);
                 done |= window_mask<R, 2>();
                 exchange<R, 2, 3>(l, lds, tl);
                 exchange<R, 2, 3>(c, lds, tl);
-                if constexpr (kHam) {
-                    add_pair_terms<R, 3>(c, l, lds, tl, G, done, field);
-                }
+                high_pair_terms<R, 3, kHam>(c, l, lds, tl, G, done, field);
                 grad_window<R, 3>(c, l, lc, G, row_acc, lane, rz_tab);
                 prefetch_next();
                 ry_inv_window<R, 3>(l, tile_coef);
@@ -1885,17 +2140,17 @@ __global__ __launch_bounds__(Tile<R>::THREADS, low_gen_min_waves<R>()) void bwd_
             }
             __syncthreads();
         }
-        add_pair_terms<R, 0, true>(c, l, lds, tl, G, 0u, field);
+        add_pair_terms<R, 0, Pairs::kFullTile>(c, l, lds, tl, G, 0u, field);
         grad_window<R, 0, true, true>(c, l, lc, G, row_acc, lane, rz_tab);
         constexpr uint32_t w0 = window_mask<R, 0>();
         constexpr uint32_t w1 = window_mask<R, 1>();
         exchange<R, 0, 1>(l, lds, tl);
         exchange<R, 0, 1>(c, lds, tl);
-        add_pair_terms<R, 1, true>(c, l, lds, tl, G, w0, field);
+        add_pair_terms<R, 1, Pairs::kFullTile>(c, l, lds, tl, G, w0, field);
         grad_window<R, 1, true, true>(c, l, lc, G, row_acc, lane, rz_tab);
         exchange<R, 1, 2>(l, lds, tl);
         exchange<R, 1, 2>(c, lds, tl);
-        add_pair_terms<R, 2, true>(c, l, lds, tl, G, w0 | w1, field);
+        add_pair_terms<R, 2, Pairs::kFullTile>(c, l, lds, tl, G, w0 | w1, field);
         grad_window<R, 2, true, true>(c, l, lc, G, row_acc, lane, rz_tab);
         if constexpr (TL::P == 3) {
             // sweep 2: lambda back to mapping 0 under RY^dagger (tangent
@@ -1910,7 +2165,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, low_gen_min_waves<R>()) void bwd_
             constexpr uint32_t w2 = window_mask<R, 2>();
             exchange<R, 2, 3>(l, lds, tl);
             exchange<R, 2, 3>(c, lds, tl);
-            add_pair_terms<R, 3, true>(c, l, lds, tl, G, w0 | w1 | w2, field);
+            add_pair_terms<R, 3, Pairs::kFullTile>(c, l, lds, tl, G, w0 | w1 | w2, field);
             grad_window<R, 3, true, true>(c, l, lc, G, row_acc, lane, rz_tab);
             ry_inv_window<R, 3>(l, tile_coef);
             exchange<R, 3, 2>(l, lds, tl);
@@ -1974,7 +2229,7 @@ template <int R>
 static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const double2 *cur_in,
                               const double2 *lam_in, double2 *cur_out, double2 *lam_out,
                               const WireCoef *lc, const PassGeom &g, double *partials, int grid,
-                              hipStream_t s, bool ham, double field, const CMat2 *gen_tab,
+                              hipStream_t s, int ham, double field, const CMat2 *gen_tab,
                               const CMat2 *gen_utab, bool prefetch, bool phase_free) {
     constexpr int TH = Tile<R>::THREADS;
     const bool gen = gen_tab != nullptr;
@@ -1992,13 +2247,22 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
             throw std::invalid_argument("lambda layouts: pass or geometry outside their scope");
         }
     }
-    if (phase_free && (R != 4 || gather || !gen || ham || write_cur || !write_lam)) {
+    if (phase_free &&
+        (R != 4 || gather || !gen || ham != kHamNone || write_cur || !write_lam)) {
         // the tables leave the pass's own phases out only for this sweep
         throw std::invalid_argument(
             "phase-free sweep: generated lambda-only high pass of shape 4 without pair terms");
     }
     if (phase_free && (g.tile_in == nullptr || g.tile_out == nullptr)) {
         throw std::invalid_argument("phase-free sweep: no per-tile lambda address tables");
+    }
+    if (ham == kHamStart && (!gather || g.a != Tile<R>::T || g.rot_lo != 0)) {
+        throw std::invalid_argument("lambda starts in a low pass");
+    }
+    if (ham_folds(ham) && (gather || gen || g.a != 3 || g.rot_lo != 4 || g.pair_lo != 4 ||
+                           (ham == kHamFoldTop && g.h0 + 9 != g.n))) {
+        // the wire below the group at tile bit 3, wire n - 1 at tile bit 11
+        throw std::invalid_argument("fold terms: geometry without the wires they reach");
     }
     if (!write_cur && write_lam) {  // the state is not rewritten: lambda-only sweep
         if (!gather && R == 4 && (g.a != 3 || g.rot_lo < 3)) {
@@ -2007,12 +2271,12 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
         }
         if constexpr (R == 4) {
             if (phase_free && prefetch) {
-                bwd_lam_kernel<R, false, false, true, true, true><<<grid, TH, 0, s>>>(
+                bwd_lam_kernel<R, false, kHamNone, true, true, true><<<grid, TH, 0, s>>>(
                     cur_in, lam_in, lam_out, lc, g, partials, field, gen_tab, gen_utab);
                 return;
             }
             if (phase_free) {
-                bwd_lam_kernel<R, false, false, true, false, true><<<grid, TH, 0, s>>>(
+                bwd_lam_kernel<R, false, kHamNone, true, false, true><<<grid, TH, 0, s>>>(
                     cur_in, lam_in, lam_out, lc, g, partials, field, gen_tab, gen_utab);
                 return;
             }
@@ -2024,18 +2288,24 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
             cur_in, lam_in, lam_out, lc, g, partials, field, gen_tab, gen_utab);             \
         return;                                                                              \
     }
-        RIE_BWD_LAM(true, false, false, false)
-        RIE_BWD_LAM(false, false, false, false)
-        RIE_BWD_LAM(true, true, false, false)
-        RIE_BWD_LAM(false, true, false, false)
-        RIE_BWD_LAM(false, false, true, false)
-        RIE_BWD_LAM(false, true, true, false)
-        RIE_BWD_LAM(true, false, false, true)
-        RIE_BWD_LAM(true, true, false, true)
-        RIE_BWD_LAM(false, false, false, true)
-        RIE_BWD_LAM(false, true, false, true)
-        RIE_BWD_LAM(false, false, true, true)
-        RIE_BWD_LAM(false, true, true, true)
+        RIE_BWD_LAM(true, kHamNone, false, false)
+        RIE_BWD_LAM(false, kHamNone, false, false)
+        RIE_BWD_LAM(true, kHamPairs, false, false)
+        RIE_BWD_LAM(true, kHamStart, false, false)
+        RIE_BWD_LAM(false, kHamPairs, false, false)
+        RIE_BWD_LAM(false, kHamFold, false, false)
+        RIE_BWD_LAM(false, kHamFoldTop, false, false)
+        RIE_BWD_LAM(false, kHamNone, true, false)
+        RIE_BWD_LAM(false, kHamPairs, true, false)
+        RIE_BWD_LAM(true, kHamNone, false, true)
+        RIE_BWD_LAM(true, kHamPairs, false, true)
+        RIE_BWD_LAM(true, kHamStart, false, true)
+        RIE_BWD_LAM(false, kHamNone, false, true)
+        RIE_BWD_LAM(false, kHamPairs, false, true)
+        RIE_BWD_LAM(false, kHamFold, false, true)
+        RIE_BWD_LAM(false, kHamFoldTop, false, true)
+        RIE_BWD_LAM(false, kHamNone, true, true)
+        RIE_BWD_LAM(false, kHamPairs, true, true)
 #undef RIE_BWD_LAM
     }
     if (gen) {
@@ -2051,29 +2321,35 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
             cur_in, lam_in, cur_out, lam_out, lc, g, partials, field);                       \
         return;                                                                              \
     }
-    RIE_BWD(true, true, true, false)
-    RIE_BWD(false, true, true, false)
-    RIE_BWD(true, false, true, false)
-    RIE_BWD(false, false, true, false)
-    RIE_BWD(true, true, true, true)
-    RIE_BWD(false, true, true, true)
-    RIE_BWD(true, false, true, true)
-    RIE_BWD(false, false, true, true)
+    RIE_BWD(true, true, true, kHamNone)
+    RIE_BWD(false, true, true, kHamNone)
+    RIE_BWD(true, false, true, kHamNone)
+    RIE_BWD(false, false, true, kHamNone)
+    RIE_BWD(true, true, true, kHamPairs)
+    RIE_BWD(false, true, true, kHamPairs)
+    RIE_BWD(true, false, true, kHamPairs)
+    RIE_BWD(false, false, true, kHamPairs)
+    RIE_BWD(false, true, true, kHamFold)
+    RIE_BWD(false, false, true, kHamFold)
+    RIE_BWD(false, true, true, kHamFoldTop)
+    RIE_BWD(false, false, true, kHamFoldTop)
+    RIE_BWD(true, true, true, kHamStart)
+    RIE_BWD(true, false, true, kHamStart)
 #undef RIE_BWD
 }
 
 void launch_bwd_pass(int R, bool gather, bool write_cur, bool write_lam, const double2 *cur_in,
                      const double2 *lam_in, double2 *cur_out, double2 *lam_out,
                      const WireCoef *layer_coef, const PassGeom &g, double *partials, int grid,
-                     hipStream_t s, bool ham_pairs, double field, const CMat2 *gen_tab,
+                     hipStream_t s, int ham, double field, const CMat2 *gen_tab,
                      const CMat2 *gen_utab, bool prefetch, bool phase_free) {
     if (R == 4) {
         launch_bwd_pass_r<4>(gather, write_cur, write_lam, cur_in, lam_in, cur_out, lam_out,
-                             layer_coef, g, partials, grid, s, ham_pairs, field, gen_tab,
+                             layer_coef, g, partials, grid, s, ham, field, gen_tab,
                              gen_utab, prefetch, phase_free);
     } else {
         launch_bwd_pass_r<3>(gather, write_cur, write_lam, cur_in, lam_in, cur_out, lam_out,
-                             layer_coef, g, partials, grid, s, ham_pairs, field, gen_tab,
+                             layer_coef, g, partials, grid, s, ham, field, gen_tab,
                              gen_utab, prefetch, phase_free);
     }
 }
@@ -2860,9 +3136,9 @@ __global__ __launch_bounds__(256, 2) void bwd_top_l0_kernel(
         double2 c[TL::REGS];
         double2 l[TL::REGS];
         // lambda's address of the tile in its layout from the per-tile table
-        // (layer0_top_factor_kernel), so the layout is not evaluated here
-        bwd_load_tile<R, false, false, true>(c, l, nullptr, lam_in, base, ta, G, lds, tl, 0.0,
-                                             gen_tab, gen_chunks, gen_utab + 2 * g, lam_tile[g],
+        // (launch_chain_prep), so the layout is not evaluated here
+        bwd_load_tile<R, false, kHamNone, true>(c, l, nullptr, lam_in, base, ta, G, lds, tl, 0.0,
+                                             nullptr, row_acc, gen_tab, gen_chunks, gen_utab + 2 * g, lam_tile[g],
                                              &ta_in);
         // the sweep of the lambda-only high pass (bwd_lam_kernel, R = 4), the
         // state generated without the group's phases
@@ -3131,6 +3407,17 @@ __global__ __launch_bounds__(256) void reduce_kernel(GradReduce jobs, int T, Lay
         double acc = 0.0;
         for (int b = t; b < J.blocks; b += 256) {
             acc += J.partials[(uint64_t)b * (2 * T) + col];
+        }
+        // what fold terms of later passes add: wires 0 and 1, the group's top wire
+        if (J.top != nullptr && col < 4) {
+            for (int b = t; b < J.top_blocks; b += 256) {
+                acc += J.top[(uint64_t)b * (2 * T) + col];
+            }
+        }
+        if (J.above != nullptr && c >= J.cols - 2) {
+            for (int b = t; b < J.above_blocks; b += 256) {
+                acc += J.above[(uint64_t)b * (2 * T) + 4 + (col & 1)];
+            }
         }
         acc = wave_sum(acc);
         if ((t & 63) == 0) {

@@ -38,6 +38,8 @@ struct PassGeom {
     // transverse-field terms a fused adjoint pass adds before un-rotating.
     int pair_lo;
     int pair_hi;
+    // Fold passes (kHamFold): the wire below the group is un-rotated already.
+    bool fold_unrotated;
     // Scattered tile (Hamiltonian pass only): when sc_n > 0, offset bits
     // [a, a + sc_n) are the index bits sc[0] < sc[1] < ... (all >= a), and h0
     // is unused.
@@ -55,6 +57,16 @@ struct PassGeom {
     const uint64_t *tile_in = nullptr;
     const uint64_t *tile_out = nullptr;
 };
+
+// Hamiltonian terms that an adjoint pass adds (launch_bwd_pass).
+constexpr int kHamNone = 0;
+constexpr int kHamPairs = 1;  // the pairs of G's range
+constexpr int kHamStart = 2;  // low pass: lambda starts here, as H's diagonal and
+                              // every pair inside the tile (lam_in is not read)
+constexpr int kHamFold = 3;   // high pass (rot_lo = 4): its pairs and the one below the
+                              // group (tile bits 3, 4)
+constexpr int kHamFoldTop = 4;  // top group: those and wire n - 1's X_0 X_1 X_{n-1} (tile
+                                // bits 0, 1, 11; wires 0 and 1 un-rotated)
 
 // Address of index i in layout L (a bit permutation, so lay_addr(x | y) =
 // lay_addr(x) | lay_addr(y) for disjoint x, y, and strides map bit by bit).
@@ -357,7 +369,7 @@ void launch_gen_layer1(int R, double2 *out, const CMat2 *tab, const CMat2 *utab,
 void launch_bwd_pass(int R, bool gather, bool write_cur, bool write_lam, const double2 *cur_in,
                      const double2 *lam_in, double2 *cur_out, double2 *lam_out,
                      const WireCoef *layer_coef, const PassGeom &g, double *partials, int grid,
-                     hipStream_t s, bool ham_pairs = false, double field = 0.0,
+                     hipStream_t s, int ham = kHamNone, double field = 0.0,
                      const CMat2 *gen_tab = nullptr, const CMat2 *gen_utab = nullptr,
                      bool prefetch = false, bool phase_free = false);
 
@@ -405,6 +417,10 @@ struct GradReduceJob {
     int cols;                // 2 (rot_hi - rot_lo)
     int a;                   // tile bit j is wire j (j < a) or h0 + j - a
     int h0;
+    const double *top;       // the top group's pass (kHamFoldTop), or null
+    int top_blocks;
+    const double *above;     // the pass of the group above (fold_unrotated), or null
+    int above_blocks;
 };
 constexpr int kGradReduceJobs = 16;
 struct GradReduce {
