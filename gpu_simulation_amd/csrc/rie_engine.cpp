@@ -461,6 +461,47 @@ void Engine::kt_flush() {
 // Structured adjoint: tile-pass path (n > 12)
 // ---------------------------------------------------------------------------
 
+// Forward pass p of layer l (gen: it generates the layer-0 state); with
+// fwd_energy the last layer's passes add the energy's terms.
+void Engine::launch_fwd(int l, size_t p, bool gen, const double2 *in, double2 *out,
+                        hipStream_t s) {
+    const PassPlan &pp = passes[p];
+    const WireCoef *lc = d_coef + (size_t)l * n;
+    const double S = (double)sizeof(double2) * (double)N;
+    const bool low = p == 0;
+    kt_begin(s);
+    if (fwd_energy && l == L - 1) {
+        PassGeom g = pp.g;
+        g.fold_unrotated = p == 1;  // wire 11 rotates in the low pass, which comes last
+        g.fold_top = p + 1 == passes.size();
+        launch_fwd_energy(low, in, out, lc, g, pp.grid, s, h, d_epartials + energy_partials);
+        energy_partials += (size_t)pp.grid;
+    } else {
+        const int kind = gen ? RIE_PASS_FWD_GEN : low ? RIE_PASS_FWD_LOW : RIE_PASS_FWD_HIGH;
+        launch_fwd_pass(pass_r[kind], low, gen, in, out, lc, d_coef, pp.g, pp.grid, s);
+    }
+    check_launch(low ? "fwd_pass scatter" : "fwd_pass");
+    kt_end(s, low ? "fwd_pass_low_cnot" : gen ? "fwd_pass_high_gen_init" : "fwd_pass_high",
+           gen ? S : 2 * S);
+}
+
+// Forward with the energy's partial sums in d_epartials: from the last layer's
+// passes where they hold every term, else from passes over the final state.
+void Engine::structured_energy(hipStream_t s, bool save_ckpts, const double *params) {
+    fwd_energy = fuse_enabled && fold_ready;
+    energy_partials = 0;
+    try {
+        structured_forward(s, save_ckpts, params);
+    } catch (...) {
+        fwd_energy = false;
+        throw;
+    }
+    if (!fwd_energy) {
+        structured_hamiltonian(s, false);
+    }
+    fwd_energy = false;
+}
+
 void Engine::structured_forward(hipStream_t s, bool save_ckpts, const double *params) {
     const double S = (double)sizeof(double2) * (double)N;
     const int K = (int)passes.size() - 1;  // high passes per layer (>= 1 for n > 12)
@@ -483,7 +524,6 @@ void Engine::structured_forward(hipStream_t s, bool save_ckpts, const double *pa
         // layer 1 is one pass that writes only its output).
         const double2 *in = nullptr;
         for (int l = 1; l < L; ++l) {
-            const WireCoef *lc = d_coef + (size_t)l * n;
             if (l == 1 && gen_fwd) {
                 kt_begin(s);
                 launch_gen_layer1(pass_r[RIE_PASS_FWD_GEN], fbuf(1, K), d_chain, d_chain_u,
@@ -494,21 +534,10 @@ void Engine::structured_forward(hipStream_t s, bool save_ckpts, const double *pa
                 continue;
             }
             for (int j = 0; j < K; ++j) {
-                const bool gen = (l == 1 && j == 0);
-                kt_begin(s);
-                launch_fwd_pass(pass_r[gen ? RIE_PASS_FWD_GEN : RIE_PASS_FWD_HIGH], false, gen, in,
-                                fbuf(l, j), lc, d_coef, passes[1 + j].g,
-                                passes[1 + j].grid, s);
-                check_launch("fwd_pass");
-                kt_end(s, gen ? "fwd_pass_high_gen_init" : "fwd_pass_high", gen ? S : 2 * S);
+                launch_fwd(l, (size_t)(1 + j), l == 1 && j == 0, in, fbuf(l, j), s);
                 in = fbuf(l, j);
             }
-            kt_begin(s);
-            launch_fwd_pass(pass_r[RIE_PASS_FWD_LOW], true, false, in, fbuf(l, K), lc, d_coef,
-                            passes[0].g,
-                            passes[0].grid, s);
-            check_launch("fwd_pass scatter");
-            kt_end(s, "fwd_pass_low_cnot", 2 * S);
+            launch_fwd(l, 0, false, in, fbuf(l, K), s);
             in = fbuf(l, K);
         }
         final_cur = -1;
@@ -522,17 +551,10 @@ void Engine::structured_forward(hipStream_t s, bool save_ckpts, const double *pa
     const double2 *cur = nullptr;
     int cur_buf = -1;  // -1: generated (layer 1, first pass) or a checkpoint buffer
     for (int l = 1; l < L; ++l) {
-        const WireCoef *lc = d_coef + (size_t)l * n;
         const bool gen_layer = (l == 1 && gen_fwd);
         for (int j = 0; j < (gen_layer ? 0 : K); ++j) {
-            const bool gen = (l == 1 && j == 0);
             double2 *out = (cur_buf >= 0) ? pool[cur_buf] : pool[0];
-            kt_begin(s);
-            launch_fwd_pass(pass_r[gen ? RIE_PASS_FWD_GEN : RIE_PASS_FWD_HIGH], false, gen, cur,
-                            out, lc, d_coef, passes[1 + j].g,
-                            passes[1 + j].grid, s);
-            check_launch("fwd_pass");
-            kt_end(s, gen ? "fwd_pass_high_gen_init" : "fwd_pass_high", gen ? S : 2 * S);
+            launch_fwd(l, (size_t)(1 + j), l == 1 && j == 0, cur, out, s);
             if (cur_buf < 0) {
                 cur_buf = 0;
             }
@@ -550,17 +572,14 @@ void Engine::structured_forward(hipStream_t s, bool save_ckpts, const double *pa
             out_buf = (cur_buf == 0) ? 1 : 0;
             out = pool[out_buf];
         }
-        kt_begin(s);
         if (gen_layer) {
+            kt_begin(s);
             launch_gen_layer1(pass_r[RIE_PASS_FWD_GEN], out, d_chain, d_chain_u, passes[0].g,
                               passes[0].grid, s);
             check_launch("gen_layer1");
             kt_end(s, "fwd_layer1_gen", S);
         } else {
-            launch_fwd_pass(pass_r[RIE_PASS_FWD_LOW], true, false, cur, out, lc, d_coef,
-                            passes[0].g, passes[0].grid, s);
-            check_launch("fwd_pass scatter");
-            kt_end(s, "fwd_pass_low_cnot", 2 * S);
+            launch_fwd(l, 0, false, cur, out, s);
         }
         cur = out;
         cur_buf = out_buf;
@@ -1373,10 +1392,14 @@ void Engine::forward_device(const double *params, double *energy, hipStream_t s,
         resident = true;
         return;
     }
-    structured_forward(s, ckpt_every > 0, prep);
     // the adjoint passes form lambda themselves where they can
     lam_deferred = keep_lam && fuse_enabled && fold_ready;
-    structured_hamiltonian(s, keep_lam && !lam_deferred);
+    if (keep_lam && !lam_deferred) {
+        structured_forward(s, ckpt_every > 0, prep);
+        structured_hamiltonian(s, true);
+    } else {
+        structured_energy(s, ckpt_every > 0, prep);
+    }
     if (lam_deferred) {
         take_lam();
     }
@@ -1499,12 +1522,16 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         structured_eval_fused(s, prep, nullptr, h_energy, true);
     } else {
         const bool gate = !on_tiles;
+        // the last layer's forward passes take the energy's terms
+        const bool from_forward = !gate && !want_grad && fuse_enabled && fold_ready;
         stage_begin(s);
         const double *prep = start_coefs(h_params, s);
         stage_end(s, "zero_state_ms");
         stage_begin(s);
         if (gate) {
             gate_forward(s);
+        } else if (from_forward) {
+            structured_energy(s, false, prep);
         } else {
             structured_forward(s, want_grad && ckpt_every > 0, prep);
         }
@@ -1512,7 +1539,7 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
         stage_begin(s);
         if (gate) {
             gate_hamiltonian(s);
-        } else {
+        } else if (!from_forward) {
             structured_hamiltonian(s, want_grad);
         }
         stage_end(s, "hamiltonian_ms");

@@ -223,6 +223,9 @@ struct Engine {
     void stage_end(hipStream_t s, const char *name);
 
     void structured_forward(hipStream_t s, bool save_ckpts, const double *params = nullptr);
+    void launch_fwd(int l, size_t p, bool gen, const double2 *in, double2 *out, hipStream_t s);
+    void structured_energy(hipStream_t s, bool save_ckpts, const double *params);
+    bool fwd_energy = false;  // the running forward's last layer adds the energy's terms
     void structured_hamiltonian(hipStream_t s, bool write_lam);
     bool fused_eval() const;
     double2 *take_lam();

@@ -348,6 +348,219 @@ void launch_init_product_cnot(double2 *out, const WireCoef *coef_layer0, int n, 
 }
 
 // ---------------------------------------------------------------------------
+// Terms of H whose wires are not all rotated yet, and energies.
+// ---------------------------------------------------------------------------
+
+// X_w X_v terms whose lower wire v a pass before this one has un-rotated: in the
+// frame of the state as it is now, X_v is O = U^dagger X U with the wire's
+// rotations U = RZ(phi) RY(theta),
+//   O = [[z, w], [conj(w), -z]], z = sin theta cos phi,
+//   w = cos theta cos phi + i sin phi.
+// The pass before took v's gradients without these terms; their part is
+// <c| dO/dtheta X_w |c> and <c| dO/dphi X_w |c>, formed here.
+struct FoldOp {
+    double z;
+    double wr;
+    double wi;
+    double tz;  // dO/dtheta (its w is real)
+    double tw;
+    double pz;  // dO/dphi
+    double pwr;
+    double pwi;
+};
+
+__device__ __forceinline__ FoldOp fold_op(const WireCoef &k) {
+    const double cp = k.ch * k.ch - k.sh * k.sh;
+    const double sp = 2.0 * k.ch * k.sh;
+    const double ct = k.c * k.c - k.s * k.s;
+    const double st = 2.0 * k.c * k.s;
+    return {st * cp, ct * cp, sp, ct * cp, -st * cp, -st * sp, -ct * sp, cp};
+}
+
+// An operator as one bit value sees it: (O c) = z a + w b with its own amplitude
+// a and the other one b (z and Im w change sign where the bit is set).
+struct FoldSide {
+    double z;
+    double wr;
+    double wi;
+};
+
+__device__ __forceinline__ FoldSide fold_side(const FoldOp &o, bool bit) {
+    return {bit ? -o.z : o.z, o.wr, bit ? -o.wi : o.wi};
+}
+
+__device__ __forceinline__ double2 fold_apply(const FoldSide &o, double2 a, double2 b) {
+    return make_double2(o.z * a.x + o.wr * b.x - o.wi * b.y,
+                        o.z * a.y + o.wr * b.y + o.wi * b.x);
+}
+
+// The expectation parts of <y| O |.>: sums of z's, Re w's and Im w's factors,
+// signs as for the bit clear.
+struct FoldSums {
+    double z = 0.0;
+    double wr = 0.0;
+    double wi = 0.0;
+    __device__ __forceinline__ void add(double2 y, double2 a, double2 b) {
+        z += y.x * a.x + y.y * a.y;
+        wr += y.x * b.x + y.y * b.y;
+        wi += y.y * b.x - y.x * b.y;
+    }
+    // gradient parts (times f), summed over the row into slots at, at + 1
+    __device__ __forceinline__ void finish(const FoldOp &o, bool bit, double f,
+                                           double *__restrict__ row_acc, int at, int lane) const {
+        const double sz = bit ? -z : z;
+        const double si = bit ? -wi : wi;
+        const double r = row_sums2(f * (o.tz * sz + o.tw * wr),
+                                   f * (o.pz * sz + o.pwr * wr + o.pwi * si), lane);
+        if ((lane & 15) < 2) {
+            row_acc[at + (lane & 1)] += r;
+        }
+    }
+};
+
+// Operators of a high pass's fold terms: ops[0] the wire below the group,
+// ops[1], ops[2] wires 0 and 1.
+__device__ __forceinline__ void build_fold_ops(FoldOp *ops, const WireCoef *__restrict__ lc,
+                                               const PassGeom &G, uint32_t t) {
+    if (t < 3) {
+        const int wire = t > 0 ? (int)t - 1 : tile_wire(3, G);
+        // a lower wire that is still rotated: plain X, no gradient part
+        ops[t] = t == 0 && !G.fold_unrotated ? FoldOp{0.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}
+                                             : fold_op(lc[wire]);
+    }
+}
+
+__device__ __forceinline__ double2 lane_xor8(double2 v) {
+    return make_double2(dpp_move<0x128>(v.x), dpp_move<0x128>(v.y));
+}
+
+__device__ __forceinline__ double2 lane_xor1(double2 v) {
+    return make_double2(dpp_move<0xB1>(v.x), dpp_move<0xB1>(v.y));
+}
+
+__device__ __forceinline__ double2 lane_xor2(double2 v) {
+    return make_double2(dpp_move<0x4E>(v.x), dpp_move<0x4E>(v.y));
+}
+
+// Energy terms of the forward passes.  Each term's expectation stays what it is
+// under the rotations of other wires that come later, so a pass takes the terms
+// whose wires its tile holds once they are rotated (those rotated later through
+// their operators O, FoldOp), and no pass over the finished state is needed.
+__device__ __forceinline__ double re_dot(double2 a, double2 b) { return a.x * b.x + a.y * b.y; }
+
+// Re <v| X_j X_{j+1} |v> of adjacent register bits rb, rb + 1 over the thread's
+// registers, each pair of amplitudes once.
+template <int R>
+__device__ __forceinline__ double pair_energy(const double2 (&v)[Tile<R>::REGS], int rb) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < Tile<R>::REGS; ++k) {
+        if ((k & (1 << rb)) == 0) {
+            s += re_dot(v[k], v[k ^ (3 << rb)]);
+        }
+    }
+    return s;
+}
+
+// v of the lane 16 apart.
+__device__ __forceinline__ double lane_xor16(double v, bool odd_row) {
+    const unsigned lo = (unsigned)__double2loint(v);
+    const unsigned hi = (unsigned)__double2hiint(v);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __hiloint2double((int)(odd_row ? h[0] : h[1]), (int)(odd_row ? l[0] : l[1]));
+}
+
+// X terms of a high pass (R = 4) after mapping 0's rotations: the pairs of tile
+// bits 8..11 and the top group's X_0 X_1 X_{n-1}.
+__device__ __forceinline__ double energy_high0(const double2 (&v)[16], uint32_t t,
+                                               const PassGeom &G, const FoldOp *ops) {
+    double e = 0.0;
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+        e += (9 + rb < G.pair_hi ? 2.0 : 0.0) * pair_energy<4>(v, rb);
+    }
+    if (G.fold_top) {
+        const FoldSide o0 = fold_side(ops[1], (t & 1u) != 0);
+        const FoldSide o1 = fold_side(ops[2], (t & 2u) != 0);
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const double2 u = fold_apply(o0, v[k], lane_xor1(v[k]));
+            s += re_dot(v[k ^ 8], fold_apply(o1, u, lane_xor2(u)));
+        }
+        e += 2.0 * s;
+    }
+    return e;
+}
+
+// The others after mapping 2's: the pairs of tile bits 4..7, (7, 8) (bit 8 is
+// lane bit 4) and (3, 4) (bit 3 is lane bit 3).
+__device__ __forceinline__ double energy_high2(const double2 (&v)[16], uint32_t t,
+                                               const PassGeom &G, const FoldOp *ops) {
+    double e = 0.0;
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+        e += (5 + rb < G.pair_hi ? 2.0 : 0.0) * pair_energy<4>(v, rb);
+    }
+    const bool odd_row = (t & 16u) != 0;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const double2 p = make_double2(lane_xor16(v[k ^ 8].x, odd_row),
+                                       lane_xor16(v[k ^ 8].y, odd_row));
+        s += re_dot(v[k], p);
+    }
+    e += (8 < G.pair_hi ? 2.0 : 0.0) * s;
+    const FoldSide o = fold_side(ops[0], (t & 8u) != 0);
+    s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; k += 2) {
+        s += re_dot(v[k], fold_apply(o, v[k ^ 1], lane_xor8(v[k ^ 1])));
+    }
+    return e + 2.0 * s;
+}
+
+// The finished low tile (R = 4) in the frame after the ring CNOT: v holds offsets
+// t | k << 8 (index run + (k << 8), the upper half of the registers run1), lds
+// the tile in offset order.  The ZZ diagonal and the X terms of wires 0..10:
+// register bits, lane bits 0, 1, 3 by DPP, the other thread bits from LDS, two of
+// them at a time: of the pairs under bits a and b an amplitude reads a's where its
+// bits a and b are equal and b's where they differ, which covers each pair once.
+__device__ __forceinline__ void energy_low(const double2 (&v)[16], const double2 *lds, uint32_t t,
+                                           uint64_t run, uint64_t run1, int n, double &diag,
+                                           double &flips) {
+    constexpr uint32_t kStep = 256 + 16;  // slots from register to register
+    double once = 0.0;  // each pair once
+    double both = 0.0;  // each pair from both sides
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const uint64_t idx = (k < 8 ? run : run1) + ((uint64_t)k << 8);
+        diag += ham_diag(idx, n) * re_dot(v[k], v[k]);
+#pragma unroll
+        for (int rb = 0; rb < 3; ++rb) {
+            if ((k & (1 << rb)) == 0) {
+                once += re_dot(v[k], v[k ^ (1 << rb)]);
+            }
+        }
+        both += re_dot(v[k], lane_xor1(v[k])) + re_dot(v[k], lane_xor2(v[k])) +
+                re_dot(v[k], lane_xor8(v[k]));
+    }
+    auto mask_of = [&](int a, int b) {
+        return (((t >> a) ^ (t >> b)) & 1u) == 0 ? 1u << a : 1u << b;
+    };
+    const double2 *p0 = lds + lds_slot<4>(t ^ mask_of(2, 4));
+    const double2 *p1 = lds + lds_slot<4>(t ^ mask_of(5, 6));
+    const double2 *p2 = lds + lds_slot<4>(t ^ (1u << 7));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        once += re_dot(v[k], p0[k * kStep]) + re_dot(v[k], p1[k * kStep]);
+        both += re_dot(v[k], p2[k * kStep]);
+    }
+    flips += 2.0 * once + both;
+}
+
+// ---------------------------------------------------------------------------
 // Forward tile pass.
 // ---------------------------------------------------------------------------
 
@@ -361,11 +574,13 @@ constexpr int tile_min_blocks() {
 // Stores a low tile (a == T) held in mapping M through the ring-CNOT
 // permutation: P(base ^ o) = P(base) ^ P_T(o) ^ (parity(o) ? hi : 0), and bit
 // T-1 of P_T(o) is parity(o), so the image is two contiguous runs.  The tile
-// is placed at P_T(o) in LDS and written out run by run.
-template <int R, int M>
-__device__ __forceinline__ void store_ring_scatter(const double2 (&v)[Tile<R>::REGS],
+// is placed at P_T(o) in LDS and written out run by run.  kEnergy: with the energy
+// terms of energy_low added to diag and flips.
+template <int R, int M, bool kEnergy>
+__device__ __forceinline__ void store_ring_scatter(double2 (&v)[Tile<R>::REGS],
                                                    double2 *lds, uint32_t t, uint64_t base,
-                                                   const PassGeom &G, double2 *out) {
+                                                   const PassGeom &G, double2 *out, double &diag,
+                                                   double &flips) {
     using TL = Tile<R>;
     __syncthreads();
 #pragma unroll
@@ -382,12 +597,16 @@ __device__ __forceinline__ void store_ring_scatter(const double2 (&v)[Tile<R>::R
     double2 *dst1 = out + (run ^ G.hi_mask);
 #pragma unroll
     for (int k = 0; k < TL::REGS; ++k) {
-        const double2 val = lds[lds_slot<R>(omap<R, 0>(t, k))];
+        v[k] = lds[lds_slot<R>(omap<R, 0>(t, k))];
         if (k < TL::REGS / 2) {
-            dst0[(uint64_t)k << (TL::T - R)] = val;
+            dst0[(uint64_t)k << (TL::T - R)] = v[k];
         } else {
-            dst1[(uint64_t)k << (TL::T - R)] = val;
+            dst1[(uint64_t)k << (TL::T - R)] = v[k];
         }
+    }
+    if constexpr (kEnergy) {
+        static_assert(R == 4, "energy_low: register shape 4");
+        energy_low(v, lds, t, run, run ^ G.hi_mask, G.n, diag, flips);
     }
 }
 
@@ -396,18 +615,30 @@ __device__ __forceinline__ void store_ring_scatter(const double2 (&v)[Tile<R>::R
 // generated from nibble tables of the layer-0 factors (lc0).
 constexpr int kInitNibbles = 9;  // covers n <= 36
 
-template <int R, bool kScatter, bool kGenInit>
+// kEnergy: the last layer's passes of an energy evaluation (launch_fwd_energy),
+// register shape 4 (the 512-thread shape spills: 291 us instead of 247 for the
+// evaluation below).  Three passes over the finished state go: 23 qubits x 3
+// layers 337 -> 275 us, 20 x 4 through autograd 248 -> 237 us.
+template <int R, bool kScatter, bool kGenInit, bool kEnergy = false>
 __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void fwd_pass_kernel(
     const double2 *in, double2 *out, const WireCoef *__restrict__ lc,
-    const WireCoef *__restrict__ lc0, PassGeom G) {
+    const WireCoef *__restrict__ lc0, PassGeom G, double field, double *__restrict__ e_partials) {
     using TL = Tile<R>;
     __shared__ double2 lds[TL::SLOTS];
     __shared__ double2 nib[kGenInit ? kInitNibbles : 1][16];
     __shared__ double2 rz_tab[TL::P * TL::REGS];
     __shared__ WireCoef tile_coef[TL::T];
+    __shared__ FoldOp fold_ops[kEnergy && !kScatter ? 3 : 1];
+    __shared__ double red[kEnergy ? TL::WAVES : 1];
+    static_assert(!kEnergy || (!kGenInit && R == 4), "energy terms: register shape 4");
+    double e_diag = 0.0;
+    double e_flips = 0.0;
     const uint32_t t = threadIdx.x;
     const TileAddr ta = tile_addr<R>(t, G);
     build_rz_tables<R>(rz_tab, lc, G, t);
+    if constexpr (kEnergy && !kScatter) {
+        build_fold_ops(fold_ops, lc, G, t);
+    }
     if (t < (uint32_t)TL::T) {
         const bool rot = (int)t >= G.rot_lo && (int)t < G.rot_hi;
         tile_coef[t] = rot ? lc[tile_wire((int)t, G)] : WireCoef{1.0, 0.0, 1.0, 0.0};
@@ -504,7 +735,13 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void fwd_pa
         }
         constexpr bool kHigh = !kScatter;  // high passes: tile bits 0..2 ride along
         phase_fwd<R, 0, kHigh>(v, tile_coef, rz_tab);
-        if constexpr (TL::P == 3) {
+        if constexpr (kEnergy && !kScatter) {
+            // the fold geometry: tile bit 3 is not rotated, so no window 1
+            e_flips += energy_high0(v, t, G, fold_ops);
+            exchange<R, 0, 2>(v, lds, t);
+            phase_fwd<R, 2, kHigh>(v, tile_coef, rz_tab);
+            e_flips += energy_high2(v, t, G, fold_ops);
+        } else if constexpr (TL::P == 3) {
             exchange<R, 0, 1>(v, lds, t);
             phase_fwd<R, 1, kHigh>(v, tile_coef, rz_tab);
             exchange<R, 1, 2>(v, lds, t);
@@ -528,7 +765,21 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void fwd_pa
                 dst[k * ta.strideC] = v[k];
             }
         } else {
-            store_ring_scatter<R, TL::P - 1>(v, lds, t, base, G, out);
+            store_ring_scatter<R, TL::P - 1, kEnergy>(v, lds, t, base, G, out, e_diag, e_flips);
+        }
+    }
+    if constexpr (kEnergy) {
+        const double ws = wave_sum(e_diag - field * e_flips);
+        if ((t & (kWave - 1)) == 0) {
+            red[t / kWave] = ws;
+        }
+        __syncthreads();
+        if (t == 0) {
+            double acc = 0.0;
+            for (int w = 0; w < TL::WAVES; ++w) {
+                acc += red[w];
+            }
+            e_partials[blockIdx.x] = acc;
         }
     }
 }
@@ -544,14 +795,14 @@ static void launch_fwd_pass_r(bool scatter, bool gen_init, const double2 *in, do
     }
     if (gen_init) {
         if (scatter) {
-            fwd_pass_kernel<R, true, true><<<grid, TH, 0, s>>>(in, out, lc, lc0, g);
+            fwd_pass_kernel<R, true, true><<<grid, TH, 0, s>>>(in, out, lc, lc0, g, 0.0, nullptr);
         } else {
-            fwd_pass_kernel<R, false, true><<<grid, TH, 0, s>>>(in, out, lc, lc0, g);
+            fwd_pass_kernel<R, false, true><<<grid, TH, 0, s>>>(in, out, lc, lc0, g, 0.0, nullptr);
         }
     } else if (scatter) {
-        fwd_pass_kernel<R, true, false><<<grid, TH, 0, s>>>(in, out, lc, lc0, g);
+        fwd_pass_kernel<R, true, false><<<grid, TH, 0, s>>>(in, out, lc, lc0, g, 0.0, nullptr);
     } else {
-        fwd_pass_kernel<R, false, false><<<grid, TH, 0, s>>>(in, out, lc, lc0, g);
+        fwd_pass_kernel<R, false, false><<<grid, TH, 0, s>>>(in, out, lc, lc0, g, 0.0, nullptr);
     }
 }
 
@@ -562,6 +813,22 @@ void launch_fwd_pass(int R, bool scatter, bool gen_init, const double2 *in, doub
         launch_fwd_pass_r<4>(scatter, gen_init, in, out, layer_coef, layer0_coef, g, grid, s);
     } else {
         launch_fwd_pass_r<3>(scatter, gen_init, in, out, layer_coef, layer0_coef, g, grid, s);
+    }
+}
+
+void launch_fwd_energy(bool scatter, const double2 *in, double2 *out, const WireCoef *layer_coef,
+                       const PassGeom &g, int grid, hipStream_t s, double field,
+                       double *e_partials) {
+    if (scatter ? g.a != Tile<4>::T || g.rot_lo != 0
+                : g.a != 3 || g.rot_lo != 4 || g.pair_lo != 4 || (g.fold_top && g.h0 + 9 != g.n)) {
+        throw std::invalid_argument("forward energy pass: low tile or fold geometry");
+    }
+    if (scatter) {
+        fwd_pass_kernel<4, true, false, true><<<grid, Tile<4>::THREADS, 0, s>>>(
+            in, out, layer_coef, nullptr, g, field, e_partials);
+    } else {
+        fwd_pass_kernel<4, false, false, true><<<grid, Tile<4>::THREADS, 0, s>>>(
+            in, out, layer_coef, nullptr, g, field, e_partials);
     }
 }
 
@@ -796,7 +1063,8 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void gen_la
         const CMat2 y = chain_y_low<R>(tab, utab + 2 * g, base + omap<R, 0>(tl, 0));
         double2 v[TL::REGS];
         chain_fill<R>(v, tab, y);
-        store_ring_scatter<R, 0>(v, lds, tl, base, G, out);
+        double none = 0.0;
+        store_ring_scatter<R, 0, false>(v, lds, tl, base, G, out, none, none);
     }
 }
 
@@ -919,97 +1187,6 @@ __device__ __forceinline__ void gather_pair_terms(const double2 (&c)[Tile<R>::RE
     } else if constexpr (kHam == kHamPairs && gather_pairs_reach<R, M>()) {
         add_pair_terms<R, M>(c, l, lds, t, G, done, field);
     }
-}
-
-// X_w X_v terms whose lower wire v a pass before this one has un-rotated: in the
-// frame of the state as it is now, X_v is O = U^dagger X U with the wire's
-// rotations U = RZ(phi) RY(theta),
-//   O = [[z, w], [conj(w), -z]], z = sin theta cos phi,
-//   w = cos theta cos phi + i sin phi.
-// The pass before took v's gradients without these terms; their part is
-// <c| dO/dtheta X_w |c> and <c| dO/dphi X_w |c>, formed here.
-struct FoldOp {
-    double z;
-    double wr;
-    double wi;
-    double tz;  // dO/dtheta (its w is real)
-    double tw;
-    double pz;  // dO/dphi
-    double pwr;
-    double pwi;
-};
-
-__device__ __forceinline__ FoldOp fold_op(const WireCoef &k) {
-    const double cp = k.ch * k.ch - k.sh * k.sh;
-    const double sp = 2.0 * k.ch * k.sh;
-    const double ct = k.c * k.c - k.s * k.s;
-    const double st = 2.0 * k.c * k.s;
-    return {st * cp, ct * cp, sp, ct * cp, -st * cp, -st * sp, -ct * sp, cp};
-}
-
-// An operator as one bit value sees it: (O c) = z a + w b with its own amplitude
-// a and the other one b (z and Im w change sign where the bit is set).
-struct FoldSide {
-    double z;
-    double wr;
-    double wi;
-};
-
-__device__ __forceinline__ FoldSide fold_side(const FoldOp &o, bool bit) {
-    return {bit ? -o.z : o.z, o.wr, bit ? -o.wi : o.wi};
-}
-
-__device__ __forceinline__ double2 fold_apply(const FoldSide &o, double2 a, double2 b) {
-    return make_double2(o.z * a.x + o.wr * b.x - o.wi * b.y,
-                        o.z * a.y + o.wr * b.y + o.wi * b.x);
-}
-
-// The expectation parts of <y| O |.>: sums of z's, Re w's and Im w's factors,
-// signs as for the bit clear.
-struct FoldSums {
-    double z = 0.0;
-    double wr = 0.0;
-    double wi = 0.0;
-    __device__ __forceinline__ void add(double2 y, double2 a, double2 b) {
-        z += y.x * a.x + y.y * a.y;
-        wr += y.x * b.x + y.y * b.y;
-        wi += y.y * b.x - y.x * b.y;
-    }
-    // gradient parts (times f), summed over the row into slots at, at + 1
-    __device__ __forceinline__ void finish(const FoldOp &o, bool bit, double f,
-                                           double *__restrict__ row_acc, int at, int lane) const {
-        const double sz = bit ? -z : z;
-        const double si = bit ? -wi : wi;
-        const double r = row_sums2(f * (o.tz * sz + o.tw * wr),
-                                   f * (o.pz * sz + o.pwr * wr + o.pwi * si), lane);
-        if ((lane & 15) < 2) {
-            row_acc[at + (lane & 1)] += r;
-        }
-    }
-};
-
-// Operators of a high pass's fold terms: ops[0] the wire below the group,
-// ops[1], ops[2] wires 0 and 1.
-__device__ __forceinline__ void build_fold_ops(FoldOp *ops, const WireCoef *__restrict__ lc,
-                                               const PassGeom &G, uint32_t t) {
-    if (t < 3) {
-        const int wire = t > 0 ? (int)t - 1 : tile_wire(3, G);
-        // a lower wire that is still rotated: plain X, no gradient part
-        ops[t] = t == 0 && !G.fold_unrotated ? FoldOp{0.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0}
-                                             : fold_op(lc[wire]);
-    }
-}
-
-__device__ __forceinline__ double2 lane_xor8(double2 v) {
-    return make_double2(dpp_move<0x128>(v.x), dpp_move<0x128>(v.y));
-}
-
-__device__ __forceinline__ double2 lane_xor1(double2 v) {
-    return make_double2(dpp_move<0xB1>(v.x), dpp_move<0xB1>(v.y));
-}
-
-__device__ __forceinline__ double2 lane_xor2(double2 v) {
-    return make_double2(dpp_move<0x4E>(v.x), dpp_move<0x4E>(v.y));
 }
 
 // The fold passes' further terms (tile bit 4 the group's lowest wire, bit 3 the wire below

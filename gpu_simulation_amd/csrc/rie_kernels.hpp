@@ -40,6 +40,7 @@ struct PassGeom {
     int pair_hi;
     // Fold passes (kHamFold): the wire below the group is un-rotated already.
     bool fold_unrotated;
+    bool fold_top;  // launch_fwd_energy: the top group's pass (wire n - 1's term)
     // Scattered tile (Hamiltonian pass only): when sc_n > 0, offset bits
     // [a, a + sc_n) are the index bits sc[0] < sc[1] < ... (all >= a), and h0
     // is unused.
@@ -261,6 +262,15 @@ void launch_init_product_cnot(double2 *out, const WireCoef *coef_layer0, int n, 
 void launch_fwd_pass(int R, bool scatter, bool gen_init, const double2 *in, double2 *out,
                      const WireCoef *layer_coef, const WireCoef *layer0_coef, const PassGeom &g,
                      int grid, hipStream_t s);
+
+// The same passes in the last layer of an energy evaluation, with the energy
+// terms whose wires they hold (per-workgroup partials): the low pass the ZZ
+// diagonal and the X terms of wires 0..10, a high pass its pairs, the one below
+// the group and, the top one, wire n - 1's.  Register shape 4; high passes in the
+// fold geometry (rot_lo = 4).
+void launch_fwd_energy(bool scatter, const double2 *in, double2 *out, const WireCoef *layer_coef,
+                       const PassGeom &g, int grid, hipStream_t s, double field,
+                       double *e_partials);
 
 // Layer-1 states from the parameters (chain_site in rie_device.hpp): the
 // state at index i is Tr(run[i's run bits] Y(i)), where the run is the pass's
