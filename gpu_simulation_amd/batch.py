@@ -136,13 +136,12 @@ def main(argv=None) -> None:
     p.add_argument("--evals", type=int, default=3)
     p.add_argument("--dense-only", action="store_true", help="keep only the n <= 8 circuits")
     p.add_argument("--dense-max", type=int, default=8,
-                   help="circuits with n <= this take dense_scan (the autotuner's choice on the "
-                        "2048-circuit mix is 4)")
-    p.add_argument("--threads", type=int, default=256)
+                   help="circuits with n <= this take dense_scan")
+    p.add_argument("--threads", type=int, default=256, help="checked and reported only")
     p.add_argument("--chunks", default="3,3,3,3,3,3,3,3,3,2,2,3,4,4,4",
-                   help="rotation chunk width per qubit count 0..14")
-    p.add_argument("--dense-tile", type=int, default=64)
-    p.add_argument("--grid", type=int, default=128, help="structured persistent workgroups")
+                   help="per qubit count 0..14: checked and reported only")
+    p.add_argument("--dense-tile", type=int, default=64, help="checked and reported only")
+    p.add_argument("--grid", type=int, default=128, help="workgroups of the 14-qubit adjoint launch")
     p.add_argument("--autotune", action="store_true", help="autotune instead of the fixed config")
     args = p.parse_args(argv)
     specs, params = uneven_mix(args.count, seed=args.seed)

@@ -11,7 +11,8 @@
 //    low tile (index bits [0, T)) is two contiguous runs, so the permutation
 //    rides on the last LDS exchange of the forward low pass (scatter) and on
 //    the first exchange of the backward low pass (gather).
-//  * Small circuits (n <= 12) run entirely in one workgroup's LDS.
+//  * Small circuits (n <= 12) run entirely in one workgroup's registers
+//    (rie_regcircuit.hip).
 //  * Reductions (energy, gradients) are per-workgroup partials followed by a
 //    fixed-order reduction kernel: results are bitwise reproducible.
 #include "rie_kernels.hpp"
@@ -618,7 +619,7 @@ constexpr int kInitNibbles = 9;  // covers n <= 36
 // kEnergy: the last layer's passes of an energy evaluation (launch_fwd_energy),
 // register shape 4 (the 512-thread shape spills: 291 us instead of 247 for the
 // evaluation below).  Three passes over the finished state go: 23 qubits x 3
-// layers 337 -> 275 us, 20 x 4 through autograd 248 -> 237 us.
+// layers 337 -> 257 us, 20 x 4 through autograd 248 -> 234 us.
 template <int R, bool kScatter, bool kGenInit, bool kEnergy = false>
 __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void fwd_pass_kernel(
     const double2 *in, double2 *out, const WireCoef *__restrict__ lc,
@@ -1577,7 +1578,7 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
 // kAllBits: the window's gradients of every bit, without the uniform
 // rot_lo / rot_hi tests: the generating low pass rotates every tile bit, and
 // the generated start's high passes leave only gradient slots that
-// reduce_grad never reads (it takes the columns of [rot_lo, rot_hi)).
+// reduce_kernel never reads (it takes the columns of [rot_lo, rot_hi)).
 template <int R, int M, bool kPhased = true, bool kAllBits = false>
 __device__ __forceinline__ void grad_window(double2 (&c)[Tile<R>::REGS],
                                             double2 (&l)[Tile<R>::REGS],
@@ -1647,7 +1648,7 @@ __device__ __forceinline__ void grad_window(double2 (&c)[Tile<R>::REGS],
         }
         // lane s (s < 8) of each row holds slot 2 * P0 + s: bit P0 + s / 2,
         // dt for s even, dp for s odd.  The slots of unrotated bits are
-        // accumulated too and never read (reduce_grad takes the columns of
+        // accumulated too and never read (reduce_kernel takes the columns of
         // [rot_lo, rot_hi) only).
         const double r = row_sums8_rest(u, lane);
         if ((lane & 15) < 8) {
