@@ -2717,33 +2717,42 @@ void launch_ham_pass(int R, bool diag, bool read_lam, bool write_lam, const doub
 // Fixed-order reductions.
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void reduce_sum_kernel(const double *__restrict__ values,
-                                                         int count, double *__restrict__ out,
-                                                         const double *__restrict__ scale) {
-    __shared__ double red[4];
+// One workgroup, bound by the latency of its loads: 1024 threads, four loads in
+// flight each (6144 partials of a 23-qubit energy: 9.6 us with 256 threads and one
+// load at a time, 4.3 so).
+__global__ __launch_bounds__(1024) void reduce_sum_kernel(const double *__restrict__ values,
+                                                          int count, double *__restrict__ out,
+                                                          const double *__restrict__ scale) {
+    __shared__ double red[16];
     const int t = threadIdx.x;
-    double acc = 0.0;
-    for (int i = t; i < count; i += 256) {
-        acc += values[i];
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int i = t; i < count; i += 4096) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int at = i + 1024 * u;
+            acc[u] += at < count ? values[at] : 0.0;
+        }
     }
-    acc = wave_sum(acc);
+    const double sum = wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
     if ((t & 63) == 0) {
-        red[t >> 6] = acc;
+        red[t >> 6] = sum;
     }
     __syncthreads();
-    if (t == 0) {
-        const double f = scale != nullptr ? *scale : 1.0;
-        *out = (red[0] + red[1] + red[2] + red[3]) * f;
+    if (t < 64) {
+        const double total = wave_sum(t < 16 ? red[t] : 0.0);
+        if (t == 0) {
+            *out = total * (scale != nullptr ? *scale : 1.0);
+        }
     }
 }
 
 void launch_reduce_sum(const double *values, int count, double *out, hipStream_t s) {
-    reduce_sum_kernel<<<1, 256, 0, s>>>(values, count, out, nullptr);
+    reduce_sum_kernel<<<1, 1024, 0, s>>>(values, count, out, nullptr);
 }
 
 void launch_reduce_to(const double *partials, int count, double *out, const double *scale,
                       hipStream_t s) {
-    reduce_sum_kernel<<<1, 256, 0, s>>>(partials, count, out, scale);
+    reduce_sum_kernel<<<1, 1024, 0, s>>>(partials, count, out, scale);
 }
 
 __global__ __launch_bounds__(256) void drift_kernel(const double2 *__restrict__ state,
