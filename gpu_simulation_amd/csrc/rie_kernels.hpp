@@ -242,7 +242,6 @@ void launch_mlp_forward(const float *X, const float *W, const float *bias, float
 void launch_mlp_output_loss(const float *X, const float *W, const float *bias, const float *T,
                             float *dY, int rows, int cols, int K, float *partials,
                             float *loss_out, hipStream_t s);
-size_t mlp_mse_partials(int rows, int cols);
 // dZ = (dY W^T) * GELU'(Z) (rows x cols; dY: rows x K, W: cols x K).
 void launch_mlp_backward_data(const float *dY, const float *W, const float *Z, float *dZ, int rows,
                               int cols, int K, hipStream_t s);

@@ -17,6 +17,7 @@
 #include "rie.h"
 #include "rie_engine_internal.hpp"
 #include "rie_kernels.hpp"
+#include "rie_mlp_shape.hpp"
 
 namespace rie {
 
@@ -53,7 +54,8 @@ struct Mlp {
 };
 
 Mlp::Mlp(int in_, int hidden_, int out_, uint64_t seed) : in(in_), hidden(hidden_), out(out_) {
-    if (in < 1 || hidden < 1 || out < 1 || in > 4096 || hidden > 4096 || out > 4096) {
+    if (in < 1 || hidden < 1 || out < 1 || in > kMlpMaxWidth || hidden > kMlpMaxWidth ||
+        out > kMlpMaxWidth) {
         fail(RIE_INVALID_ARGUMENT, "MLP sizes must be in [1, 4096].");
     }
     o_w1 = 0;
@@ -109,7 +111,7 @@ Mlp::~Mlp() {
 }
 
 void Mlp::ensure_rows(int rows) {
-    if (rows < 1 || rows > (1 << 22)) {
+    if (rows < 1 || rows > kMlpMaxRows) {
         fail(RIE_INVALID_ARGUMENT, "MLP batches need 1 <= rows <= 2^22.");
     }
     if (rows <= cap) {

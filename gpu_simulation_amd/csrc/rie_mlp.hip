@@ -20,9 +20,8 @@
 // a serial loss sum; 135 us now.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "rie_kernels.hpp"
+#include "rie_mlp_shape.hpp"
 
 namespace rie {
 
@@ -74,8 +73,12 @@ __global__ __launch_bounds__(256) void mlp_gemm_kernel(MlpGemm g) {
     const int wave = t >> 6;
     const int i = lane & 15;
     const int q = lane >> 4;
-    const int m0 = blockIdx.y * 16 * kSub;
+    const unsigned row_tile = blockIdx.z * gridDim.y + blockIdx.y;
+    const int m0 = (int)row_tile * 16 * kSub;
     const int n0 = blockIdx.x * 16 * kSub;
+    if (m0 >= g.M) {
+        return;
+    }
     float4_t acc[kSub][kSub];
 #pragma unroll
     for (int a = 0; a < kSub; ++a) {
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(256) void mlp_gemm_kernel(MlpGemm g) {
         }
         __syncthreads();
         if (t == 0) {
-            g.partials[blockIdx.y * gridDim.x + blockIdx.x] =
+            g.partials[row_tile * gridDim.x + blockIdx.x] =
                 (red[0] + red[1]) + (red[2] + red[3]);
         }
     }
@@ -222,20 +225,11 @@ __global__ __launch_bounds__(256) void mlp_loss_kernel(const float *__restrict__
 
 namespace {
 
-// 32 x 32 tiles read each operand half as often; below 512 of them the chip has
-// idle CUs and the shorter tiles win.
-constexpr int kWideTiles = 512;
-
-int sub_for(int M, int N) {
-    return (long)((M + 31) / 32) * ((N + 31) / 32) >= kWideTiles ? 2 : 1;
-}
-
 template <bool kTA, bool kTB, int kEpi>
 void gemm(const MlpGemm &g, hipStream_t s) {
-    const int sub = sub_for(g.M, g.N);
-    const int tile = 16 * sub;
-    dim3 grid((g.N + tile - 1) / tile, (g.M + tile - 1) / tile);
-    if (sub == 2) {
+    const MlpGrid shape = mlp_grid(g.M, g.N);
+    const dim3 grid(shape.x, shape.y, shape.z);
+    if (shape.sub == 2) {
         mlp_gemm_kernel<kTA, kTB, kEpi, 2><<<grid, 256, 0, s>>>(g);
     } else {
         mlp_gemm_kernel<kTA, kTB, kEpi, 1><<<grid, 256, 0, s>>>(g);
@@ -247,13 +241,6 @@ bool wide_rows(const float *p, int ld) {
 }
 
 }  // namespace
-
-size_t mlp_mse_partials(int rows, int cols) {
-    // the 16 x 16 grid of fewer rows may be the larger one
-    const size_t wide = (size_t)((rows + 31) / 32) * ((cols + 31) / 32);
-    return std::max<size_t>(wide, 4 * (size_t)kWideTiles + (size_t)(cols + 15) / 16 * 2 +
-                                      (size_t)(rows + 15) / 16 * 2);
-}
 
 void launch_mlp_forward(const float *X, const float *W, const float *bias, float *Z, float *act,
                         int rows, int cols, int K, hipStream_t s) {
@@ -272,9 +259,8 @@ void launch_mlp_output_loss(const float *X, const float *W, const float *bias, c
     MlpGemm g{X, W, dY, rows, cols, K, 0, wide_rows(X, K), 0, bias, nullptr, T, partials,
               2.0f / (float)count};
     gemm<false, false, kMlpEpiMse>(g, s);
-    const int tile = 16 * sub_for(rows, cols);
-    const int n = ((rows + tile - 1) / tile) * ((cols + tile - 1) / tile);
-    mlp_loss_kernel<<<1, 256, 0, s>>>(partials, n, count, loss_out);
+    const MlpGrid grid = mlp_grid(rows, cols);
+    mlp_loss_kernel<<<1, 256, 0, s>>>(partials, (int)(grid.rows * grid.x), count, loss_out);
 }
 
 void launch_mlp_backward_data(const float *dY, const float *W, const float *Z, float *dZ, int rows,
