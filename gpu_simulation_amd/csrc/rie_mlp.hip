@@ -204,7 +204,8 @@ __global__ __launch_bounds__(256) void mlp_gemm_kernel(MlpGemm g) {
 
 // loss = sum of the workgroups' squares / count, in a fixed order.
 __global__ __launch_bounds__(256) void mlp_loss_kernel(const float *__restrict__ partials, int n,
-                                                       int count, float *__restrict__ loss_out) {
+                                                       long long count,
+                                                       float *__restrict__ loss_out) {
     __shared__ float red[4];
     float acc = 0.0f;
     for (int i = threadIdx.x; i < n; i += 256) {
@@ -255,7 +256,7 @@ void launch_mlp_forward(const float *X, const float *W, const float *bias, float
 void launch_mlp_output_loss(const float *X, const float *W, const float *bias, const float *T,
                             float *dY, int rows, int cols, int K, float *partials,
                             float *loss_out, hipStream_t s) {
-    const int count = rows * cols;
+    const long long count = mlp_elements(rows, cols);
     MlpGemm g{X, W, dY, rows, cols, K, 0, wide_rows(X, K), 0, bias, nullptr, T, partials,
               2.0f / (float)count};
     gemm<false, false, kMlpEpiMse>(g, s);

@@ -42,4 +42,7 @@ constexpr size_t mlp_mse_partials(int rows, int cols) {
     return wide > 4 * (size_t)kMlpWideTiles ? wide : 4 * (size_t)kMlpWideTiles;
 }
 
+// Values that the loss is the mean of: up to 2^34.
+constexpr long long mlp_elements(int rows, int cols) { return (long long)rows * cols; }
+
 }  // namespace rie

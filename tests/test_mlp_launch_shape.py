@@ -25,7 +25,8 @@ int main() {
     int m, n;
     while (std::scanf("%d %d", &m, &n) == 2) {
         const rie::MlpGrid g = rie::mlp_grid(m, n);
-        std::printf("%d %u %u %u %u %zu\n", g.sub, g.rows, g.x, g.y, g.z, rie::mlp_mse_partials(m, n));
+        std::printf("%d %u %u %u %u %zu %lld\n", g.sub, g.rows, g.x, g.y, g.z,
+                    rie::mlp_mse_partials(m, n), rie::mlp_elements(m, n));
     }
 }
 """
@@ -50,7 +51,7 @@ def shapes(tmp_path_factory):
 def test_grids_stay_within_the_launch_limits(shapes):
     # row calls (rows x width) and weight gradients (width + 1 x width)
     pairs = [(m, n) for m in ROWS for n in SIZES] + [(m + 1, n) for m in SIZES for n in SIZES]
-    for (m, n), (sub, row_tiles, x, y, z, _) in zip(pairs, shapes(pairs)):
+    for (m, n), (sub, row_tiles, x, y, z, _, _) in zip(pairs, shapes(pairs)):
         tile = 16 * sub
         assert 1 <= y <= 65535 and 1 <= z <= 65535 and x * 256 < 1 << 32, (m, n)
         assert (row_tiles - 1) * tile < m <= row_tiles * tile, (m, n)
@@ -62,6 +63,13 @@ def test_grids_stay_within_the_launch_limits(shapes):
 def test_loss_partials_hold_every_smaller_grid(shapes, cols):
     rows = sorted({1, 2, 511, 512, 513, 8191, 8192, 16384, 16385, *ROWS})
     out = shapes([(m, cols) for m in rows])
-    for k, (*_, room) in enumerate(out):
-        for _, row_tiles, x, _, _, _ in out[:k + 1]:
+    for k, (*_, room, _) in enumerate(out):
+        for _, row_tiles, x, *_ in out[:k + 1]:
             assert row_tiles * x <= room, (rows[k], cols)
+
+
+def test_the_loss_is_a_mean_over_all_values(shapes):
+    # 2^22 rows of 4096 outputs: more values than 32 bits count
+    pairs = [(m, n) for m in ROWS for n in SIZES]
+    for (m, n), (*_, elements) in zip(pairs, shapes(pairs)):
+        assert elements == m * n
