@@ -44,6 +44,17 @@ namespace rie {
 namespace {
 
 constexpr int kMaxN = kBatchMaxQubits;
+constexpr size_t kStateAmps = (size_t)1 << kMaxN;  // of a 14-qubit circuit
+
+// An evaluation holds the layers' records (up to 1 KB each) and 256 KB for every
+// 14-qubit circuit.  Large batches run in slices that use that memory in turn.  A
+// slice ends at a gigabyte once it has sixteen circuits for each CU, enough
+// for the tail between two slices not to count (8192 circuits of 14 qubits x 2
+// layers in three slices 12.1 ms, in one 11.9; 260 circuits of 4 qubits x 8192
+// layers, cut at a gigabyte too, would take 18.6 ms instead of 11.3), and in
+// any case at a quarter of the free device memory (at least a quarter gigabyte).
+constexpr size_t kSliceBytes = (size_t)1 << 30;
+constexpr int kSliceCircuitsPerCu = 16;
 
 }  // namespace
 
@@ -92,28 +103,38 @@ struct Batch {
         int first;  // in d_reg_g / d_reg_e
         int count;
     };
-    std::vector<RegGroup> reg_groups;   // largest n first
+    // circuits evaluated together: their records and states share d_rec and
+    // d_psi with the other slices'
+    struct Slice {
+        int first_layer = 0;  // in d_layer_job
+        int layers = 0;
+        int g_first = 0;      // in d_jobs_g / d_jobs_e
+        int g_count = 0;
+        int grid = 0;         // workgroups of the 14-qubit adjoint launch
+        int begin_off = 0;    // its schedule in d_wg_begin
+        std::vector<RegGroup> groups;  // largest n first
+    };
+    std::vector<Slice> slices;
     std::vector<RegJob> reg_jobs;       // with gradients, grouped, deepest first
     std::vector<RecordJob> reg_rec;     // indexed like reg_jobs
     std::vector<RecordJob> rec_jobs;    // every structured circuit
     std::vector<int> reg_of;            // circuit -> reg_jobs index, or -1
-    int reg_layers = 0;                 // records of one evaluation
     RegJob *d_reg_g = nullptr;
     RegJob *d_reg_e = nullptr;
     RecordJob *d_rec_jobs = nullptr;
     int *d_layer_job = nullptr;
     double *d_rec = nullptr;
     // 14 qubits
-    std::vector<int> gids;
-    std::vector<Reg14Job> jobs_g;    // with gradients, indexed like gids
-    std::vector<RecordJob> jobs_rec; // indexed like gids
+    std::vector<int> gid_of;         // circuit -> jobs_g index, or -1
+    std::vector<Reg14Job> jobs_g;    // with gradients
+    std::vector<RecordJob> jobs_rec; // indexed like jobs_g
     Reg14Job *d_jobs_g = nullptr;
     Reg14Job *d_jobs_e = nullptr;  // energy only
     double2 *d_psi = nullptr;      // forward results of the 14-qubit circuits
     int *d_order = nullptr;
     int *d_wg_begin = nullptr;
     double2 *d_scratch = nullptr;
-    int grid = 0;
+    int grid = 0;  // the slices' largest
     int threads = 512;  // reported only, like chunk_by_n and dense_tile below:
                         // the kernels have one shape per qubit count
     int grid_limit = 0;  // 0: every CU
@@ -142,6 +163,7 @@ struct Batch {
     void release_structured();
     void invalidate_graph();
     void issue_eval(hipStream_t s, bool want_grad);
+    void issue_slice(hipStream_t s, bool want_grad, const Slice &sl, bool with_dense);
     void issue_step(hipStream_t s, int optimizer, double lr, int capacity);
     void launch_graph(int kind, double lr, int capacity, hipStream_t s);
     void run(hipStream_t s, bool want_grad);
@@ -154,7 +176,7 @@ struct Batch {
     void ensure_adam();
     std::string config_json() const;
     // whether anything runs beside the persistent launch
-    bool parts_beside() const { return !dids.empty() || !reg_groups.empty(); }
+    bool parts_beside() const { return !dids.empty() || !reg_jobs.empty(); }
 };
 
 Batch::Batch(size_t count_, const int *nq, const int *nl, const double *fields, int dense_max_qubits)
@@ -292,11 +314,10 @@ void Batch::release_structured() {
     d_rec_jobs = nullptr;
     d_layer_job = nullptr;
     d_rec = nullptr;
-    reg_groups.clear();
+    slices.clear();
     reg_jobs.clear();
     rec_jobs.clear();
     reg_rec.clear();
-    reg_layers = 0;
     d_jobs_g = d_jobs_e = nullptr;
     d_order = d_wg_begin = nullptr;
     d_scratch = nullptr;
@@ -308,6 +329,7 @@ void Batch::release_structured() {
 void Batch::build_register_jobs() {
     std::vector<int> ids = sids;
     reg_of.assign(count, -1);
+    gid_of.assign(count, -1);
     if (ids.empty()) {
         return;
     }
@@ -315,36 +337,85 @@ void Batch::build_register_jobs() {
         return n[(size_t)a] != n[(size_t)b] ? n[(size_t)a] > n[(size_t)b]
                                             : L[(size_t)a] > L[(size_t)b];
     });
-    size_t bytes = 0;
-    for (int i : ids) {
-        bytes += circuit_record_bytes(n[(size_t)i], L[(size_t)i]);
-    }
-    d_rec = (double *)device_alloc(bytes, "alloc batch records");
     std::vector<int> layer_job;
-    double *rec = d_rec;
+    std::vector<size_t> place;  // record offsets of rec_jobs in their slice
+    size_t rec_bytes = 0;       // of the running slice
+    size_t psi_bytes = 0;
+    int in_slice = 0;
+    size_t rec_top = 0;         // of the largest
+    size_t psi_top = 0;
+    size_t most = 0;  // a quarter of the free memory, asked for where it can matter
     for (int i : ids) {
         const int q = n[(size_t)i];
         const int layers = L[(size_t)i];
-        const RegJob job{rec, d_energy + i, d_grad + poff[(size_t)i], nullptr, nullptr,
+        const bool large = q > kRegMaxQubits;
+        const size_t bytes = circuit_record_bytes(q, layers);
+        const size_t state = large ? sizeof(double2) * kStateAmps : 0;
+        const size_t held = rec_bytes + bytes + psi_bytes + state;
+        if (held > kSliceBytes / 4 && most == 0) {
+            size_t free_b = 0;
+            size_t total_b = 0;
+            check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+            most = std::max(free_b, kSliceBytes) / 4;
+        }
+        if (slices.empty() || (most > 0 && held > most) ||
+            (held > kSliceBytes && in_slice >= kSliceCircuitsPerCu * num_cus)) {
+            Slice next;
+            next.first_layer = (int)layer_job.size();
+            next.g_first = (int)jobs_g.size();
+            slices.push_back(next);
+            rec_bytes = 0;
+            psi_bytes = 0;
+            in_slice = 0;
+        }
+        in_slice += 1;
+        Slice &sl = slices.back();
+        const RegJob job{nullptr, d_energy + i, d_grad + poff[(size_t)i], nullptr, nullptr,
                          h[(size_t)i], layers, 0};
-        const RecordJob record{d_params + poff[(size_t)i], rec, q, reg_layers};
+        const RecordJob record{d_params + poff[(size_t)i], nullptr, q, sl.layers};
         layer_job.insert(layer_job.end(), (size_t)layers, (int)rec_jobs.size());
         rec_jobs.push_back(record);
-        reg_layers += layers;
-        rec += circuit_record_bytes(q, layers) / sizeof(double);
-        if (q > kRegMaxQubits) {
-            gids.push_back(i);
+        place.push_back(rec_bytes / sizeof(double));
+        sl.layers += layers;
+        rec_bytes += bytes;
+        rec_top = std::max(rec_top, rec_bytes);
+        if (large) {
+            gid_of[(size_t)i] = (int)jobs_g.size();
             jobs_g.push_back({job, nullptr});
             jobs_rec.push_back(record);
+            sl.g_count += 1;
+            psi_bytes += state;
+            psi_top = std::max(psi_top, psi_bytes);
             continue;
         }
-        if (reg_groups.empty() || reg_groups.back().n != q) {
-            reg_groups.push_back({q, (int)reg_jobs.size(), 0});
+        if (sl.groups.empty() || sl.groups.back().n != q) {
+            sl.groups.push_back({q, (int)reg_jobs.size(), 0});
         }
-        reg_groups.back().count += 1;
+        sl.groups.back().count += 1;
         reg_of[(size_t)i] = (int)reg_jobs.size();
         reg_jobs.push_back(job);
         reg_rec.push_back(record);
+    }
+    d_rec = (double *)device_alloc(rec_top, "alloc batch records");
+    if (psi_top > 0) {
+        d_psi = (double2 *)device_alloc(psi_top, "alloc batch states");
+    }
+    for (size_t k = 0; k < rec_jobs.size(); ++k) {
+        double *rec = d_rec + place[k];
+        const size_t i = (size_t)ids[k];
+        rec_jobs[k].rec = rec;
+        if (gid_of[i] >= 0) {
+            jobs_g[(size_t)gid_of[i]].base.rec = rec;
+            jobs_rec[(size_t)gid_of[i]].rec = rec;
+        } else {
+            reg_jobs[(size_t)reg_of[i]].rec = rec;
+            reg_rec[(size_t)reg_of[i]].rec = rec;
+        }
+    }
+    for (const Slice &sl : slices) {
+        for (int k = 0; k < sl.g_count; ++k) {
+            jobs_g[(size_t)(sl.g_first + k)].psi = d_psi + kStateAmps * (size_t)k;
+        }
     }
     std::vector<RegJob> energy_only = reg_jobs;
     for (auto &j : energy_only) {
@@ -369,50 +440,52 @@ void Batch::build_register_jobs() {
           "upload batch layers");
 }
 
-// Jobs and records, and a longest-first schedule of the 14-qubit circuits'
-// adjoint sweeps over `grid` workgroups.
+// Jobs and records, and for each slice a longest-first schedule of its 14-qubit
+// circuits' adjoint sweeps over its workgroups.
 void Batch::build_structured() {
     invalidate_graph();
     release_structured();
     jobs_g.clear();
     jobs_rec.clear();
-    gids.clear();
     build_register_jobs();
-    if (gids.empty()) {
+    if (jobs_g.empty()) {
         return;
     }
     const int cap = grid_limit > 0 ? grid_limit : num_cus;
-    grid = (int)std::min<size_t>(gids.size(), (size_t)std::max(1, cap));
-    constexpr size_t kAmps = (size_t)1 << kMaxN;
-    d_psi = (double2 *)device_alloc(sizeof(double2) * kAmps * gids.size(), "alloc batch states");
-    for (size_t k = 0; k < gids.size(); ++k) {
-        jobs_g[k].psi = d_psi + kAmps * k;
-    }
-    // LPT: heaviest first onto the least-loaded workgroup
-    std::vector<int> idx(gids.size());
-    for (size_t k = 0; k < idx.size(); ++k) {
-        idx[k] = (int)k;
-    }
-    auto cost = [&](int k) { return (double)jobs_g[(size_t)k].base.layers; };
-    std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return cost(a) > cost(b); });
-    using Slot = std::pair<double, int>;
-    std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> heap;
-    for (int b = 0; b < grid; ++b) {
-        heap.push({0.0, b});
-    }
-    std::vector<std::vector<int>> lists((size_t)grid);
-    for (int k : idx) {
-        Slot s = heap.top();
-        heap.pop();
-        lists[(size_t)s.second].push_back(k);
-        s.first += cost(k);
-        heap.push(s);
-    }
-    std::vector<int> order;
-    std::vector<int> begin(1, 0);
-    for (const auto &lst : lists) {
-        order.insert(order.end(), lst.begin(), lst.end());
+    std::vector<int> order;  // places in the slice's jobs
+    std::vector<int> begin;
+    for (Slice &sl : slices) {
+        if (sl.g_count == 0) {
+            continue;
+        }
+        sl.grid = std::min(sl.g_count, std::max(1, cap));
+        grid = std::max(grid, sl.grid);
+        // LPT: heaviest first onto the least-loaded workgroup
+        std::vector<int> idx((size_t)sl.g_count);
+        for (size_t k = 0; k < idx.size(); ++k) {
+            idx[k] = (int)k;
+        }
+        auto cost = [&](int k) { return (double)jobs_g[(size_t)(sl.g_first + k)].base.layers; };
+        std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return cost(a) > cost(b); });
+        using Slot = std::pair<double, int>;
+        std::priority_queue<Slot, std::vector<Slot>, std::greater<Slot>> heap;
+        for (int b = 0; b < sl.grid; ++b) {
+            heap.push({0.0, b});
+        }
+        std::vector<std::vector<int>> lists((size_t)sl.grid);
+        for (int k : idx) {
+            Slot top = heap.top();
+            heap.pop();
+            lists[(size_t)top.second].push_back(k);
+            top.first += cost(k);
+            heap.push(top);
+        }
+        sl.begin_off = (int)begin.size();
         begin.push_back((int)order.size());
+        for (auto &lst : lists) {
+            order.insert(order.end(), lst.begin(), lst.end());
+            begin.push_back((int)order.size());
+        }
     }
     std::vector<Reg14Job> jobs_e = jobs_g;
     for (auto &j : jobs_e) {
@@ -448,13 +521,24 @@ void Batch::build_dense() {
 }
 
 void Batch::issue_eval(hipStream_t s, bool want_grad) {
-    if (reg_layers > 0) {
-        launch_circuit_records(d_rec_jobs, RecordJob{}, d_layer_job, reg_layers, s);
+    for (size_t k = 0; k < std::max<size_t>(1, slices.size()); ++k) {
+        issue_slice(s, want_grad, k < slices.size() ? slices[k] : Slice{}, k == 0);
+    }
+}
+
+// One slice's records and circuits, the first with the dense circuits beside
+// them.  Everything has joined s again at the end: the next slice writes the
+// same records and states.
+void Batch::issue_slice(hipStream_t s, bool want_grad, const Slice &sl, bool with_dense) {
+    if (sl.layers > 0) {
+        launch_circuit_records(d_rec_jobs, RecordJob{}, d_layer_job + sl.first_layer, sl.layers,
+                               s);
         check_launch("batch records");
     }
+    const bool dense_here = with_dense && !dids.empty();
     // part i of the evaluation runs on stream i mod 4 (0: s itself): the
     // largest circuits first, each stream's parts one after the other
-    const int parts = (gids.empty() ? 0 : 1) + (dids.empty() ? 0 : 1) + (int)reg_groups.size();
+    const int parts = (sl.g_count > 0 ? 1 : 0) + (dense_here ? 1 : 0) + (int)sl.groups.size();
     const int used = std::min(parts - 1, kAux);
     if (used > 0) {
         check(hipEventRecord(ev_fork, s), "record fork");
@@ -467,15 +551,15 @@ void Batch::issue_eval(hipStream_t s, bool want_grad) {
         const int k = part++ % (kAux + 1);
         return k == 0 ? s : s_aux[k - 1];
     };
-    if (!gids.empty()) {
-        launch_reg14(want_grad ? d_jobs_g : d_jobs_e, Reg14Job{}, d_order, d_wg_begin,
-                     (int)gids.size(), grid, d_scratch, next_stream());
+    if (sl.g_count > 0) {
+        launch_reg14((want_grad ? d_jobs_g : d_jobs_e) + sl.g_first, Reg14Job{}, d_order,
+                     d_wg_begin + sl.begin_off, sl.g_count, sl.grid, d_scratch, next_stream());
         check_launch("batch 14 qubits");
     }
-    if (!dids.empty()) {
+    if (dense_here) {
         dense.run(next_stream(), want_grad);
     }
-    for (const RegGroup &g : reg_groups) {
+    for (const RegGroup &g : sl.groups) {
         launch_regcircuit(g.n, (want_grad ? d_reg_g : d_reg_e) + g.first, RegJob{}, g.count,
                           next_stream());
         check_launch("batch circuits");
@@ -586,7 +670,7 @@ void Batch::run_per_circuit(hipStream_t s, bool want_grad) {
             dense_single[di++]->run(s, want_grad);
             continue;
         }
-        const size_t k = (size_t)(std::find(gids.begin(), gids.end(), (int)i) - gids.begin());
+        const size_t k = (size_t)gid_of[i];
         Reg14Job j = jobs_g[k];
         RecordJob r = jobs_rec[k];
         r.first_layer = 0;
@@ -690,7 +774,7 @@ void Batch::autotune(size_t repeats) {
             repartition(split);
         }
         std::vector<int> grid_opts;
-        if (!gids.empty()) {
+        if (!jobs_g.empty()) {
             if (parts_beside()) {
                 for (int f : {1, 2, 3, 4}) {
                     grid_opts.push_back(num_cus * f / 4);
