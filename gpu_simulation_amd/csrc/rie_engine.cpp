@@ -215,14 +215,21 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     check(hipEventCreateWithFlags(&ev_last, hipEventDisableTiming), "hipEventCreate");
     build_plan();
     // The gate-level strategy's results are those of the structured sweeps, so
-    // it runs on the same kernels; above kGateTileQubits, where their four state
-    // buffers and tables would take memory that two buffers leave free, gate by
-    // gate.  15 qubits x 2 layers through the host call: 849 us gate by gate
-    // (about 250 launches), 75 us on the tile passes.
+    // it runs on the same kernels: 15 qubits x 2 layers through the host call 849
+    // us gate by gate (about 250 launches), 75 us on the tile passes, 26 x 2 187
+    // and 1.9 ms.  These hold four state buffers and tables of 1/64 of them
+    // where gate by gate takes two buffers, so it stays gate by gate above
+    // kGateTileQubits and where they are not free.
     const bool gate = strategy == RIE_STRATEGY_INVERSE_WALK_GATE;
+    size_t free_b = 0;
+    if (!small && strategy != RIE_STRATEGY_DENSE_SCAN && (!gate || n <= kGateTileQubits)) {
+        size_t total_b = 0;
+        check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    }
+    const size_t tile_bytes = (4 * sizeof(double2) + 1) * N + ((size_t)32 << 20);
     whole = small && (gate || strategy == RIE_STRATEGY_STRUCTURED_ADJOINT);
     on_tiles = !small && (strategy == RIE_STRATEGY_STRUCTURED_ADJOINT ||
-                       (gate && n <= kGateTileQubits));
+                           (gate && n <= kGateTileQubits && tile_bytes <= free_b));
 
     d_params = (double *)device_alloc(sizeof(double) * num_params, "alloc params");
     d_grad = (double *)device_alloc(sizeof(double) * num_params, "alloc gradient");
@@ -243,9 +250,6 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     } else if (on_tiles) {
         // The stored schedule keeps every forward pass output; use it when it
         // fits comfortably in free device memory, else walk back by inverse gates.
-        size_t free_b = 0;
-        size_t total_b = 0;
-        check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
         const double need = (double)stored_buffer_count() * (double)sizeof(double2) * (double)N;
         schedule = (!gate && L > 1 && need <= 0.85 * (double)free_b) ? RIE_SCHEDULE_STORED
                                                                      : RIE_SCHEDULE_INVERSE_WALK;

@@ -56,7 +56,8 @@ struct PassPlan {
 
 class DensePlan;  // dense_scan buffers and launches (rie_dense.hpp)
 
-// Largest size that the gate-level strategy runs on the tile passes.
+// Largest size that the gate-level strategy runs on the tile passes: 4 GiB of state
+// buffers, where gate by gate takes 2.  The gap doubles with each qubit.
 constexpr int kGateTileQubits = 26;
 
 struct Engine {
