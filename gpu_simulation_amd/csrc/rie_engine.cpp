@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -56,6 +57,59 @@ void device_free(void *p) {
         (void)hipFree(p);
     }
 }
+
+namespace {
+
+// Pinned blocks of the host calls, for every engine of the process: kCount of
+// kBytes, allocated at the first host call that asks for one and kept.  An engine
+// takes one at its own first host call and gives it back when it goes; larger
+// ones, and more engines than blocks, get memory of their own.  Pinning a block
+// costs 30 us and freeing it up to 250: one-shot calls of 4 qubits x 2 layers
+// take 71 us, 99 with a block of their own pinned and freed each time.
+template <size_t kBytes, int kCount>
+class HostBlocks {
+  public:
+    void *take(size_t bytes) {
+        if (bytes > kBytes) {
+            return nullptr;
+        }
+        const std::lock_guard<std::mutex> hold(lock_);
+        if (slab_ == nullptr) {
+            // seen by every device
+            check(hipHostMalloc((void **)&slab_, kBytes * kCount, hipHostMallocPortable),
+                  "alloc host staging");
+        }
+        for (int i = 0; i < kCount; ++i) {
+            if (!((used_ >> i) & 1u)) {
+                used_ |= uint64_t{1} << i;
+                return slab_ + kBytes * (size_t)i;
+            }
+        }
+        return nullptr;
+    }
+
+    // false: not one of these blocks
+    bool give(void *block) {
+        const std::lock_guard<std::mutex> hold(lock_);
+        const uintptr_t at = (uintptr_t)block - (uintptr_t)slab_;
+        if (slab_ == nullptr || at >= kBytes * kCount) {
+            return false;
+        }
+        used_ &= ~(uint64_t{1} << (at / kBytes));
+        return true;
+    }
+
+  private:
+    static_assert(kCount <= 64, "bits of used_");
+    std::mutex lock_;
+    char *slab_ = nullptr;  // until the process ends
+    uint64_t used_ = 0;
+};
+
+HostBlocks<4096, 64> g_small_blocks;   // up to 255 parameters
+HostBlocks<65536, 16> g_large_blocks;  // up to 4095: deep circuits on few qubits
+
+}  // namespace
 
 int parse_strategy(const std::string &name) {
     // reference: cpp/ising_cuda_backend.cu:249-264
@@ -234,10 +288,6 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
     d_params = (double *)device_alloc(sizeof(double) * num_params, "alloc params");
     d_grad = (double *)device_alloc(sizeof(double) * num_params, "alloc gradient");
     grad_dst = d_grad;
-    check(hipHostMalloc((void **)&h_params, sizeof(double) * (2 * num_params + 1), 0),
-          "alloc host staging");
-    h_grad = h_params + num_params;
-    h_energy = h_grad + num_params;
     d_energy = (double *)device_alloc(sizeof(double) * 4, "alloc energy");
     if (whole) {
         // the whole circuit lives in one workgroup's registers
@@ -324,7 +374,7 @@ Engine::~Engine() {
     }
     device_free(d_params);
     device_free(d_grad);
-    if (h_params != nullptr) {
+    if (h_params != nullptr && !g_small_blocks.give(h_params) && !g_large_blocks.give(h_params)) {
         (void)hipHostFree(h_params);
     }
     device_free(d_energy);
@@ -1472,6 +1522,24 @@ void Engine::eval_device(const double *params, double *energy, double *grad, hip
 // Host-pointer driver with stage profiling
 // ---------------------------------------------------------------------------
 
+// The host calls' pinned block, from the engine's first of them on.
+void Engine::host_staging() {
+    if (h_params != nullptr) {
+        return;
+    }
+    const size_t bytes = sizeof(double) * (2 * num_params + 1);
+    void *block = g_small_blocks.take(bytes);
+    if (block == nullptr) {
+        block = g_large_blocks.take(bytes);
+    }
+    if (block == nullptr) {
+        check(hipHostMalloc(&block, bytes, 0), "alloc host staging");
+    }
+    h_params = (double *)block;
+    h_grad = h_params + num_params;
+    h_energy = h_grad + num_params;
+}
+
 void Engine::energy_and_grad_host(const double *params, size_t count, bool want_grad,
                                   bool profile, double *energy_out, double *grad_out) {
     if (count != num_params) {
@@ -1480,14 +1548,17 @@ void Engine::energy_and_grad_host(const double *params, size_t count, bool want_
     if (params == nullptr || energy_out == nullptr || (want_grad && grad_out == nullptr)) {
         fail(RIE_INVALID_ARGUMENT, "null pointer argument.");
     }
+    host_staging();
     hipStream_t s = own_stream;
     order_begin(s);
     timings.clear();
     profiling = profile;
     auto t0 = std::chrono::steady_clock::now();
     // Parameters, energy and gradient pass through pinned memory that the
-    // kernels read and write themselves (each value once): three copies of
-    // pageable memory cost 20 to 65 us a call, most of a small circuit's time.
+    // kernels read and write themselves, each result once, each parameter once or,
+    // on the tile passes, layers 0 and 1 once per workgroup of the preparation
+    // (start_coefs): three copies of pageable memory cost 20 to 65 us a call,
+    // most of a small circuit's time.
     std::memcpy(h_params, params, sizeof(double) * num_params);
     const GradTarget target(*this, h_grad);
     if (profile) {

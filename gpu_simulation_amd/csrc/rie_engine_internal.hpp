@@ -143,7 +143,8 @@ struct Engine {
     double *d_params = nullptr;
     double *d_grad = nullptr;
     double *grad_dst = nullptr;  // where the current call's gradient goes
-    double *h_params = nullptr;  // pinned: parameters, gradient, energy of host calls
+    // pinned, from the first host call on: its parameters, gradient, energy
+    double *h_params = nullptr;
     double *h_grad = nullptr;
     double *h_energy = nullptr;
     double *d_energy = nullptr;
@@ -271,6 +272,7 @@ struct Engine {
     void forward_device(const double *params, double *energy, hipStream_t s, bool keep_lam);
     void backward_device(const double *params, const double *scale, double *grad, hipStream_t s);
     void eval_device(const double *params, double *energy, double *grad, hipStream_t s);
+    void host_staging();
     void energy_and_grad_host(const double *params, size_t count, bool want_grad, bool profile,
                               double *energy_out, double *grad_out);
     double inverse_walk_drift(const double *params, size_t count);
