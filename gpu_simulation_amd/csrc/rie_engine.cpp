@@ -363,9 +363,8 @@ Engine::Engine(size_t num_qubits, size_t num_layers, double field, const std::st
 }
 
 Engine::~Engine() {
-    if (own_stream != nullptr) {
-        (void)hipStreamSynchronize(own_stream);
-    }
+    // (the wait fails while another thread captures a stream in the global mode)
+    const bool idle = own_stream == nullptr || hipStreamSynchronize(own_stream) == hipSuccess;
     for (auto &c : ckpts) {
         device_free(c);
     }
@@ -374,7 +373,10 @@ Engine::~Engine() {
     }
     device_free(d_params);
     device_free(d_grad);
-    if (h_params != nullptr && !g_small_blocks.give(h_params) && !g_large_blocks.give(h_params)) {
+    // kernels of a failed host call may still write to the block: then nobody
+    // else gets it
+    if (idle && h_params != nullptr && !g_small_blocks.give(h_params) &&
+        !g_large_blocks.give(h_params)) {
         (void)hipHostFree(h_params);
     }
     device_free(d_energy);
