@@ -113,8 +113,10 @@ class RingIsingBatch:
                                            int(stream)))
 
     def autotune(self, repeats: int = 3, choose_split: bool = True) -> dict:
-        """Tune kernel shapes, and with choose_split which circuits with
-        num_qubits <= dense_max_qubits take dense_scan, on this batch."""
+        """Tune the workgroups of the 14-qubit adjoint launch, and with choose_split
+        which circuits with num_qubits <= dense_max_qubits take dense_scan, on this
+        batch.  ``threads``, ``chunk_by_n`` and ``dense_tile`` of the returned
+        configuration are the values of ``set_config``: nothing tunes them."""
         self._b.set_tune_split(int(bool(choose_split)))
         return self._b.autotune(int(repeats))
 

@@ -813,9 +813,10 @@ std::string Batch::config_json() const {
       << ", \"dense_tile\": " << dense_tile << ", \"measured\": " << (measured ? "true" : "false")
       << ", \"structured_circuits\": " << sids.size() << ", \"dense_circuits\": " << dids.size()
       << ", \"chunk_by_n\": {";
+    const int widest = threads >= 1024 ? 2 : threads >= 512 ? 3 : 4;  // of that workgroup size
     bool first = true;
     for (int q = 2; q <= kMaxN; ++q) {
-        o << (first ? "" : ", ") << "\"" << q << "\": " << chunk_by_n[q];
+        o << (first ? "" : ", ") << "\"" << q << "\": " << std::min(chunk_by_n[q], widest);
         first = false;
     }
     o << "}, \"autotune\": " << report << "}";
