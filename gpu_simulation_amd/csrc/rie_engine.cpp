@@ -793,7 +793,7 @@ void Engine::launch_bwd(int l, bool gather, bool write_cur, const double2 *cur_i
     // (lam of a high pass, the state of the gather pass) behind the current
     // one; the walk's one-sweep passes do not
     const bool prefetch = double_buffer && !write_cur;
-    launch_bwd_pass(pass_r[gather ? RIE_PASS_BWD_LOW : RIE_PASS_BWD_HIGH], gather, write_cur, true,
+    launch_bwd_pass(pass_r[gather ? RIE_PASS_BWD_LOW : RIE_PASS_BWD_HIGH], gather, write_cur,
                     cur_in, lam_in, cur_out, lam_out, lc, folded, pass_partials(), pp.grid, s, ham,
                     ham != kHamNone ? h : 0.0, gen_tab, gen_utab, prefetch, phase_free);
 }

@@ -1425,7 +1425,7 @@ __device__ __forceinline__ void bwd_load_tile(double2 (&c)[Tile<R>::REGS],
     }
 }
 
-template <int R, bool kGather, bool kWriteCur, bool kWriteLam, int kHam>
+template <int R, bool kGather, int kHam>
 __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pass_kernel(
     const double2 *cur_in, const double2 *lam_in, double2 *cur_out, double2 *lam_out,
     const WireCoef *__restrict__ lc, PassGeom G, double *__restrict__ partials, double field) {
@@ -1493,12 +1493,8 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
 #pragma unroll
             for (int k = 0; k < TL::REGS; ++k) {
                 const uint64_t idx = row + k * ta.strideA;
-                if constexpr (kWriteCur) {
-                    cur_out[idx] = c[k];
-                }
-                if constexpr (kWriteLam) {
-                    lam_out[idx] = l[k];
-                }
+                cur_out[idx] = c[k];
+                lam_out[idx] = l[k];
             }
         } else {
             constexpr uint32_t w0 = window_mask<R, 0>();
@@ -1544,12 +1540,8 @@ __global__ __launch_bounds__(Tile<R>::THREADS, tile_min_blocks<R>()) void bwd_pa
 #pragma unroll
             for (int k = 0; k < TL::REGS; ++k) {
                 const uint64_t idx = row + k * ta.strideC;
-                if constexpr (kWriteCur) {
-                    cur_out[idx] = c[k];
-                }
-                if constexpr (kWriteLam) {
-                    lam_out[idx] = l[k];
-                }
+                cur_out[idx] = c[k];
+                lam_out[idx] = l[k];
             }
         }
     }
@@ -2404,7 +2396,7 @@ void launch_bwd_low_gen(int R, double2 *lam_out, const WireCoef *layer_coef, con
 }
 
 template <int R>
-static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const double2 *cur_in,
+static void launch_bwd_pass_r(bool gather, bool write_cur, const double2 *cur_in,
                               const double2 *lam_in, double2 *cur_out, double2 *lam_out,
                               const WireCoef *lc, const PassGeom &g, double *partials, int grid,
                               hipStream_t s, int ham, double field, const CMat2 *gen_tab,
@@ -2420,13 +2412,12 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
         // lambda layouts: lambda-only high passes whose register bits the
         // layouts keep contiguous
         const int first = g.h0 + (Tile<R>::T - R - g.a);
-        if (gather || write_cur || !write_lam || g.a != 3 || !lay_fits(g.lay_in, g.n, first, R) ||
+        if (gather || write_cur || g.a != 3 || !lay_fits(g.lay_in, g.n, first, R) ||
             !lay_fits(g.lay_out, g.n, first, R)) {
             throw std::invalid_argument("lambda layouts: pass or geometry outside their scope");
         }
     }
-    if (phase_free &&
-        (R != 4 || gather || !gen || ham != kHamNone || write_cur || !write_lam)) {
+    if (phase_free && (R != 4 || gather || !gen || ham != kHamNone || write_cur)) {
         // the tables leave the pass's own phases out only for this sweep
         throw std::invalid_argument(
             "phase-free sweep: generated lambda-only high pass of shape 4 without pair terms");
@@ -2442,7 +2433,7 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
         // the wire below the group at tile bit 3, wire n - 1 at tile bit 11
         throw std::invalid_argument("fold terms: geometry without the wires they reach");
     }
-    if (!write_cur && write_lam) {  // the state is not rewritten: lambda-only sweep
+    if (!write_cur) {  // the state is not rewritten: lambda-only sweep
         if (!gather && R == 4 && (g.a != 3 || g.rot_lo < 3)) {
             // the sweep takes tile bit 3 across lanes and no other bit of window 1
             throw std::invalid_argument("high pass geometry: tile bits 0..2 must ride along");
@@ -2493,40 +2484,34 @@ static void launch_bwd_pass_r(bool gather, bool write_cur, bool write_lam, const
         // the one-sweep high pass skips tile bits 0..2 at compile time
         throw std::invalid_argument("high pass geometry: tile bits 0..2 must ride along");
     }
-#define RIE_BWD(GA, WC, WL, HM)                                                              \
-    if (gather == GA && write_cur == WC && write_lam == WL && ham == HM) {                   \
-        bwd_pass_kernel<R, GA, WC, WL, HM><<<grid, TH, 0, s>>>(                              \
-            cur_in, lam_in, cur_out, lam_out, lc, g, partials, field);                       \
+#define RIE_BWD(GA, HM)                                                                      \
+    if (write_cur && gather == GA && ham == HM) {                                            \
+        bwd_pass_kernel<R, GA, HM><<<grid, TH, 0, s>>>(cur_in, lam_in, cur_out, lam_out, lc, \
+                                                       g, partials, field);                  \
         return;                                                                              \
     }
-    RIE_BWD(true, true, true, kHamNone)
-    RIE_BWD(false, true, true, kHamNone)
-    RIE_BWD(true, false, true, kHamNone)
-    RIE_BWD(false, false, true, kHamNone)
-    RIE_BWD(true, true, true, kHamPairs)
-    RIE_BWD(false, true, true, kHamPairs)
-    RIE_BWD(true, false, true, kHamPairs)
-    RIE_BWD(false, false, true, kHamPairs)
-    RIE_BWD(false, true, true, kHamFold)
-    RIE_BWD(false, false, true, kHamFold)
-    RIE_BWD(false, true, true, kHamFoldTop)
-    RIE_BWD(false, false, true, kHamFoldTop)
-    RIE_BWD(true, true, true, kHamStart)
-    RIE_BWD(true, false, true, kHamStart)
+    RIE_BWD(true, kHamNone)
+    RIE_BWD(false, kHamNone)
+    RIE_BWD(true, kHamPairs)
+    RIE_BWD(false, kHamPairs)
+    RIE_BWD(false, kHamFold)
+    RIE_BWD(false, kHamFoldTop)
+    RIE_BWD(true, kHamStart)
 #undef RIE_BWD
+    throw std::invalid_argument("adjoint pass: no kernel for this combination");
 }
 
-void launch_bwd_pass(int R, bool gather, bool write_cur, bool write_lam, const double2 *cur_in,
+void launch_bwd_pass(int R, bool gather, bool write_cur, const double2 *cur_in,
                      const double2 *lam_in, double2 *cur_out, double2 *lam_out,
                      const WireCoef *layer_coef, const PassGeom &g, double *partials, int grid,
                      hipStream_t s, int ham, double field, const CMat2 *gen_tab,
                      const CMat2 *gen_utab, bool prefetch, bool phase_free) {
     if (R == 4) {
-        launch_bwd_pass_r<4>(gather, write_cur, write_lam, cur_in, lam_in, cur_out, lam_out,
+        launch_bwd_pass_r<4>(gather, write_cur, cur_in, lam_in, cur_out, lam_out,
                              layer_coef, g, partials, grid, s, ham, field, gen_tab,
                              gen_utab, prefetch, phase_free);
     } else {
-        launch_bwd_pass_r<3>(gather, write_cur, write_lam, cur_in, lam_in, cur_out, lam_out,
+        launch_bwd_pass_r<3>(gather, write_cur, cur_in, lam_in, cur_out, lam_out,
                              layer_coef, g, partials, grid, s, ham, field, gen_tab,
                              gen_utab, prefetch, phase_free);
     }

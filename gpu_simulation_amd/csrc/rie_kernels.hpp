@@ -363,19 +363,21 @@ void launch_gen_layer1(int R, double2 *out, const CMat2 *tab, const CMat2 *utab,
 
 // Adjoint tile pass: un-rotates the pass's wires on (cur, lam) and writes
 // per-workgroup gradient partials [grid][2T].  gather = apply the inverse
-// ring-CNOT on load (low pass, out of place); write_cur / write_lam = store
-// the un-rotated state / adjoint state.
-// ham_pairs: before un-rotating, add the transverse-field terms of the
-// tile-bit pairs [g.pair_lo, g.pair_hi) to lam (-field * X_j X_{j+1} cur).  In
-// the pre-CNOT frame of the last layer these pairs are the X terms X_j of H;
-// their energy is not summed here (the layer-0 contraction yields the whole
-// energy once lambda = H psi is complete).
+// ring-CNOT on load (low pass, out of place); write_cur = store the
+// un-rotated state too (the walk), else only the adjoint state (the lambda-only
+// sweep).
+// ham (kHamNone ..): the terms of H that the pass adds to lam before
+// un-rotating.  kHamPairs: the transverse-field terms of the tile-bit pairs
+// [g.pair_lo, g.pair_hi) (-field * X_j X_{j+1} cur).  In the pre-CNOT frame of
+// the last layer these pairs are the X terms X_j of H; their energy is not summed
+// here (the layer-0 contraction yields the whole energy once lambda = H psi is
+// complete).
 // gen_tab, gen_utab (layer 1, high pass on the lambda-only sweep): the state
 // is not read from cur_in but generated from a chain table set whose run is
 // mapping 0's register wires, and that set's per-tile segments.
 // prefetch (high passes on the lambda-only sweep): each workgroup loads its
 // next tile's lam into the registers the current tile's state frees.
-void launch_bwd_pass(int R, bool gather, bool write_cur, bool write_lam, const double2 *cur_in,
+void launch_bwd_pass(int R, bool gather, bool write_cur, const double2 *cur_in,
                      const double2 *lam_in, double2 *cur_out, double2 *lam_out,
                      const WireCoef *layer_coef, const PassGeom &g, double *partials, int grid,
                      hipStream_t s, int ham = kHamNone, double field = 0.0,
