@@ -1694,14 +1694,25 @@ void Engine::set_checkpoint_interval(size_t every) {
         device_free(c);
     }
     ckpts.clear();
-    ckpt_every = every;
+    // the interval counts only where its buffers are: a forward sweep on the tile
+    // passes writes to them, also the gate-level strategy's, which has none
+    ckpt_every = 0;
     if (every == 0 || small || strategy != RIE_STRATEGY_STRUCTURED_ADJOINT) {
         return;
     }
     const size_t count = (size_t)(L - 1) / every;
-    for (size_t i = 0; i < count; ++i) {
-        ckpts.push_back((double2 *)device_alloc(sizeof(double2) * N, "alloc checkpoint"));
+    try {
+        for (size_t i = 0; i < count; ++i) {
+            ckpts.push_back((double2 *)device_alloc(sizeof(double2) * N, "alloc checkpoint"));
+        }
+    } catch (...) {
+        for (auto &c : ckpts) {
+            device_free(c);
+        }
+        ckpts.clear();
+        throw;
     }
+    ckpt_every = count > 0 ? every : 0;
 }
 
 // Tile register shapes and backward schedule for the caller's parameters.
