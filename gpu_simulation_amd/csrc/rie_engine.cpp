@@ -1697,6 +1697,7 @@ void Engine::set_checkpoint_interval(size_t every) {
     // the interval counts only where its buffers are: a forward sweep on the tile
     // passes writes to them, also the gate-level strategy's, which has none
     ckpt_every = 0;
+    resident = false;  // a forward before this has not written the new ones
     if (every == 0 || small || strategy != RIE_STRATEGY_STRUCTURED_ADJOINT) {
         return;
     }

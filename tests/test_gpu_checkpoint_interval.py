@@ -61,3 +61,24 @@ def test_gate_level_module_with_checkpoints(oracle):
     energy.backward()
     _check({"energy": energy.item(), "gradient": params.grad.cpu().numpy().reshape(-1)},
            (e_ref, g_ref))
+
+
+def test_interval_set_between_forward_and_backward(oracle, backend_module):
+    import torch
+
+    n, layers = 16, 5
+    p = np.random.default_rng(93).uniform(0, 2 * np.pi, (layers, n, 2))
+    ref = oracle.energy_and_grad(n, layers, 1.0, p)
+    eng = backend_module.RingIsingCudaBackend(n, layers, 1.0, "structured_adjoint", 8, False)
+    eng.set_schedule("inverse_walk")
+    d = torch.from_numpy(p.reshape(-1)).cuda()
+    e = torch.zeros(1, dtype=torch.float64, device="cuda")
+    g = torch.zeros_like(d)
+    stream = torch.cuda.current_stream().cuda_stream
+    for every in (2, 0, 1):
+        print(f"case interval {every} between forward and backward", flush=True)
+        eng.forward_device(d.data_ptr(), e.data_ptr(), stream)
+        eng.set_checkpoint_interval(every)
+        eng.backward_device(d.data_ptr(), 0, g.data_ptr(), stream)
+        torch.cuda.synchronize()
+        _check({"energy": e.item(), "gradient": g.cpu().numpy()}, ref)
