@@ -1535,7 +1535,7 @@ void Engine::host_staging() {
         block = g_large_blocks.take(bytes);
     }
     if (block == nullptr) {
-        check(hipHostMalloc(&block, bytes, 0), "alloc host staging");
+        check(hipHostMalloc(&block, bytes, hipHostMallocPortable), "alloc host staging");
     }
     h_params = (double *)block;
     h_grad = h_params + num_params;
