@@ -1252,7 +1252,8 @@ void Engine::structured_backward(hipStream_t s, const double *scale, bool full_w
         kt_begin(s);
         launch_bwd(l, true, low_cur, cur_in, pool[lam], pool[ncur], pool[nlam], 0, s);
         check_launch("bwd_pass gather");
-        kt_end(s, "bwd_pass_low_cnot", S * (3.0 + (low_cur ? 1.0 : 0.0)));
+        kt_end(s, "bwd_pass_low_cnot",
+               S * (2.0 + (starts_lam(l) ? 0.0 : 1.0) + (low_cur ? 1.0 : 0.0)));
         queue_grad(passes[0], l, scale, s);
         cur = ncur;
         lam = nlam;
@@ -1333,7 +1334,7 @@ void Engine::structured_backward_stored(hipStream_t s, const double *scale) {
         kt_begin(s);
         launch_bwd(l, true, false, fbuf(l, K), lbuf(a), nullptr, lbuf(b), 0, s);
         check_launch("bwd_pass gather");
-        kt_end(s, "bwd_pass_low_cnot", 3 * S);
+        kt_end(s, "bwd_pass_low_cnot", (starts_lam(l) ? 2 : 3) * S);
         queue_grad(passes[0], l, scale, s);
         for (int j = K - 1; j >= 0; --j) {
             const PassPlan &pp = passes[1 + j];

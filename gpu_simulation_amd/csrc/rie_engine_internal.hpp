@@ -106,6 +106,8 @@ struct Engine {
     // the state alone, so no Hamiltonian pass runs and lambda is not read there.
     bool fold_ready = false;    // the plan supports it
     bool fold_start = false;    // the running backward does so
+    // the low adjoint pass of layer l starts lambda instead of reading it
+    bool starts_lam(int l) const { return fold_start && l == fuse_layer; }
     bool fold_upwards = false;  // its high passes run from the lowest group up
     bool lam_deferred = false;  // the last forward left lambda to the backward
     // Layer-1 generation (L >= 2, n <= kChainMaxQubits): every state inside
