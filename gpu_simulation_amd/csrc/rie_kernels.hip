@@ -1200,7 +1200,10 @@ __device__ __forceinline__ void gather_pair_terms(const double2 (&c)[Tile<R>::RE
 // 12.8 -> 11.9 ms; low pass 1.53 -> 1.41 ms, the Hamiltonian's 0.86 ms gone, the
 // top group's pass 1.61 -> 1.98 ms, the other group's 1.61 -> 1.43 with its
 // loads' steps formed per tile).  One kernel per combination of terms: with
-// branches around them the register arrays were copied and spilled (2.8 ms).
+// branches around them the register arrays were copied and spilled (2.8 ms).  The
+// lambda-only kernels still spill 35 values (144 bytes a lane), with the next tile
+// prefetched 225 (392 bytes): 27 qubits x 3 layers take 14.3 ms with
+// double_buffer, 12.0 without (14.6 and 13.0 with a Hamiltonian pass).
 // Wire n - 1's term (kHamFoldTop): mapping 0.  kStart: l becomes the term before
 // its factor -field, which the caller adds lambda to, else the term is added.
 template <int R, bool kStart>

@@ -211,7 +211,12 @@ constexpr size_t kReg14Scratch = (size_t)4 << 14;
 void launch_reg14(const Reg14Job *d_jobs, const Reg14Job &single, const int *d_order,
                   const int *d_wg_begin, int count, int grid, double2 *scratch, hipStream_t s);
 
-constexpr int kEngineWholeQubits = 12;  // an engine's whole-circuit path (tile passes above)
+// An engine's whole-circuit path; tile passes above.  The line is where final_state,
+// schedules and checkpoints begin: they need a state in memory, which the
+// whole-circuit kernels do not leave.  It is not where the times cross: at 13 qubits
+// the tile passes take 69, 179 and 692 us for 2, 4 and 16 layers, one circuit in
+// registers 59, 104 and 372.
+constexpr int kEngineWholeQubits = 12;
 constexpr int kBatchMaxQubits = 14;     // whole-circuit kernels
 
 // Coefficient table from device parameters: coef[i] from params[2i], params[2i+1].

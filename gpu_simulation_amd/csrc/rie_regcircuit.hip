@@ -10,7 +10,9 @@
 // layer of one circuit, forward and back, takes 1.0 us at 4 qubits, 2.5 at 8,
 // 11 at 12 and 22 at 13 (128 layers).  Before, with psi and lambda in LDS (a
 // sweep per chunk of wires, one barrier each, pair indexes computed per group)
-// or at 13 qubits in L2: 8, 15, 23 and 102 us.
+// or at 13 qubits in L2: 8, 15, 23 and 102 us.  13 qubits pay for spills too:
+// with 128 of a lane's 256 VGPRs taken by psi and lambda, 105 values go through
+// scratch (336 bytes a lane).
 #include <hip/hip_runtime.h>
 
 #include "rie_regstate.hpp"
@@ -277,8 +279,9 @@ __global__ __launch_bounds__(RegState<n>::kThreads) __attribute__((
 // (L2 / MALL) once a layer: the read applies the inverse ring CNOT and, as it
 // meets both halves, un-rotates the top wire of the layer before.
 //
-// Bound by latency and L2: a layer of one circuit takes 69 us forward and back
-// against 212 for sweeps of chunks of three wires over the scratch.
+// Bound by latency, L2 and spills: the adjoint kernel keeps 318 values of its 256
+// VGPRs in scratch (1076 bytes a lane).  A layer of one circuit takes 69 us forward
+// and back against 212 for sweeps of chunks of three wires over the scratch.
 // ---------------------------------------------------------------------------
 
 constexpr uint32_t kHalf14 = 1u << 13;

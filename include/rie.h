@@ -313,7 +313,8 @@ rie_status rie_engine_autotune(rie_engine *engine, const double *params, size_t 
 /* Store the statevector at every k-th layer boundary during the forward pass
  * and restore it there during the backward sweep instead of continuing the
  * inverse walk (k = 0 disables).  Costs one extra state buffer per stored
- * boundary. */
+ * boundary.  structured_adjoint above 12 qubits; other engines accept it and
+ * keep no checkpoints. */
 rie_status rie_engine_set_checkpoint_interval(rie_engine *engine, size_t every_k_layers);
 
 /* Run energy_and_grad with a full inverse walk through layer 0 and report
@@ -345,9 +346,11 @@ rie_status rie_engine_copy_state(rie_engine *engine, double *host_out, size_t nu
  * dense_max_qubits (0..8) use dense_scan, the others structured_adjoint.
  * All circuits are evaluated together: the structured ones in one launch per
  * qubit count (14 qubits: one persistent launch), the dense ones level by
- * level in grouped FP64-MFMA GEMM launches, concurrently.  Parameters, energies and gradients live in device arrays
- * owned by the batch; circuit i's 2*n_i*L_i parameters (and gradients) start
- * at offsets[i] and follow the single-circuit layout. */
+ * level in grouped FP64-MFMA GEMM launches, concurrently; large batches in
+ * slices that share about a gigabyte of workspace.  Parameters, energies and
+ * gradients live in device arrays owned by the batch; circuit i's 2*n_i*L_i
+ * parameters (and gradients) start at offsets[i] and follow the single-circuit
+ * layout. */
 typedef struct rie_batch rie_batch;
 
 rie_status rie_batch_create(size_t count, const int *num_qubits, const int *num_layers,
@@ -396,9 +399,9 @@ rie_status rie_batch_optimize(rie_batch *batch, int optimizer, double learning_r
 /* Autotuner: for each split of the circuits between dense_scan (num_qubits <=
  * s) and the whole-circuit kernels, s from the dense_max_qubits given at creation
  * down to 0 (see rie_batch_set_tune_split), and each share of the CUs for the
- * 14-qubit adjoint launch, times the whole evaluation and keeps the fastest.  The reference fixes the
- * strategy per call and its kernel shapes by qubit-count thresholds
- * (cpp/ising_cuda_rotation_kernels.cu:562-575). */
+ * 14-qubit adjoint launch, times the whole evaluation and keeps the fastest.
+ * The reference fixes the strategy per call and its kernel shapes by
+ * qubit-count thresholds (cpp/ising_cuda_rotation_kernels.cu:562-575). */
 rie_status rie_batch_autotune(rie_batch *batch, size_t repeats);
 /* Whether rie_batch_autotune may move circuits between dense_scan and the
  * whole-circuit kernel (default 1; 0 keeps num_qubits <= dense_max_qubits on
@@ -406,10 +409,10 @@ rie_status rie_batch_autotune(rie_batch *batch, size_t repeats);
 rie_status rie_batch_set_tune_split(rie_batch *batch, int enabled);
 /* Manual configuration: threads 256/512/1024; chunk_by_n (15 values,
  * indexed by num_qubits, each 1..4) or NULL to keep; dense_tile 32/64;
- * structured_grid = workgroups of the persistent launch (0: one per CU).
- * structured_grid bounds the 14-qubit adjoint launch.  The kernels have one
- * shape per qubit count: threads, chunk_by_n and dense_tile are checked and
- * reported, nothing more. */
+ * structured_grid = workgroups of the persistent launch, the 14-qubit adjoint
+ * one (0: one per CU).  The kernels have one shape per qubit count: threads,
+ * chunk_by_n and dense_tile are checked and reported (the widths cut to what
+ * the workgroup size allows), nothing more. */
 rie_status rie_batch_set_config(rie_batch *batch, int threads, const int *chunk_by_n,
                                 size_t chunk_len, int dense_tile, int structured_grid);
 /* Current configuration and the last autotuning measurements as JSON. */
